@@ -77,9 +77,10 @@ __device__ __forceinline__ void wave_reduce(Acc &a, float &m) {
   }
 }
 
-// Reduces (a, m) over the block; the result is valid in thread 0.
+// Reduces (a, m) over a block of kW waves; the result is valid in thread 0.
+template <int kW = kWaves>
 __device__ __forceinline__ void block_reduce(Acc &a, float &m) {
-  __shared__ float ls[kWaves], lc[kWaves], lm[kWaves];
+  __shared__ float ls[kW], lc[kW], lm[kW];
   wave_reduce(a, m);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0) {
@@ -94,7 +95,7 @@ __device__ __forceinline__ void block_reduce(Acc &a, float &m) {
     t.c = lc[0];
     float mm = lm[0];
 #pragma unroll
-    for (int w = 1; w < kWaves; ++w) {
+    for (int w = 1; w < kW; ++w) {
       t.merge(ls[w], lc[w]);
       mm = nanmax(mm, lm[w]);
     }
@@ -202,52 +203,124 @@ __global__ __launch_bounds__(kBlock) void reduce_all_kernel(const float *__restr
 }
 
 // ----------------------------------------------------------------------------- rows
-// One workgroup per row: row sum (compensated FP32, rounded once), row max, and the FP64
-// partial of the row for the total.
-template <bool kVec>
-__global__ __launch_bounds__(kBlock) void reduce_rows_kernel(const float *__restrict__ in, int64_t rows,
-                                                             int64_t cols, float *row_sum, float *row_max,
-                                                             double *partial64) {
-  const int64_t row = blockIdx.x;
-  const float *p = in + row * cols;
-  Acc a;
-  float m = __builtin_nanf("");
-  if (kVec) {
-    const f4 *p4 = reinterpret_cast<const f4 *>(p);
-    const int64_t nv = cols / 4;
-    int64_t i = threadIdx.x;
-    for (; i + 3 * kBlock < nv; i += 4 * kBlock) {
-      f4 v[4];
+// A row starts at any 4-byte boundary (cols need not be a multiple of 4): 16-byte loads take
+// four-byte alignment on this hardware, so rows are read in vectors of four from their first
+// element, with cols % 4 single elements at the end.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// Adds four elements: pairwise inside the vector, then one compensated add.
+__device__ __forceinline__ void add_vector(f4u v, Acc &a, float &m) {
+  float s01, e01, s23, e23, s, e;
+  two_sum(v.x, v.y, s01, e01);
+  two_sum(v.z, v.w, s23, e23);
+  two_sum(s01, s23, s, e);
+  a.merge(s, e + e01 + e23);
+  m = nanmax(m, nanmax(nanmax(v.x, v.y), nanmax(v.z, v.w)));
+}
+
+// One row's share of a lane: vectors lane, lane + kStep, ... of p, four loads in flight. The
+// cols % 4 elements after the last whole vector are the end of one more vector that overlaps it,
+// so that they ride with the other loads.
+template <int kStep>
+__device__ __forceinline__ void read_row(const float *__restrict__ p, int64_t cols, int lane, Acc &a, float &m) {
+  const f4u *p4 = reinterpret_cast<const f4u *>(p);
+  const int64_t nv = cols / 4;
+  int64_t i = lane;
+  for (; i + 3 * kStep < nv; i += 4 * kStep) {
+    f4u v[4];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) v[k] = __builtin_nontemporal_load(p4 + i + k * kBlock);
+    for (int k = 0; k < 4; ++k) v[k] = __builtin_nontemporal_load(p4 + i + k * kStep);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        // pairwise inside the vector, then one compensated add
-        float s01, e01, s23, e23, s, e;
-        two_sum(v[k].x, v[k].y, s01, e01);
-        two_sum(v[k].z, v[k].w, s23, e23);
-        two_sum(s01, s23, s, e);
-        a.merge(s, e + e01 + e23);
-        m = nanmax(m, nanmax(nanmax(v[k].x, v[k].y), nanmax(v[k].z, v[k].w)));
-      }
+    for (int k = 0; k < 4; ++k) add_vector(v[k], a, m);
+  }
+  const int tail = static_cast<int>(cols % 4);
+  if (nv == 0) {
+    for (int j = lane; j < tail; j += kStep) {
+      a.add(p[j]);
+      m = nanmax(m, p[j]);
     }
-    for (; i < nv; i += kBlock) {
-      f4 v = __builtin_nontemporal_load(p4 + i);
-      a.add(v.x); a.add(v.y); a.add(v.z); a.add(v.w);
-      m = nanmax(m, nanmax(nanmax(v.x, v.y), nanmax(v.z, v.w)));
-    }
-  } else {
-    for (int64_t i = threadIdx.x; i < cols; i += kBlock) {
-      float x = p[i];
-      a.add(x);
-      m = nanmax(m, x);
+    return;
+  }
+  const int64_t all = nv + (tail ? 1 : 0);
+  if (i >= all) return;
+  f4u v[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int64_t c = i + k * kStep;
+    if (c < all) v[k] = __builtin_nontemporal_load(reinterpret_cast<const f4u *>(p + (c < nv ? 4 * c : cols - 4)));
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int64_t c = i + k * kStep;
+    if (c < nv) {
+      a.add(v[k].x), a.add(v[k].y), a.add(v[k].z), a.add(v[k].w);
+      m = nanmax(m, nanmax(nanmax(v[k].x, v[k].y), nanmax(v[k].z, v[k].w)));
+    } else if (c < all) {
+      // the last `tail` of the vector's elements; the others were added with the one before
+      a.add(v[k].w);
+      m = nanmax(m, v[k].w);
+      if (tail > 1) a.add(v[k].z), m = nanmax(m, v[k].z);
+      if (tail > 2) a.add(v[k].y), m = nanmax(m, v[k].y);
     }
   }
-  block_reduce(a, m);
+}
+
+// One workgroup per row: row sum (compensated FP32, rounded once), row max, and the FP64
+// partial of the row for the total.
+template <int kThreads>
+__global__ __launch_bounds__(kThreads) void reduce_rows_kernel(const float *__restrict__ in, int64_t cols,
+                                                               float *row_sum, float *row_max, double *partial64) {
+  const int64_t row = blockIdx.x;
+  Acc a;
+  float m = __builtin_nanf("");
+  read_row<kThreads>(in + row * cols, cols, threadIdx.x, a, m);
+  block_reduce<kThreads / 64>(a, m);
   if (threadIdx.x == 0) {
     if (row_sum) row_sum[row] = a.result();
     if (row_max) row_max[row] = m;
     if (partial64) partial64[row] = a.result64();
+  }
+}
+
+// Short rows: kG lanes per row, kBlock / kG consecutive rows per workgroup at a time, so that a
+// wave reads whole rows one after another; `tiles` such groups of rows per workgroup. The FP64
+// values of its rows are added in a fixed order into one partial per workgroup. Bound by HBM once
+// the grid fills the chip: 120011 x 77 (37 MB) takes 12.5 us with its combine, 3.0 TB/s, against
+// 109 us when every row had a workgroup; 16000 x 1025 15.7 us (4.2 TB/s) against 25.2.
+template <int kG>
+__global__ __launch_bounds__(kBlock) void reduce_short_rows_kernel(const float *__restrict__ in, int64_t rows,
+                                                                   int64_t cols, int tiles, float *row_sum,
+                                                                   float *row_max, double *partial64) {
+  __shared__ double lw[kWaves];
+  const int lane = threadIdx.x % kG, group = threadIdx.x / kG;
+  double total = 0.0;  // of this lane's rows
+  for (int t = 0; t < tiles; ++t) {
+    const int64_t row = (int64_t(blockIdx.x) * tiles + t) * (kBlock / kG) + group;
+    Acc a;
+    float m = __builtin_nanf("");
+    if (row < rows) read_row<kG>(in + row * cols, cols, lane, a, m);
+#pragma unroll
+    for (int off = kG / 2; off >= 1; off >>= 1) {
+      const float s2 = __shfl_xor(a.s, off, 64), c2 = __shfl_xor(a.c, off, 64), m2 = __shfl_xor(m, off, 64);
+      a.merge(s2, c2);
+      m = nanmax(m, m2);
+    }
+    if (lane == 0 && row < rows) {
+      if (row_sum) row_sum[row] = a.result();
+      if (row_max) row_max[row] = m;
+      total += a.result64();
+    }
+  }
+  if (!partial64) return;
+#pragma unroll
+  for (int off = 32; off >= kG; off >>= 1) total += __shfl_xor(total, off, 64);  // lane 0 of each row group holds a value
+  if ((threadIdx.x & 63) == 0) lw[threadIdx.x >> 6] = total;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double s = lw[0];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) s += lw[w];
+    partial64[blockIdx.x] = s;
   }
 }
 
@@ -390,6 +463,72 @@ double *noalloc_scratch(cs_device *device) {
 }
 }  // namespace
 
+namespace {
+// How a [rows, cols] matrix is cut for the row kernels.
+struct RowPlan {
+  int lanes = 0;        // lanes per row of the short-row kernel; 0: a workgroup per row
+  bool wide = false;    // with a workgroup per row: 1024 threads instead of 256
+  int tiles = 1;        // groups of kBlock / lanes rows per workgroup
+  int64_t grid = 0;     // workgroups, each with one FP64 partial
+};
+
+// Where the lines lie (whole calls with the total, in us: a workgroup per row against the rule):
+//   * up to 2048 columns a row is 8 vectors per lane of one wave, so a workgroup per row spends
+//     its time starting and combining: 120011 x 77 109.0 / 12.5, 524288 x 8 463 / 9.4,
+//     60000 x 128 57.8 / 9.4, 16384 x 1024 19.3 / 14.8, 16000 x 1025 21.6 / 15.7; equal at
+//     2047 columns (15.4 / 15.6); at 4096 the workgroup per row is ahead (43.3 / 45.8).
+//   * as many lanes as take a row in at most four vectors each, all in flight together: half as
+//     many (eight vectors) 14.1 at 120011 x 77 against 12.4, twice as many 15.5.
+//   * at most 8192 partials, which the combine adds in one round of loads.
+//   * at most one row per CU and long rows: 1024 threads per row, since nothing else fills the
+//     chip (64 x 65536 14.9 / 9.0, 256 x 16384 7.4 / 6.5); from two rows per CU on 256 threads
+//     are ahead (512 x 16384 8.8 against 9.4, 2000 x 8192 13.4 against 16.9).
+constexpr int64_t kShortCols = 2048, kMaxPartials = 8192, kWideCols = 8192;
+
+RowPlan plan_rows(cs_stream *stream, int64_t rows, int64_t cols) {
+  RowPlan p;
+  if (cols > kShortCols) {
+    p.grid = rows;
+    p.wide = rows <= stream->device->props.multiProcessorCount && cols >= kWideCols;
+    return p;
+  }
+  p.lanes = 2;
+  while (p.lanes < 64 && p.lanes * 16 < cols) p.lanes *= 2;
+  const int64_t per = kBlock / p.lanes, groups = (rows + per - 1) / per;
+  p.tiles = static_cast<int>((groups + kMaxPartials - 1) / kMaxPartials);
+  p.grid = (groups + p.tiles - 1) / p.tiles;
+  return p;
+}
+
+template <int kG>
+void launch_short_rows(cs_stream *stream, const RowPlan &p, const float *in, int64_t rows, int64_t cols,
+                       float *row_sum, float *row_max, double *partial64) {
+  hipLaunchKernelGGL(reduce_short_rows_kernel<kG>, dim3(static_cast<unsigned>(p.grid)), dim3(kBlock), 0,
+                     stream->stream, in, rows, cols, p.tiles, row_sum, row_max, partial64);
+}
+
+// The row pass of a plan and, when partial64 is not null, the combine of its plan.grid partials.
+void launch_rows(cs_stream *stream, const RowPlan &p, const float *in, int64_t rows, int64_t cols, float *row_sum,
+                 float *row_max, double *partial64, float *total, double *total64) {
+  switch (p.lanes) {
+    case 2: launch_short_rows<2>(stream, p, in, rows, cols, row_sum, row_max, partial64); break;
+    case 4: launch_short_rows<4>(stream, p, in, rows, cols, row_sum, row_max, partial64); break;
+    case 8: launch_short_rows<8>(stream, p, in, rows, cols, row_sum, row_max, partial64); break;
+    case 16: launch_short_rows<16>(stream, p, in, rows, cols, row_sum, row_max, partial64); break;
+    case 32: launch_short_rows<32>(stream, p, in, rows, cols, row_sum, row_max, partial64); break;
+    case 64: launch_short_rows<64>(stream, p, in, rows, cols, row_sum, row_max, partial64); break;
+    default:
+      if (p.wide)
+        hipLaunchKernelGGL(reduce_rows_kernel<1024>, dim3(static_cast<unsigned>(p.grid)), dim3(1024), 0,
+                           stream->stream, in, cols, row_sum, row_max, partial64);
+      else
+        hipLaunchKernelGGL(reduce_rows_kernel<kBlock>, dim3(static_cast<unsigned>(p.grid)), dim3(kBlock), 0,
+                           stream->stream, in, cols, row_sum, row_max, partial64);
+  }
+  if (partial64) launch_finish_sum(stream, partial64, p.grid, total, total64);
+}
+}  // namespace
+
 static int reduce_grid(cs_stream *stream, int64_t n) {
   int cus = stream->device->props.multiProcessorCount;
   int64_t want = (n / 4 + kBlock * 4 - 1) / (kBlock * 4);  // >= 4 vectors per thread
@@ -452,14 +591,9 @@ cs_status cs_reduce_rows(cs_stream *stream, const float *in, int64_t rows, int64
       CS_HIP(hipGetLastError());
       return;
     }
-    ReduceScratch s = scratch_for(stream, want_total ? static_cast<size_t>(rows) : 0);
-    bool vec = cols % 4 == 0 && (reinterpret_cast<uintptr_t>(in) & 15) == 0;
-    auto k = vec ? reduce_rows_kernel<true> : reduce_rows_kernel<false>;
-    hipLaunchKernelGGL(k, dim3(static_cast<unsigned>(rows)), dim3(kBlock), 0, stream->stream, in, rows, cols,
-                       row_sum, row_max, want_total ? s.partial64 : nullptr);
-    if (want_total)
-      hipLaunchKernelGGL(finish_sum_kernel, dim3(1), dim3(kFinish), 0, stream->stream, s.partial64, rows, total,
-                         total64);
+    const RowPlan plan = plan_rows(stream, rows, cols);
+    ReduceScratch s = scratch_for(stream, want_total ? static_cast<size_t>(plan.grid) : 0);
+    launch_rows(stream, plan, in, rows, cols, row_sum, row_max, want_total ? s.partial64 : nullptr, total, total64);
     CS_HIP(hipGetLastError());
   });
 }
@@ -486,13 +620,7 @@ cs_status cs_reduce_rows_noalloc(cs_stream *stream, const float *in, int64_t row
     }
     // every partial the combine reads is written by this call's row kernel first
     double *partial64 = want_total ? noalloc_scratch(stream->device) : nullptr;
-    const bool vec = cols % 4 == 0 && (reinterpret_cast<uintptr_t>(in) & 15) == 0;
-    auto k = vec ? reduce_rows_kernel<true> : reduce_rows_kernel<false>;
-    hipLaunchKernelGGL(k, dim3(static_cast<unsigned>(rows)), dim3(kBlock), 0, stream->stream, in, rows, cols,
-                       row_sum, row_max, partial64);
-    if (want_total)
-      hipLaunchKernelGGL(finish_sum_kernel, dim3(1), dim3(kFinish), 0, stream->stream, partial64, rows, total,
-                         total64);
+    launch_rows(stream, plan_rows(stream, rows, cols), in, rows, cols, row_sum, row_max, partial64, total, total64);
     CS_HIP(hipGetLastError());
   });
 }

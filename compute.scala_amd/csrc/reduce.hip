@@ -19,6 +19,7 @@
 // two (Tensors.scala:375-387); these kernels sum every element.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 
@@ -325,88 +326,116 @@ __global__ __launch_bounds__(kBlock) void reduce_short_rows_kernel(const float *
 }
 
 // ----------------------------------------------------------------------------- columns
-// Column sums: thread = column, blockIdx.y = a slice of rows; FP64 partials per slice, then
-// one thread per column adds its slices in order. Rows are read eight at a time, all eight
-// loads in flight before the first addition (the additions stay in row order).
+// Column sums. A thread owns four adjacent columns (16-byte loads at any 4-byte boundary; the
+// last four columns overlap the group before when cols % 4 != 0) and every `lanes`-th row of the
+// workgroup's slice of rows: `across` threads side by side, kBlock / across row lanes, so that a
+// workgroup reads whole rows of a narrow matrix. Eight rows of loads are in flight before the
+// first addition. The row lanes meet in LDS in FP64, in order: one partial per column and slice
+// (or, with one slice, the column's sum itself). Bound by HBM: 16384 x 4096 takes 45.7 us with its
+// combine (5.9 TB/s), 20011 x 1003 19.0 us against 26.3 us with one column per thread and one
+// thread per column in the combine, 524288 x 8 9.9 us against 169 us (a wave with two active
+// lanes).
 __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(const float *__restrict__ in, int64_t rows,
-                                                             int64_t cols, int64_t rows_per_slice,
-                                                             double *partial64) {
-  const int64_t col = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-  if (col >= cols) return;
+                                                             int64_t cols, int across, int64_t rows_per_slice,
+                                                             double *partial64, float *col_sum) {
+  __shared__ double part[kBlock * 4];
+  const int lanes = kBlock / across;
+  const int rl = threadIdx.x / across, cl = threadIdx.x % across;
+  const int64_t first = (int64_t(blockIdx.x) * across + cl) * 4;  // of this thread's four columns
   const int64_t r0 = int64_t(blockIdx.y) * rows_per_slice;
   const int64_t r1 = r0 + rows_per_slice < rows ? r0 + rows_per_slice : rows;
-  Acc a;
-  const float *p = in + r0 * cols + col;
-  int64_t r = r0;
-  for (; r + 8 <= r1; r += 8, p += 8 * cols) {
-    float v[8];
+  Acc a[4];
+  if (rl < lanes && first < cols) {
+    if (cols >= 4) {
+      const int64_t c = first + 4 <= cols ? first : cols - 4;
+      const int64_t step = int64_t(lanes) * cols;
+      int64_t r = r0 + rl;
+      const float *p = in + r * cols + c;
+      for (; r + 7 * lanes < r1; r += 8 * lanes, p += 8 * step) {
+        f4u v[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = __builtin_nontemporal_load(p + k * cols);
+        for (int k = 0; k < 8; ++k) v[k] = __builtin_nontemporal_load(reinterpret_cast<const f4u *>(p + k * step));
 #pragma unroll
-    for (int k = 0; k < 8; ++k) a.add(v[k]);
-  }
-  for (; r < r1; ++r, p += cols) a.add(__builtin_nontemporal_load(p));
-  partial64[int64_t(blockIdx.y) * cols + col] = a.result64();
-}
-
-// Four adjacent columns per thread with 16-byte loads, when cols is a multiple of 4 and the
-// input is 16-byte aligned; the same row order per column as above. One wave per workgroup:
-// many small workgroups spread evenly over the CUs.
-constexpr int kColsBlock = 64;
-__global__ __launch_bounds__(kColsBlock) void reduce_cols4_kernel(const float *__restrict__ in, int64_t rows,
-                                                                  int64_t cols, int64_t rows_per_slice,
-                                                                  double *partial64) {
-  const int64_t c = (int64_t(blockIdx.x) * kColsBlock + threadIdx.x) * 4;
-  if (c >= cols) return;
-  const int64_t r0 = int64_t(blockIdx.y) * rows_per_slice;
-  const int64_t r1 = r0 + rows_per_slice < rows ? r0 + rows_per_slice : rows;
-  Acc a0, a1, a2, a3;
-  const int64_t step = cols / 4;  // one row, in 16-byte vectors
-  const f4 *p = reinterpret_cast<const f4 *>(in + r0 * cols + c);
-  int64_t r = r0;
-  for (; r + 8 <= r1; r += 8, p += 8 * step) {
-    f4 v[8];
+        for (int k = 0; k < 8; ++k) {
+          a[0].add(v[k].x);
+          a[1].add(v[k].y);
+          a[2].add(v[k].z);
+          a[3].add(v[k].w);
+        }
+      }
+      f4u v[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = __builtin_nontemporal_load(p + k * step);
+      for (int k = 0; k < 8; ++k)
+        if (r + k * lanes < r1) v[k] = __builtin_nontemporal_load(reinterpret_cast<const f4u *>(p + k * step));
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      a0.add(v[k].x);
-      a1.add(v[k].y);
-      a2.add(v[k].z);
-      a3.add(v[k].w);
+      for (int k = 0; k < 8; ++k)
+        if (r + k * lanes < r1) {
+          a[0].add(v[k].x);
+          a[1].add(v[k].y);
+          a[2].add(v[k].z);
+          a[3].add(v[k].w);
+        }
+    } else {
+      for (int64_t r = r0 + rl; r < r1; r += lanes) {
+        a[0].add(in[r * cols]);
+        if (cols > 1) a[1].add(in[r * cols + 1]);
+        if (cols > 2) a[2].add(in[r * cols + 2]);
+      }
     }
   }
-  for (; r < r1; ++r, p += step) {
-    const f4 v = __builtin_nontemporal_load(p);
-    a0.add(v.x);
-    a1.add(v.y);
-    a2.add(v.z);
-    a3.add(v.w);
+  if (rl < lanes) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) part[(rl * across + cl) * 4 + k] = a[k].result64();
   }
-  double *o = partial64 + int64_t(blockIdx.y) * cols + c;
-  o[0] = a0.result64();
-  o[1] = a1.result64();
-  o[2] = a2.result64();
-  o[3] = a3.result64();
+  __syncthreads();
+  const int t = threadIdx.x;
+  if (t < across * 4) {
+    // thread t adds column t of the workgroup's columns; in an overlapping group the column sits
+    // nearer to the group's end
+    const int64_t col = int64_t(blockIdx.x) * across * 4 + t;
+    if (col < cols) {
+      const int64_t group = col - t % 4;
+      const int k = cols >= 4 && group + 4 > cols ? static_cast<int>(col - (cols - 4)) : t % 4;
+      double s = part[(t / 4) * 4 + k];
+      for (int l = 1; l < lanes; ++l) s += part[(l * across + t / 4) * 4 + k];
+      if (col_sum) col_sum[col] = float(s);
+      else partial64[int64_t(blockIdx.y) * cols + col] = s;
+    }
+  }
 }
 
-// One thread per column adds its slices in order, eight loads in flight.
+// Adds each column's slices: `lanes` threads per column take every lanes-th slice in order, eight
+// loads in flight, and meet in LDS in order.
 __global__ __launch_bounds__(kBlock) void finish_cols_kernel(const double *__restrict__ partial64, int64_t cols,
-                                                             int64_t slices, float *col_sum) {
-  const int64_t col = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-  if (col >= cols) return;
+                                                             int64_t slices, int lanes, float *col_sum) {
+  __shared__ double part[kBlock];
+  const int width = kBlock / lanes, cl = threadIdx.x % width, sl = threadIdx.x / width;
+  const int64_t col = int64_t(blockIdx.x) * width + cl;
   double s = 0.0;
-  const double *p = partial64 + col;
-  int64_t y = 0;
-  for (; y + 8 <= slices; y += 8, p += 8 * cols) {
+  if (col < cols) {
+    const double *p = partial64 + int64_t(sl) * cols + col;
+    const int64_t step = int64_t(lanes) * cols;
+    int64_t y = sl;
+    for (; y + 7 * lanes < slices; y += 8 * lanes, p += 8 * step) {
+      double v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = p[k * step];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) s += v[k];
+    }
     double v[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = p[k * cols];
+    for (int k = 0; k < 8; ++k) v[k] = y + k * lanes < slices ? p[k * step] : 0.0;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) s += v[k];
+    for (int k = 0; k < 8; ++k)
+      if (y + k * lanes < slices) s += v[k];
   }
-  for (; y < slices; ++y, p += cols) s += *p;
-  col_sum[col] = float(s);
+  part[threadIdx.x] = s;
+  __syncthreads();
+  if (sl == 0 && col < cols) {
+    for (int l = 1; l < lanes; ++l) s += part[l * width + cl];
+    col_sum[col] = float(s);
+  }
 }
 
 }  // namespace
@@ -529,6 +558,51 @@ void launch_rows(cs_stream *stream, const RowPlan &p, const float *in, int64_t r
 }
 }  // namespace
 
+namespace {
+// How a [rows, cols] matrix is cut for column sums.
+struct ColPlan {
+  int across = 1;          // threads side by side, four columns each
+  int64_t groups = 1;      // workgroups side by side
+  int64_t slices = 1, rows_per_slice = 1;
+  int finish_lanes = 1;    // threads per column of the combine
+};
+
+// Where the lines lie (whole calls, in us):
+//   * one workgroup per CU, never a few more: four waves of eight rows of loads keep the memory
+//     busy, and each further slice adds partials to write and read (20011 x 1003: 19.0 with one,
+//     19.5 with two, 20.3 with four per CU; 16384 x 4096: 45.8, 51.0, 55.8). Rounding the slices
+//     up left a second round of a few workgroups (10000 x 3000: 31.2 against 25.6).
+//   * at least eight rows per row lane (60000 x 128: 11.0; with 32 13.8).
+//   * up to 32 rows per row lane in one slice, which needs no combine (116 x 2588: 4.2 against
+//     6.8 with two launches); 128 leave one workgroup busy too long (1000 x 100: 13.3 against 6.7).
+//   * 64 threads across, for whole rows of 1 KiB per wave; up to 1024 rows fewer, down to 16, as
+//     long as that brings workgroups (300 x 16384: 6.1 against 7.9; 116 x 2588: 4.2 against 6.4).
+//     Taller matrices lose by it (20011 x 1003: 22.8 against 19.0).
+constexpr int64_t kMinRowsPerLane = 8, kOneSliceRowsPerLane = 32, kNarrowRows = 1024;
+
+ColPlan plan_cols(cs_stream *stream, int64_t rows, int64_t cols) {
+  ColPlan p;
+  const int64_t cus = stream->device->props.multiProcessorCount;
+  const int64_t quads = (cols + 3) / 4;
+  int64_t most = 64;
+  while (rows <= kNarrowRows && most > 16 && (quads + most - 1) / most < cus) most /= 2;
+  p.groups = (quads + most - 1) / most;
+  if (p.groups > 0x7fffffff) fail(CS_INVALID_VALUE, "too many columns");
+  p.across = static_cast<int>((quads + p.groups - 1) / p.groups);
+  const int64_t lanes = kBlock / p.across;
+  if (rows > lanes * kOneSliceRowsPerLane) {
+    int64_t slices = std::min(cus / p.groups, rows / (lanes * kMinRowsPerLane));
+    slices = std::max<int64_t>(1, std::min<int64_t>(slices, 65535));
+    p.rows_per_slice = (rows + slices - 1) / slices;
+    p.slices = (rows + p.rows_per_slice - 1) / p.rows_per_slice;
+  } else {
+    p.rows_per_slice = std::max<int64_t>(rows, 1);
+  }
+  while (p.finish_lanes < 32 && p.finish_lanes * 8 < p.slices) p.finish_lanes *= 2;
+  return p;
+}
+}  // namespace
+
 static int reduce_grid(cs_stream *stream, int64_t n) {
   int cus = stream->device->props.multiProcessorCount;
   int64_t want = (n / 4 + kBlock * 4 - 1) / (kBlock * 4);  // >= 4 vectors per thread
@@ -632,29 +706,19 @@ cs_status cs_reduce_cols(cs_stream *stream, const float *in, int64_t rows, int64
     if (cols == 0) return;
     if (!col_sum || (rows > 0 && !in)) fail(CS_INVALID_VALUE, "null pointer");
     set_device(stream->device);
-    const bool vec = cols % 4 == 0 && (reinterpret_cast<uintptr_t>(in) & 15) == 0;
-    const int64_t per_block = vec ? int64_t(kColsBlock) * 4 : kBlock;  // columns per workgroup
-    int64_t groups = (cols + per_block - 1) / per_block;
-    if (groups > 0x7fffffff) fail(CS_INVALID_VALUE, "too many columns");
-    int cus = stream->device->props.multiProcessorCount;
-    // about 8 waves per CU, and at least 128 rows per slice so that the partials stay few
-    int64_t slices = (int64_t(cus) * (vec ? 32 : 8) + groups - 1) / groups;
-    int64_t max_slices = (rows + 127) / 128;
-    if (slices > max_slices) slices = max_slices;
-    if (slices < 1) slices = 1;
-    if (slices > 65535) slices = 65535;
-    int64_t per = (rows + slices - 1) / slices;
-    if (per < 1) per = 1;
-    slices = rows > 0 ? (rows + per - 1) / per : 1;
-    ReduceScratch s = scratch_for(stream, static_cast<size_t>(slices * cols));
-    const dim3 grid(static_cast<unsigned>(groups), static_cast<unsigned>(slices));
-    if (vec)
-      hipLaunchKernelGGL(reduce_cols4_kernel, grid, dim3(kColsBlock), 0, stream->stream, in, rows, cols, per,
-                         s.partial64);
-    else
-      hipLaunchKernelGGL(reduce_cols_kernel, grid, dim3(kBlock), 0, stream->stream, in, rows, cols, per, s.partial64);
-    hipLaunchKernelGGL(finish_cols_kernel, dim3(static_cast<unsigned>((cols + kBlock - 1) / kBlock)), dim3(kBlock), 0,
-                       stream->stream, s.partial64, cols, slices, col_sum);
+    const ColPlan p = plan_cols(stream, rows, cols);
+    const dim3 grid(static_cast<unsigned>(p.groups), static_cast<unsigned>(p.slices));
+    if (p.slices == 1) {
+      hipLaunchKernelGGL(reduce_cols_kernel, grid, dim3(kBlock), 0, stream->stream, in, rows, cols, p.across,
+                         p.rows_per_slice, static_cast<double *>(nullptr), col_sum);
+    } else {
+      ReduceScratch s = scratch_for(stream, static_cast<size_t>(p.slices * cols));
+      hipLaunchKernelGGL(reduce_cols_kernel, grid, dim3(kBlock), 0, stream->stream, in, rows, cols, p.across,
+                         p.rows_per_slice, s.partial64, static_cast<float *>(nullptr));
+      const int64_t width = kBlock / p.finish_lanes;
+      hipLaunchKernelGGL(finish_cols_kernel, dim3(static_cast<unsigned>((cols + width - 1) / width)), dim3(kBlock), 0,
+                         stream->stream, s.partial64, cols, p.slices, p.finish_lanes, col_sum);
+    }
     CS_HIP(hipGetLastError());
   });
 }

@@ -13,13 +13,14 @@
 //                   each row of A and each column of B (amax / 448 rounded up to 2^e),
 //                   applied by v_mfma_scale_f32_32x32x64_f8f6f4, FP32 accumulate
 //
-// A pre-pass converts A to a K-contiguous operand X[Mp][.] and B to its transpose Y[Np][.]
+// Small products run on gemm_direct_kernel, straight from A and B (prefer_direct, below). For the
+// others a pre-pass converts A to a K-contiguous operand X[Mp][.] and B to its transpose Y[Np][.]
 // (zero padded to the tile sizes; split, interleaved or quantised as the variant needs) in
 // the stream's scratch; the main kernel computes C[m][n] = sum_k X[m][k] Y[n][k] with 256
 // threads (4 wave64s in 2x2) per 256x256 output tile, each wave owning 128x128 as 4x4 MFMA
 // tiles of 32x32 (256 FP32 accumulators per lane).
 //
-// All variants share one pipeline. A K stage is 128 bytes of every operand row (32 FP32
+// All variants share one pipeline there. A K stage is 128 bytes of every operand row (32 FP32
 // values, 64 BF16 values, 32 hi/lo pairs or 128 e4m3 values); two stages live in LDS (128 KiB).
 // The next stage streams global -> LDS directly (buffer_load ... lds, no registers) while
 // the MFMAs of the current one run; inside a stage the fragments of the next MFMA step are
@@ -28,6 +29,7 @@
 // (the lanes the LDS serves in one cycle) hit 16 different bank groups.
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstdint>
 #include <type_traits>
 
@@ -705,6 +707,242 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_lds_kernel(int M, int N, int
       }
 }
 
+// ------------------------------------------------------------------------ direct kernel
+// Products too small to fill the chip with 256 x 256 tiles. A wave owns a (16 T) x (16 T) tile of
+// C and reads its operands from A and B as they lie, without a pre-pass and without LDS: per K
+// step a lane holds kVals consecutive K values of one row of each 16-row tile of A (16-byte loads
+// along K) and, for each of those K, T consecutive columns of B (one load of 4 T bytes along N).
+// MFMA tile j takes the columns n0 + T c + j, c = 0..15, so a lane's T columns are the T tiles of
+// its 16 x 16 column c, and its results are T consecutive columns too. kWK waves of a workgroup
+// take every kWK-th K step of the same tile and add their sums through LDS, in wave order; with
+// kWK = 1 the four waves take four tiles below one another instead. The operands of the next step
+// load while the current one's MFMAs run.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
+
+template <int KIND>
+constexpr int kDirectVals = KIND == kF32 ? 4 : KIND == kFP8 ? 32 : 8;
+
+template <int KIND, int T>
+struct DirectFrags {
+  float a[T][kDirectVals<KIND>], b[T][kDirectVals<KIND>];
+};
+
+__device__ __forceinline__ bf16x8 to_bf16x8(const float (&v)[8]) {
+  i32x4 h;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) h[e] = int(bf16x2(v[2 * e], v[2 * e + 1]));
+  return __builtin_bit_cast(bf16x8, h);
+}
+
+__device__ __forceinline__ void split_bf16x8(const float (&v)[8], bf16x8 &hi, bf16x8 &lo) {
+  i32x4 h, l;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t w = bf16x2(v[2 * e], v[2 * e + 1]);
+    h[e] = int(w);
+    l[e] = int(bf16x2(v[2 * e] - __uint_as_float(w << 16), v[2 * e + 1] - __uint_as_float(w & 0xffff0000u)));
+  }
+  hi = __builtin_bit_cast(bf16x8, h);
+  lo = __builtin_bit_cast(bf16x8, l);
+}
+
+// 32 values of a 128-wide K block whose other 96 are in lanes 16, 32 and 48 away: quantised with
+// the block's scale, as the pre-pass does.
+__device__ __forceinline__ i32x8 to_fp8x32(const float (&v)[32], int &scale) {
+  float m = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 32; ++e) m = fmaxf(m, fabsf(v[e]));
+  m = fmaxf(m, __shfl_xor(m, 16, 64));
+  m = fmaxf(m, __shfl_xor(m, 32, 64));
+  const int e = fp8_scale_exponent(m);
+  const float inv = ldexpf(1.0f, -e);
+  i32x8 w;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) w[j] = int(fp8x4(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3], inv));
+  scale = e + 127;
+  return w;
+}
+
+template <int KIND, int T>
+__device__ __forceinline__ void direct_mma(const DirectFrags<KIND, T> &f, f32x4 (&acc)[T][T]) {
+  if constexpr (KIND == kF32) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < T; ++i)
+#pragma unroll
+        for (int j = 0; j < T; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.a[i][t], f.b[j][t], acc[i][j], 0, 0, 0);
+  } else if constexpr (KIND == kBF16) {
+    bf16x8 a[T], b[T];
+#pragma unroll
+    for (int i = 0; i < T; ++i) a[i] = to_bf16x8(f.a[i]), b[i] = to_bf16x8(f.b[i]);
+#pragma unroll
+    for (int i = 0; i < T; ++i)
+#pragma unroll
+      for (int j = 0; j < T; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+  } else if constexpr (KIND == kBF16X3) {
+    bf16x8 ah[T], al[T], bh[T], bl[T];
+#pragma unroll
+    for (int i = 0; i < T; ++i) split_bf16x8(f.a[i], ah[i], al[i]), split_bf16x8(f.b[i], bh[i], bl[i]);
+#pragma unroll
+    for (int part = 0; part < 3; ++part)
+#pragma unroll
+      for (int i = 0; i < T; ++i)
+#pragma unroll
+        for (int j = 0; j < T; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(part == 0 ? al[i] : ah[i], part == 1 ? bl[j] : bh[j],
+                                                              acc[i][j], 0, 0, 0);
+  } else {
+    i32x8 a[T], b[T];
+    int sa[T], sb[T];
+#pragma unroll
+    for (int i = 0; i < T; ++i) a[i] = to_fp8x32(f.a[i], sa[i]), b[i] = to_fp8x32(f.b[i], sb[i]);
+#pragma unroll
+    for (int i = 0; i < T; ++i)
+#pragma unroll
+      for (int j = 0; j < T; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a[i], b[j], acc[i][j], 0, 0, 0, sa[i], 0, sb[j]);
+  }
+}
+
+template <int KIND, int T, int kWK>
+__global__ __launch_bounds__(kWK == 1 ? 256 : 64 * kWK) void gemm_direct_kernel(
+    int M, int N, int K, const float *__restrict__ A, int lda, const float *__restrict__ B, int ldb,
+    float *__restrict__ C, int ldc, int tiles_m) {
+  constexpr int kVals = kDirectVals<KIND>, kStep = 4 * kVals;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4;
+  const int tm = int(blockIdx.x) % tiles_m, tn = int(blockIdx.x) / tiles_m;
+  const int m0 = (kWK == 1 ? tm * 4 + wave : tm) * 16 * T, n0 = tn * 16 * T;
+  const int nb = n0 + T * l16;  // this lane's T columns
+  const bool inside = nb + T <= N;
+  const float *arow[T];  // rows past the end repeat the last one: their results are not stored
+#pragma unroll
+  for (int i = 0; i < T; ++i) arow[i] = A + int64_t(min(m0 + 16 * i + l16, M - 1)) * lda + quad * kVals;
+  int ncol[T];
+#pragma unroll
+  for (int j = 0; j < T; ++j) ncol[j] = min(nb + j, N - 1);
+
+  auto load = [&](int step, DirectFrags<KIND, T> &f) {
+    const int k0 = step * kStep, k = k0 + quad * kVals;  // this lane's K values: k .. k + kVals - 1
+    const float *brow = B + int64_t(k) * ldb;
+    if (k + kVals <= K) {
+#pragma unroll
+      for (int i = 0; i < T; ++i)
+#pragma unroll
+        for (int t = 0; t < kVals; t += 4) {
+          const f4u v = *reinterpret_cast<const f4u *>(arow[i] + k0 + t);
+          f.a[i][t] = v.x, f.a[i][t + 1] = v.y, f.a[i][t + 2] = v.z, f.a[i][t + 3] = v.w;
+        }
+      if (inside) {
+#pragma unroll
+        for (int t = 0; t < kVals; ++t) {
+          const float *q = brow + int64_t(t) * ldb + nb;
+          if constexpr (T == 4) {
+            const f4u v = *reinterpret_cast<const f4u *>(q);
+            f.b[0][t] = v.x, f.b[1][t] = v.y, f.b[2][t] = v.z, f.b[3][t] = v.w;
+          } else if constexpr (T == 2) {
+            const f2u v = *reinterpret_cast<const f2u *>(q);
+            f.b[0][t] = v.x, f.b[1][t] = v.y;
+          } else {
+            f.b[0][t] = *q;
+          }
+        }
+      } else {
+#pragma unroll
+        for (int t = 0; t < kVals; ++t)
+#pragma unroll
+          for (int j = 0; j < T; ++j) f.b[j][t] = brow[int64_t(t) * ldb + ncol[j]];
+      }
+    } else {
+      // past the end of K: zeros in both operands
+#pragma unroll
+      for (int t = 0; t < kVals; ++t) {
+#pragma unroll
+        for (int i = 0; i < T; ++i) f.a[i][t] = k + t < K ? arow[i][k0 + t] : 0.0f;
+#pragma unroll
+        for (int j = 0; j < T; ++j) f.b[j][t] = k + t < K ? brow[int64_t(t) * ldb + ncol[j]] : 0.0f;
+      }
+    }
+    CSMI_SCHED_FENCE();  // the loads go out before the MFMAs of the step before
+  };
+
+  f32x4 acc[T][T];
+#pragma unroll
+  for (int i = 0; i < T; ++i)
+#pragma unroll
+    for (int j = 0; j < T; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const int steps = (K + kStep - 1) / kStep;
+  int step = kWK == 1 ? 0 : wave;
+  if (step < steps) {
+    DirectFrags<KIND, T> f[2];
+    load(step, f[0]);
+    for (;;) {
+      if (step + kWK >= steps) {
+        direct_mma<KIND, T>(f[0], acc);
+        break;
+      }
+      load(step + kWK, f[1]);
+      direct_mma<KIND, T>(f[0], acc);
+      step += kWK;
+      if (step + kWK >= steps) {
+        direct_mma<KIND, T>(f[1], acc);
+        break;
+      }
+      load(step + kWK, f[0]);
+      direct_mma<KIND, T>(f[1], acc);
+      step += kWK;
+    }
+  }
+
+  // acc[i][j][e] is row m0 + 16 i + 4 quad + e, column nb + j
+  auto store = [&](int row, int col, const float (&v)[T]) {
+    if (row >= M) return;
+    float *c = C + int64_t(row) * ldc + col;
+    if (T == 4 && col + 4 <= N) {
+      *reinterpret_cast<f4u *>(c) = f4u{v[0], v[1 % T], v[2 % T], v[3 % T]};
+      return;
+    }
+#pragma unroll
+    for (int j = 0; j < T; ++j)
+      if (col + j < N) c[j] = v[j];
+  };
+  if constexpr (kWK == 1) {
+#pragma unroll
+    for (int i = 0; i < T; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float v[T];
+#pragma unroll
+        for (int j = 0; j < T; ++j) v[j] = acc[i][j][e];
+        store(m0 + 16 * i + 4 * quad + e, nb, v);
+      }
+  } else {
+    // part[wave][(i, e, j)][lane]
+    extern __shared__ float part[];
+    constexpr int kRuns = 4 * T;  // runs of T columns per lane
+#pragma unroll
+    for (int i = 0; i < T; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int j = 0; j < T; ++j) part[((wave * kRuns + 4 * i + e) * T + j) * 64 + lane] = acc[i][j][e];
+    __syncthreads();
+    for (int run = wave; run < kRuns; run += kWK) {
+      float v[T];
+#pragma unroll
+      for (int j = 0; j < T; ++j) v[j] = part[(run * T + j) * 64 + lane];
+      for (int w = 1; w < kWK; ++w)
+#pragma unroll
+        for (int j = 0; j < T; ++j) v[j] += part[((w * kRuns + run) * T + j) * 64 + lane];
+      store(m0 + 16 * (run / 4) + 4 * quad + run % 4, nb, v);
+    }
+  }
+}
+
 int64_t round_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 
 __global__ __launch_bounds__(256) void zero_matrix_kernel(float *__restrict__ C, int M, int N, int ldc) {
@@ -765,6 +1003,102 @@ void run_lds(cs_stream *stream, int M, int N, int K, const float *A, int lda, co
   CS_HIP(hipGetLastError());
 }
 
+template <int KIND, int T, int kWK>
+void run_direct(cs_stream *stream, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
+                int ldc) {
+  const int64_t rows = 16 * T * (kWK == 1 ? 4 : 1);  // of C per workgroup
+  const int64_t tiles_m = (M + rows - 1) / rows, tiles_n = (N + 16 * T - 1) / (16 * T);
+  const size_t lds = kWK == 1 ? 0 : size_t(kWK) * 256 * T * T * sizeof(float);
+  hipLaunchKernelGGL((gemm_direct_kernel<KIND, T, kWK>), dim3(unsigned(tiles_m * tiles_n)),
+                     dim3(kWK == 1 ? 256 : 64 * kWK), lds, stream->stream, M, N, K, A, lda, B, ldb, C, ldc,
+                     int(tiles_m));
+  CS_HIP(hipGetLastError());
+}
+
+// The direct kernel's launch shape. Where the lines lie (FP32 calls, in us, "T.kWK"):
+//   * the largest T that still gives a tile per CU: 300x200x1000 (247 tiles of T = 1) 1.16 5.8,
+//     2.8 10.7, 4.4 28.2; 512^3 (256 of T = 2) 2.8 5.8, 1.4 7.1, 4.4 13.1; 1000^3 (256 of T = 4)
+//     4.4 29.1, 2.4 33.0, 1.4 51.4. T stays where a larger one would pad the result by more than
+//     a third (65536x8x8: 1.1 4.2, 4.1 5.6).
+//   * waves per tile as long as they are needed to fill the SIMDs and have a K step each:
+//     300x200x1000 1.16 5.8, 1.4 7.2, 1.1 22.2; 2000x64x500 (500 tiles) 1.4 5.4, 1.16 6.5;
+//     2048^3 (1024 tiles of T = 4) 4.1 155.9, 4.4 164.5; 65536x8x8 1.1 4.2, 1.4 5.0.
+// FP8 holds 32 K values of every row and column per lane: more than T = 2 or than 4 waves per
+// tile spills (300x200x1000: 1.4 10.8, 1.16 22.2, 4.4 71.1).
+struct DirectPlan {
+  int t = 1, wk = 1;
+};
+
+DirectPlan plan_direct(int kind, int64_t cus, int64_t M, int64_t N, int64_t K) {
+  auto up = [](int64_t v, int64_t a) { return (v + a - 1) / a; };
+  DirectPlan p;
+  for (int t = kind == kFP8 ? 2 : 4; t > 1; t /= 2) {
+    const int64_t e = 16 * t, area = up(M, e) * up(N, e) * e * e;
+    if (up(M, e) * up(N, e) >= cus && area * 3 <= up(M, 16) * up(N, 16) * 256 * 4) {
+      p.t = t;
+      break;
+    }
+  }
+  const int64_t tiles = up(M, 16 * p.t) * up(N, 16 * p.t);
+  const int64_t steps = up(K, kind == kF32 ? 16 : kind == kFP8 ? 128 : 32);
+  if (steps < 3 || tiles > (p.t == 4 ? 2 : 4) * cus) return p;
+  p.wk = 4;
+  if (kind != kFP8 && p.t < 4 && tiles <= cus && steps > 4) p.wk = p.t == 1 ? 16 : 8;
+  return p;
+}
+
+// Whether two ranges of device memory meet.
+bool overlap(const float *a, int64_t rows_a, int64_t cols_a, int lda, const float *c, int64_t rows_c, int64_t cols_c,
+             int ldc) {
+  const float *a1 = a + (rows_a - 1) * lda + cols_a, *c1 = c + (rows_c - 1) * ldc + cols_c;
+  return a < c1 && c < a1;
+}
+
+// Direct or packed. The packed kernel's time is a round of 256 x 256 tiles over K for every 256
+// workgroups begun, however few there are, on top of the pre-pass and a second launch; the direct
+// one's follows the flops. In us, direct / packed:
+//   FP32: 300x200x1000 5.8 / 242, 1000^3 29.1 / 250, 2048^3 156 / 481, 1024x1024x4096 81 / 936
+//   BF16: 300x200x1000 5.6 / 33, 1000^3 18.7 / 37.6, 1024x1024x4096 62 / 99, 2048^3 122 / 61
+//   BF16x3: 1000^3 20.4 / 73.9, 2048^3 85 / 130;  FP8: 512^3 6.5 / 19.6, 1000^3 43 / 30
+// The packed path copies the operands first, so a C that overlaps A or B always takes it.
+template <int KIND>
+bool prefer_direct(int64_t cus, int64_t M, int64_t N, int64_t K, const DirectPlan &p) {
+  const double packed_per_k = KIND == kF32 ? 0.225 : KIND == kBF16 ? 0.0217 : KIND == kBF16X3 ? 0.054 : 0.0125;  // us
+  const double direct_tflops =
+      KIND == kF32 ? 105.0 : KIND == kBF16 ? 135.0 : KIND == kBF16X3 ? 160.0 : p.t == 2 ? 40.0 : 25.0;
+  const double e = 16.0 * p.t;
+  const double area = std::ceil(M / e) * std::ceil(N / e) * e * e, out = double(M) * double(N);
+  // the direct kernel's stores of C come in shorter runs (4096x4096x16 in BF16: 20.5 / 18.7)
+  const double direct = 2e-6 * area * double(K) / direct_tflops + (KIND == kF32 ? 0.8e-6 : 1.2e-6) * out;
+  const double rounds = std::ceil(std::ceil(M / 256.0) * std::ceil(N / 256.0) / double(cus));
+  const double pack = double(M + N) * double(K) * 1.5e-6;
+  return direct < 8.0 + pack + rounds * packed_per_k * double(K) + 0.5e-6 * out;
+}
+
+template <int KIND>
+void run(cs_stream *stream, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C, int ldc) {
+  const int64_t cus = stream->device->props.multiProcessorCount;
+  const DirectPlan p = plan_direct(KIND, cus, M, N, K);
+  if (!prefer_direct<KIND>(cus, M, N, K, p) || overlap(A, M, K, lda, C, M, N, ldc) ||
+      overlap(B, K, N, ldb, C, M, N, ldc))
+    return run_lds<KIND>(stream, M, N, K, A, lda, B, ldb, C, ldc);
+  switch (p.t * 100 + p.wk) {
+    case 101: return run_direct<KIND, 1, 1>(stream, M, N, K, A, lda, B, ldb, C, ldc);
+    case 104: return run_direct<KIND, 1, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc);
+    case 201: return run_direct<KIND, 2, 1>(stream, M, N, K, A, lda, B, ldb, C, ldc);
+    case 204: return run_direct<KIND, 2, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc);
+  }
+  if constexpr (KIND != kFP8) {
+    switch (p.t * 100 + p.wk) {
+      case 116: return run_direct<KIND, 1, 16>(stream, M, N, K, A, lda, B, ldb, C, ldc);
+      case 208: return run_direct<KIND, 2, 8>(stream, M, N, K, A, lda, B, ldb, C, ldc);
+      case 401: return run_direct<KIND, 4, 1>(stream, M, N, K, A, lda, B, ldb, C, ldc);
+      case 404: return run_direct<KIND, 4, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc);
+    }
+  }
+  fail(CS_INVALID_OPERATION, "no direct GEMM kernel for this plan");
+}
+
 }  // namespace
 }  // namespace csmi
 
@@ -792,10 +1126,10 @@ extern "C" cs_status cs_gemm(cs_stream *stream, int variant, int M, int N, int K
     if (int64_t(M) * K >= (int64_t(1) << 31) || int64_t(N) * K >= (int64_t(1) << 31))
       fail(CS_INVALID_VALUE, "operands are limited to 2^31 elements");
     switch (variant) {
-      case CS_GEMM_FP32: run_lds<kF32>(stream, M, N, K, A, lda, B, ldb, C, ldc); break;
-      case CS_GEMM_BF16: run_lds<kBF16>(stream, M, N, K, A, lda, B, ldb, C, ldc); break;
-      case CS_GEMM_BF16X3: run_lds<kBF16X3>(stream, M, N, K, A, lda, B, ldb, C, ldc); break;
-      case CS_GEMM_FP8: run_lds<kFP8>(stream, M, N, K, A, lda, B, ldb, C, ldc); break;
+      case CS_GEMM_FP32: run<kF32>(stream, M, N, K, A, lda, B, ldb, C, ldc); break;
+      case CS_GEMM_BF16: run<kBF16>(stream, M, N, K, A, lda, B, ldb, C, ldc); break;
+      case CS_GEMM_BF16X3: run<kBF16X3>(stream, M, N, K, A, lda, B, ldb, C, ldc); break;
+      case CS_GEMM_FP8: run<kFP8>(stream, M, N, K, A, lda, B, ldb, C, ldc); break;
     }
   });
 }

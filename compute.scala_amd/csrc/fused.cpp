@@ -298,6 +298,12 @@ struct Options {
 // size (launch_bound) and launched by default at one element per vector and per thread.
 constexpr size_t kLargeBody = 256;
 
+// Rows longer than a vector of four that four does not divide are cut into vectors of four all the
+// same (Emitter::ragged). In us against the widest dividing width, at about 4 million elements: view
+// chain with rows of 5 12.1 / 17.3, of 6 11.1 / 14.1, of 10 10.8 / 14.1, of 33 10.7 / 11.1, of 510
+// 9.0 / 9.8; a*b+c 10.6 / 12.3; 2049 x 2050 transpose plus matrix 13.8 / 18.9; their sums 11.9 / 17.5.
+constexpr int64_t kRaggedRow = 5;
+
 Options resolve_options(const cs_fused_options *o, const Dag &dag) {
   Options r;
   if (o) {
@@ -318,9 +324,13 @@ Options resolve_options(const cs_fused_options *o, const Dag &dag) {
   // holds hundreds of values per element, so it defaults to 1 and 1 (the convolution idiom:
   // 9.3 us at V=1 against 25 us at V=2 and 50 us at V=4; two vectors per thread spill, 129 us).
   const bool large = dag.nodes.size() > kLargeBody;
-  if (r.V == 0) r.V = large ? 1 : 4;
-  if (r.V != 1 && r.V != 2 && r.V != 4 && r.V != 8) fail(CS_INVALID_VALUE, "vector_width must be 1, 2, 4 or 8");
-  while (r.V > 1 && last % r.V != 0) r.V /= 2;
+  if (r.V == 0 && !large && last >= kRaggedRow && last % 4 != 0) {
+    r.V = 4;  // the last vector of a row overlaps the one before (Emitter::ragged)
+  } else {
+    if (r.V == 0) r.V = large ? 1 : 4;
+    if (r.V != 1 && r.V != 2 && r.V != 4 && r.V != 8) fail(CS_INVALID_VALUE, "vector_width must be 1, 2, 4 or 8");
+    while (r.V > 1 && last % r.V != 0) r.V /= 2;
+  }
   if (r.U == 0) r.U = !large && total >= (int64_t(1) << 22) ? 2 : 1;
   if (r.U < 1 || r.U > 8) fail(CS_INVALID_VALUE, "items_per_thread must be 1..8");
   if (r.block == 0) r.block = 256;
@@ -508,8 +518,6 @@ class Emitter {
     Order ord;
     const int r = static_cast<int>(dag_.out_shape.size());
     if (o_.order == CS_ORDER_LINEAR || o_.sum || r < 2) return ord;
-    const int64_t V = o_.V;
-    if (dag_.out_shape[r - 1] % V != 0) return ord;
     std::vector<double> weight(static_cast<size_t>(r), 0.0);
     for (const cs_node &n : dag_.nodes) {
       if (n.op != CS_OP_EXTRACT) continue;
@@ -537,9 +545,9 @@ class Emitter {
       if (weight[static_cast<size_t>(x)] > 0.0 && (d < 0 || weight[static_cast<size_t>(x)] > weight[static_cast<size_t>(d)]))
         d = x;
     if (d < 0) return ord;
-    int64_t B = 1;
-    for (int x = d + 1; x < r; ++x) B *= dag_.out_shape[static_cast<size_t>(x)];
-    const int64_t Sd = dag_.out_shape[static_cast<size_t>(d)], Bv = B / V;
+    int64_t Bv = row_vectors();
+    for (int x = d + 1; x < r - 1; ++x) Bv *= dag_.out_shape[static_cast<size_t>(x)];
+    const int64_t Sd = dag_.out_shape[static_cast<size_t>(d)];
     const int64_t R = least_padding(Sd, 16, 32), C = least_padding(Bv, 8, 16);
     if (R < 4) return ord;
     const int64_t Sdp = (Sd + R - 1) / R * R, Bvp = (Bv + C - 1) / C * C;
@@ -550,12 +558,24 @@ class Emitter {
     return ord;
   }
 
+  // Rows that the vector width does not divide: a row has one vector more than fit, and the last one
+  // starts early, so that it ends with the row. Its first elements repeat the ones before with the
+  // same values (a sum leaves them out), and every vector is whole: no element takes a path of its
+  // own, and loads and stores stay 16 bytes wide, at any 4-byte boundary. The view chain of
+  // [251,37,509] takes 8.5 us this way against 10.2 us one element at a time.
+  bool ragged() const { return !dag_.out_shape.empty() && dag_.out_shape.back() % o_.V != 0; }
+  // Vectors per row of the innermost dimension.
+  int64_t row_vectors() const {
+    return dag_.out_shape.empty() ? 1 : (dag_.out_shape.back() + o_.V - 1) / o_.V;
+  }
+
   void body(std::ostringstream &s, const std::string &tile, int64_t *vectors_out) {
     const int r = static_cast<int>(dag_.out_shape.size());
     const int V = o_.V, U = o_.U;
     int64_t total = 1;
     for (auto d : dag_.out_shape) total *= d;
-    const int64_t vectors = total / V;
+    const bool rag = ragged();
+    const int64_t vectors = rag ? total / dag_.out_shape[r - 1] * row_vectors() : total / V;
     const int nout = static_cast<int>(dag_.outputs.size());
     uniform_.clear();
     fill_of_.clear();
@@ -567,6 +587,7 @@ class Emitter {
     // phase 0: vector index, validity and coordinates of element 0 of every vector
     s << "  unsigned q[" << U << "]; bool live[" << U << "];\n";
     for (int d = 0; d < r; ++d) s << "  int c" << d << "[" << U << "];\n";
+    if (rag) s << "  unsigned e0[" << U << "];" << (o_.sum ? " int again[" + std::to_string(U) + "];" : std::string()) << "\n";
     s << "#pragma unroll\n  for (int u = 0; u < " << U << "; ++u) {\n";
     s << "    q[u] = vbase + u * " << bdim_ << ";\n";
     if (!ord.tiled) {
@@ -587,8 +608,17 @@ class Emitter {
       s << "      q[u] = live[u] ? (ot * " << ord.Sd << "u + dd) * " << ord.Bv << "u + bb : " << vectors << "u;\n";
       s << "    }\n";
     }
-    s << "    unsigned rest = q[u] * " << V << "u;\n";
-    for (int d = r - 1; d >= 0; --d) {
+    if (rag) {
+      const int64_t last = dag_.out_shape[r - 1], rv = row_vectors();
+      s << "    unsigned rest = q[u] / " << rv << "u;\n";
+      s << "    const int at = (int)(q[u] - rest * " << rv << "u) * " << V << ";\n";
+      s << "    c" << r - 1 << "[u] = at < " << last - V << " ? at : " << last - V << ";\n";
+      s << "    e0[u] = rest * " << last << "u + (unsigned)c" << r - 1 << "[u];\n";
+      if (o_.sum) s << "    again[u] = at - c" << r - 1 << "[u];\n";
+    } else {
+      s << "    unsigned rest = q[u] * " << V << "u;\n";
+    }
+    for (int d = rag ? r - 2 : r - 1; d >= 0; --d) {
       if (d > 0)
         s << "    c" << d << "[u] = (int)(rest % " << dag_.out_shape[d] << "u); rest /= " << dag_.out_shape[d] << "u;\n";
       else
@@ -615,7 +645,11 @@ class Emitter {
     const int run = V * nout;
     s << "#pragma unroll\n  for (int u = 0; u < " << U << "; ++u) {\n";
     s << "    if (!live[u]) continue;\n";
-    s << "    " << gq_ << "float* __restrict__ dst = out + (unsigned long long)q[u] * " << run << "u;\n";
+    if (rag)
+      s << "    " << gq_ << "float* __restrict__ dst = out + (unsigned long long)e0[u] * " << nout << "u;\n";
+    else
+      s << "    " << gq_ << "float* __restrict__ dst = out + (unsigned long long)q[u] * " << run << "u;\n";
+    const std::string vec = rag ? "csmi_f4" : "csmi_v4";
     std::vector<std::string> vals;
     for (int v = 0; v < V; ++v)
       for (int j = 0; j < nout; ++j) vals.push_back(value_of(dag_.outputs[j], v));
@@ -623,8 +657,8 @@ class Emitter {
     while (i < run) {
       if (run % 4 == 0 && run - i >= 4) {
         s << "    " << store("dst + " + std::to_string(i),
-                             "csmi_v4{" + vals[i] + ", " + vals[i + 1] + ", " + vals[i + 2] + ", " + vals[i + 3] + "}",
-                             "csmi_v4", run)
+                             vec + "{" + vals[i] + ", " + vals[i + 1] + ", " + vals[i + 2] + ", " + vals[i + 3] + "}",
+                             vec, run)
           << "\n";
         i += 4;
       } else {
@@ -643,7 +677,9 @@ class Emitter {
     const int V = o_.V, U = o_.U;
     s << "  float csmi_s = 0.0f, csmi_c = 0.0f;\n";
     s << "#pragma unroll\n  for (int u = 0; u < " << U << "; ++u) {\n    if (!live[u]) continue;\n";
-    for (int v = 0; v < V; ++v) s << "    csmi_acc(csmi_s, csmi_c, " << value_of(dag_.outputs[0], v) << ");\n";
+    for (int v = 0; v < V; ++v)
+      s << "    " << (ragged() && v + 1 < V ? "if (again[u] <= " + std::to_string(v) + ") " : std::string())
+        << "csmi_acc(csmi_s, csmi_c, " << value_of(dag_.outputs[0], v) << ");\n";
     s << "  }\n";
     // c only while s is finite: an infinite or NaN sum stays so, and its error terms are NaN
     s << "  double csmi_d = __builtin_isfinite(csmi_s) ? (double)csmi_s + (double)csmi_c : (double)csmi_s;\n";
@@ -664,9 +700,9 @@ class Emitter {
   // written through becomes partial-line writes: those stay plain non-temporal stores.
   std::string store(const std::string &addr, const std::string &val, const std::string &type, int run) {
     if (o_.nt) {
-      const bool whole = (run == 4 && type == "csmi_v4") || (run == 1 && type == "float");
+      const bool whole = (run == 4 && type != "float") || (run == 1 && type == "float");
       if (!whole) return "__builtin_nontemporal_store(" + val + ", (" + gq_ + type + "*)(" + addr + "));";
-      const std::string op = type == "csmi_v4" ? "global_store_dwordx4" : "global_store_dword";
+      const std::string op = type != "float" ? "global_store_dwordx4" : "global_store_dword";
       return "asm volatile(\"" + op + " %0, %1, off sc1 nt\" :: \"v\"((" + gq_ + type + "*)(" + addr +
              ")), \"v\"(" + val + ") : \"memory\");";
     }
@@ -1110,7 +1146,7 @@ class Emitter {
     // leaf's base instead and are replaced by the padding: no per-element branches. Gathers of
     // one leaf that differ only in k share their chunks (a value and its translate read the
     // same row).
-    const bool window = contiguous && V % 4 == 0 && p.shape[moving] % 4 == 0 && rows[moving].others_by4 &&
+    const bool window = contiguous && !ragged() && V % 4 == 0 && p.shape[moving] % 4 == 0 && rows[moving].others_by4 &&
                         !rows[moving].upper_only;
     std::vector<std::string> chunk(static_cast<size_t>(V / 4 + 1));
     std::vector<bool> chunk_new(chunk.size(), false);

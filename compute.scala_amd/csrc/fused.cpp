@@ -298,6 +298,8 @@ struct Options {
 // size (launch_bound) and launched by default at one element per vector and per thread.
 constexpr size_t kLargeBody = 256;
 
+bool tiled_launch(const Dag &dag, const Options &o);
+
 // Rows longer than a vector of four that four does not divide are cut into vectors of four all the
 // same (Emitter::ragged). In us against the widest dividing width, at about 4 million elements: view
 // chain with rows of 5 12.1 / 17.3, of 6 11.1 / 14.1, of 10 10.8 / 14.1, of 33 10.7 / 11.1, of 510
@@ -320,9 +322,12 @@ Options resolve_options(const cs_fused_options *o, const Dag &dag) {
   int64_t last = dag.out_shape.empty() ? 1 : dag.out_shape.back();
   int64_t total = 1;
   for (auto s : dag.out_shape) total *= s;
-  // Defaults: 4 elements per vector, 2 vectors per thread from 2^22 elements. A large body
-  // holds hundreds of values per element, so it defaults to 1 and 1 (the convolution idiom:
-  // 9.3 us at V=1 against 25 us at V=2 and 50 us at V=4; two vectors per thread spill, 129 us).
+  // Defaults: 4 elements per vector, 2 vectors per thread from 2^22 elements; from 2^23 with a
+  // transcendental function outside 2-D tiles, where the arithmetic of one vector covers the loads of
+  // another wave's (us, 1 / 2 vectors: view chain of 4 million elements 7.1 / 7.6, of 32 million
+  // 57.8 / 53.5; a*b+c of 4 million 10.7 / 10.6; 2048 x 2048 transpose plus matrix 12.6 / 10.9).
+  // A large body holds hundreds of values per element, so it defaults to 1 and 1 (the convolution
+  // idiom: 9.3 us at V=1 against 25 us at V=2 and 50 us at V=4; two vectors per thread spill, 129 us).
   const bool large = dag.nodes.size() > kLargeBody;
   if (r.V == 0 && !large && last >= kRaggedRow && last % 4 != 0) {
     r.V = 4;  // the last vector of a row overlaps the one before (Emitter::ragged)
@@ -331,13 +336,21 @@ Options resolve_options(const cs_fused_options *o, const Dag &dag) {
     if (r.V != 1 && r.V != 2 && r.V != 4 && r.V != 8) fail(CS_INVALID_VALUE, "vector_width must be 1, 2, 4 or 8");
     while (r.V > 1 && last % r.V != 0) r.V /= 2;
   }
-  if (r.U == 0) r.U = !large && total >= (int64_t(1) << 22) ? 2 : 1;
+  if (r.U == 0) {
+    bool heavy = false;
+    for (const cs_node &n : dag.nodes) heavy = heavy || n.op == CS_OP_TANH || n.op == CS_OP_EXP || n.op == CS_OP_LOG;
+    const int from = heavy && !tiled_launch(dag, r) ? 23 : 22;
+    r.U = !large && total >= (int64_t(1) << from) ? 2 : 1;
+  }
   if (r.U < 1 || r.U > 8) fail(CS_INVALID_VALUE, "items_per_thread must be 1..8");
   if (r.block == 0) r.block = 256;
   if (r.block < 64 || r.block > 1024 || r.block % 64 != 0)
     fail(CS_INVALID_WORK_GROUP_SIZE, "block_size must be a multiple of 64 in 64..1024");
   return r;
 }
+
+// Whether the vector width leaves elements over at the end of every row (Emitter::ragged).
+bool ragged_rows(const Dag &dag, const Options &o) { return !dag.out_shape.empty() && dag.out_shape.back() % o.V != 0; }
 
 // Rows of a TRANSFORM matrix: the rank of the space its operand lives in.
 int transform_rows(const Dag &dag, const cs_node &n) {
@@ -470,6 +483,13 @@ class Emitter {
 
   int nleaves() const { return dag_.nleaves; }
 
+  // Whether the automatic launch order takes 2-D tiles for this expression.
+  bool tiled() const {
+    int64_t rows = 1;
+    for (size_t i = 0; i + 1 < dag_.out_shape.size(); ++i) rows *= dag_.out_shape[i];
+    return choose_order(rows * row_vectors()).tiled;
+  }
+
  private:
   void header(std::ostringstream &s, bool with_prelude) {
     const int r = static_cast<int>(dag_.out_shape.size());
@@ -559,11 +579,15 @@ class Emitter {
   }
 
   // Rows that the vector width does not divide: a row has one vector more than fit, and the last one
-  // starts early, so that it ends with the row. Its first elements repeat the ones before with the
-  // same values (a sum leaves them out), and every vector is whole: no element takes a path of its
-  // own, and loads and stores stay 16 bytes wide, at any 4-byte boundary. The view chain of
-  // [251,37,509] takes 8.5 us this way against 10.2 us one element at a time.
-  bool ragged() const { return !dag_.out_shape.empty() && dag_.out_shape.back() % o_.V != 0; }
+  // starts early, so that it ends with the row. Its first again[u] elements repeat the ones before
+  // with the same values (a sum leaves them out), so loads and stores stay 16 bytes wide, at any
+  // 4-byte boundary. The view chain of [251,37,509] takes 8.4 us this way, against 9.2 us one element
+  // at a time; without the repeated stores each row would end in a narrower one, and the partly
+  // written lines cost more than the rest together (12.1 us, with rows of 33 31 us against 11).
+  // A kernel whose output lies over one of its leaves must not repeat elements, as the repetition may
+  // read what the first computation wrote: such launches run at a width that divides the rows
+  // (LaunchKernel), and a batch's bodies, whose pointers are bound later, store no element twice.
+  bool ragged() const { return ragged_rows(dag_, o_); }
   // Vectors per row of the innermost dimension.
   int64_t row_vectors() const {
     return dag_.out_shape.empty() ? 1 : (dag_.out_shape.back() + o_.V - 1) / o_.V;
@@ -587,7 +611,7 @@ class Emitter {
     // phase 0: vector index, validity and coordinates of element 0 of every vector
     s << "  unsigned q[" << U << "]; bool live[" << U << "];\n";
     for (int d = 0; d < r; ++d) s << "  int c" << d << "[" << U << "];\n";
-    if (rag) s << "  unsigned e0[" << U << "];" << (o_.sum ? " int again[" + std::to_string(U) + "];" : std::string()) << "\n";
+    if (rag) s << "  unsigned e0[" << U << "]; int again[" << U << "];\n";
     s << "#pragma unroll\n  for (int u = 0; u < " << U << "; ++u) {\n";
     s << "    q[u] = vbase + u * " << bdim_ << ";\n";
     if (!ord.tiled) {
@@ -614,7 +638,7 @@ class Emitter {
       s << "    const int at = (int)(q[u] - rest * " << rv << "u) * " << V << ";\n";
       s << "    c" << r - 1 << "[u] = at < " << last - V << " ? at : " << last - V << ";\n";
       s << "    e0[u] = rest * " << last << "u + (unsigned)c" << r - 1 << "[u];\n";
-      if (o_.sum) s << "    again[u] = at - c" << r - 1 << "[u];\n";
+      s << "    again[u] = at - c" << r - 1 << "[u];\n";
     } else {
       s << "    unsigned rest = q[u] * " << V << "u;\n";
     }
@@ -653,6 +677,8 @@ class Emitter {
     std::vector<std::string> vals;
     for (int v = 0; v < V; ++v)
       for (int j = 0; j < nout; ++j) vals.push_back(value_of(dag_.outputs[j], v));
+    const bool mask = rag && !gq_.empty();
+    if (mask) s << "    if (again[u] == 0) {\n";
     int i = 0;
     while (i < run) {
       if (run % 4 == 0 && run - i >= 4) {
@@ -665,6 +691,15 @@ class Emitter {
         s << "    " << store("dst + " + std::to_string(i), vals[i], "float", run) << "\n";
         i += 1;
       }
+    }
+    if (mask) {
+      s << "    } else {\n";
+      for (int v = 1; v < V; ++v) {
+        s << "      if (again[u] <= " << v << ") {";
+        for (int j = 0; j < nout; ++j) s << " dst[" << v * nout + j << "] = " << vals[v * nout + j] << ";";
+        s << " }\n";
+      }
+      s << "    }\n";
     }
     s << "  }\n";
   }
@@ -692,20 +727,24 @@ class Emitter {
     s << "    partials[" << (bdim_ == "blockDim.x" ? "blockIdx.x" : "tile") << "] = t;\n  }\n";
   }
 
-  // Non-temporal stores. When one store instruction covers the wave's lanes contiguously (a
-  // run of 1 or 4 floats per vector) they also write through at device scope (`sc1 nt`, a
-  // vector store): the output is not read again, and no dirty line is left in L2 for the
-  // release at the end of the kernel, which otherwise writes it back between this launch and
-  // the next. Longer or odd runs leave each instruction every other piece of a line, which
-  // written through becomes partial-line writes: those stay plain non-temporal stores.
+  // Stores. When one store instruction covers the wave's lanes contiguously (a run of 1 or 4 floats
+  // per vector) it writes through at device scope (`sc1`, a vector store): no dirty line is left in
+  // L2 for the release at the end of the kernel, which otherwise writes it back between this launch
+  // and the next. The lines stay in L2 for a kernel that reads them, unless the caller asks for
+  // non-temporal stores (`sc1 nt`). In us, plain / written through / and non-temporal: view chain of
+  // [256,64,256] 8.9 / 7.6 / 7.5, of [251,37,509] 9.6 / 8.3 / 10.2, of [300,100,33] 6.3 / 4.0 / 4.3;
+  // a 2048 x 2048 producer followed by its consumer 21.9 / 20.7 / 23.0; a*b+c of 16 million 47.9 /
+  // 48.1 / 47.7. Longer or odd runs leave each instruction every other piece of a line, which written
+  // through becomes partial-line writes: those stay plain or plainly non-temporal, as do the bodies
+  // of a batch, whose kernel ends once.
   std::string store(const std::string &addr, const std::string &val, const std::string &type, int run) {
-    if (o_.nt) {
-      const bool whole = (run == 4 && type != "float") || (run == 1 && type == "float");
-      if (!whole) return "__builtin_nontemporal_store(" + val + ", (" + gq_ + type + "*)(" + addr + "));";
+    const bool whole = (run == 4 && type != "float") || (run == 1 && type == "float");
+    if (whole && (o_.nt || gq_.empty())) {
       const std::string op = type != "float" ? "global_store_dwordx4" : "global_store_dword";
-      return "asm volatile(\"" + op + " %0, %1, off sc1 nt\" :: \"v\"((" + gq_ + type + "*)(" + addr +
-             ")), \"v\"(" + val + ") : \"memory\");";
+      return "asm volatile(\"" + op + " %0, %1, off sc1" + (o_.nt ? " nt" : "") + "\" :: \"v\"((" + gq_ + type +
+             "*)(" + addr + ")), \"v\"(" + val + ") : \"memory\");";
     }
+    if (o_.nt) return "__builtin_nontemporal_store(" + val + ", (" + gq_ + type + "*)(" + addr + "));";
     return "*(" + gq_ + type + "*)(" + addr + ") = " + val + ";";
   }
 
@@ -1269,6 +1308,8 @@ class Emitter {
   std::map<int, std::string> in_group_;                 // gather node -> its row group
 };
 
+bool tiled_launch(const Dag &dag, const Options &o) { return Emitter(dag, o).tiled(); }
+
 // FAST mirrors -cl-unsafe-math-optimizations (OpenCL.scala:1131-1135): reassociation,
 // reciprocals, no signed zeros and contraction, but not finite-math-only, so infinities and
 // NaN keep their meaning (fmaxf/fminf still return the non-NaN operand).
@@ -1424,6 +1465,98 @@ BatchPlan plan_batch(const std::vector<BatchExpr> &members, int block, int math_
 
 }  // namespace
 
+// Compiles the kernel of `dag` under `o` into the device's cache (or takes the one another thread
+// has put there meanwhile); the caller gets a reference.
+static cs_fused *build_fused(cs_device *device, Dag dag, const Options &o, const std::string &key) {
+  int64_t vectors = 0;
+  const std::string name = kernel_name(key, o);
+  std::string src = Emitter(dag, o).generate(&vectors, name);
+  std::string log;
+  auto mod = std::make_shared<ModuleRef>();
+  mod->ordinal = device->ordinal;
+  mod->module = build_module(device, src, math_options(o.math_mode), &log);
+  std::unique_ptr<cs_fused> f(new cs_fused());
+  f->device = device;
+  f->key = key;
+  f->hash = fnv1a(key);
+  f->source = src;
+  f->module = mod;
+  CS_HIP(hipModuleGetFunction(&f->function, mod->module, name.c_str()));
+  f->nleaves = dag.nleaves;
+  int64_t total = 1;
+  for (auto d : dag.out_shape) total *= d;
+  f->out_elements = total * static_cast<int64_t>(dag.outputs.size());
+  f->vectors = vectors;
+  f->block = static_cast<uint32_t>(o.block);
+  f->max_block = launch_bound(dag, o);
+  int64_t per_block = int64_t(o.block) * o.U;
+  f->grid = static_cast<uint32_t>((vectors + per_block - 1) / per_block);
+  f->dag = std::move(dag);
+  f->opts = o;
+  std::lock_guard<std::recursive_mutex> l(device->mu);
+  auto it = device->fused_cache.find(key);
+  if (it != device->fused_cache.end()) {  // another thread won the race
+    it->second->refs++;
+    return it->second;
+  }
+  f->refs = 2;  // one for the cache, one for the caller
+  device->fused_cache.emplace(key, f.get());
+  return f.release();
+}
+
+// The kernel that a launch of `fused` into `out` runs: `fused` itself, or, where its rows are ragged
+// and the output lies over a leaf, the same expression at a width that divides the rows (compiled on
+// the first such launch, which may be under capture). Holds a reference while it lives.
+class LaunchKernel {
+ public:
+  LaunchKernel(cs_fused *fused, const void *const *leaves, const void *out) : f_(fused) {
+    if (!ragged_rows(fused->dag, fused->opts) || !over_leaf(fused, leaves, out)) {
+      f_->refs++;
+      return;
+    }
+    Options o = fused->opts;
+    const int64_t last = fused->dag.out_shape.back();
+    while (o.V > 1 && last % o.V != 0) o.V /= 2;
+    const std::string key = canonical_key(fused->dag, o);
+    cs_device *device = fused->device;
+    {
+      std::lock_guard<std::recursive_mutex> l(device->mu);
+      auto it = device->fused_cache.find(key);
+      if (it != device->fused_cache.end()) {
+        f_ = it->second;
+        f_->refs++;
+        return;
+      }
+    }
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    CS_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+    try {
+      f_ = build_fused(device, fused->dag, o, key);
+    } catch (...) {
+      (void)hipThreadExchangeStreamCaptureMode(&mode);
+      throw;
+    }
+    CS_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  }
+  ~LaunchKernel() { (void)cs_fused_release(f_); }
+  LaunchKernel(const LaunchKernel &) = delete;
+  LaunchKernel &operator=(const LaunchKernel &) = delete;
+  cs_fused *operator->() const { return f_; }
+
+ private:
+  static bool over_leaf(const cs_fused *f, const void *const *leaves, const void *out) {
+    const char *o = static_cast<const char *>(out);
+    for (int i = 0; i < f->nleaves; ++i) {
+      int64_t elements = 1;
+      for (auto d : f->dag.leaf_shape[static_cast<size_t>(i)]) elements *= d;
+      const char *p = static_cast<const char *>(leaves[i]);
+      if (o < p + 4 * elements && p < o + 4 * f->out_elements) return true;
+    }
+    return false;
+  }
+  cs_fused *f_;
+};
+
 static cs_status compile_fused(cs_device *device, const cs_node *nodes, int nnodes, const int32_t *outputs,
                                int noutputs, int out_rank, const int32_t *out_shape,
                                const cs_fused_options *options, bool sum, cs_fused **fused) {
@@ -1446,41 +1579,7 @@ static cs_status compile_fused(cs_device *device, const cs_node *nodes, int nnod
         return;
       }
     }
-    int64_t vectors = 0;
-    const std::string name = kernel_name(key, o);
-    std::string src = Emitter(dag, o).generate(&vectors, name);
-    std::string log;
-    auto mod = std::make_shared<ModuleRef>();
-    mod->ordinal = device->ordinal;
-    mod->module = build_module(device, src, math_options(o.math_mode), &log);
-    std::unique_ptr<cs_fused> f(new cs_fused());
-    f->device = device;
-    f->key = key;
-    f->hash = fnv1a(key);
-    f->source = src;
-    f->module = mod;
-    CS_HIP(hipModuleGetFunction(&f->function, mod->module, name.c_str()));
-    f->nleaves = dag.nleaves;
-    int64_t total = 1;
-    for (auto d : dag.out_shape) total *= d;
-    f->out_elements = total * static_cast<int64_t>(dag.outputs.size());
-    f->vectors = vectors;
-    f->block = static_cast<uint32_t>(o.block);
-    f->max_block = launch_bound(dag, o);
-    int64_t per_block = int64_t(o.block) * o.U;
-    f->grid = static_cast<uint32_t>((vectors + per_block - 1) / per_block);
-    f->dag = std::move(dag);
-    f->opts = o;
-    std::lock_guard<std::recursive_mutex> l(device->mu);
-    auto it = device->fused_cache.find(key);
-    if (it != device->fused_cache.end()) {  // another thread won the race
-      it->second->refs++;
-      *fused = it->second;
-      return;
-    }
-    f->refs = 2;  // one for the cache, one for the caller
-    device->fused_cache.emplace(key, f.get());
-    *fused = f.release();
+    *fused = build_fused(device, std::move(dag), o, key);
   });
 }
 
@@ -1728,9 +1827,7 @@ cs_status cs_fused_launch_block(cs_stream *stream, cs_fused *fused, const void *
     if (nleaves != fused->nleaves)
       fail(CS_INVALID_KERNEL_ARGS, "kernel takes " + std::to_string(fused->nleaves) + " leaves, got " +
                                        std::to_string(nleaves));
-    int64_t per_block = int64_t(block) * fused->opts.U;
-    uint32_t grid = static_cast<uint32_t>((fused->vectors + per_block - 1) / per_block);
-    if (grid == 0) return;
+    if (fused->grid == 0) return;
     if (!out) fail(CS_INVALID_KERNEL_ARGS, "output pointer is null");
     std::vector<const void *> vals(static_cast<size_t>(nleaves) + 1);
     std::vector<void *> args(static_cast<size_t>(nleaves) + 1);
@@ -1742,7 +1839,10 @@ cs_status cs_fused_launch_block(cs_stream *stream, cs_fused *fused, const void *
     vals[nleaves] = out;
     args[nleaves] = &vals[nleaves];
     set_device(stream->device);
-    CS_HIP(hipModuleLaunchKernel(fused->function, grid, 1, 1, static_cast<uint32_t>(block), 1, 1, 0,
+    const LaunchKernel k(fused, leaves, out);
+    const int64_t per_block = int64_t(block) * k->opts.U;
+    const uint32_t grid = static_cast<uint32_t>((k->vectors + per_block - 1) / per_block);
+    CS_HIP(hipModuleLaunchKernel(k->function, grid, 1, 1, static_cast<uint32_t>(block), 1, 1, 0,
                                  stream->stream, args.data(), nullptr));
   });
 }
@@ -1803,7 +1903,8 @@ cs_status cs_fused_launch(cs_stream *stream, cs_fused *fused, const void *const 
     vals[nleaves] = out;
     args[nleaves] = &vals[nleaves];
     set_device(stream->device);
-    CS_HIP(hipModuleLaunchKernel(fused->function, fused->grid, 1, 1, fused->block, 1, 1, 0,
+    const LaunchKernel k(fused, leaves, out);
+    CS_HIP(hipModuleLaunchKernel(k->function, k->grid, 1, 1, k->block, 1, 1, 0,
                                  stream->stream, args.data(), nullptr));
   });
 }
@@ -1829,13 +1930,14 @@ cs_status cs_fused_launch_timed(cs_stream *stream, cs_fused *fused, const void *
     vals[nleaves] = out;
     args[nleaves] = &vals[nleaves];
     set_device(stream->device);
+    const LaunchKernel k(fused, leaves, out);
     hipEvent_t ea = nullptr, eb = nullptr;
     hipError_t r = hipEventCreate(&ea);
     if (r == hipSuccess) r = hipEventCreate(&eb);
     // hipExtModuleLaunchKernel takes the grid in work items; the events carry the
     // dispatch's own start and end
     if (r == hipSuccess)
-      r = hipExtModuleLaunchKernel(fused->function, fused->grid * fused->block, 1, 1, fused->block, 1, 1, 0,
+      r = hipExtModuleLaunchKernel(k->function, k->grid * k->block, 1, 1, k->block, 1, 1, 0,
                                    stream->stream, args.data(), nullptr, ea, eb, 0);
     if (r != hipSuccess) {
       if (ea) (void)hipEventDestroy(ea);

@@ -75,6 +75,22 @@ def test_stores_stay_inside(items, block):
             t.release()
 
 
+@pytest.mark.parametrize("hw", [(3, 5), (257, 7), (64, 1021), (1, 1000003)])
+def test_result_over_a_leaf(hw):
+    """The output in the memory of a leaf that is read at its own place."""
+    with Tensors(0) as T:
+        a, b = _leaf(T, hw, 1).doCache(), _leaf(T, hw, 2).doCache()
+        e = a * b + a
+        want = e.flatArray()
+        f, leaves, _ = T.compile(e.closure, e.shape)
+        ptrs = (ctypes.c_void_p * len(leaves))(*[leaf.id.buffer.ptr for leaf in leaves])
+        capi.check(capi.lib.cs_fused_launch(T.stream, f, ptrs, len(leaves), a.buffer.ptr))
+        assert np.array_equal(a.flatArray().view(np.uint32), want.view(np.uint32))
+        capi.lib.cs_fused_release(f)
+        for t in (a, b):
+            t.release()
+
+
 def test_in_a_batch():
     """The same kernels as members of a persistent batch."""
     with Tensors(0) as T:

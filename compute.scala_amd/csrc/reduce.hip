@@ -160,10 +160,18 @@ __global__ __launch_bounds__(kFinish) void finish_max_kernel(const float *__rest
   }
 }
 
+// A pass of a single workgroup writes its result itself, as the combine of one partial would.
+__device__ __forceinline__ void write_total(double total, float *out, double *out64) {
+  if (out) *out = float(total);
+  if (out64) *out64 = total;
+}
+
 // ----------------------------------------------------------------------------- full sum/max
+// With one workgroup *out and *out64 get the result, else each workgroup its partial.
 template <bool kMax>
 __global__ __launch_bounds__(kBlock) void reduce_all_kernel(const float *__restrict__ in, int64_t n,
-                                                            double *partial64, float *partialmax) {
+                                                            double *partial64, float *partialmax, float *out,
+                                                            double *out64) {
   Acc a;
   float m = __builtin_nanf("");
   const int64_t nvec = ((reinterpret_cast<uintptr_t>(in) & 15) == 0) ? n / 4 : 0;
@@ -198,8 +206,14 @@ __global__ __launch_bounds__(kBlock) void reduce_all_kernel(const float *__restr
   }
   block_reduce(a, m);
   if (threadIdx.x == 0) {
-    if (kMax) partialmax[blockIdx.x] = m;
-    else partial64[blockIdx.x] = a.result64();
+    if (gridDim.x == 1) {
+      if (kMax) *out = m;
+      else write_total(a.result64(), out, out64);
+    } else if (kMax) {
+      partialmax[blockIdx.x] = m;
+    } else {
+      partial64[blockIdx.x] = a.result64();
+    }
   }
 }
 
@@ -270,7 +284,8 @@ __device__ __forceinline__ void read_row(const float *__restrict__ p, int64_t co
 // partial of the row for the total.
 template <int kThreads>
 __global__ __launch_bounds__(kThreads) void reduce_rows_kernel(const float *__restrict__ in, int64_t cols,
-                                                               float *row_sum, float *row_max, double *partial64) {
+                                                               float *row_sum, float *row_max, double *partial64,
+                                                               float *total, double *total64) {
   const int64_t row = blockIdx.x;
   Acc a;
   float m = __builtin_nanf("");
@@ -279,7 +294,8 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_kernel(const float *__re
   if (threadIdx.x == 0) {
     if (row_sum) row_sum[row] = a.result();
     if (row_max) row_max[row] = m;
-    if (partial64) partial64[row] = a.result64();
+    if (partial64 && gridDim.x == 1) write_total(a.result64(), total, total64);
+    else if (partial64) partial64[row] = a.result64();
   }
 }
 
@@ -291,10 +307,11 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_kernel(const float *__re
 template <int kG>
 __global__ __launch_bounds__(kBlock) void reduce_short_rows_kernel(const float *__restrict__ in, int64_t rows,
                                                                    int64_t cols, int tiles, float *row_sum,
-                                                                   float *row_max, double *partial64) {
+                                                                   float *row_max, double *partial64, float *total,
+                                                                   double *total64) {
   __shared__ double lw[kWaves];
   const int lane = threadIdx.x % kG, group = threadIdx.x / kG;
-  double total = 0.0;  // of this lane's rows
+  double sum = 0.0;  // of this lane's rows
   for (int t = 0; t < tiles; ++t) {
     const int64_t row = (int64_t(blockIdx.x) * tiles + t) * (kBlock / kG) + group;
     Acc a;
@@ -309,19 +326,20 @@ __global__ __launch_bounds__(kBlock) void reduce_short_rows_kernel(const float *
     if (lane == 0 && row < rows) {
       if (row_sum) row_sum[row] = a.result();
       if (row_max) row_max[row] = m;
-      total += a.result64();
+      sum += a.result64();
     }
   }
   if (!partial64) return;
 #pragma unroll
-  for (int off = 32; off >= kG; off >>= 1) total += __shfl_xor(total, off, 64);  // lane 0 of each row group holds a value
-  if ((threadIdx.x & 63) == 0) lw[threadIdx.x >> 6] = total;
+  for (int off = 32; off >= kG; off >>= 1) sum += __shfl_xor(sum, off, 64);  // lane 0 of each row group holds a value
+  if ((threadIdx.x & 63) == 0) lw[threadIdx.x >> 6] = sum;
   __syncthreads();
   if (threadIdx.x == 0) {
     double s = lw[0];
 #pragma unroll
     for (int w = 1; w < kWaves; ++w) s += lw[w];
-    partial64[blockIdx.x] = s;
+    if (gridDim.x == 1) write_total(s, total, total64);
+    else partial64[blockIdx.x] = s;
   }
 }
 
@@ -531,30 +549,31 @@ RowPlan plan_rows(cs_stream *stream, int64_t rows, int64_t cols) {
 
 template <int kG>
 void launch_short_rows(cs_stream *stream, const RowPlan &p, const float *in, int64_t rows, int64_t cols,
-                       float *row_sum, float *row_max, double *partial64) {
+                       float *row_sum, float *row_max, double *partial64, float *total, double *total64) {
   hipLaunchKernelGGL(reduce_short_rows_kernel<kG>, dim3(static_cast<unsigned>(p.grid)), dim3(kBlock), 0,
-                     stream->stream, in, rows, cols, p.tiles, row_sum, row_max, partial64);
+                     stream->stream, in, rows, cols, p.tiles, row_sum, row_max, partial64, total, total64);
 }
 
-// The row pass of a plan and, when partial64 is not null, the combine of its plan.grid partials.
+// The row pass of a plan and, when partial64 is not null, the combine of its plan.grid partials (one
+// workgroup writes the total itself).
 void launch_rows(cs_stream *stream, const RowPlan &p, const float *in, int64_t rows, int64_t cols, float *row_sum,
                  float *row_max, double *partial64, float *total, double *total64) {
   switch (p.lanes) {
-    case 2: launch_short_rows<2>(stream, p, in, rows, cols, row_sum, row_max, partial64); break;
-    case 4: launch_short_rows<4>(stream, p, in, rows, cols, row_sum, row_max, partial64); break;
-    case 8: launch_short_rows<8>(stream, p, in, rows, cols, row_sum, row_max, partial64); break;
-    case 16: launch_short_rows<16>(stream, p, in, rows, cols, row_sum, row_max, partial64); break;
-    case 32: launch_short_rows<32>(stream, p, in, rows, cols, row_sum, row_max, partial64); break;
-    case 64: launch_short_rows<64>(stream, p, in, rows, cols, row_sum, row_max, partial64); break;
+    case 2: launch_short_rows<2>(stream, p, in, rows, cols, row_sum, row_max, partial64, total, total64); break;
+    case 4: launch_short_rows<4>(stream, p, in, rows, cols, row_sum, row_max, partial64, total, total64); break;
+    case 8: launch_short_rows<8>(stream, p, in, rows, cols, row_sum, row_max, partial64, total, total64); break;
+    case 16: launch_short_rows<16>(stream, p, in, rows, cols, row_sum, row_max, partial64, total, total64); break;
+    case 32: launch_short_rows<32>(stream, p, in, rows, cols, row_sum, row_max, partial64, total, total64); break;
+    case 64: launch_short_rows<64>(stream, p, in, rows, cols, row_sum, row_max, partial64, total, total64); break;
     default:
       if (p.wide)
         hipLaunchKernelGGL(reduce_rows_kernel<1024>, dim3(static_cast<unsigned>(p.grid)), dim3(1024), 0,
-                           stream->stream, in, cols, row_sum, row_max, partial64);
+                           stream->stream, in, cols, row_sum, row_max, partial64, total, total64);
       else
         hipLaunchKernelGGL(reduce_rows_kernel<kBlock>, dim3(static_cast<unsigned>(p.grid)), dim3(kBlock), 0,
-                           stream->stream, in, cols, row_sum, row_max, partial64);
+                           stream->stream, in, cols, row_sum, row_max, partial64, total, total64);
   }
-  if (partial64) launch_finish_sum(stream, partial64, p.grid, total, total64);
+  if (partial64 && p.grid > 1) launch_finish_sum(stream, partial64, p.grid, total, total64);
 }
 }  // namespace
 
@@ -624,9 +643,8 @@ cs_status cs_reduce_sum(cs_stream *stream, const float *in, int64_t n, float *ou
     int grid = reduce_grid(stream, n);
     ReduceScratch s = scratch_for(stream, static_cast<size_t>(grid));
     hipLaunchKernelGGL(reduce_all_kernel<false>, dim3(grid), dim3(kBlock), 0, stream->stream, in, n,
-                       s.partial64, s.partialmax);
-    hipLaunchKernelGGL(finish_sum_kernel, dim3(1), dim3(kFinish), 0, stream->stream, s.partial64,
-                       int64_t(grid), out, out64);
+                       s.partial64, s.partialmax, out, out64);
+    if (grid > 1) launch_finish_sum(stream, s.partial64, grid, out, out64);
     CS_HIP(hipGetLastError());
   });
 }
@@ -641,9 +659,10 @@ cs_status cs_reduce_max(cs_stream *stream, const float *in, int64_t n, float *ou
     int grid = reduce_grid(stream, n);
     ReduceScratch s = scratch_for(stream, static_cast<size_t>(grid));
     hipLaunchKernelGGL(reduce_all_kernel<true>, dim3(grid), dim3(kBlock), 0, stream->stream, in, n,
-                       s.partial64, s.partialmax);
-    hipLaunchKernelGGL(finish_max_kernel, dim3(1), dim3(kFinish), 0, stream->stream, s.partialmax,
-                       int64_t(grid), out);
+                       s.partial64, s.partialmax, out, static_cast<double *>(nullptr));
+    if (grid > 1)
+      hipLaunchKernelGGL(finish_max_kernel, dim3(1), dim3(kFinish), 0, stream->stream, s.partialmax,
+                         int64_t(grid), out);
     CS_HIP(hipGetLastError());
   });
 }

@@ -58,18 +58,20 @@ class PendingBuffer(object):
 
     __slots__ = ("tensors", "handle", "ptr", "nbytes", "_released")
 
-    def __init__(self, tensors, handle, nbytes):
+    def __init__(self, tensors, handle, nbytes, ptr=None):
         self.tensors = tensors
         self.handle = handle
-        p = ctypes.c_void_p()
-        check(lib.cs_buffer_device_ptr(handle, ctypes.byref(p)), "cs_buffer_device_ptr")
-        self.ptr = p.value
+        if ptr is None:
+            p = ctypes.c_void_p()
+            check(lib.cs_buffer_device_ptr(handle, ctypes.byref(p)), "cs_buffer_device_ptr")
+            ptr = p.value
+        self.ptr = ptr
         self.nbytes = nbytes
         self._released = False
 
     def retain(self):
         check(lib.cs_buffer_retain(self.handle), "cs_buffer_retain")
-        return PendingBuffer(self.tensors, self.handle, self.nbytes)
+        return PendingBuffer(self.tensors, self.handle, self.nbytes, self.ptr)
 
     def release(self):
         if self._released:
@@ -81,7 +83,7 @@ class PendingBuffer(object):
         out = np.empty(count, dtype=np.float32)
         if count:
             check(lib.cs_buffer_read(self.tensors._stream, self.handle, 0,
-                                     out.ctypes.data_as(ctypes.c_void_p), count * 4), "cs_buffer_read")
+                                     out.__array_interface__["data"][0], count * 4), "cs_buffer_read")
         return out
 
     def __enter__(self):
@@ -954,6 +956,8 @@ class Tensors(object):
         """autoBroadcast / autoBroadcastShape (Tensors.scala:202-222): leading dimensions
         align."""
         s1, s2 = a.shape, b.shape
+        if s1 == s2:
+            return a, b
         shape = []
         for i in range(max(len(s1), len(s2))):
             if i >= len(s1) or s1[i] == 1:

@@ -9,6 +9,7 @@ shares the computation (the export memo of Trees.scala:220 works by identity).
 by first visit in depth-first, left-to-right order, which is both the alpha conversion
 (Trees.scala:807-822) and the kernel argument order (Tensors.scala:230-251).
 """
+import ctypes
 import struct
 
 from . import _capi as capi
@@ -136,83 +137,85 @@ def parameters(tree):
     return out
 
 
+_NODE_BYTES = ctypes.sizeof(capi.CsNode)
+_SHAPE_AT = capi.CsNode.shape.offset
+_MATRIX_AT = capi.CsNode.matrix.offset
+_HEAD = struct.Struct("=4ifi")  # op, a, b, param, value, rank
+_INTS = [struct.Struct("=%di" % k) for k in range(capi.MAX_RANK + 1)]
+_DOUBLES = [struct.Struct("=%dd" % k) for k in range(capi.MAX_RANK * (capi.MAX_RANK + 1) + 1)]
+
+
 def serialize(tree):
     """Returns (nodes, outputs, leaves): a ctypes array of CsNode, the output node indices
     and the ArrayParameter leaves in slot order."""
-    index = {}
-    records = []
-    leaves = []
+    index = {}  # id of a node -> its record
+    records = []  # nodes, operands before their users
+    leaves = []  # numbered by first visit, depth first
     roots = tree.elements if isinstance(tree, Concatenate) else (tree,)
-
-    def visit(root):
-        # Iterative: pre-order numbers the leaves, post-order emits the nodes.
-        stack = [(root, False)]
-        while stack:
-            node, done = stack.pop()
-            key = id(node)
-            if key in index:
-                continue
-            if not done:
-                if isinstance(node, ArrayParameter):
-                    leaves.append(node)
-                    slot = len(leaves) - 1
-                    index[key] = len(records)
-                    records.append(("param", node, slot))
-                    continue
-                stack.append((node, True))
-                for child in reversed(node.children()):
-                    if id(child) not in index:
-                        stack.append((child, False))
-                continue
-            index[key] = len(records)
-            records.append(("node", node, None))
-
     for r in roots:
         if isinstance(r, Concatenate):
             raise ValueError("nested tuples are not supported")
-        visit(r)
+        # Iterative: a node is met once before its operands and once after them.
+        stack = [r]
+        opened = set()
+        while stack:
+            node = stack[-1]
+            key = id(node)
+            if key in index:
+                stack.pop()
+                continue
+            cls = type(node)
+            if cls is ArrayParameter:
+                leaves.append(node)
+            elif key not in opened:
+                opened.add(key)
+                if cls is Binary:
+                    if id(node.rhs) not in index:
+                        stack.append(node.rhs)
+                    if id(node.lhs) not in index:
+                        stack.append(node.lhs)
+                else:
+                    for c in node.children():  # at most one: a tuple's elements are roots
+                        if id(c) not in index:
+                            stack.append(c)
+                continue
+            stack.pop()
+            index[key] = len(records)
+            records.append(node)
 
-    nodes = (capi.CsNode * len(records))()
-    for i, (kind, node, slot) in enumerate(records):
-        n = nodes[i]
-        n.a = n.b = -1
-        if kind == "param":
-            n.op = capi.OP_PARAMETER
-            n.param = slot
-            n.value = node.padding
-            n.rank = len(node.shape)
-            if n.rank > capi.MAX_RANK:
-                raise ValueError("rank %d exceeds %d" % (n.rank, capi.MAX_RANK))
-            for d, s in enumerate(node.shape):
-                n.shape[d] = s
-        elif isinstance(node, FloatLiteral):
-            n.op = capi.OP_LITERAL
-            n.value = node.value
-        elif isinstance(node, Transform):
-            n.op = capi.OP_TRANSFORM
-            n.a = index[id(node.array)]
-            n.rank = node.rank
+    data = bytearray(_NODE_BYTES * len(records))
+    pack = _HEAD.pack_into
+    slot = 0
+    at = 0
+    for node in records:
+        cls = type(node)
+        if cls is Binary:
+            pack(data, at, BINARY[node.op], index[id(node.lhs)], index[id(node.rhs)], 0, 0.0, 0)
+        elif cls is Unary:
+            pack(data, at, UNARY[node.op], index[id(node.operand)], -1, 0, 0.0, 0)
+        elif cls is Extract:
+            pack(data, at, capi.OP_EXTRACT, index[id(node.array)], -1, 0, 0.0, 0)
+        elif cls is Transform:
             if node.rank > capi.MAX_RANK:
                 raise ValueError("rank %d exceeds %d" % (node.rank, capi.MAX_RANK))
-            for j, m in enumerate(node.matrix):
-                n.matrix[j] = m
-        elif isinstance(node, Fill):
-            n.op = capi.OP_FILL
-            n.a = index[id(node.element)]
-        elif isinstance(node, Extract):
-            n.op = capi.OP_EXTRACT
-            n.a = index[id(node.array)]
-        elif isinstance(node, Unary):
-            n.op = UNARY[node.op]
-            n.a = index[id(node.operand)]
-        elif isinstance(node, Binary):
-            n.op = BINARY[node.op]
-            n.a = index[id(node.lhs)]
-            n.b = index[id(node.rhs)]
+            pack(data, at, capi.OP_TRANSFORM, index[id(node.array)], -1, 0, 0.0, node.rank)
+            _DOUBLES[len(node.matrix)].pack_into(data, at + _MATRIX_AT, *node.matrix)
+        elif cls is ArrayParameter:
+            rank = len(node.shape)
+            if rank > capi.MAX_RANK:
+                raise ValueError("rank %d exceeds %d" % (rank, capi.MAX_RANK))
+            pack(data, at, capi.OP_PARAMETER, -1, -1, slot, node.padding, rank)
+            _INTS[rank].pack_into(data, at + _SHAPE_AT, *node.shape)
+            slot += 1
+        elif cls is FloatLiteral:
+            pack(data, at, capi.OP_LITERAL, -1, -1, 0, node.value, 0)
+        elif cls is Fill:
+            pack(data, at, capi.OP_FILL, index[id(node.element)], -1, 0, 0.0, 0)
         else:
             raise TypeError("cannot serialize %r" % (node,))
-    outputs = [index[id(r)] for r in roots]
-    return nodes, outputs, leaves
+        at += _NODE_BYTES
+    nodes = (capi.CsNode * len(records)).from_buffer(data)
+    return nodes, [index[id(r)] for r in roots], leaves
 
 
 def structural_key(tree):

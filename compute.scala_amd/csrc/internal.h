@@ -66,7 +66,8 @@ struct Slab {
   size_t in_use = 0;
 };
 
-// An event recorded on a stream (nullptr: the null stream) when a block was released.
+// An event recorded on a stream (nullptr: the null stream) when a block was released; without an
+// event, the block is free once all work queued on the stream by then is done.
 struct StreamEvent {
   hipStream_t stream;
   hipEvent_t event;

@@ -4,7 +4,8 @@
 // product and join that unrolls into one elementwise kernel (README.md:301-362,
 // TensorsSpec.scala:468-528), so every output is a sequential FP32 dot product. Here:
 //
-//   CS_GEMM_FP32    FP32 operands on v_mfma_f32_32x32x2_f32 (FP32 products and sums)
+//   CS_GEMM_FP32    FP32 operands: on the FP32 MFMA where the product is small, and from three BF16
+//                   parts of each operand, exact together, where it is large (gemm_split_kernel)
 //   CS_GEMM_BF16    operands rounded to BF16, v_mfma_f32_32x32x16_bf16, FP32 accumulate
 //   CS_GEMM_BF16X3  split-BF16x3 (Henry, Tang & Heinecke 2019): A = Ah + Al, B = Bh + Bl
 //                   with Ah = bf16(A), Al = bf16(A - Ah); C = Al.Bh + Ah.Bl + Ah.Bh, all
@@ -29,6 +30,7 @@
 // (the lanes the LDS serves in one cycle) hit 16 different bank groups.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <type_traits>
@@ -808,15 +810,13 @@ __device__ __forceinline__ void direct_mma(const DirectFrags<KIND, T> &f, f32x4 
   }
 }
 
-template <int KIND, int T, int kWK>
-__global__ __launch_bounds__(kWK == 1 ? 256 : 64 * kWK) void gemm_direct_kernel(
-    int M, int N, int K, const float *__restrict__ A, int lda, const float *__restrict__ B, int ldb,
-    float *__restrict__ C, int ldc, int tiles_m) {
+// The sums of K steps first, first + stride, ... of the tile at (m0, n0).
+template <int KIND, int T>
+__device__ __forceinline__ void direct_tile(int M, int N, int K, const float *__restrict__ A, int lda,
+                                            const float *__restrict__ B, int ldb, int m0, int n0, int lane, int first,
+                                            int stride, f32x4 (&acc)[T][T]) {
   constexpr int kVals = kDirectVals<KIND>, kStep = 4 * kVals;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4;
-  const int tm = int(blockIdx.x) % tiles_m, tn = int(blockIdx.x) / tiles_m;
-  const int m0 = (kWK == 1 ? tm * 4 + wave : tm) * 16 * T, n0 = tn * 16 * T;
+  const int l16 = lane & 15, quad = lane >> 4;
   const int nb = n0 + T * l16;  // this lane's T columns
   const bool inside = nb + T <= N;
   const float *arow[T];  // rows past the end repeat the last one: their results are not stored
@@ -870,56 +870,76 @@ __global__ __launch_bounds__(kWK == 1 ? 256 : 64 * kWK) void gemm_direct_kernel(
     CSMI_SCHED_FENCE();  // the loads go out before the MFMAs of the step before
   };
 
-  f32x4 acc[T][T];
 #pragma unroll
   for (int i = 0; i < T; ++i)
 #pragma unroll
     for (int j = 0; j < T; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   const int steps = (K + kStep - 1) / kStep;
-  int step = kWK == 1 ? 0 : wave;
+  int step = first;
   if (step < steps) {
     DirectFrags<KIND, T> f[2];
     load(step, f[0]);
     for (;;) {
-      if (step + kWK >= steps) {
+      if (step + stride >= steps) {
         direct_mma<KIND, T>(f[0], acc);
         break;
       }
-      load(step + kWK, f[1]);
+      load(step + stride, f[1]);
       direct_mma<KIND, T>(f[0], acc);
-      step += kWK;
-      if (step + kWK >= steps) {
+      step += stride;
+      if (step + stride >= steps) {
         direct_mma<KIND, T>(f[1], acc);
         break;
       }
-      load(step + kWK, f[0]);
+      load(step + stride, f[0]);
       direct_mma<KIND, T>(f[1], acc);
-      step += kWK;
+      step += stride;
     }
   }
 
-  // acc[i][j][e] is row m0 + 16 i + 4 quad + e, column nb + j
-  auto store = [&](int row, int col, const float (&v)[T]) {
-    if (row >= M) return;
-    float *c = C + int64_t(row) * ldc + col;
-    if (T == 4 && col + 4 <= N) {
-      *reinterpret_cast<f4u *>(c) = f4u{v[0], v[1 % T], v[2 % T], v[3 % T]};
-      return;
+}
+
+// acc[i][j][e] of a direct tile is row m0 + 16 i + 4 quad + e, column n0 + T l16 + j.
+template <int T>
+__device__ __forceinline__ void store_run(int M, int N, float *__restrict__ C, int ldc, int row, int col,
+                                          const float (&v)[T]) {
+  if (row >= M) return;
+  float *c = C + int64_t(row) * ldc + col;
+  if (T == 4 && col + 4 <= N) {
+    *reinterpret_cast<f4u *>(c) = f4u{v[0], v[1 % T], v[2 % T], v[3 % T]};
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < T; ++j)
+    if (col + j < N) c[j] = v[j];
+}
+
+template <int T>
+__device__ __forceinline__ void store_tile(int M, int N, float *__restrict__ C, int ldc, int m0, int n0, int lane,
+                                           const f32x4 (&acc)[T][T]) {
+#pragma unroll
+  for (int i = 0; i < T; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float v[T];
+#pragma unroll
+      for (int j = 0; j < T; ++j) v[j] = acc[i][j][e];
+      store_run<T>(M, N, C, ldc, m0 + 16 * i + 4 * (lane >> 4) + e, n0 + T * (lane & 15), v);
     }
-#pragma unroll
-    for (int j = 0; j < T; ++j)
-      if (col + j < N) c[j] = v[j];
-  };
+}
+
+template <int KIND, int T, int kWK>
+__global__ __launch_bounds__(kWK == 1 ? 256 : 64 * kWK) void gemm_direct_kernel(
+    int M, int N, int K, const float *__restrict__ A, int lda, const float *__restrict__ B, int ldb,
+    float *__restrict__ C, int ldc, int tiles_m) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int tm = int(blockIdx.x) % tiles_m, tn = int(blockIdx.x) / tiles_m;
+  const int m0 = (kWK == 1 ? tm * 4 + wave : tm) * 16 * T, n0 = tn * 16 * T;
+  f32x4 acc[T][T];
+  direct_tile<KIND, T>(M, N, K, A, lda, B, ldb, m0, n0, lane, kWK == 1 ? 0 : wave, kWK, acc);
   if constexpr (kWK == 1) {
-#pragma unroll
-    for (int i = 0; i < T; ++i)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float v[T];
-#pragma unroll
-        for (int j = 0; j < T; ++j) v[j] = acc[i][j][e];
-        store(m0 + 16 * i + 4 * quad + e, nb, v);
-      }
+    store_tile<T>(M, N, C, ldc, m0, n0, lane, acc);
   } else {
     // part[wave][(i, e, j)][lane]
     extern __shared__ float part[];
@@ -938,9 +958,256 @@ __global__ __launch_bounds__(kWK == 1 ? 256 : 64 * kWK) void gemm_direct_kernel(
       for (int w = 1; w < kWK; ++w)
 #pragma unroll
         for (int j = 0; j < T; ++j) v[j] += part[((w * kRuns + run) * T + j) * 64 + lane];
-      store(m0 + 16 * (run / 4) + 4 * quad + run % 4, nb, v);
+      store_run<T>(M, N, C, ldc, m0 + 16 * (run / 4) + 4 * (lane >> 4) + run % 4, n0 + T * (lane & 15), v);
     }
   }
+}
+
+// ------------------------------------------------------------------------ FP32 from three parts
+// Large FP32 products on the BF16 matrix cores, which do 16 times the FP32 ones' work per cycle. A
+// 24-bit significand is exactly three 8-bit ones, x = h + m + l (each the BF16 nearest to what is
+// left; Henry, Tang & Heinecke 2019), and of the nine products the six of hh, hm, mh, mm, hl and lh
+// are summed in FP32: what the others would add is below 2^-25 of |a||b|, half an FP32 rounding of
+// one product. The error against FP64 is that of the FP32 matrix cores or less, since 16 products
+// meet in one rounding instead of two: relative to |C|, U(-1,1), K = 16 3.2e-8 / 7.4e-8, 256
+// 2.3e-7 / 2.9e-7, 1024 4.8e-7 / 5.7e-7, 4096 1.0e-6 / 1.1e-6.
+// The split is exact, and the products' sums are FP32's, only in a range: not for infinities and
+// NaN, values that round to an infinite BF16, parts below BF16's normal range and products near
+// FP32's. The pre-pass keeps the least exponent of each of its pieces of A and B (0 for values out of
+// range), and a tile of C whose rows or columns leave the range is computed from A and B on the FP32
+// matrix cores (direct_tile).
+constexpr int kSplitK = 16;                        // K values of a stage
+constexpr int kPartB = kTile * kSplitK * 2;        // one part of an operand's stage: 8 KiB
+constexpr int kSplitPanelB = 3 * kPartB;           // h, m, l
+constexpr int kSplitStageB = 2 * kSplitPanelB;     // both operands: 48 KiB
+constexpr size_t kSplitLds = size_t(3) * kSplitStageB;  // three stages: 144 KiB
+// Least exponents (biased) of the operands, and of a product of both, that stay on the BF16 path.
+constexpr unsigned kMinExponent = 24, kMinProduct = 254 - 110;
+
+struct SplitArgs {
+  const float *a, *b;
+  int m, n, k, lda, ldb, mp, np, kp, vec_a;
+  char *x, *y;         // [kp / 16][3][mp or np][16] BF16
+  uint8_t *ea, *eb;    // least exponents: [mp / 256][chunks][4] and [np / 256][chunks][4], chunks of 64 K
+  unsigned row_blocks;
+};
+
+// Splits 16 consecutive K values of one row of an operand, stores them and returns their least
+// exponent: 255 for zeros, 0 for a value out of range.
+__device__ __forceinline__ unsigned split_store(const float (&v)[16], char *dst, int64_t part_stride) {
+  unsigned least = 255;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const uint32_t bits = __float_as_uint(v[e]) & 0x7fffffffu;
+    const unsigned x = bits >= 0x7f7f8000u ? 0u : bits == 0 ? 255u : bits >> 23;
+    least = min(least, x);
+  }
+  float r[16];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) r[e] = v[e];
+#pragma unroll
+  for (int part = 0; part < 3; ++part) {
+    i32x4 w[2];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t h = bf16x2(r[2 * e], r[2 * e + 1]);
+      w[e / 4][e % 4] = int(h);
+      r[2 * e] -= __uint_as_float(h << 16);
+      r[2 * e + 1] -= __uint_as_float(h & 0xffff0000u);
+    }
+    *reinterpret_cast<i32x4 *>(dst + part * part_stride) = w[0];
+    *reinterpret_cast<i32x4 *>(dst + part * part_stride + 16) = w[1];
+  }
+  return least;
+}
+
+// Workgroups [0, row_blocks) split 64 rows x 64 K of A (a thread per 16 K of a row), the others 64
+// columns x 64 K of B (a thread per 16 K of a column: each load of a wave is 256 contiguous bytes).
+// Rows, columns and K values past the source are zeros.
+__global__ __launch_bounds__(256) void split_operands_kernel(SplitArgs p) {
+  __shared__ unsigned least;
+  const int t = threadIdx.x;
+  if (t == 0) least = 255;
+  __syncthreads();
+  const unsigned chunks = unsigned(p.kp + 63) / 64;
+  const bool is_a = blockIdx.x < p.row_blocks;
+  const unsigned block = is_a ? blockIdx.x : blockIdx.x - p.row_blocks;
+  const unsigned strip = is_a ? block / chunks : block % unsigned(p.np / 64);
+  const unsigned chunk = is_a ? block % chunks : block / unsigned(p.np / 64);
+  const int row = int(strip) * 64 + (is_a ? t / 4 : t % 64), k = int(chunk) * 64 + 16 * (is_a ? t % 4 : t / 64);
+  if (k < p.kp) {
+    float v[16];
+    if (is_a) {
+      const float *src = p.a + int64_t(row) * p.lda + k;
+      if (p.vec_a && row < p.m && k + 16 <= p.k) {
+#pragma unroll
+        for (int e = 0; e < 16; e += 4) {
+          const float4 x = *reinterpret_cast<const float4 *>(src + e);
+          v[e] = x.x, v[e + 1] = x.y, v[e + 2] = x.z, v[e + 3] = x.w;
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = row < p.m && k + e < p.k ? src[e] : 0.0f;
+      }
+    } else {
+      const float *src = p.b + int64_t(k) * p.ldb + row;
+      if (row < p.n && k + 16 <= p.k) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = src[int64_t(e) * p.ldb];
+      } else {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = row < p.n && k + e < p.k ? src[int64_t(e) * p.ldb] : 0.0f;
+      }
+    }
+    const int64_t part_stride = int64_t(is_a ? p.mp : p.np) * 32;
+    char *dst = (is_a ? p.x : p.y) + int64_t(k / 16) * 3 * part_stride + int64_t(row) * 32;
+    const unsigned e = split_store(v, dst, part_stride);
+    if (e < 255) atomicMin(&least, e);
+  }
+  __syncthreads();
+  if (t == 0)
+    (is_a ? p.ea : p.eb)[(int64_t(strip / 4) * chunks + chunk) * 4 + strip % 4] = static_cast<uint8_t>(least);
+}
+
+// 256 threads (4 waves in 2x2) per 256 x 256 tile, each wave 128 x 128 as 4 x 4 MFMA tiles, as in
+// gemm_lds_kernel. A stage is 16 K values: 96 MFMAs per wave, in six groups of 16 that use every
+// accumulator once. Three stages live in LDS: while stage s computes, the fragments of s + 1 replace
+// those of s as their last group has issued, and stage s + 2 streams into the buffer of s - 1. The
+// operands are packed so that each part of a stage is 8 KiB in a row: DMA and fragment reads are
+// linear in LDS, without bank conflicts.
+__global__ __launch_bounds__(kThreads, 1) void gemm_split_kernel(int M, int N, int K, int Kp, int Mp, int Np,
+                                                                 const char *__restrict__ X, const char *__restrict__ Y,
+                                                                 const uint8_t *__restrict__ ea,
+                                                                 const uint8_t *__restrict__ eb,
+                                                                 const float *__restrict__ A, int lda,
+                                                                 const float *__restrict__ B, int ldb,
+                                                                 float *__restrict__ C, int ldc) {
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int wm = wave >> 1, wn = wave & 1, half = lane >> 5, l32 = lane & 31;
+  int tm, tn;
+  tile_coords(blockIdx.x, Mp / kTile, Np / kTile, tm, tn);
+  const int m0 = tm * kTile, n0 = tn * kTile;
+
+  {
+    unsigned *const least = reinterpret_cast<unsigned *>(lds);
+    if (threadIdx.x < 2) least[threadIdx.x] = 255;
+    __syncthreads();
+    const int pieces = (Kp + 63) / 64 * 4;
+    unsigned la = 255, lb = 255;
+    for (int i = threadIdx.x; i < pieces; i += kThreads) {
+      la = min(la, unsigned(ea[int64_t(tm) * pieces + i]));
+      lb = min(lb, unsigned(eb[int64_t(tn) * pieces + i]));
+    }
+    atomicMin(&least[0], la);
+    atomicMin(&least[1], lb);
+    __syncthreads();
+    la = least[0], lb = least[1];
+    __syncthreads();  // before the stages overwrite them
+    if (la < kMinExponent || lb < kMinExponent || la + lb < kMinProduct) {
+      for (int sub = 0; sub < 4; ++sub) {
+        const int ms = m0 + wm * 128 + (sub >> 1) * 64, ns = n0 + wn * 128 + (sub & 1) * 64;
+        if (ms >= M || ns >= N) continue;
+        f32x4 acc[4][4];
+        direct_tile<kF32, 4>(M, N, K, A, lda, B, ldb, ms, ns, lane, 0, 1, acc);
+        store_tile<4>(M, N, C, ldc, ms, ns, lane, acc);
+      }
+      return;
+    }
+  }
+
+  // Waves 0 and 1 stream A's panel, 2 and 3 B's: 12 chunks of 1 KiB each per stage.
+  const int rows_p = wave < 2 ? Mp : Np;
+  const char *const from = wave < 2 ? X + int64_t(m0) * 32 : Y + int64_t(n0) * 32;
+  const int part_stride = rows_p * 32;
+  const int stages = Kp / kSplitK;
+  const unsigned voff = unsigned(lane) * 16;
+  auto dma = [&](int ks, int buf) {
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char *>(from) + int64_t(ks) * 3 * part_stride, 0, 2 * part_stride + kPartB, 0x00020000);
+    char *const l = lds + buf + (wave >> 1) * kSplitPanelB;
+#pragma unroll
+    for (int i = 0; i < 12; ++i) {
+      const int q = (wave & 1) * 12 + i;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)(l + q * 1024), 16, voff,
+                                               unsigned((q >> 3) * part_stride + (q & 7) * 1024), 0, 0);
+    }
+  };
+  const int arow = (wm * 128 + l32) * 32 + half * 16, brow = kSplitPanelB + (wn * 128 + l32) * 32 + half * 16;
+  auto frags = [&](bf16x8 (&f)[kWaveTiles], int buf, int row, int part) {
+#pragma unroll
+    for (int i = 0; i < kWaveTiles; ++i)
+      f[i] = *reinterpret_cast<const bf16x8 *>(lds + buf + part * kPartB + row + i * 1024);
+  };
+
+  f32x16 acc[kWaveTiles][kWaveTiles];
+#pragma unroll
+  for (int i = 0; i < kWaveTiles; ++i)
+#pragma unroll
+    for (int j = 0; j < kWaveTiles; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+  auto group = [&](const bf16x8 (&a)[kWaveTiles], const bf16x8 (&b)[kWaveTiles]) {
+    CSMI_SCHED_FENCE();
+#pragma unroll
+    for (int i = 0; i < kWaveTiles; ++i)
+#pragma unroll
+      for (int j = 0; j < kWaveTiles; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+    CSMI_SCHED_FENCE();
+  };
+
+  int cur = 0, nxt = kSplitStageB, nn = 2 * kSplitStageB;  // buffers of stages s, s + 1, s + 2
+  dma(0, cur);
+  if (stages > 1) dma(1, nxt);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  bf16x8 ah[kWaveTiles], am[kWaveTiles], al[kWaveTiles], bm[kWaveTiles], bl[kWaveTiles], bh[2][kWaveTiles];
+  frags(al, cur, arow, 2);
+  frags(bh[0], cur, brow, 0);
+  frags(bl, cur, brow, 2);
+  frags(am, cur, arow, 1);
+  frags(bm, cur, brow, 1);
+  auto stage = [&](int ks, auto parity) {
+    constexpr int P = decltype(parity)::value;
+    frags(ah, cur, arow, 0);
+    if (ks + 2 < stages) dma(ks + 2, nn);
+    // past the last stage the reads below fetch what no MFMA uses
+    group(al, bh[P]);
+    frags(al, nxt, arow, 2);
+    group(ah, bl);
+    frags(bl, nxt, brow, 2);
+    group(am, bm);
+    frags(bh[P ^ 1], nxt, brow, 0);
+    group(am, bh[P]);
+    frags(am, nxt, arow, 1);
+    group(ah, bm);
+    frags(bm, nxt, brow, 1);
+    group(ah, bh[P]);
+    // stage s + 2 has landed (own DMAs, then everybody's), and nobody reads stage s any more
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    const int free = cur;
+    cur = nxt, nxt = nn, nn = free;
+  };
+  int ks = 0;
+  for (; ks + 1 < stages; ks += 2) {
+    stage(ks, std::integral_constant<int, 0>());
+    stage(ks + 1, std::integral_constant<int, 1>());
+  }
+  if (ks < stages) stage(ks, std::integral_constant<int, 0>());
+
+  // acc[i][j][e]: row = 8*(e/4) + 4*half + e%4, col = l32 of the 32x32 tile (i, j)
+#pragma unroll
+  for (int i = 0; i < kWaveTiles; ++i)
+#pragma unroll
+    for (int j = 0; j < kWaveTiles; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int r = m0 + wm * 128 + i * 32 + 8 * (e / 4) + 4 * half + (e % 4);
+        const int c = n0 + wn * 128 + j * 32 + l32;
+        if (r < M && c < N) C[int64_t(r) * ldc + c] = acc[i][j][e];
+      }
 }
 
 int64_t round_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
@@ -951,15 +1218,21 @@ __global__ __launch_bounds__(256) void zero_matrix_kernel(float *__restrict__ C,
   C[(i / N) * ldc + i % N] = 0.0f;
 }
 
+// The packed kernel's row offsets are 32 bits wide; K is held to that on every path.
+template <int KIND>
+void check_depth(int K) {
+  using P = Pipe<KIND>;
+  if (round_up(K, P::kK) * P::kBytesPerK * kTile >= (int64_t(1) << 31))
+    fail(CS_INVALID_VALUE, "K = " + std::to_string(K) + " is too large for this GEMM variant (K * bytes per "
+                           "value must stay below 8 MiB)");
+}
+
 template <int KIND>
 void run_lds(cs_stream *stream, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
              int ldc) {
   using P = Pipe<KIND>;
   const int64_t Mp = round_up(M, kTile), Np = round_up(N, kTile), Kp = round_up(K, P::kK);
   const int64_t rowb = Kp * P::kBytesPerK;
-  if (rowb * kTile >= (int64_t(1) << 31))
-    fail(CS_INVALID_VALUE, "K = " + std::to_string(K) + " is too large for this GEMM variant (K * bytes per "
-                           "value must stay below 8 MiB)");
   const int64_t xbytes = Mp * rowb, ybytes = Np * rowb;
   int64_t total = xbytes + ybytes + 4096;
   if (KIND == kFP8) total += (Mp + Np) * (Kp / 128) + 4096;
@@ -1001,6 +1274,34 @@ void run_lds(cs_stream *stream, int M, int N, int K, const float *A, int lda, co
   hipLaunchKernelGGL(gemm_lds_kernel<KIND>, dim3(grid), dim3(kThreads), kLdsBytes, s, M, N, int(Kp), int(Mp),
                      int(Np), x, y, sx, sy, C, ldc);
   CS_HIP(hipGetLastError());
+}
+
+// FP32 from three BF16 parts. False when the operands are too tall for its 32-bit offsets.
+bool run_split(cs_stream *stream, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
+               int ldc) {
+  const int64_t Mp = round_up(M, kTile), Np = round_up(N, kTile), Kp = round_up(K, kSplitK);
+  if (std::max(Mp, Np) * 96 >= (int64_t(1) << 31)) return false;
+  const int64_t xbytes = Mp * Kp * 6, ybytes = Np * Kp * 6, pieces = (Kp + 63) / 64 * 4;
+  const int64_t ebytes = (Mp + Np) / kTile * pieces;
+  char *base = static_cast<char *>(stream_scratch(stream, static_cast<size_t>(xbytes + ybytes + ebytes + 4096)));
+  SplitArgs p;
+  p.a = A, p.b = B, p.m = M, p.n = N, p.k = K, p.lda = lda, p.ldb = ldb, p.mp = int(Mp), p.np = int(Np), p.kp = int(Kp);
+  p.vec_a = (lda % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0) ? 1 : 0;
+  p.x = base, p.y = base + xbytes;
+  p.ea = reinterpret_cast<uint8_t *>(base + xbytes + ybytes), p.eb = p.ea + Mp / kTile * pieces;
+  p.row_blocks = unsigned(Mp / 64 * (pieces / 4));
+  const int64_t blocks = int64_t(p.row_blocks) + Np / 64 * (pieces / 4);
+  hipLaunchKernelGGL(split_operands_kernel, dim3(unsigned(blocks)), dim3(256), 0, stream->stream, p);
+  static const bool configured = [] {
+    CS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_split_kernel),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kSplitLds)));
+    return true;
+  }();
+  (void)configured;
+  hipLaunchKernelGGL(gemm_split_kernel, dim3(unsigned((Mp / kTile) * (Np / kTile))), dim3(kThreads), kSplitLds,
+                     stream->stream, M, N, K, int(Kp), int(Mp), int(Np), p.x, p.y, p.ea, p.eb, A, lda, B, ldb, C, ldc);
+  CS_HIP(hipGetLastError());
+  return true;
 }
 
 template <int KIND, int T, int kWK>
@@ -1057,13 +1358,14 @@ bool overlap(const float *a, int64_t rows_a, int64_t cols_a, int lda, const floa
 // Direct or packed. The packed kernel's time is a round of 256 x 256 tiles over K for every 256
 // workgroups begun, however few there are, on top of the pre-pass and a second launch; the direct
 // one's follows the flops. In us, direct / packed:
-//   FP32: 300x200x1000 5.8 / 242, 1000^3 29.1 / 250, 2048^3 156 / 481, 1024x1024x4096 81 / 936
+//   FP32 (packed as three BF16 parts): 300x200x1000 5.8 / 140, 1000^3 29.1 / 145, 2048^3 156 / 300,
+//     3000x3000x1000 251 / 155
 //   BF16: 300x200x1000 5.6 / 33, 1000^3 18.7 / 37.6, 1024x1024x4096 62 / 99, 2048^3 122 / 61
 //   BF16x3: 1000^3 20.4 / 73.9, 2048^3 85 / 130;  FP8: 512^3 6.5 / 19.6, 1000^3 43 / 30
 // The packed path copies the operands first, so a C that overlaps A or B always takes it.
 template <int KIND>
 bool prefer_direct(int64_t cus, int64_t M, int64_t N, int64_t K, const DirectPlan &p) {
-  const double packed_per_k = KIND == kF32 ? 0.225 : KIND == kBF16 ? 0.0217 : KIND == kBF16X3 ? 0.054 : 0.0125;  // us
+  const double packed_per_k = KIND == kF32 ? 0.134 : KIND == kBF16 ? 0.0217 : KIND == kBF16X3 ? 0.054 : 0.0125;  // us
   const double direct_tflops =
       KIND == kF32 ? 105.0 : KIND == kBF16 ? 135.0 : KIND == kBF16X3 ? 160.0 : p.t == 2 ? 40.0 : 25.0;
   const double e = 16.0 * p.t;
@@ -1071,17 +1373,21 @@ bool prefer_direct(int64_t cus, int64_t M, int64_t N, int64_t K, const DirectPla
   // the direct kernel's stores of C come in shorter runs (4096x4096x16 in BF16: 20.5 / 18.7)
   const double direct = 2e-6 * area * double(K) / direct_tflops + (KIND == kF32 ? 0.8e-6 : 1.2e-6) * out;
   const double rounds = std::ceil(std::ceil(M / 256.0) * std::ceil(N / 256.0) / double(cus));
-  const double pack = double(M + N) * double(K) * 1.5e-6;
+  const double pack = double(M + N) * double(K) * (KIND == kF32 ? 1.8e-6 : 1.5e-6);
   return direct < 8.0 + pack + rounds * packed_per_k * double(K) + 0.5e-6 * out;
 }
 
 template <int KIND>
 void run(cs_stream *stream, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C, int ldc) {
+  check_depth<KIND>(K);
   const int64_t cus = stream->device->props.multiProcessorCount;
   const DirectPlan p = plan_direct(KIND, cus, M, N, K);
-  if (!prefer_direct<KIND>(cus, M, N, K, p) || overlap(A, M, K, lda, C, M, N, ldc) ||
-      overlap(B, K, N, ldb, C, M, N, ldc))
+  if (overlap(A, M, K, lda, C, M, N, ldc) || overlap(B, K, N, ldb, C, M, N, ldc))
     return run_lds<KIND>(stream, M, N, K, A, lda, B, ldb, C, ldc);
+  if (!prefer_direct<KIND>(cus, M, N, K, p)) {
+    if (KIND == kF32 && run_split(stream, M, N, K, A, lda, B, ldb, C, ldc)) return;
+    return run_lds<KIND>(stream, M, N, K, A, lda, B, ldb, C, ldc);
+  }
   switch (p.t * 100 + p.wk) {
     case 101: return run_direct<KIND, 1, 1>(stream, M, N, K, A, lda, B, ldb, C, ldc);
     case 104: return run_direct<KIND, 1, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc);

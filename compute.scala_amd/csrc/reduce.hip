@@ -235,19 +235,11 @@ __device__ __forceinline__ void add_vector(f4u v, Acc &a, float &m) {
 
 // One row's share of a lane: vectors lane, lane + kStep, ... of p, four loads in flight. The
 // cols % 4 elements after the last whole vector are the end of one more vector that overlaps it,
-// so that they ride with the other loads.
-template <int kStep>
-__device__ __forceinline__ void read_row(const float *__restrict__ p, int64_t cols, int lane, Acc &a, float &m) {
-  const f4u *p4 = reinterpret_cast<const f4u *>(p);
-  const int64_t nv = cols / 4;
-  int64_t i = lane;
-  for (; i + 3 * kStep < nv; i += 4 * kStep) {
-    f4u v[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = __builtin_nontemporal_load(p4 + i + k * kStep);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) add_vector(v[k], a, m);
-  }
+// so that they ride with the other loads. kShort: at most one vector per lane; what a launch of few
+// short rows waits for is mostly its own instructions, so it gets a kernel of few.
+template <int kStep, bool kShort, class Index>
+__device__ __forceinline__ void read_row(const float *__restrict__ p, Index cols, int lane, Acc &a, float &m) {
+  const Index nv = cols / 4;
   const int tail = static_cast<int>(cols % 4);
   if (nv == 0) {
     for (int j = lane; j < tail; j += kStep) {
@@ -256,40 +248,50 @@ __device__ __forceinline__ void read_row(const float *__restrict__ p, int64_t co
     }
     return;
   }
-  const int64_t all = nv + (tail ? 1 : 0);
-  if (i >= all) return;
-  f4u v[4];
+  Index i = lane;
+  if (!kShort) {
+    const f4u *p4 = reinterpret_cast<const f4u *>(p);
+    for (; i + 3 * kStep < nv; i += 4 * kStep) {
+      f4u v[4];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int64_t c = i + k * kStep;
+      for (int k = 0; k < 4; ++k) v[k] = __builtin_nontemporal_load(p4 + i + k * kStep);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) add_vector(v[k], a, m);
+    }
+  }
+  constexpr int kVecs = kShort ? 1 : 4;
+  const Index all = nv + (tail ? 1 : 0);
+  if (i >= all) return;
+  f4u v[kVecs];
+#pragma unroll
+  for (int k = 0; k < kVecs; ++k) {
+    const Index c = i + k * kStep;
     if (c < all) v[k] = __builtin_nontemporal_load(reinterpret_cast<const f4u *>(p + (c < nv ? 4 * c : cols - 4)));
   }
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int64_t c = i + k * kStep;
-    if (c < nv) {
-      a.add(v[k].x), a.add(v[k].y), a.add(v[k].z), a.add(v[k].w);
-      m = nanmax(m, nanmax(nanmax(v[k].x, v[k].y), nanmax(v[k].z, v[k].w)));
-    } else if (c < all) {
-      // the last `tail` of the vector's elements; the others were added with the one before
-      a.add(v[k].w);
-      m = nanmax(m, v[k].w);
-      if (tail > 1) a.add(v[k].z), m = nanmax(m, v[k].z);
-      if (tail > 2) a.add(v[k].y), m = nanmax(m, v[k].y);
+  for (int k = 0; k < kVecs; ++k) {
+    const Index c = i + k * kStep;
+    if (c < all) {
+      const int again = c < nv ? 0 : 4 - tail;  // elements that the vector before has added
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        a.add(e >= again ? v[k][e] : 0.0f);
+        m = nanmax(m, e >= again ? v[k][e] : __builtin_nanf(""));
+      }
     }
   }
 }
 
 // One workgroup per row: row sum (compensated FP32, rounded once), row max, and the FP64
 // partial of the row for the total.
-template <int kThreads>
+template <int kThreads, bool kShort>
 __global__ __launch_bounds__(kThreads) void reduce_rows_kernel(const float *__restrict__ in, int64_t cols,
                                                                float *row_sum, float *row_max, double *partial64,
                                                                float *total, double *total64) {
   const int64_t row = blockIdx.x;
   Acc a;
   float m = __builtin_nanf("");
-  read_row<kThreads>(in + row * cols, cols, threadIdx.x, a, m);
+  read_row<kThreads, kShort>(in + row * cols, cols, threadIdx.x, a, m);
   block_reduce<kThreads / 64>(a, m);
   if (threadIdx.x == 0) {
     if (row_sum) row_sum[row] = a.result();
@@ -304,7 +306,7 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_kernel(const float *__re
 // values of its rows are added in a fixed order into one partial per workgroup. Bound by HBM once
 // the grid fills the chip: 120011 x 77 (37 MB) takes 12.5 us with its combine, 3.0 TB/s, against
 // 109 us when every row had a workgroup; 16000 x 1025 15.7 us (4.2 TB/s) against 25.2.
-template <int kG>
+template <int kG, bool kShort>
 __global__ __launch_bounds__(kBlock) void reduce_short_rows_kernel(const float *__restrict__ in, int64_t rows,
                                                                    int64_t cols, int tiles, float *row_sum,
                                                                    float *row_max, double *partial64, float *total,
@@ -316,7 +318,7 @@ __global__ __launch_bounds__(kBlock) void reduce_short_rows_kernel(const float *
     const int64_t row = (int64_t(blockIdx.x) * tiles + t) * (kBlock / kG) + group;
     Acc a;
     float m = __builtin_nanf("");
-    if (row < rows) read_row<kG>(in + row * cols, cols, lane, a, m);
+    if (row < rows) read_row<kG, kShort>(in + row * cols, static_cast<int>(cols), lane, a, m);
 #pragma unroll
     for (int off = kG / 2; off >= 1; off >>= 1) {
       const float s2 = __shfl_xor(a.s, off, 64), c2 = __shfl_xor(a.c, off, 64), m2 = __shfl_xor(m, off, 64);
@@ -524,55 +526,69 @@ struct RowPlan {
 //     its time starting and combining: 120011 x 77 109.0 / 12.5, 524288 x 8 463 / 9.4,
 //     60000 x 128 57.8 / 9.4, 16384 x 1024 19.3 / 14.8, 16000 x 1025 21.6 / 15.7; equal at
 //     2047 columns (15.4 / 15.6); at 4096 the workgroup per row is ahead (43.3 / 45.8).
+//   * few rows (at most 8 per CU, all resident at once) of more than 256 columns keep a workgroup
+//     per row, since nothing else fills the chip: 2000 x 2000 7.5 / 7.2.
 //   * as many lanes as take a row in at most four vectors each, all in flight together: half as
 //     many (eight vectors) 14.1 at 120011 x 77 against 12.4, twice as many 15.5.
+//     More where the rows leave the chip idle otherwise, down to one vector each.
 //   * at most 8192 partials, which the combine adds in one round of loads.
 //   * at most one row per CU and long rows: 1024 threads per row, since nothing else fills the
 //     chip (64 x 65536 14.9 / 9.0, 256 x 16384 7.4 / 6.5); from two rows per CU on 256 threads
 //     are ahead (512 x 16384 8.8 against 9.4, 2000 x 8192 13.4 against 16.9).
-constexpr int64_t kShortCols = 2048, kMaxPartials = 8192, kWideCols = 8192;
+constexpr int64_t kShortCols = 2048, kMaxPartials = 8192, kWideCols = 8192, kFewRows = 8;
 
 RowPlan plan_rows(cs_stream *stream, int64_t rows, int64_t cols) {
   RowPlan p;
-  if (cols > kShortCols) {
+  const int64_t cus = stream->device->props.multiProcessorCount;
+  if (cols > kShortCols || (rows <= kFewRows * cus && cols > 256)) {
     p.grid = rows;
-    p.wide = rows <= stream->device->props.multiProcessorCount && cols >= kWideCols;
+    p.wide = rows <= cus && cols >= kWideCols;
     return p;
   }
   p.lanes = 2;
   while (p.lanes < 64 && p.lanes * 16 < cols) p.lanes *= 2;
+  while (p.lanes < 64 && p.lanes * 4 < cols && rows * p.lanes < 2 * cus * kBlock) p.lanes *= 2;
   const int64_t per = kBlock / p.lanes, groups = (rows + per - 1) / per;
   p.tiles = static_cast<int>((groups + kMaxPartials - 1) / kMaxPartials);
   p.grid = (groups + p.tiles - 1) / p.tiles;
   return p;
 }
 
-template <int kG>
+template <int kG, bool kShort>
 void launch_short_rows(cs_stream *stream, const RowPlan &p, const float *in, int64_t rows, int64_t cols,
                        float *row_sum, float *row_max, double *partial64, float *total, double *total64) {
-  hipLaunchKernelGGL(reduce_short_rows_kernel<kG>, dim3(static_cast<unsigned>(p.grid)), dim3(kBlock), 0,
+  hipLaunchKernelGGL((reduce_short_rows_kernel<kG, kShort>), dim3(static_cast<unsigned>(p.grid)), dim3(kBlock), 0,
                      stream->stream, in, rows, cols, p.tiles, row_sum, row_max, partial64, total, total64);
+}
+
+template <int kThreads, bool kShort>
+void launch_long_rows(cs_stream *stream, const RowPlan &p, const float *in, int64_t cols, float *row_sum,
+                      float *row_max, double *partial64, float *total, double *total64) {
+  hipLaunchKernelGGL((reduce_rows_kernel<kThreads, kShort>), dim3(static_cast<unsigned>(p.grid)), dim3(kThreads), 0,
+                     stream->stream, in, cols, row_sum, row_max, partial64, total, total64);
 }
 
 // The row pass of a plan and, when partial64 is not null, the combine of its plan.grid partials (one
 // workgroup writes the total itself).
 void launch_rows(cs_stream *stream, const RowPlan &p, const float *in, int64_t rows, int64_t cols, float *row_sum,
                  float *row_max, double *partial64, float *total, double *total64) {
+#define CSMI_ROWS(kG) \
+  (cols <= 4 * kG ? launch_short_rows<kG, true> : launch_short_rows<kG, false>)(stream, p, in, rows, cols, row_sum, \
+                                                                             row_max, partial64, total, total64)
   switch (p.lanes) {
-    case 2: launch_short_rows<2>(stream, p, in, rows, cols, row_sum, row_max, partial64, total, total64); break;
-    case 4: launch_short_rows<4>(stream, p, in, rows, cols, row_sum, row_max, partial64, total, total64); break;
-    case 8: launch_short_rows<8>(stream, p, in, rows, cols, row_sum, row_max, partial64, total, total64); break;
-    case 16: launch_short_rows<16>(stream, p, in, rows, cols, row_sum, row_max, partial64, total, total64); break;
-    case 32: launch_short_rows<32>(stream, p, in, rows, cols, row_sum, row_max, partial64, total, total64); break;
-    case 64: launch_short_rows<64>(stream, p, in, rows, cols, row_sum, row_max, partial64, total, total64); break;
+    case 2: CSMI_ROWS(2); break;
+    case 4: CSMI_ROWS(4); break;
+    case 8: CSMI_ROWS(8); break;
+    case 16: CSMI_ROWS(16); break;
+    case 32: CSMI_ROWS(32); break;
+    case 64: CSMI_ROWS(64); break;
     default:
-      if (p.wide)
-        hipLaunchKernelGGL(reduce_rows_kernel<1024>, dim3(static_cast<unsigned>(p.grid)), dim3(1024), 0,
-                           stream->stream, in, cols, row_sum, row_max, partial64, total, total64);
-      else
-        hipLaunchKernelGGL(reduce_rows_kernel<kBlock>, dim3(static_cast<unsigned>(p.grid)), dim3(kBlock), 0,
-                           stream->stream, in, cols, row_sum, row_max, partial64, total, total64);
+      (p.wide                ? launch_long_rows<1024, false>
+       : cols <= 4 * kBlock  ? launch_long_rows<kBlock, true>
+                             : launch_long_rows<kBlock, false>)(stream, p, in, cols, row_sum, row_max, partial64,
+                                                                total, total64);
   }
+#undef CSMI_ROWS
   if (partial64 && p.grid > 1) launch_finish_sum(stream, partial64, p.grid, total, total64);
 }
 }  // namespace

@@ -14,15 +14,16 @@
 //                   each row of A and each column of B (amax / 448 rounded up to 2^e),
 //                   applied by v_mfma_scale_f32_32x32x64_f8f6f4, FP32 accumulate
 //
-// Small products run on gemm_direct_kernel, straight from A and B (prefer_direct, below). For the
+// Small products run on gemm_direct_kernel, straight from A and B (choose_path, below). For the
 // others a pre-pass converts A to a K-contiguous operand X[Mp][.] and B to its transpose Y[Np][.]
 // (zero padded to the tile sizes; split, interleaved or quantised as the variant needs) in
 // the stream's scratch; the main kernel computes C[m][n] = sum_k X[m][k] Y[n][k] with 256
-// threads (4 wave64s in 2x2) per 256x256 output tile, each wave owning 128x128 as 4x4 MFMA
-// tiles of 32x32 (256 FP32 accumulators per lane).
+// threads (4 wave64s in 2x2) per output tile: 256x256, each wave owning 128x128 as 4x4 MFMA
+// tiles of 32x32 (256 FP32 accumulators per lane), or, where such tiles leave CUs idle, 128x128
+// (2048^3 in BF16: 64 tiles 61 us, 256 tiles 37 us).
 //
 // All variants share one pipeline there. A K stage is 128 bytes of every operand row (32 FP32
-// values, 64 BF16 values, 32 hi/lo pairs or 128 e4m3 values); two stages live in LDS (128 KiB).
+// values, 64 BF16 values, 32 hi/lo pairs or 128 e4m3 values); two stages live in LDS (128 or 64 KiB).
 // The next stage streams global -> LDS directly (buffer_load ... lds, no registers) while
 // the MFMAs of the current one run; inside a stage the fragments of the next MFMA step are
 // read from LDS while the current step's MFMAs issue. Each 128-byte LDS row R stores its
@@ -48,9 +49,9 @@ typedef __attribute__((address_space(3))) void lds_void;
 
 enum Kind { kF32 = 0, kBF16 = 1, kBF16X3 = 2, kFP8 = 3 };
 
-constexpr int kTile = 256;     // output tile edge (rows and columns)
-constexpr int kThreads = 256;  // 4 waves
-constexpr int kWaveTiles = 4;  // 4x4 MFMA tiles of 32x32 per wave
+constexpr int kThreads = 256;  // 4 waves, in 2x2
+// W x W MFMA tiles of 32x32 per wave make an output tile of tile_edge(W) rows and columns.
+constexpr int tile_edge(int W) { return 64 * W; }
 
 // Blocks are dispatched round-robin over the 8 XCDs, each with its own L2. The tile of
 // block b: the XCDs get contiguous ranges of tiles, walked in groups of 4 tile rows (column
@@ -401,9 +402,9 @@ __global__ __launch_bounds__(256) void pack_operands_kernel(PackArgs p) {
 
 // ------------------------------------------------------------------------ main kernel
 constexpr int kRowB = 128;                          // bytes of one operand row per K stage
-constexpr int kPanelB = kTile * kRowB;              // 32 KiB: one operand's rows of a stage
-constexpr int kStageB = 2 * kPanelB;                // X and Y panels
-constexpr size_t kLdsBytes = size_t(2) * kStageB;   // two stages in flight: 128 KiB
+// One operand's rows of a stage (W = 4: 32 KiB, W = 2: 16 KiB), and two stages of both.
+constexpr int panel_bytes(int W) { return tile_edge(W) * kRowB; }
+constexpr size_t lds_bytes(int W) { return size_t(4) * panel_bytes(W); }
 
 template <int KIND>
 struct Pipe;
@@ -454,8 +455,8 @@ __device__ __forceinline__ void run_stages(int stages, Stage &stage) {
 
 // X: [Mp] rows of Kp * kBytesPerK bytes, Y: [Np] rows likewise. sx / sy: FP8 scales
 // [Kp/128][Mp] and [Kp/128][Np]. Host guarantees 256 * row bytes < 2^31.
-template <int KIND>
-__global__ __launch_bounds__(kThreads, 1) void gemm_lds_kernel(int M, int N, int Kp, int Mp, int Np,
+template <int KIND, int W>
+__global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_lds_kernel(int M, int N, int Kp, int Mp, int Np,
                                                                const char *__restrict__ X,
                                                                const char *__restrict__ Y,
                                                                const uint8_t *__restrict__ sx,
@@ -463,6 +464,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_lds_kernel(int M, int N, int
                                                                float *__restrict__ C, int ldc) {
   using P = Pipe<KIND>;
   using F = typename P::Frag;
+  constexpr int kTile = tile_edge(W), kWaveRows = 32 * W, kPanelB = panel_bytes(W), kStageB = 2 * kPanelB;
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -475,9 +477,9 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_lds_kernel(int M, int N, int
 
   // Global -> LDS. One DMA instruction of a wave fills a 1 KiB chunk = 8 rows of a panel,
   // lane l writing LDS bytes 16 l .. 16 l + 15: slot l & 7 of row l >> 3 of the chunk. Row R
-  // of a panel stores its piece p at slot p ^ ((R >> 1) & 7). DMA d (0..15) of a stage:
+  // of a panel stores its piece p at slot p ^ ((R >> 1) & 7). DMA d (0..4W - 1) of a stage:
   // operand d & 1, chunk c = 4 (d >> 1) + wave, i.e. rows R = 8 c + (l >> 3), whose key
-  // (R >> 1) & 7 = 4 (wave & 1) + (l >> 4) is the same for all 8 DMAs of a lane.
+  // (R >> 1) & 7 = 4 (wave & 1) + (l >> 4) is the same for all DMAs of a lane.
   const int drow = lane >> 3;
   const int dkey = 4 * (wave & 1) + (drow >> 1);
   const unsigned voff = unsigned((drow + 8 * wave) * rowb + (((lane & 7) ^ dkey) << 4));
@@ -492,12 +494,12 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_lds_kernel(int M, int N, int
     __builtin_amdgcn_raw_ptr_buffer_load_lds((d & 1) ? ry : rx, (lds_void *)(l), 16, voff, soff, 0, 0);
   };
 
-  // Fragment reads: lane (half, l32) of tile i reads row R = wm*128 + 32 i + l32 (A) or
-  // wn*128 + 32 i + l32 (B); piece p sits at slot p ^ ((R >> 1) & 7) = p ^ ((l32 >> 1) & 7).
+  // Fragment reads: lane (half, l32) of tile i reads row R = wm*32W + 32 i + l32 (A) or
+  // wn*32W + 32 i + l32 (B); piece p sits at slot p ^ ((R >> 1) & 7) = p ^ ((l32 >> 1) & 7).
   // The LDS serves 16 lanes per cycle over 64 banks (two 128-byte rows): lanes l32 .. l32 + 15
   // have 16 different (R & 1, (R >> 1) & 7), so they hit 16 different bank groups.
   const int sw = (l32 >> 1) & 7;
-  const int arow = (wm * 128 + l32) * kRowB, brow = kPanelB + (wn * 128 + l32) * kRowB;
+  const int arow = (wm * kWaveRows + l32) * kRowB, brow = kPanelB + (wn * kWaveRows + l32) * kRowB;
   auto piece = [&](int buf, int row, int p) -> i32x4 {
     return *reinterpret_cast<const i32x4 *>(lds + buf * kStageB + row + ((p ^ sw) << 4));
   };
@@ -518,23 +520,23 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_lds_kernel(int M, int N, int
     }
   };
 
-  f32x16 acc[kWaveTiles][kWaveTiles];
+  f32x16 acc[W][W];
 #pragma unroll
-  for (int i = 0; i < kWaveTiles; ++i)
+  for (int i = 0; i < W; ++i)
 #pragma unroll
-    for (int j = 0; j < kWaveTiles; ++j)
+    for (int j = 0; j < W; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
 
   // FP8 scales of the current stage (set 0) and of the next one (set 1, loaded one stage
   // ahead and moved to set 0 at the stage boundary).
-  int sa[2][kWaveTiles], sb[2][kWaveTiles];
+  int sa[2][W], sb[2][W];
   auto scales = [&](int ks, int set) {
 #pragma unroll
-    for (int i = 0; i < kWaveTiles; ++i) {
+    for (int i = 0; i < W; ++i) {
       if constexpr (KIND == kFP8) {
-        sa[set][i] = sx[int64_t(ks) * Mp + m0 + wm * 128 + i * 32 + l32];
-        sb[set][i] = sy[int64_t(ks) * Np + n0 + wn * 128 + i * 32 + l32];
+        sa[set][i] = sx[int64_t(ks) * Mp + m0 + wm * kWaveRows + i * 32 + l32];
+        sb[set][i] = sy[int64_t(ks) * Np + n0 + wn * kWaveRows + i * 32 + l32];
       } else {
         sa[set][i] = sb[set][i] = 0;
       }
@@ -545,14 +547,14 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_lds_kernel(int M, int N, int
   // twice the cycles (a group of 4 spans 256 of the stage's 2048).
   auto dma_slot = [&](int group, int ks_next, int buf) {
     constexpr int kPer = KIND == kFP8 ? 8 : 4;
-    if (group < 16 / kPer) {
+    if (group < 4 * W / kPer) {
 #pragma unroll
       for (int e = 0; e < kPer; ++e) dma(kPer * group + e, ks_next, buf);
     }
   };
 
 #pragma unroll
-  for (int d = 0; d < 16; ++d) dma(d, 0, 0);
+  for (int d = 0; d < 4 * W; ++d) dma(d, 0, 0);
   scales(0, 0);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
@@ -561,9 +563,9 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_lds_kernel(int M, int N, int
     // Fragments: al, ah, bl single; bh double (it is used by the first and the last MFMA
     // group of a step). Order per step: A = Al.Bh, B = Ah.Bl, C = Ah.Bh. Ah, Bl of step s
     // are read at its start (used from group B on); Al, Bh of step s + 1 right after group A.
-    F al[kWaveTiles], ah[kWaveTiles], bl[kWaveTiles], bh[2][kWaveTiles];
+    F al[W], ah[W], bl[W], bh[2][W];
 #pragma unroll
-    for (int i = 0; i < kWaveTiles; ++i) {
+    for (int i = 0; i < W; ++i) {
       al[i] = frag(0, arow + i * 32 * kRowB, 0, 1);
       bh[0][i] = frag(0, brow + i * 32 * kRowB, 0, 0);
     }
@@ -573,21 +575,21 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_lds_kernel(int M, int N, int
 #pragma unroll
       for (int s = 0; s < P::kSteps; ++s) {
 #pragma unroll
-        for (int i = 0; i < kWaveTiles; ++i) {
+        for (int i = 0; i < W; ++i) {
           ah[i] = frag(buf, arow + i * 32 * kRowB, s, 0);
           bl[i] = frag(buf, brow + i * 32 * kRowB, s, 1);
         }
         CSMI_SCHED_FENCE();
 #pragma unroll
-        for (int g = 0; g < kWaveTiles; ++g) {
+        for (int g = 0; g < W; ++g) {
 #pragma unroll
-          for (int j = 0; j < kWaveTiles; ++j) mma<KIND>(al[g], bh[s & 1][j], acc[g][j], 0, 0);
+          for (int j = 0; j < W; ++j) mma<KIND>(al[g], bh[s & 1][j], acc[g][j], 0, 0);
           if (kMore && s == 0) dma_slot(g, ks + 1, buf ^ 1);
           CSMI_SCHED_FENCE();
         }
         if (s + 1 < P::kSteps) {
 #pragma unroll
-          for (int i = 0; i < kWaveTiles; ++i) {
+          for (int i = 0; i < W; ++i) {
             al[i] = frag(buf, arow + i * 32 * kRowB, s + 1, 1);
             bh[(s + 1) & 1][i] = frag(buf, brow + i * 32 * kRowB, s + 1, 0);
           }
@@ -599,7 +601,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_lds_kernel(int M, int N, int
           __syncthreads();
           if (kMore) {
 #pragma unroll
-            for (int i = 0; i < kWaveTiles; ++i) {
+            for (int i = 0; i < W; ++i) {
               al[i] = frag(buf ^ 1, arow + i * 32 * kRowB, 0, 1);
               bh[0][i] = frag(buf ^ 1, brow + i * 32 * kRowB, 0, 0);
             }
@@ -607,15 +609,15 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_lds_kernel(int M, int N, int
         }
         CSMI_SCHED_FENCE();
 #pragma unroll
-        for (int g = 0; g < kWaveTiles; ++g) {
+        for (int g = 0; g < W; ++g) {
 #pragma unroll
-          for (int j = 0; j < kWaveTiles; ++j) mma<KIND>(ah[g], bl[j], acc[g][j], 0, 0);
+          for (int j = 0; j < W; ++j) mma<KIND>(ah[g], bl[j], acc[g][j], 0, 0);
           CSMI_SCHED_FENCE();
         }
 #pragma unroll
-        for (int g = 0; g < kWaveTiles; ++g) {
+        for (int g = 0; g < W; ++g) {
 #pragma unroll
-          for (int j = 0; j < kWaveTiles; ++j) mma<KIND>(ah[g], bh[s & 1][j], acc[g][j], 0, 0);
+          for (int j = 0; j < W; ++j) mma<KIND>(ah[g], bh[s & 1][j], acc[g][j], 0, 0);
           CSMI_SCHED_FENCE();
         }
       }
@@ -624,9 +626,9 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_lds_kernel(int M, int N, int
   } else {
     // Fragments double-buffered across the K steps of a stage (kSteps is even, so step 0
     // of every stage uses set 0).
-    F fa[2][kWaveTiles], fb[2][kWaveTiles];
+    F fa[2][W], fb[2][W];
 #pragma unroll
-    for (int i = 0; i < kWaveTiles; ++i) {
+    for (int i = 0; i < W; ++i) {
       fa[0][i] = frag(0, arow + i * 32 * kRowB, 0, 0);
       fb[0][i] = frag(0, brow + i * 32 * kRowB, 0, 0);
     }
@@ -638,7 +640,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_lds_kernel(int M, int N, int
       for (int s = 0; s < P::kSteps; ++s) {
         if (s + 1 < P::kSteps) {
 #pragma unroll
-          for (int i = 0; i < kWaveTiles; ++i) {
+          for (int i = 0; i < W; ++i) {
             fa[(s + 1) & 1][i] = frag(buf, arow + i * 32 * kRowB, s + 1, 0);
             fb[(s + 1) & 1][i] = frag(buf, brow + i * 32 * kRowB, s + 1, 0);
           }
@@ -650,7 +652,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_lds_kernel(int M, int N, int
           __syncthreads();
           if (kMore) {
 #pragma unroll
-            for (int i = 0; i < kWaveTiles; ++i) {
+            for (int i = 0; i < W; ++i) {
               fa[0][i] = frag(buf ^ 1, arow + i * 32 * kRowB, 0, 0);
               fb[0][i] = frag(buf ^ 1, brow + i * 32 * kRowB, 0, 0);
             }
@@ -664,30 +666,30 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_lds_kernel(int M, int N, int
 #pragma unroll
           for (int t = 0; t < 4; ++t) {
 #pragma unroll
-            for (int g = 0; g < kWaveTiles; ++g) {
+            for (int g = 0; g < W; ++g) {
 #pragma unroll
-              for (int j = 0; j < kWaveTiles; ++j)
+              for (int j = 0; j < W; ++j)
                 acc[g][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__int_as_float(fa[s & 1][g][t]),
                                                                  __int_as_float(fb[s & 1][j][t]),
                                                                  acc[g][j], 0, 0, 0);
-              if (kMore && t == 0) dma_slot(s * kWaveTiles + g, ks + 1, buf ^ 1);
+              if (kMore && t == 0) dma_slot(s * W + g, ks + 1, buf ^ 1);
               CSMI_SCHED_FENCE();
             }
           }
         } else {
 #pragma unroll
-          for (int g = 0; g < kWaveTiles; ++g) {
+          for (int g = 0; g < W; ++g) {
 #pragma unroll
-            for (int j = 0; j < kWaveTiles; ++j)
+            for (int j = 0; j < W; ++j)
               mma<KIND>(fa[s & 1][g], fb[s & 1][j], acc[g][j], sa[0][g], sb[0][j]);
-            if (kMore) dma_slot(s * kWaveTiles + g, ks + 1, buf ^ 1);
+            if (kMore) dma_slot(s * W + g, ks + 1, buf ^ 1);
             CSMI_SCHED_FENCE();
           }
         }
       }
       if (kMore) {
 #pragma unroll
-        for (int i = 0; i < kWaveTiles; ++i) {
+        for (int i = 0; i < W; ++i) {
           sa[0][i] = sa[1][i];
           sb[0][i] = sb[1][i];
         }
@@ -698,13 +700,13 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_lds_kernel(int M, int N, int
 
   // acc[i][j][e]: row = 8*(e/4) + 4*half + e%4, col = l32 of the 32x32 tile (i, j)
 #pragma unroll
-  for (int i = 0; i < kWaveTiles; ++i)
+  for (int i = 0; i < W; ++i)
 #pragma unroll
-    for (int j = 0; j < kWaveTiles; ++j)
+    for (int j = 0; j < W; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const int r = m0 + wm * 128 + i * 32 + 8 * (e / 4) + 4 * half + (e % 4);
-        const int c = n0 + wn * 128 + j * 32 + l32;
+        const int r = m0 + wm * kWaveRows + i * 32 + 8 * (e / 4) + 4 * half + (e % 4);
+        const int c = n0 + wn * kWaveRows + j * 32 + l32;
         if (r < M && c < N) C[int64_t(r) * ldc + c] = acc[i][j][e];
       }
 }
@@ -976,11 +978,11 @@ __global__ __launch_bounds__(kWK == 1 ? 256 : 64 * kWK) void gemm_direct_kernel(
 // FP32's. The pre-pass keeps the least exponent of each of its pieces of A and B (0 for values out of
 // range), and a tile of C whose rows or columns leave the range is computed from A and B on the FP32
 // matrix cores (direct_tile).
-constexpr int kSplitK = 16;                        // K values of a stage
-constexpr int kPartB = kTile * kSplitK * 2;        // one part of an operand's stage: 8 KiB
-constexpr int kSplitPanelB = 3 * kPartB;           // h, m, l
-constexpr int kSplitStageB = 2 * kSplitPanelB;     // both operands: 48 KiB
-constexpr size_t kSplitLds = size_t(3) * kSplitStageB;  // three stages: 144 KiB
+constexpr int kSplitK = 16;  // K values of a stage
+// One part of an operand's stage (W = 4: 8 KiB); h, m and l of both operands are a stage (48 KiB), and
+// three stages are in LDS (144 KiB).
+constexpr int part_bytes(int W) { return tile_edge(W) * kSplitK * 2; }
+constexpr size_t split_lds_bytes(int W) { return size_t(18) * part_bytes(W); }
 // Least exponents (biased) of the operands, and of a product of both, that stay on the BF16 path.
 constexpr unsigned kMinExponent = 24, kMinProduct = 254 - 110;
 
@@ -988,7 +990,7 @@ struct SplitArgs {
   const float *a, *b;
   int m, n, k, lda, ldb, mp, np, kp, vec_a;
   char *x, *y;         // [kp / 16][3][mp or np][16] BF16
-  uint8_t *ea, *eb;    // least exponents: [mp / 256][chunks][4] and [np / 256][chunks][4], chunks of 64 K
+  uint8_t *ea, *eb;    // least exponents: [mp / 64][chunks] and [np / 64][chunks], chunks of 64 K
   unsigned row_blocks;
 };
 
@@ -1066,22 +1068,24 @@ __global__ __launch_bounds__(256) void split_operands_kernel(SplitArgs p) {
   }
   __syncthreads();
   if (t == 0)
-    (is_a ? p.ea : p.eb)[(int64_t(strip / 4) * chunks + chunk) * 4 + strip % 4] = static_cast<uint8_t>(least);
+    (is_a ? p.ea : p.eb)[int64_t(strip) * chunks + chunk] = static_cast<uint8_t>(least);
 }
 
-// 256 threads (4 waves in 2x2) per 256 x 256 tile, each wave 128 x 128 as 4 x 4 MFMA tiles, as in
-// gemm_lds_kernel. A stage is 16 K values: 96 MFMAs per wave, in six groups of 16 that use every
-// accumulator once. Three stages live in LDS: while stage s computes, the fragments of s + 1 replace
+// 4 waves in 2x2 per output tile, W x W MFMA tiles each, as in gemm_lds_kernel. A stage is 16 K
+// values: (W = 4) 96 MFMAs per wave, in six groups of 16 that use every accumulator once. Three stages live in LDS: while stage s computes, the fragments of s + 1 replace
 // those of s as their last group has issued, and stage s + 2 streams into the buffer of s - 1. The
-// operands are packed so that each part of a stage is 8 KiB in a row: DMA and fragment reads are
+// operands are packed so that each part of a stage is contiguous: DMA and fragment reads are
 // linear in LDS, without bank conflicts.
-__global__ __launch_bounds__(kThreads, 1) void gemm_split_kernel(int M, int N, int K, int Kp, int Mp, int Np,
+template <int W>
+__global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_split_kernel(int M, int N, int K, int Kp, int Mp, int Np,
                                                                  const char *__restrict__ X, const char *__restrict__ Y,
                                                                  const uint8_t *__restrict__ ea,
                                                                  const uint8_t *__restrict__ eb,
                                                                  const float *__restrict__ A, int lda,
                                                                  const float *__restrict__ B, int ldb,
                                                                  float *__restrict__ C, int ldc) {
+  constexpr int kTile = tile_edge(W), kWaveRows = 32 * W, kPartB = part_bytes(W), kSplitPanelB = 3 * kPartB,
+                kSplitStageB = 2 * kSplitPanelB;
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -1094,7 +1098,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_split_kernel(int M, int N, i
     unsigned *const least = reinterpret_cast<unsigned *>(lds);
     if (threadIdx.x < 2) least[threadIdx.x] = 255;
     __syncthreads();
-    const int pieces = (Kp + 63) / 64 * 4;
+    const int pieces = (Kp + 63) / 64 * W;  // of the tile's rows, and of its columns
     unsigned la = 255, lb = 255;
     for (int i = threadIdx.x; i < pieces; i += kThreads) {
       la = min(la, unsigned(ea[int64_t(tm) * pieces + i]));
@@ -1106,8 +1110,8 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_split_kernel(int M, int N, i
     la = least[0], lb = least[1];
     __syncthreads();  // before the stages overwrite them
     if (la < kMinExponent || lb < kMinExponent || la + lb < kMinProduct) {
-      for (int sub = 0; sub < 4; ++sub) {
-        const int ms = m0 + wm * 128 + (sub >> 1) * 64, ns = n0 + wn * 128 + (sub & 1) * 64;
+      for (int sub = 0; sub < W * W / 4; ++sub) {
+        const int ms = m0 + wm * kWaveRows + sub / (W / 2) * 64, ns = n0 + wn * kWaveRows + sub % (W / 2) * 64;
         if (ms >= M || ns >= N) continue;
         f32x4 acc[4][4];
         direct_tile<kF32, 4>(M, N, K, A, lda, B, ldb, ms, ns, lane, 0, 1, acc);
@@ -1117,7 +1121,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_split_kernel(int M, int N, i
     }
   }
 
-  // Waves 0 and 1 stream A's panel, 2 and 3 B's: 12 chunks of 1 KiB each per stage.
+  // Waves 0 and 1 stream A's panel, 2 and 3 B's: 3W chunks of 1 KiB each per stage.
   const int rows_p = wave < 2 ? Mp : Np;
   const char *const from = wave < 2 ? X + int64_t(m0) * 32 : Y + int64_t(n0) * 32;
   const int part_stride = rows_p * 32;
@@ -1128,32 +1132,32 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_split_kernel(int M, int N, i
         const_cast<char *>(from) + int64_t(ks) * 3 * part_stride, 0, 2 * part_stride + kPartB, 0x00020000);
     char *const l = lds + buf + (wave >> 1) * kSplitPanelB;
 #pragma unroll
-    for (int i = 0; i < 12; ++i) {
-      const int q = (wave & 1) * 12 + i;
+    for (int i = 0; i < 3 * W; ++i) {
+      const int q = (wave & 1) * 3 * W + i;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)(l + q * 1024), 16, voff,
-                                               unsigned((q >> 3) * part_stride + (q & 7) * 1024), 0, 0);
+                                               unsigned(q / (2 * W) * part_stride + q % (2 * W) * 1024), 0, 0);
     }
   };
-  const int arow = (wm * 128 + l32) * 32 + half * 16, brow = kSplitPanelB + (wn * 128 + l32) * 32 + half * 16;
-  auto frags = [&](bf16x8 (&f)[kWaveTiles], int buf, int row, int part) {
+  const int arow = (wm * kWaveRows + l32) * 32 + half * 16, brow = kSplitPanelB + (wn * kWaveRows + l32) * 32 + half * 16;
+  auto frags = [&](bf16x8 (&f)[W], int buf, int row, int part) {
 #pragma unroll
-    for (int i = 0; i < kWaveTiles; ++i)
+    for (int i = 0; i < W; ++i)
       f[i] = *reinterpret_cast<const bf16x8 *>(lds + buf + part * kPartB + row + i * 1024);
   };
 
-  f32x16 acc[kWaveTiles][kWaveTiles];
+  f32x16 acc[W][W];
 #pragma unroll
-  for (int i = 0; i < kWaveTiles; ++i)
+  for (int i = 0; i < W; ++i)
 #pragma unroll
-    for (int j = 0; j < kWaveTiles; ++j)
+    for (int j = 0; j < W; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-  auto group = [&](const bf16x8 (&a)[kWaveTiles], const bf16x8 (&b)[kWaveTiles]) {
+  auto group = [&](const bf16x8 (&a)[W], const bf16x8 (&b)[W]) {
     CSMI_SCHED_FENCE();
 #pragma unroll
-    for (int i = 0; i < kWaveTiles; ++i)
+    for (int i = 0; i < W; ++i)
 #pragma unroll
-      for (int j = 0; j < kWaveTiles; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+      for (int j = 0; j < W; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
     CSMI_SCHED_FENCE();
   };
 
@@ -1162,7 +1166,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_split_kernel(int M, int N, i
   if (stages > 1) dma(1, nxt);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  bf16x8 ah[kWaveTiles], am[kWaveTiles], al[kWaveTiles], bm[kWaveTiles], bl[kWaveTiles], bh[2][kWaveTiles];
+  bf16x8 ah[W], am[W], al[W], bm[W], bl[W], bh[2][W];
   frags(al, cur, arow, 2);
   frags(bh[0], cur, brow, 0);
   frags(bl, cur, brow, 2);
@@ -1199,13 +1203,13 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_split_kernel(int M, int N, i
 
   // acc[i][j][e]: row = 8*(e/4) + 4*half + e%4, col = l32 of the 32x32 tile (i, j)
 #pragma unroll
-  for (int i = 0; i < kWaveTiles; ++i)
+  for (int i = 0; i < W; ++i)
 #pragma unroll
-    for (int j = 0; j < kWaveTiles; ++j)
+    for (int j = 0; j < W; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const int r = m0 + wm * 128 + i * 32 + 8 * (e / 4) + 4 * half + (e % 4);
-        const int c = n0 + wn * 128 + j * 32 + l32;
+        const int r = m0 + wm * kWaveRows + i * 32 + 8 * (e / 4) + 4 * half + (e % 4);
+        const int c = n0 + wn * kWaveRows + j * 32 + l32;
         if (r < M && c < N) C[int64_t(r) * ldc + c] = acc[i][j][e];
       }
 }
@@ -1222,15 +1226,16 @@ __global__ __launch_bounds__(256) void zero_matrix_kernel(float *__restrict__ C,
 template <int KIND>
 void check_depth(int K) {
   using P = Pipe<KIND>;
-  if (round_up(K, P::kK) * P::kBytesPerK * kTile >= (int64_t(1) << 31))
+  if (round_up(K, P::kK) * P::kBytesPerK * tile_edge(4) >= (int64_t(1) << 31))
     fail(CS_INVALID_VALUE, "K = " + std::to_string(K) + " is too large for this GEMM variant (K * bytes per "
                            "value must stay below 8 MiB)");
 }
 
-template <int KIND>
+template <int KIND, int W>
 void run_lds(cs_stream *stream, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
              int ldc) {
   using P = Pipe<KIND>;
+  constexpr int kTile = tile_edge(W);
   const int64_t Mp = round_up(M, kTile), Np = round_up(N, kTile), Kp = round_up(K, P::kK);
   const int64_t rowb = Kp * P::kBytesPerK;
   const int64_t xbytes = Mp * rowb, ybytes = Np * rowb;
@@ -1265,40 +1270,42 @@ void run_lds(cs_stream *stream, int M, int N, int K, const float *A, int lda, co
     hipLaunchKernelGGL(pack_operands_kernel<KIND>, dim3(unsigned(blocks)), dim3(256), 0, s, pa);
   }
   static const bool configured = [] {
-    CS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_lds_kernel<KIND>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kLdsBytes)));
+    CS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_lds_kernel<KIND, W>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes(W))));
     return true;
   }();
   (void)configured;
   const unsigned grid = static_cast<unsigned>((Mp / kTile) * (Np / kTile));
-  hipLaunchKernelGGL(gemm_lds_kernel<KIND>, dim3(grid), dim3(kThreads), kLdsBytes, s, M, N, int(Kp), int(Mp),
+  hipLaunchKernelGGL((gemm_lds_kernel<KIND, W>), dim3(grid), dim3(kThreads), lds_bytes(W), s, M, N, int(Kp), int(Mp),
                      int(Np), x, y, sx, sy, C, ldc);
   CS_HIP(hipGetLastError());
 }
 
 // FP32 from three BF16 parts. False when the operands are too tall for its 32-bit offsets.
+template <int W>
 bool run_split(cs_stream *stream, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
                int ldc) {
+  constexpr int kTile = tile_edge(W);
   const int64_t Mp = round_up(M, kTile), Np = round_up(N, kTile), Kp = round_up(K, kSplitK);
   if (std::max(Mp, Np) * 96 >= (int64_t(1) << 31)) return false;
-  const int64_t xbytes = Mp * Kp * 6, ybytes = Np * Kp * 6, pieces = (Kp + 63) / 64 * 4;
-  const int64_t ebytes = (Mp + Np) / kTile * pieces;
+  const int64_t xbytes = Mp * Kp * 6, ybytes = Np * Kp * 6, chunks = (Kp + 63) / 64;
+  const int64_t ebytes = (Mp + Np) / 64 * chunks;
   char *base = static_cast<char *>(stream_scratch(stream, static_cast<size_t>(xbytes + ybytes + ebytes + 4096)));
   SplitArgs p;
   p.a = A, p.b = B, p.m = M, p.n = N, p.k = K, p.lda = lda, p.ldb = ldb, p.mp = int(Mp), p.np = int(Np), p.kp = int(Kp);
   p.vec_a = (lda % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0) ? 1 : 0;
   p.x = base, p.y = base + xbytes;
-  p.ea = reinterpret_cast<uint8_t *>(base + xbytes + ybytes), p.eb = p.ea + Mp / kTile * pieces;
-  p.row_blocks = unsigned(Mp / 64 * (pieces / 4));
-  const int64_t blocks = int64_t(p.row_blocks) + Np / 64 * (pieces / 4);
+  p.ea = reinterpret_cast<uint8_t *>(base + xbytes + ybytes), p.eb = p.ea + Mp / 64 * chunks;
+  p.row_blocks = unsigned(Mp / 64 * chunks);
+  const int64_t blocks = int64_t(p.row_blocks) + Np / 64 * chunks;
   hipLaunchKernelGGL(split_operands_kernel, dim3(unsigned(blocks)), dim3(256), 0, stream->stream, p);
   static const bool configured = [] {
-    CS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_split_kernel),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kSplitLds)));
+    CS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_split_kernel<W>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(split_lds_bytes(W))));
     return true;
   }();
   (void)configured;
-  hipLaunchKernelGGL(gemm_split_kernel, dim3(unsigned((Mp / kTile) * (Np / kTile))), dim3(kThreads), kSplitLds,
+  hipLaunchKernelGGL(gemm_split_kernel<W>, dim3(unsigned((Mp / kTile) * (Np / kTile))), dim3(kThreads), split_lds_bytes(W),
                      stream->stream, M, N, K, int(Kp), int(Mp), int(Np), p.x, p.y, p.ea, p.eb, A, lda, B, ldb, C, ldc);
   CS_HIP(hipGetLastError());
   return true;
@@ -1342,7 +1349,7 @@ DirectPlan plan_direct(int kind, int64_t cus, int64_t M, int64_t N, int64_t K) {
   }
   const int64_t tiles = up(M, 16 * p.t) * up(N, 16 * p.t);
   const int64_t steps = up(K, kind == kF32 ? 16 : kind == kFP8 ? 128 : 32);
-  if (steps < 3 || tiles > (p.t == 4 ? 2 : 4) * cus) return p;
+  if (steps < 3 || tiles > (p.t == 4 ? 3 : 4) * cus) return p;
   p.wk = 4;
   if (kind != kFP8 && p.t < 4 && tiles <= cus && steps > 4) p.wk = p.t == 1 ? 16 : 8;
   return p;
@@ -1355,26 +1362,49 @@ bool overlap(const float *a, int64_t rows_a, int64_t cols_a, int lda, const floa
   return a < c1 && c < a1;
 }
 
-// Direct or packed. The packed kernel's time is a round of 256 x 256 tiles over K for every 256
-// workgroups begun, however few there are, on top of the pre-pass and a second launch; the direct
-// one's follows the flops. In us, direct / packed:
-//   FP32 (packed as three BF16 parts): 300x200x1000 5.8 / 140, 1000^3 29.1 / 145, 2048^3 156 / 300,
-//     3000x3000x1000 251 / 155
-//   BF16: 300x200x1000 5.6 / 33, 1000^3 18.7 / 37.6, 1024x1024x4096 62 / 99, 2048^3 122 / 61
-//   BF16x3: 1000^3 20.4 / 73.9, 2048^3 85 / 130;  FP8: 512^3 6.5 / 19.6, 1000^3 43 / 30
-// The packed path copies the operands first, so a C that overlaps A or B always takes it.
+// The path of a product: 0 direct, else the W of the packed kernels' tiles. Each path's time is
+// estimated from what it was measured to take (us): the direct kernel's from the flops of its padded
+// tiles at the rate of its tile size, with the CUs its last round leaves idle; the packed kernels'
+// from two launches, the pre-pass and one round of tiles over K for every 256 workgroups begun (two
+// of W = 2 share a CU). Over 68 shapes from 512^3 to 4096^3 the choice was within 3% of the fastest in
+// 65 and within 12% in the others. Measured direct / W = 2 / W = 4:
+//   FP32    300x200x1000 5.8 / - / 140, 1000^3 28 / 53 / 130, 2048^3 162 / 103 / 243, 4096^3 1277 /
+//           635 / 613
+//   BF16    1000^3 20 / 22 / 38, 2048^3 123 / 37 / 61, 4096^3 1005 / 154 / 147
+//   BF16x3  1000^3 20 / 37 / 74, 2048^3 85 / 65 / 131, 4096^3 654 / 364 / 331
+//   FP8     512^3 6.5 / 10 / 19, 2048^3 261 / 28 / 46, 4096^3 2069 / 100 / 97
 template <int KIND>
-bool prefer_direct(int64_t cus, int64_t M, int64_t N, int64_t K, const DirectPlan &p) {
-  const double packed_per_k = KIND == kF32 ? 0.134 : KIND == kBF16 ? 0.0217 : KIND == kBF16X3 ? 0.054 : 0.0125;  // us
-  const double direct_tflops =
-      KIND == kF32 ? 105.0 : KIND == kBF16 ? 135.0 : KIND == kBF16X3 ? 160.0 : p.t == 2 ? 40.0 : 25.0;
-  const double e = 16.0 * p.t;
-  const double area = std::ceil(M / e) * std::ceil(N / e) * e * e, out = double(M) * double(N);
-  // the direct kernel's stores of C come in shorter runs (4096x4096x16 in BF16: 20.5 / 18.7)
-  const double direct = 2e-6 * area * double(K) / direct_tflops + (KIND == kF32 ? 0.8e-6 : 1.2e-6) * out;
-  const double rounds = std::ceil(std::ceil(M / 256.0) * std::ceil(N / 256.0) / double(cus));
-  const double pack = double(M + N) * double(K) * (KIND == kF32 ? 1.8e-6 : 1.5e-6);
-  return direct < 8.0 + pack + rounds * packed_per_k * double(K) + 0.5e-6 * out;
+int choose_path(double cus, double M, double N, double K, const DirectPlan &p) {
+  struct Rates {
+    double direct[3];  // TFLOP/s of T = 1, 2, 4
+    double base;       // of a packed call, and what W = 4 adds
+    double base_w4;
+    double pack;       // of a value of A or B
+    double w4, w4_few;  // of one K of a round: W = 4 on all CUs, on at most three quarters (a higher clock)
+    double w2, w2_pair;  // W = 2: one workgroup on a CU, two together
+  };
+  constexpr Rates r = KIND == kF32      ? Rates{{45, 80, 110}, 13, -2, 1.8e-6, 0.134, 0.112, 0.038, 0.068}
+                      : KIND == kBF16   ? Rates{{50, 85, 140}, 7, 1.5, 0.9e-6, 0.0254, 0.0245, 0.0107, 0.0165}
+                      : KIND == kBF16X3 ? Rates{{50, 90, 190}, 7, 1.5, 1.35e-6, 0.0655, 0.058, 0.0228, 0.0360}
+                                        : Rates{{25, 60, 60}, 7, 1.5, 0.85e-6, 0.0137, 0.0137, 0.0066, 0.0076};
+  auto tiles = [&](double edge) { return std::ceil(M / edge) * std::ceil(N / edge); };
+  auto rounds = [&](double n) { return std::ceil(n / cus); };
+  const double e = 16.0 * p.t, blocks = p.wk == 1 ? std::ceil(std::ceil(M / e) / 4) * std::ceil(N / e) : tiles(e);
+  const double direct = 4 + 2e-6 * tiles(e) * e * e * K / r.direct[p.t / 2] * rounds(blocks) * cus / blocks +
+                        (KIND == kF32 ? 0.5e-6 : 1.2e-6) * M * N;
+  const double packed = r.base + r.pack * (M + N) * K + 0.5e-6 * M * N;
+  const double t4 = tiles(256), r2 = rounds(tiles(128)), pairs = std::floor(r2 / 2);
+  const double w4 = packed + r.base_w4 + K * rounds(t4) * (t4 <= 0.75 * cus ? r.w4_few : r.w4);
+  const double w2 = packed + K * (pairs * r.w2_pair + (r2 - 2 * pairs) * r.w2);
+  return direct <= w2 && direct <= w4 ? 0 : w2 <= w4 ? 2 : 4;
+}
+
+template <int KIND, int W>
+void run_packed(cs_stream *stream, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
+                int ldc, bool over) {
+  if constexpr (KIND == kF32)
+    if (!over && run_split<W>(stream, M, N, K, A, lda, B, ldb, C, ldc)) return;
+  run_lds<KIND, W>(stream, M, N, K, A, lda, B, ldb, C, ldc);
 }
 
 template <int KIND>
@@ -1382,12 +1412,12 @@ void run(cs_stream *stream, int M, int N, int K, const float *A, int lda, const 
   check_depth<KIND>(K);
   const int64_t cus = stream->device->props.multiProcessorCount;
   const DirectPlan p = plan_direct(KIND, cus, M, N, K);
-  if (overlap(A, M, K, lda, C, M, N, ldc) || overlap(B, K, N, ldb, C, M, N, ldc))
-    return run_lds<KIND>(stream, M, N, K, A, lda, B, ldb, C, ldc);
-  if (!prefer_direct<KIND>(cus, M, N, K, p)) {
-    if (KIND == kF32 && run_split(stream, M, N, K, A, lda, B, ldb, C, ldc)) return;
-    return run_lds<KIND>(stream, M, N, K, A, lda, B, ldb, C, ldc);
-  }
+  // A C that overlaps A or B is written only from copies of both.
+  const bool over = overlap(A, M, K, lda, C, M, N, ldc) || overlap(B, K, N, ldb, C, M, N, ldc);
+  int path = choose_path<KIND>(double(cus), M, N, K, p);
+  if (over && path == 0) path = 2;
+  if (path == 4) return run_packed<KIND, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc, over);
+  if (path == 2) return run_packed<KIND, 2>(stream, M, N, K, A, lda, B, ldb, C, ldc, over);
   switch (p.t * 100 + p.wk) {
     case 101: return run_direct<KIND, 1, 1>(stream, M, N, K, A, lda, B, ldb, C, ldc);
     case 104: return run_direct<KIND, 1, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc);

@@ -71,3 +71,32 @@ def test_direct_special_values(gpu_tensors, mnk):
     assert np.array_equal(download(T, bc, M * N).reshape(M, N), want, equal_nan=True)
     for h in (ba, bb, bc):
         h.release()
+
+
+@pytest.mark.parametrize("variant", sorted(VARIANTS))
+@pytest.mark.parametrize("mnk", [(1500, 1400, 260), (2049, 1031, 300), (640, 4097, 515)])
+def test_tiles_of_128(gpu_tensors, variant, mnk):
+    """The packed kernels on 128 x 128 tiles: remainders in every dimension."""
+    T = gpu_tensors
+    M, N, K = mnk
+    a, b = inputs.uniform(M * K, 4051).reshape(M, K), inputs.uniform(K * N, 4052).reshape(K, N)
+    ba, bb = upload(T, a), upload(T, b)
+    bc = upload(T, np.full(M * N + 8, 7.0, np.float32))
+    capi.check(capi.lib.cs_gemm(T.stream, VARIANTS[variant], M, N, K, ba.ptr, K, bb.ptr, N, bc.ptr, N))
+    got = download(T, bc, M * N + 8)
+    assert np.all(got[M * N:] == 7.0)
+    c = got[:M * N].reshape(M, N)
+    assert fp64.gemm_normalized_error(c, a, b) <= BOUND[variant]
+    for h in (ba, bb, bc):
+        h.release()
+
+
+def test_depth_is_limited_on_every_path(gpu_tensors):
+    """A K whose packed rows pass the 32-bit offsets is refused for small products too."""
+    T = gpu_tensors
+    K = 1 << 21
+    a, b, c = alloc(T, K), alloc(T, K), alloc(T, 1)
+    with pytest.raises(capi.InvalidValue):
+        capi.check(capi.lib.cs_gemm(T.stream, capi.GEMM_FP32, 1, 1, K, a.ptr, K, b.ptr, 1, c.ptr, 1))
+    for h in (a, b, c):
+        h.release()

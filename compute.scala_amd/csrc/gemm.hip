@@ -23,8 +23,8 @@
 // (2048^3 in BF16: 64 tiles 61 us, 256 tiles 37 us).
 //
 // All variants share one pipeline there. A K stage is 128 bytes of every operand row (32 FP32
-// values, 64 BF16 values, 32 hi/lo pairs or 128 e4m3 values); two stages live in LDS (128 or 64 KiB).
-// The next stage streams global -> LDS directly (buffer_load ... lds, no registers) while
+// values, 64 BF16 values, 32 hi/lo pairs or 128 e4m3 values); two stages live in LDS (128 or 64 KiB),
+// or four of a 128x128 tile. The next stages stream global -> LDS directly (buffer_load ... lds, no registers) while
 // the MFMAs of the current one run; inside a stage the fragments of the next MFMA step are
 // read from LDS while the current step's MFMAs issue. Each 128-byte LDS row R stores its
 // 16-byte piece p at slot p ^ ((R >> 1) & 7), so the fragment reads of 16 consecutive rows
@@ -402,9 +402,9 @@ __global__ __launch_bounds__(256) void pack_operands_kernel(PackArgs p) {
 
 // ------------------------------------------------------------------------ main kernel
 constexpr int kRowB = 128;                          // bytes of one operand row per K stage
-// One operand's rows of a stage (W = 4: 32 KiB, W = 2: 16 KiB), and two stages of both.
+// One operand's rows of a stage (W = 4: 32 KiB, W = 2: 16 KiB), and the stages held of both.
 constexpr int panel_bytes(int W) { return tile_edge(W) * kRowB; }
-constexpr size_t lds_bytes(int W) { return size_t(4) * panel_bytes(W); }
+constexpr size_t lds_bytes(int W, int bufs) { return size_t(2) * bufs * panel_bytes(W); }
 
 template <int KIND>
 struct Pipe;
@@ -445,18 +445,30 @@ __device__ __forceinline__ void mma(const typename Pipe<KIND>::Frag &a, const ty
   }
 }
 
-// Runs stage(ks, more) for ks = 0 .. stages - 1 with `more` (a next stage exists) as a
-// compile-time constant.
-template <class Stage>
+// Waits until at most kLeft of this wave's memory instructions are in flight and its LDS accesses are
+// done, then for the other waves. (__syncthreads would wait for every DMA.)
+template <int kLeft>
+__device__ __forceinline__ void publish_stage() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kLeft) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// Runs stage(ks, fill, more) for ks = 0 .. stages - 1. Compile-time constants: fill, stage ks + kAhead
+// exists, to be fetched meanwhile; more, stage ks + 1 exists.
+template <int kAhead, class Stage>
 __device__ __forceinline__ void run_stages(int stages, Stage &stage) {
-  for (int ks = 0; ks + 1 < stages; ++ks) stage(ks, std::true_type());
-  stage(stages - 1, std::false_type());
+  int ks = 0;
+  for (; ks + kAhead < stages; ++ks) stage(ks, std::true_type(), std::true_type());
+  if constexpr (kAhead > 1)
+    for (; ks + 1 < stages; ++ks) stage(ks, std::false_type(), std::true_type());
+  stage(ks, std::false_type(), std::false_type());
 }
 
 // X: [Mp] rows of Kp * kBytesPerK bytes, Y: [Np] rows likewise. sx / sy: FP8 scales
 // [Kp/128][Mp] and [Kp/128][Np]. Host guarantees 256 * row bytes < 2^31.
-template <int KIND, int W>
-__global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_lds_kernel(int M, int N, int Kp, int Mp, int Np,
+template <int KIND, int W, int kBufs>
+__global__ __launch_bounds__(kThreads, W * kBufs == 4 ? 2 : 1) void gemm_lds_kernel(int M, int N, int Kp, int Mp, int Np,
                                                                const char *__restrict__ X,
                                                                const char *__restrict__ Y,
                                                                const uint8_t *__restrict__ sx,
@@ -465,6 +477,8 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_lds_kernel(int 
   using P = Pipe<KIND>;
   using F = typename P::Frag;
   constexpr int kTile = tile_edge(W), kWaveRows = 32 * W, kPanelB = panel_bytes(W), kStageB = 2 * kPanelB;
+  constexpr int kAhead = kBufs - 1;  // stages fetched ahead of the one in use
+  constexpr int kDmas = 4 * W;                                 // of a wave, per stage
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -528,9 +542,11 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_lds_kernel(int 
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
 
-  // FP8 scales of the current stage (set 0) and of the next one (set 1, loaded one stage
-  // ahead and moved to set 0 at the stage boundary).
-  int sa[2][W], sb[2][W];
+  // FP8 scales of the current stage (set 0) and of the next kScales (set i moves to set i - 1 at the
+  // stage boundary). They are loaded before the DMAs of stages that may still be in flight when they
+  // are needed, since loads return in order.
+  constexpr int kScales = kAhead > 1 ? kAhead - 1 : 1;
+  int sa[kScales + 1][W], sb[kScales + 1][W];
   auto scales = [&](int ks, int set) {
 #pragma unroll
     for (int i = 0; i < W; ++i) {
@@ -553,11 +569,19 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_lds_kernel(int 
     }
   };
 
+  // Stage 0 and its scales have landed once at most those of the stages after it are in flight.
 #pragma unroll
-  for (int d = 0; d < 4 * W; ++d) dma(d, 0, 0);
-  scales(0, 0);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
+  for (int i = 0; i < kScales; ++i) scales(min(i, stages - 1), i);
+#pragma unroll
+  for (int i = 0; i < kAhead; ++i)
+    if (i < stages) {
+#pragma unroll
+      for (int d = 0; d < kDmas; ++d) dma(d, i, i);
+    }
+  if (stages >= kAhead)
+    publish_stage<(kAhead - 1) * kDmas>();
+  else
+    publish_stage<0>();
 
   if constexpr (KIND == kBF16X3) {
     // Fragments: al, ah, bl single; bh double (it is used by the first and the last MFMA
@@ -569,9 +593,9 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_lds_kernel(int 
       al[i] = frag(0, arow + i * 32 * kRowB, 0, 1);
       bh[0][i] = frag(0, brow + i * 32 * kRowB, 0, 0);
     }
-    auto stage = [&](int ks, auto more_tag) {
-      constexpr bool kMore = decltype(more_tag)::value;
-      const int buf = ks & 1;
+    auto stage = [&](int ks, auto fill_tag, auto more_tag) {
+      constexpr bool kFill = decltype(fill_tag)::value, kMore = decltype(more_tag)::value;
+      const int buf = ks & (kBufs - 1), next = (ks + 1) & (kBufs - 1);
 #pragma unroll
       for (int s = 0; s < P::kSteps; ++s) {
 #pragma unroll
@@ -584,7 +608,7 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_lds_kernel(int 
         for (int g = 0; g < W; ++g) {
 #pragma unroll
           for (int j = 0; j < W; ++j) mma<KIND>(al[g], bh[s & 1][j], acc[g][j], 0, 0);
-          if (kMore && s == 0) dma_slot(g, ks + 1, buf ^ 1);
+          if (kFill && s == 0) dma_slot(g, ks + kAhead, (ks + kAhead) & (kBufs - 1));
           CSMI_SCHED_FENCE();
         }
         if (s + 1 < P::kSteps) {
@@ -597,13 +621,12 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_lds_kernel(int 
           // Every read of this stage's buffer has been issued (Ah, Bl above): publish the next
           // stage (own DMAs landed, then the barrier) and read its first fragments while the
           // remaining two groups run.
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-          __syncthreads();
+          publish_stage<kFill ? (kAhead - 1) * kDmas : 0>();
           if (kMore) {
 #pragma unroll
             for (int i = 0; i < W; ++i) {
-              al[i] = frag(buf ^ 1, arow + i * 32 * kRowB, 0, 1);
-              bh[0][i] = frag(buf ^ 1, brow + i * 32 * kRowB, 0, 0);
+              al[i] = frag(next, arow + i * 32 * kRowB, 0, 1);
+              bh[0][i] = frag(next, brow + i * 32 * kRowB, 0, 0);
             }
           }
         }
@@ -622,7 +645,7 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_lds_kernel(int 
         }
       }
     };
-    run_stages(stages, stage);
+    run_stages<kAhead>(stages, stage);
   } else {
     // Fragments double-buffered across the K steps of a stage (kSteps is even, so step 0
     // of every stage uses set 0).
@@ -632,10 +655,10 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_lds_kernel(int 
       fa[0][i] = frag(0, arow + i * 32 * kRowB, 0, 0);
       fb[0][i] = frag(0, brow + i * 32 * kRowB, 0, 0);
     }
-    auto stage = [&](int ks, auto more_tag) {
-      constexpr bool kMore = decltype(more_tag)::value;
-      const int buf = ks & 1;
-      if (kMore) scales(ks + 1, 1);
+    auto stage = [&](int ks, auto fill_tag, auto more_tag) {
+      constexpr bool kFill = decltype(fill_tag)::value, kMore = decltype(more_tag)::value;
+      const int buf = ks & (kBufs - 1), next = (ks + 1) & (kBufs - 1);
+      if (kMore) scales(min(ks + kScales, stages - 1), kScales);
 #pragma unroll
       for (int s = 0; s < P::kSteps; ++s) {
         if (s + 1 < P::kSteps) {
@@ -648,13 +671,12 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_lds_kernel(int 
           // The last step's fragments were read during the previous step, so this stage's
           // buffer is no longer read: publish the next stage (own DMAs and scale loads landed,
           // then the barrier) and read its first fragments while this step's MFMAs run.
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-          __syncthreads();
+          publish_stage<kFill ? (kAhead - 1) * kDmas : 0>();
           if (kMore) {
 #pragma unroll
             for (int i = 0; i < W; ++i) {
-              fa[0][i] = frag(buf ^ 1, arow + i * 32 * kRowB, 0, 0);
-              fb[0][i] = frag(buf ^ 1, brow + i * 32 * kRowB, 0, 0);
+              fa[0][i] = frag(next, arow + i * 32 * kRowB, 0, 0);
+              fb[0][i] = frag(next, brow + i * 32 * kRowB, 0, 0);
             }
           }
         }
@@ -672,7 +694,7 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_lds_kernel(int 
                 acc[g][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__int_as_float(fa[s & 1][g][t]),
                                                                  __int_as_float(fb[s & 1][j][t]),
                                                                  acc[g][j], 0, 0, 0);
-              if (kMore && t == 0) dma_slot(s * W + g, ks + 1, buf ^ 1);
+              if (kFill && t == 0) dma_slot(s * W + g, ks + kAhead, (ks + kAhead) & (kBufs - 1));
               CSMI_SCHED_FENCE();
             }
           }
@@ -682,20 +704,22 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_lds_kernel(int 
 #pragma unroll
             for (int j = 0; j < W; ++j)
               mma<KIND>(fa[s & 1][g], fb[s & 1][j], acc[g][j], sa[0][g], sb[0][j]);
-            if (kMore) dma_slot(s * W + g, ks + 1, buf ^ 1);
+            if (kFill) dma_slot(s * W + g, ks + kAhead, (ks + kAhead) & (kBufs - 1));
             CSMI_SCHED_FENCE();
           }
         }
       }
       if (kMore) {
 #pragma unroll
-        for (int i = 0; i < W; ++i) {
-          sa[0][i] = sa[1][i];
-          sb[0][i] = sb[1][i];
-        }
+        for (int set = 0; set < kScales; ++set)
+#pragma unroll
+          for (int i = 0; i < W; ++i) {
+            sa[set][i] = sa[set + 1][i];
+            sb[set][i] = sb[set + 1][i];
+          }
       }
     };
-    run_stages(stages, stage);
+    run_stages<kAhead>(stages, stage);
   }
 
   // acc[i][j][e]: row = 8*(e/4) + 4*half + e%4, col = l32 of the 32x32 tile (i, j)
@@ -1072,10 +1096,11 @@ __global__ __launch_bounds__(256) void split_operands_kernel(SplitArgs p) {
 }
 
 // 4 waves in 2x2 per output tile, W x W MFMA tiles each, as in gemm_lds_kernel. A stage is 16 K
-// values: (W = 4) 96 MFMAs per wave, in six groups of 16 that use every accumulator once. Three stages live in LDS: while stage s computes, the fragments of s + 1 replace
-// those of s as their last group has issued, and stage s + 2 streams into the buffer of s - 1. The
-// operands are packed so that each part of a stage is contiguous: DMA and fragment reads are
-// linear in LDS, without bank conflicts.
+// values: (W = 4) 96 MFMAs per wave, in six groups of 16 that use every accumulator once. Three stages
+// live in LDS: while stage s computes, the fragments of s + 1 replace those of s as their last group
+// has issued, and stage s + 2 streams into the buffer of s - 1 (six stages of W = 2 gain nothing:
+// 2048^3 101.9 us against 103.5). The operands are packed so that each part of a stage is contiguous:
+// DMA and fragment reads are linear in LDS, without bank conflicts.
 template <int W>
 __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_split_kernel(int M, int N, int K, int Kp, int Mp, int Np,
                                                                  const char *__restrict__ X, const char *__restrict__ Y,
@@ -1164,8 +1189,7 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_split_kernel(in
   int cur = 0, nxt = kSplitStageB, nn = 2 * kSplitStageB;  // buffers of stages s, s + 1, s + 2
   dma(0, cur);
   if (stages > 1) dma(1, nxt);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
+  publish_stage<0>();
   bf16x8 ah[W], am[W], al[W], bm[W], bl[W], bh[2][W];
   frags(al, cur, arow, 2);
   frags(bh[0], cur, brow, 0);
@@ -1189,8 +1213,7 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_split_kernel(in
     frags(bm, nxt, brow, 1);
     group(ah, bh[P]);
     // stage s + 2 has landed (own DMAs, then everybody's), and nobody reads stage s any more
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
+    publish_stage<0>();
     const int free = cur;
     cur = nxt, nxt = nn, nn = free;
   };
@@ -1231,7 +1254,7 @@ void check_depth(int K) {
                            "value must stay below 8 MiB)");
 }
 
-template <int KIND, int W>
+template <int KIND, int W, int kBufs>
 void run_lds(cs_stream *stream, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
              int ldc) {
   using P = Pipe<KIND>;
@@ -1270,13 +1293,13 @@ void run_lds(cs_stream *stream, int M, int N, int K, const float *A, int lda, co
     hipLaunchKernelGGL(pack_operands_kernel<KIND>, dim3(unsigned(blocks)), dim3(256), 0, s, pa);
   }
   static const bool configured = [] {
-    CS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_lds_kernel<KIND, W>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes(W))));
+    CS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_lds_kernel<KIND, W, kBufs>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes(W, kBufs))));
     return true;
   }();
   (void)configured;
   const unsigned grid = static_cast<unsigned>((Mp / kTile) * (Np / kTile));
-  hipLaunchKernelGGL((gemm_lds_kernel<KIND, W>), dim3(grid), dim3(kThreads), lds_bytes(W), s, M, N, int(Kp), int(Mp),
+  hipLaunchKernelGGL((gemm_lds_kernel<KIND, W, kBufs>), dim3(grid), dim3(kThreads), lds_bytes(W, kBufs), s, M, N, int(Kp), int(Mp),
                      int(Np), x, y, sx, sy, C, ldc);
   CS_HIP(hipGetLastError());
 }
@@ -1305,7 +1328,8 @@ bool run_split(cs_stream *stream, int M, int N, int K, const float *A, int lda, 
     return true;
   }();
   (void)configured;
-  hipLaunchKernelGGL(gemm_split_kernel<W>, dim3(unsigned((Mp / kTile) * (Np / kTile))), dim3(kThreads), split_lds_bytes(W),
+  hipLaunchKernelGGL(gemm_split_kernel<W>, dim3(unsigned((Mp / kTile) * (Np / kTile))), dim3(kThreads),
+                     split_lds_bytes(W),
                      stream->stream, M, N, K, int(Kp), int(Mp), int(Np), p.x, p.y, p.ea, p.eb, A, lda, B, ldb, C, ldc);
   CS_HIP(hipGetLastError());
   return true;
@@ -1362,49 +1386,64 @@ bool overlap(const float *a, int64_t rows_a, int64_t cols_a, int lda, const floa
   return a < c1 && c < a1;
 }
 
-// The path of a product: 0 direct, else the W of the packed kernels' tiles. Each path's time is
-// estimated from what it was measured to take (us): the direct kernel's from the flops of its padded
-// tiles at the rate of its tile size, with the CUs its last round leaves idle; the packed kernels'
-// from two launches, the pre-pass and one round of tiles over K for every 256 workgroups begun (two
-// of W = 2 share a CU). Over 68 shapes from 512^3 to 4096^3 the choice was within 3% of the fastest in
-// 65 and within 12% in the others. Measured direct / W = 2 / W = 4:
-//   FP32    300x200x1000 5.8 / - / 140, 1000^3 28 / 53 / 130, 2048^3 162 / 103 / 243, 4096^3 1277 /
-//           635 / 613
-//   BF16    1000^3 20 / 22 / 38, 2048^3 123 / 37 / 61, 4096^3 1005 / 154 / 147
-//   BF16x3  1000^3 20 / 37 / 74, 2048^3 85 / 65 / 131, 4096^3 654 / 364 / 331
-//   FP8     512^3 6.5 / 10 / 19, 2048^3 261 / 28 / 46, 4096^3 2069 / 100 / 97
+// How a product runs: straight from A and B, or packed with 256 x 256 tiles (two stages of them in
+// LDS), 128 x 128 tiles (two stages, two workgroups on a CU) or 128 x 128 tiles with four stages, one
+// workgroup on a CU.
+enum Path { kDirect, kTiles256, kTiles128, kDeep128 };
+
+// Each path's time is estimated from what it was measured to take (us): the direct kernel's from the
+// flops of its padded tiles at the rate of its tile size, with the CUs its last round leaves idle; the
+// packed kernels' from two launches, the pre-pass and one round of tiles over K for every 256
+// workgroups begun. Over 64 shapes from 512^3 to 4096^3 the choice was within
+// 3% of the fastest in 61 and within 7% in the others.
+// Measured direct / 128 / deep 128 / 256:
+//   FP32    300x200x1000 5.8 / - / - / 140, 1000^3 28 / 53 / - / 130, 2048^3 160 / 104 / - / 242,
+//           4096^3 1269 / 620 / - / 594
+//   BF16    1000^3 20 / 22 / 19 / 38, 2048^3 122 / 37 / 30 / 61, 2500^3 262 / 53 / 57 / 82, 4096^3
+//           982 / 151 / 165 / 144
+//   BF16x3  1000^3 20 / 38 / 32 / 74, 2048^3 83 / 65 / 56 / 130, 2500^3 244 / 105 / 112 / 164, 4096^3
+//           655 / 356 / 377 / 326
+//   FP8     512^3 6.5 / 10.2 / 9.8 / 20, 2048^3 259 / 28 / 24 / 46, 2500^3 522 / 40 / 46 / 61, 4096^3
+//           2024 / 99 / 110 / 95
+// With 128 tiles on 64 of the CUs (1024x1024x4096) a stage of two waits for the DMA of the next: BF16
+// 55 us, with four 40; FP8 38 / 29.
 template <int KIND>
-int choose_path(double cus, double M, double N, double K, const DirectPlan &p) {
+Path choose_path(double cus, double M, double N, double K, const DirectPlan &p) {
   struct Rates {
-    double direct[3];  // TFLOP/s of T = 1, 2, 4
-    double base;       // of a packed call, and what W = 4 adds
-    double base_w4;
-    double pack;       // of a value of A or B
-    double w4, w4_few;  // of one K of a round: W = 4 on all CUs, on at most three quarters (a higher clock)
-    double w2, w2_pair;  // W = 2: one workgroup on a CU, two together
+    double direct[3];   // TFLOP/s of T = 1, 2, 4
+    double base;        // of a packed call, and what 256 x 256 tiles add
+    double base_256;
+    double pack;        // of a value of A or B
+    // of one K of a round: 256 x 256 tiles on all CUs, on at most three quarters (a higher clock);
+    // 128 x 128 tiles, one on a CU, two together; the same with four stages
+    double t256, t256_few, t128, t128_pair, deep;
   };
-  constexpr Rates r = KIND == kF32      ? Rates{{45, 80, 110}, 13, -2, 1.8e-6, 0.134, 0.112, 0.038, 0.068}
-                      : KIND == kBF16   ? Rates{{50, 85, 140}, 7, 1.5, 0.9e-6, 0.0254, 0.0245, 0.0107, 0.0165}
-                      : KIND == kBF16X3 ? Rates{{50, 90, 190}, 7, 1.5, 1.35e-6, 0.0655, 0.058, 0.0228, 0.0360}
-                                        : Rates{{25, 60, 60}, 7, 1.5, 0.85e-6, 0.0137, 0.0137, 0.0066, 0.0076};
+  constexpr Rates r = KIND == kF32    ? Rates{{45, 80, 110}, 13, -2, 1.8e-6, 0.126, 0.107, 0.036, 0.066, 1e9}
+                      : KIND == kBF16 ? Rates{{50, 85, 140}, 7, 0.5, 0.9e-6, 0.0245, 0.0245, 0.0107, 0.0145, 0.0071}
+                      : KIND == kBF16X3
+                          ? Rates{{50, 90, 190}, 7, 1.5, 1.35e-6, 0.0645, 0.058, 0.0228, 0.0365, 0.0180}
+                          : Rates{{25, 60, 60}, 7, 1.5, 0.85e-6, 0.0130, 0.0130, 0.0066, 0.0078, 0.0043};
   auto tiles = [&](double edge) { return std::ceil(M / edge) * std::ceil(N / edge); };
   auto rounds = [&](double n) { return std::ceil(n / cus); };
   const double e = 16.0 * p.t, blocks = p.wk == 1 ? std::ceil(std::ceil(M / e) / 4) * std::ceil(N / e) : tiles(e);
-  const double direct = 4 + 2e-6 * tiles(e) * e * e * K / r.direct[p.t / 2] * rounds(blocks) * cus / blocks +
-                        (KIND == kF32 ? 0.5e-6 : 1.2e-6) * M * N;
   const double packed = r.base + r.pack * (M + N) * K + 0.5e-6 * M * N;
-  const double t4 = tiles(256), r2 = rounds(tiles(128)), pairs = std::floor(r2 / 2);
-  const double w4 = packed + r.base_w4 + K * rounds(t4) * (t4 <= 0.75 * cus ? r.w4_few : r.w4);
-  const double w2 = packed + K * (pairs * r.w2_pair + (r2 - 2 * pairs) * r.w2);
-  return direct <= w2 && direct <= w4 ? 0 : w2 <= w4 ? 2 : 4;
+  const double t256 = tiles(256), r128 = rounds(tiles(128)), pairs = std::floor(r128 / 2);
+  const double time[] = {
+      4 + 2e-6 * tiles(e) * e * e * K / r.direct[p.t / 2] * rounds(blocks) * cus / blocks +
+          (KIND == kF32 ? 0.5e-6 : 1.2e-6) * M * N,
+      packed + r.base_256 + K * rounds(t256) * (t256 <= 0.75 * cus ? r.t256_few : r.t256),
+      packed + K * (pairs * r.t128_pair + (r128 - 2 * pairs) * r.t128),
+      r128 == 1 ? packed + K * r.deep : 1e30,  // in several rounds nothing hides their ends
+  };
+  return Path(std::min_element(time, time + 4) - time);
 }
 
-template <int KIND, int W>
+template <int KIND, int W, int kBufs>
 void run_packed(cs_stream *stream, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
                 int ldc, bool over) {
   if constexpr (KIND == kF32)
     if (!over && run_split<W>(stream, M, N, K, A, lda, B, ldb, C, ldc)) return;
-  run_lds<KIND, W>(stream, M, N, K, A, lda, B, ldb, C, ldc);
+  run_lds<KIND, W, kBufs>(stream, M, N, K, A, lda, B, ldb, C, ldc);
 }
 
 template <int KIND>
@@ -1414,10 +1453,12 @@ void run(cs_stream *stream, int M, int N, int K, const float *A, int lda, const 
   const DirectPlan p = plan_direct(KIND, cus, M, N, K);
   // A C that overlaps A or B is written only from copies of both.
   const bool over = overlap(A, M, K, lda, C, M, N, ldc) || overlap(B, K, N, ldb, C, M, N, ldc);
-  int path = choose_path<KIND>(double(cus), M, N, K, p);
-  if (over && path == 0) path = 2;
-  if (path == 4) return run_packed<KIND, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc, over);
-  if (path == 2) return run_packed<KIND, 2>(stream, M, N, K, A, lda, B, ldb, C, ldc, over);
+  Path path = choose_path<KIND>(double(cus), M, N, K, p);
+  if (over && path == kDirect) path = kTiles128;
+  if (path == kTiles256) return run_packed<KIND, 4, 2>(stream, M, N, K, A, lda, B, ldb, C, ldc, over);
+  if (path == kTiles128) return run_packed<KIND, 2, 2>(stream, M, N, K, A, lda, B, ldb, C, ldc, over);
+  if constexpr (KIND != kF32)
+    if (path == kDeep128) return run_packed<KIND, 2, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc, over);
   switch (p.t * 100 + p.wk) {
     case 101: return run_direct<KIND, 1, 1>(stream, M, N, K, A, lda, B, ldb, C, ldc);
     case 104: return run_direct<KIND, 1, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc);

@@ -100,3 +100,19 @@ def test_depth_is_limited_on_every_path(gpu_tensors):
         capi.check(capi.lib.cs_gemm(T.stream, capi.GEMM_FP32, 1, 1, K, a.ptr, K, b.ptr, 1, c.ptr, 1))
     for h in (a, b, c):
         h.release()
+
+
+@pytest.mark.parametrize("variant", sorted(set(VARIANTS) - {"fp32"}))
+@pytest.mark.parametrize("k", [17, 65, 129, 200, 257, 400, 640])
+def test_ring_of_four_stages(gpu_tensors, variant, k):
+    """128 x 128 tiles with four stages in LDS: fewer stages than that, exactly as many, more."""
+    T = gpu_tensors
+    M, N = 1999, 1901
+    a, b = inputs.uniform(M * k, 4061).reshape(M, k), inputs.uniform(k * N, 4062).reshape(k, N)
+    ba, bb, bc = upload(T, a), upload(T, b), alloc(T, M * N)
+    for _ in range(2):
+        capi.check(capi.lib.cs_gemm(T.stream, VARIANTS[variant], M, N, k, ba.ptr, k, bb.ptr, N, bc.ptr, N))
+        c = download(T, bc, M * N).reshape(M, N)
+        assert fp64.gemm_normalized_error(c, a, b) <= BOUND[variant]
+    for h in (ba, bb, bc):
+        h.release()

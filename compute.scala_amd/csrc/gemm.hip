@@ -42,6 +42,9 @@ namespace csmi {
 namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+// Loads of four and two consecutive values at any 4-byte boundary.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
@@ -69,20 +72,22 @@ __device__ __forceinline__ void tile_coords(int b, int tiles_m, int tiles_n, int
 }
 
 // ---------------------------------------------------------------------------- pre-pass
+// Reads are 16 bytes at any 4-byte boundary, whatever the leading dimension: 4095^3 in BF16 took 169 us
+// where rows off the 16-byte grid were read value by value, and takes 153 (4096^3: 148).
 
 // FP32 operands for the FP32 kernel, zero padded to [rows_p][kp]. A (K contiguous): one
-// thread per 4 consecutive K values of a row, 16-byte loads when the source is 16-byte
-// aligned (`vec`) and 16-byte stores.
+// thread per 4 consecutive K values of a row, 16-byte loads and stores.
 __device__ __forceinline__ void pack_rows_f32(unsigned bx, const float *__restrict__ src, int rows, int cols, int ld,
-                                              int rows_p, int kp, int vec, float *__restrict__ out) {
+                                              int rows_p, int kp, float *__restrict__ out) {
   const int chunks = kp / 4;
   const int64_t idx = int64_t(bx) * 256 + threadIdx.x;
   if (idx >= int64_t(rows_p) * chunks) return;
   const int r = static_cast<int>(idx / chunks), k = static_cast<int>(idx % chunks) * 4;
   const float *p = src + int64_t(r) * ld + k;
   float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  if (vec && r < rows && k + 4 <= cols) {
-    v = *reinterpret_cast<const float4 *>(p);
+  if (r < rows && k + 4 <= cols) {
+    const f4u a = *reinterpret_cast<const f4u *>(p);
+    v = make_float4(a[0], a[1], a[2], a[3]);
   } else if (r < rows) {
     v.x = k < cols ? p[0] : 0.0f;
     v.y = k + 1 < cols ? p[1] : 0.0f;
@@ -93,53 +98,50 @@ __device__ __forceinline__ void pack_rows_f32(unsigned bx, const float *__restri
 }
 
 // A TK x TN tile of B (K x N, N contiguous): rows k0.., columns n0.., zero outside the source.
-// TN / 4 threads per row, one 16-byte load each (`vec`), so a row's 4 TN bytes are read
+// TN / 4 threads per row, one 16-byte load each, so a row's 4 TN bytes are read
 // contiguously. Column n of row k sits at (n + k) mod TN: the reads of one column down K
 // (lane l at row 4l + j or 8l + e) then spread over the 64 banks without padding.
 constexpr int kPackTN = 64;  // B-tile width of the FP32 and BF16 packs
 template <int TN>
 __device__ __forceinline__ int tile_col(int k, int n) { return (n + k) & (TN - 1); }
 
+// Four consecutive columns of row k of B from column n on.
+__device__ __forceinline__ f4u load_b4(const float *__restrict__ src, int n_src, int k_src, int ld, int n, int k) {
+  f4u a = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (k < k_src && n < n_src) {
+    const float *p = src + int64_t(k) * ld + n;
+    if (n + 4 <= n_src) {
+      a = *reinterpret_cast<const f4u *>(p);
+    } else {
+      a[0] = p[0];
+      if (n + 1 < n_src) a[1] = p[1];
+      if (n + 2 < n_src) a[2] = p[2];
+    }
+  }
+  return a;
+}
+
 template <int TK, int TN, int kThreadsT>
 __device__ __forceinline__ void load_b_tile(float (*tile)[TN], const float *__restrict__ src, int n_src, int k_src,
-                                            int ld, int n0, int k0, int vec) {
+                                            int ld, int n0, int k0) {
   constexpr int kRowsPerPass = kThreadsT / (TN / 4), kPasses = TK / kRowsPerPass;
   const int t = threadIdx.x, n = (t % (TN / 4)) * 4;
-  if (vec && n0 + TN <= n_src && k0 + TK <= k_src) {
-    // the tile lies inside the source: all loads in flight before the first LDS write
-    float4 a[kPasses];
+  // all loads in flight before the first LDS write
+  f4u a[kPasses];
+  if (n0 + TN <= n_src && k0 + TK <= k_src) {
 #pragma unroll
     for (int i = 0; i < kPasses; ++i)
-      a[i] = *reinterpret_cast<const float4 *>(src + int64_t(k0 + t / (TN / 4) + kRowsPerPass * i) * ld + (n0 + n));
+      a[i] = *reinterpret_cast<const f4u *>(src + int64_t(k0 + t / (TN / 4) + kRowsPerPass * i) * ld + (n0 + n));
+  } else {
 #pragma unroll
-    for (int i = 0; i < kPasses; ++i) {
-      const int k = t / (TN / 4) + kRowsPerPass * i;
-      tile[k][tile_col<TN>(k, n)] = a[i].x;
-      tile[k][tile_col<TN>(k, n + 1)] = a[i].y;
-      tile[k][tile_col<TN>(k, n + 2)] = a[i].z;
-      tile[k][tile_col<TN>(k, n + 3)] = a[i].w;
-    }
-    return;
+    for (int i = 0; i < kPasses; ++i)
+      a[i] = load_b4(src, n_src, k_src, ld, n0 + n, k0 + t / (TN / 4) + kRowsPerPass * i);
   }
 #pragma unroll
   for (int i = 0; i < kPasses; ++i) {
     const int k = t / (TN / 4) + kRowsPerPass * i;
-    const float *p = src + int64_t(k0 + k) * ld + (n0 + n);
-    float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (k0 + k < k_src) {
-      if (vec && n0 + n + 4 <= n_src) {
-        a = *reinterpret_cast<const float4 *>(p);
-      } else {
-        a.x = n0 + n < n_src ? p[0] : 0.0f;
-        a.y = n0 + n + 1 < n_src ? p[1] : 0.0f;
-        a.z = n0 + n + 2 < n_src ? p[2] : 0.0f;
-        a.w = n0 + n + 3 < n_src ? p[3] : 0.0f;
-      }
-    }
-    tile[k][tile_col<TN>(k, n)] = a.x;
-    tile[k][tile_col<TN>(k, n + 1)] = a.y;
-    tile[k][tile_col<TN>(k, n + 2)] = a.z;
-    tile[k][tile_col<TN>(k, n + 3)] = a.w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tile[k][tile_col<TN>(k, n + e)] = a[i][e];
   }
 }
 
@@ -147,11 +149,11 @@ __device__ __forceinline__ void load_b_tile(float (*tile)[TN], const float *__re
 // LDS, 16-byte stores along K (each row of Y gets 256 contiguous bytes per tile).
 template <int TN>
 __device__ __forceinline__ void pack_cols_f32(unsigned bx, unsigned by, const float *__restrict__ src, int n_src,
-                                              int k_src, int ld, int rows_p, int kp, int vec,
+                                              int k_src, int ld, int rows_p, int kp,
                                               float *__restrict__ out) {
   __shared__ float tile[64][TN];  // [k][rotated n]
   const int n0 = int(bx) * TN, k0 = int(by) * 64, t = threadIdx.x;
-  load_b_tile<64, TN, 256>(tile, src, n_src, k_src, ld, n0, k0, vec);
+  load_b_tile<64, TN, 256>(tile, src, n_src, k_src, ld, n0, k0);
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < TN / 16; ++i) {
@@ -193,20 +195,20 @@ __device__ __forceinline__ void store_bf16x8(const float (&v)[8], char *row, int
 }
 
 // A (rows x cols, K contiguous) -> X: one thread per 8 consecutive K values of a row, two
-// 16-byte loads when the source is 16-byte aligned (`vec`), and one (split: two) 16-byte
-// stores. Rows and K values beyond the source are zero.
+// 16-byte loads and one (split: two) 16-byte stores. Rows and K values beyond the source are zero.
 template <bool kSplit>
 __device__ __forceinline__ void pack_rows_bf16(unsigned bx, const float *__restrict__ src, int rows, int cols, int ld,
-                                               int rows_p, int kp, int vec, char *__restrict__ out) {
+                                               int rows_p, int kp, char *__restrict__ out) {
   const int chunks = kp / 8;
   const int64_t idx = int64_t(bx) * 256 + threadIdx.x;
   if (idx >= int64_t(rows_p) * chunks) return;
   const int r = static_cast<int>(idx / chunks), k = static_cast<int>(idx % chunks) * 8;
   float v[8];
   const float *p = src + int64_t(r) * ld + k;
-  if (vec && r < rows && k + 8 <= cols) {
-    const float4 a = *reinterpret_cast<const float4 *>(p), b = *reinterpret_cast<const float4 *>(p + 4);
-    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+  if (r < rows && k + 8 <= cols) {
+    const f4u a = *reinterpret_cast<const f4u *>(p), b = *reinterpret_cast<const f4u *>(p + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = a[e], v[4 + e] = b[e];
   } else {
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = (r < rows && k + e < cols) ? p[e] : 0.0f;
@@ -218,11 +220,11 @@ __device__ __forceinline__ void pack_rows_bf16(unsigned bx, const float *__restr
 // through LDS; stores are 16 bytes along K (split: 16 high and 16 low bytes).
 template <bool kSplit, int TN>
 __device__ __forceinline__ void pack_cols_bf16(unsigned bx, unsigned by, const float *__restrict__ src, int n_src,
-                                               int k_src, int ld, int rows_p, int kp, int vec,
+                                               int k_src, int ld, int rows_p, int kp,
                                                char *__restrict__ out) {
   __shared__ float tile[64][TN];  // [k][rotated n]
   const int n0 = int(bx) * TN, k0 = int(by) * 64, t = threadIdx.x;
-  load_b_tile<64, TN, 256>(tile, src, n_src, k_src, ld, n0, k0, vec);
+  load_b_tile<64, TN, 256>(tile, src, n_src, k_src, ld, n0, k0);
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < TN / 32; ++i) {
@@ -257,10 +259,10 @@ __device__ __forceinline__ uint32_t fp8x4(float x0, float x1, float x2, float x3
 }
 
 // A (rows x cols, K contiguous) -> X[rows_p][kp] e4m3 plus scales[kb * rows_p + r]: 16 lanes
-// per 128-wide block of a row, 8 consecutive values per lane (two 16-byte loads when the
-// source is 16-byte aligned, `vec`), one 8-byte store per lane.
+// per 128-wide block of a row, 8 consecutive values per lane (two 16-byte loads), one 8-byte
+// store per lane.
 __device__ __forceinline__ void quantize_rows_fp8(unsigned bx, const float *__restrict__ src, int rows, int cols,
-                                                  int ld, int rows_p, int kp, int vec, uint8_t *__restrict__ q,
+                                                  int ld, int rows_p, int kp, uint8_t *__restrict__ q,
                                                   uint8_t *__restrict__ scales) {
   const int64_t group = (int64_t(bx) * 256 + threadIdx.x) / 16;
   const int l16 = threadIdx.x % 16;
@@ -270,9 +272,10 @@ __device__ __forceinline__ void quantize_rows_fp8(unsigned bx, const float *__re
   const int k = kb * 128 + 8 * l16;
   const float *p = src + int64_t(r) * ld + k;
   float v[8];
-  if (vec && r < rows && k + 8 <= cols) {
-    const float4 a = *reinterpret_cast<const float4 *>(p), b = *reinterpret_cast<const float4 *>(p + 4);
-    v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+  if (r < rows && k + 8 <= cols) {
+    const f4u a = *reinterpret_cast<const f4u *>(p), b = *reinterpret_cast<const f4u *>(p + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = a[e], v[4 + e] = b[e];
   } else {
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = (r < rows && k + e < cols) ? p[e] : 0.0f;
@@ -290,51 +293,29 @@ __device__ __forceinline__ void quantize_rows_fp8(unsigned bx, const float *__re
 }
 
 // B (K x N, N contiguous) -> Y[rows_p][kp] e4m3 (row n = column n of B) plus
-// scales[kb * rows_p + n]: a block stages 128 K x 64 N in LDS (16-byte loads along N when
-// `vec`, all in flight when the tile lies inside the source), then 4 lanes quantise one
+// scales[kb * rows_p + n]: a block stages 128 K x 64 N in LDS (16-byte loads along N, all
+// in flight together), then 4 lanes quantise one
 // column's 128-wide block, 32 consecutive K values per lane and two 16-byte stores each (the
 // column's 128 bytes are contiguous in Y).
 __device__ __forceinline__ void quantize_cols_fp8(unsigned bx, unsigned by, const float *__restrict__ src, int n_src,
-                                                  int k_src, int ld, int rows_p, int kp, int vec,
+                                                  int k_src, int ld, int rows_p, int kp,
                                                   uint8_t *__restrict__ q_out, uint8_t *__restrict__ scales) {
   __shared__ float tile[128][65];  // [k][n]; row stride 65 words: read j of lane (n, q) hits bank 32q + j + n
   const int n0 = int(bx) * 64, kb = int(by), k0 = kb * 128, t = threadIdx.x;
   const int c4 = (t % 16) * 4;  // first of the four columns this thread loads
-  if (vec && n0 + 64 <= n_src && k0 + 128 <= k_src) {
-    float4 a[8];
+  f4u a[8];
+  if (n0 + 64 <= n_src && k0 + 128 <= k_src) {
 #pragma unroll
     for (int i = 0; i < 8; ++i)
-      a[i] = *reinterpret_cast<const float4 *>(src + int64_t(k0 + t / 16 + 16 * i) * ld + (n0 + c4));
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int k = t / 16 + 16 * i;
-      tile[k][c4] = a[i].x;
-      tile[k][c4 + 1] = a[i].y;
-      tile[k][c4 + 2] = a[i].z;
-      tile[k][c4 + 3] = a[i].w;
-    }
+      a[i] = *reinterpret_cast<const f4u *>(src + int64_t(k0 + t / 16 + 16 * i) * ld + (n0 + c4));
   } else {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int k = t / 16 + 16 * i;
-      const float *p = src + int64_t(k0 + k) * ld + (n0 + c4);
-      float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      if (k0 + k < k_src) {
-        if (vec && n0 + c4 + 4 <= n_src) {
-          a = *reinterpret_cast<const float4 *>(p);
-        } else {
-          a.x = n0 + c4 < n_src ? p[0] : 0.0f;
-          a.y = n0 + c4 + 1 < n_src ? p[1] : 0.0f;
-          a.z = n0 + c4 + 2 < n_src ? p[2] : 0.0f;
-          a.w = n0 + c4 + 3 < n_src ? p[3] : 0.0f;
-        }
-      }
-      tile[k][c4] = a.x;
-      tile[k][c4 + 1] = a.y;
-      tile[k][c4 + 2] = a.z;
-      tile[k][c4 + 3] = a.w;
-    }
+    for (int i = 0; i < 8; ++i) a[i] = load_b4(src, n_src, k_src, ld, n0 + c4, k0 + t / 16 + 16 * i);
   }
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tile[t / 16 + 16 * i][c4 + e] = a[i][e];
   __syncthreads();
   // 4 lanes per column, 32 consecutive K values each: lane q of column n quantises K rows
   // 32q..32q+31 of the tile and stores them as 32 contiguous bytes of Y's row n.
@@ -366,11 +347,11 @@ __device__ __forceinline__ void quantize_cols_fp8(unsigned bx, unsigned by, cons
 // the call pays one dispatch instead of two.
 struct PackArgs {
   const float *a;
-  int m, k, lda, mp, kp, vec_a;
+  int m, k, lda, mp, kp;
   void *x;
   unsigned row_blocks;
   const float *b;
-  int n, ldb, np, vec_b;
+  int n, ldb, np;
   void *y;
   unsigned cols_gx;
   uint8_t *sx, *sy;  // FP8: the scales of A's rows and B's columns
@@ -381,23 +362,23 @@ __global__ __launch_bounds__(256) void pack_operands_kernel(PackArgs p) {
   const unsigned b = blockIdx.x;
   if (b < p.row_blocks) {
     if constexpr (KIND == kFP8)
-      quantize_rows_fp8(b, p.a, p.m, p.k, p.lda, p.mp, p.kp, p.vec_a, static_cast<uint8_t *>(p.x), p.sx);
+      quantize_rows_fp8(b, p.a, p.m, p.k, p.lda, p.mp, p.kp, static_cast<uint8_t *>(p.x), p.sx);
     else if constexpr (KIND == kF32)
-      pack_rows_f32(b, p.a, p.m, p.k, p.lda, p.mp, p.kp, p.vec_a, static_cast<float *>(p.x));
+      pack_rows_f32(b, p.a, p.m, p.k, p.lda, p.mp, p.kp, static_cast<float *>(p.x));
     else
-      pack_rows_bf16<KIND == kBF16X3>(b, p.a, p.m, p.k, p.lda, p.mp, p.kp, p.vec_a, static_cast<char *>(p.x));
+      pack_rows_bf16<KIND == kBF16X3>(b, p.a, p.m, p.k, p.lda, p.mp, p.kp, static_cast<char *>(p.x));
     return;
   }
   const unsigned c = b - p.row_blocks;
   if constexpr (KIND == kFP8)
-    quantize_cols_fp8(c % p.cols_gx, c / p.cols_gx, p.b, p.n, p.k, p.ldb, p.np, p.kp, p.vec_b,
+    quantize_cols_fp8(c % p.cols_gx, c / p.cols_gx, p.b, p.n, p.k, p.ldb, p.np, p.kp,
                       static_cast<uint8_t *>(p.y), p.sy);
   else if constexpr (KIND == kF32)
-    pack_cols_f32<kPackTN>(c % p.cols_gx, c / p.cols_gx, p.b, p.n, p.k, p.ldb, p.np, p.kp, p.vec_b,
+    pack_cols_f32<kPackTN>(c % p.cols_gx, c / p.cols_gx, p.b, p.n, p.k, p.ldb, p.np, p.kp,
                            static_cast<float *>(p.y));
   else
     pack_cols_bf16<KIND == kBF16X3, kPackTN>(c % p.cols_gx, c / p.cols_gx, p.b, p.n, p.k, p.ldb, p.np, p.kp,
-                                              p.vec_b, static_cast<char *>(p.y));
+                                              static_cast<char *>(p.y));
 }
 
 // ------------------------------------------------------------------------ main kernel
@@ -746,8 +727,6 @@ __global__ __launch_bounds__(kThreads, W * kBufs == 4 ? 2 : 1) void gemm_lds_ker
 // kWK = 1 the four waves take four tiles below one another instead. The operands of the next step
 // load while the current one's MFMAs run.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
 
 template <int KIND>
 constexpr int kDirectVals = KIND == kF32 ? 4 : KIND == kFP8 ? 32 : 8;
@@ -1012,7 +991,7 @@ constexpr unsigned kMinExponent = 24, kMinProduct = 254 - 110;
 
 struct SplitArgs {
   const float *a, *b;
-  int m, n, k, lda, ldb, mp, np, kp, vec_a;
+  int m, n, k, lda, ldb, mp, np, kp;
   char *x, *y;         // [kp / 16][3][mp or np][16] BF16
   uint8_t *ea, *eb;    // least exponents: [mp / 64][chunks] and [np / 64][chunks], chunks of 64 K
   unsigned row_blocks;
@@ -1065,11 +1044,11 @@ __global__ __launch_bounds__(256) void split_operands_kernel(SplitArgs p) {
     float v[16];
     if (is_a) {
       const float *src = p.a + int64_t(row) * p.lda + k;
-      if (p.vec_a && row < p.m && k + 16 <= p.k) {
+      if (row < p.m && k + 16 <= p.k) {
 #pragma unroll
         for (int e = 0; e < 16; e += 4) {
-          const float4 x = *reinterpret_cast<const float4 *>(src + e);
-          v[e] = x.x, v[e + 1] = x.y, v[e + 2] = x.z, v[e + 3] = x.w;
+          const f4u x = *reinterpret_cast<const f4u *>(src + e);
+          v[e] = x[0], v[e + 1] = x[1], v[e + 2] = x[2], v[e + 3] = x[3];
         }
       } else {
 #pragma unroll
@@ -1268,16 +1247,14 @@ void run_lds(cs_stream *stream, int M, int N, int K, const float *A, int lda, co
   char *x = base, *y = base + xbytes;
   uint8_t *sx = nullptr, *sy = nullptr;
   hipStream_t s = stream->stream;
-  const int vec_a = (lda % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0) ? 1 : 0;
-  const int vec_b = (ldb % 4 == 0 && reinterpret_cast<uintptr_t>(B) % 16 == 0) ? 1 : 0;
   if constexpr (KIND == kFP8) {
     sx = reinterpret_cast<uint8_t *>(base + xbytes + ybytes);
     sy = sx + Mp * (Kp / 128);
   }
   {
     PackArgs pa;
-    pa.a = A, pa.m = M, pa.k = K, pa.lda = lda, pa.mp = int(Mp), pa.kp = int(Kp), pa.vec_a = vec_a, pa.x = x;
-    pa.b = B, pa.n = N, pa.ldb = ldb, pa.np = int(Np), pa.vec_b = vec_b, pa.y = y;
+    pa.a = A, pa.m = M, pa.k = K, pa.lda = lda, pa.mp = int(Mp), pa.kp = int(Kp), pa.x = x;
+    pa.b = B, pa.n = N, pa.ldb = ldb, pa.np = int(Np), pa.y = y;
     pa.sx = sx, pa.sy = sy;
     int64_t col_tiles_k;
     if constexpr (KIND == kFP8) {  // 16 lanes per 128-wide block of a row; 128 K x 64 N column tiles
@@ -1316,7 +1293,6 @@ bool run_split(cs_stream *stream, int M, int N, int K, const float *A, int lda, 
   char *base = static_cast<char *>(stream_scratch(stream, static_cast<size_t>(xbytes + ybytes + ebytes + 4096)));
   SplitArgs p;
   p.a = A, p.b = B, p.m = M, p.n = N, p.k = K, p.lda = lda, p.ldb = ldb, p.mp = int(Mp), p.np = int(Np), p.kp = int(Kp);
-  p.vec_a = (lda % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0) ? 1 : 0;
   p.x = base, p.y = base + xbytes;
   p.ea = reinterpret_cast<uint8_t *>(base + xbytes + ybytes), p.eb = p.ea + Mp / 64 * chunks;
   p.row_blocks = unsigned(Mp / 64 * chunks);

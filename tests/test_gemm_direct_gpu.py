@@ -116,3 +116,23 @@ def test_ring_of_four_stages(gpu_tensors, variant, k):
         assert fp64.gemm_normalized_error(c, a, b) <= BOUND[variant]
     for h in (ba, bb, bc):
         h.release()
+
+
+@pytest.mark.parametrize("variant", sorted(VARIANTS))
+@pytest.mark.parametrize("shift", [1, 2, 3])
+def test_packed_at_any_4_byte_boundary(gpu_tensors, variant, shift):
+    """Packed operands whose rows start off the 16-byte grid, inside larger matrices."""
+    T = gpu_tensors
+    M, N, K = 1800, 1700, 133
+    lda, ldb = K + shift, N + shift
+    a = inputs.uniform(M * lda, 4071).reshape(M, lda)
+    b = inputs.uniform(K * ldb, 4072).reshape(K, ldb)
+    ba = upload(T, np.concatenate([np.full(shift, np.nan), a.ravel()]))
+    bb = upload(T, np.concatenate([np.full(shift, np.nan), b.ravel()]))
+    bc = alloc(T, M * N)
+    capi.check(capi.lib.cs_gemm(T.stream, VARIANTS[variant], M, N, K, ba.ptr + 4 * shift, lda, bb.ptr + 4 * shift, ldb,
+                                bc.ptr, N))
+    c = download(T, bc, M * N).reshape(M, N)
+    assert fp64.gemm_normalized_error(c, a[:, :K].copy(), b[:, :N].copy()) <= BOUND[variant]
+    for h in (ba, bb, bc):
+        h.release()

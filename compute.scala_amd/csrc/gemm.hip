@@ -446,15 +446,18 @@ __device__ __forceinline__ void run_stages(int stages, Stage &stage) {
   stage(ks, std::false_type(), std::false_type());
 }
 
+// The first of slice i's stages, of n stages cut into `slices` runs.
+__device__ __forceinline__ int slice_begin(int n, unsigned i, int slices) {
+  return slices == 1 ? int(i) * n : int(int64_t(n) * i / slices);
+}
+
+// Slice blockIdx.y of K; several slices write partial results C[slice][M][ldc].
 // X: [Mp] rows of Kp * kBytesPerK bytes, Y: [Np] rows likewise. sx / sy: FP8 scales
 // [Kp/128][Mp] and [Kp/128][Np]. Host guarantees 256 * row bytes < 2^31.
 template <int KIND, int W, int kBufs>
-__global__ __launch_bounds__(kThreads, W * kBufs == 4 ? 2 : 1) void gemm_lds_kernel(int M, int N, int Kp, int Mp, int Np,
-                                                               const char *__restrict__ X,
-                                                               const char *__restrict__ Y,
-                                                               const uint8_t *__restrict__ sx,
-                                                               const uint8_t *__restrict__ sy,
-                                                               float *__restrict__ C, int ldc) {
+__global__ __launch_bounds__(kThreads, W * kBufs == 4 ? 2 : 1) void gemm_lds_kernel(
+    int M, int N, int Kp, int Mp, int Np, const char *__restrict__ X, const char *__restrict__ Y,
+    const uint8_t *__restrict__ sx, const uint8_t *__restrict__ sy, float *__restrict__ C, int ldc, int slices) {
   using P = Pipe<KIND>;
   using F = typename P::Frag;
   constexpr int kTile = tile_edge(W), kWaveRows = 32 * W, kPanelB = panel_bytes(W), kStageB = 2 * kPanelB;
@@ -468,7 +471,9 @@ __global__ __launch_bounds__(kThreads, W * kBufs == 4 ? 2 : 1) void gemm_lds_ker
   tile_coords(blockIdx.x, Mp / kTile, Np / kTile, tm, tn);
   const int m0 = tm * kTile, n0 = tn * kTile;
   const int rowb = Kp * P::kBytesPerK;
-  const int stages = Kp / P::kK;
+  const int first = slice_begin(Kp / P::kK, blockIdx.y, slices);
+  const int stages = slice_begin(Kp / P::kK, blockIdx.y + 1, slices) - first;
+  C += int64_t(blockIdx.y) * M * ldc;
 
   // Global -> LDS. One DMA instruction of a wave fills a 1 KiB chunk = 8 rows of a panel,
   // lane l writing LDS bytes 16 l .. 16 l + 15: slot l & 7 of row l >> 3 of the chunk. Row R
@@ -484,7 +489,7 @@ __global__ __launch_bounds__(kThreads, W * kBufs == 4 ? 2 : 1) void gemm_lds_ker
       __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(Y) + int64_t(n0) * rowb, 0, kTile * rowb, 0x00020000);
   auto dma = [&](int d, int ks, int buf) {
     const int j = d >> 1;
-    const unsigned soff = unsigned(32 * j * rowb + ks * kRowB);
+    const unsigned soff = unsigned(32 * j * rowb + (first + ks) * kRowB);
     char *l = lds + buf * kStageB + (d & 1) * kPanelB + (4 * j + wave) * 1024;
     __builtin_amdgcn_raw_ptr_buffer_load_lds((d & 1) ? ry : rx, (lds_void *)(l), 16, voff, soff, 0, 0);
   };
@@ -532,8 +537,8 @@ __global__ __launch_bounds__(kThreads, W * kBufs == 4 ? 2 : 1) void gemm_lds_ker
 #pragma unroll
     for (int i = 0; i < W; ++i) {
       if constexpr (KIND == kFP8) {
-        sa[set][i] = sx[int64_t(ks) * Mp + m0 + wm * kWaveRows + i * 32 + l32];
-        sb[set][i] = sy[int64_t(ks) * Np + n0 + wn * kWaveRows + i * 32 + l32];
+        sa[set][i] = sx[int64_t(first + ks) * Mp + m0 + wm * kWaveRows + i * 32 + l32];
+        sb[set][i] = sy[int64_t(first + ks) * Np + n0 + wn * kWaveRows + i * 32 + l32];
       } else {
         sa[set][i] = sb[set][i] = 0;
       }
@@ -936,13 +941,15 @@ __device__ __forceinline__ void store_tile(int M, int N, float *__restrict__ C, 
 template <int KIND, int T, int kWK>
 __global__ __launch_bounds__(kWK == 1 ? 256 : 64 * kWK) void gemm_direct_kernel(
     int M, int N, int K, const float *__restrict__ A, int lda, const float *__restrict__ B, int ldb,
-    float *__restrict__ C, int ldc, int tiles_m) {
+    float *__restrict__ C, int ldc, int tiles_m, int slices) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int tm = int(blockIdx.x) % tiles_m, tn = int(blockIdx.x) / tiles_m;
   const int m0 = (kWK == 1 ? tm * 4 + wave : tm) * 16 * T, n0 = tn * 16 * T;
   f32x4 acc[T][T];
-  direct_tile<KIND, T>(M, N, K, A, lda, B, ldb, m0, n0, lane, kWK == 1 ? 0 : wave, kWK, acc);
+  direct_tile<KIND, T>(M, N, K, A, lda, B, ldb, m0, n0, lane, int(blockIdx.y) * kWK + (kWK == 1 ? 0 : wave),
+                       kWK * slices, acc);
+  C += int64_t(blockIdx.y) * M * ldc;
   if constexpr (kWK == 1) {
     store_tile<T>(M, N, C, ldc, m0, n0, lane, acc);
   } else {
@@ -1081,13 +1088,10 @@ __global__ __launch_bounds__(256) void split_operands_kernel(SplitArgs p) {
 // 2048^3 101.9 us against 103.5). The operands are packed so that each part of a stage is contiguous:
 // DMA and fragment reads are linear in LDS, without bank conflicts.
 template <int W>
-__global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_split_kernel(int M, int N, int K, int Kp, int Mp, int Np,
-                                                                 const char *__restrict__ X, const char *__restrict__ Y,
-                                                                 const uint8_t *__restrict__ ea,
-                                                                 const uint8_t *__restrict__ eb,
-                                                                 const float *__restrict__ A, int lda,
-                                                                 const float *__restrict__ B, int ldb,
-                                                                 float *__restrict__ C, int ldc) {
+__global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_split_kernel(
+    int M, int N, int K, int Kp, int Mp, int Np, const char *__restrict__ X, const char *__restrict__ Y,
+    const uint8_t *__restrict__ ea, const uint8_t *__restrict__ eb, const float *__restrict__ A, int lda,
+    const float *__restrict__ B, int ldb, float *__restrict__ C, int ldc, int slices) {
   constexpr int kTile = tile_edge(W), kWaveRows = 32 * W, kPartB = part_bytes(W), kSplitPanelB = 3 * kPartB,
                 kSplitStageB = 2 * kSplitPanelB;
   extern __shared__ __attribute__((aligned(1024))) char lds[];
@@ -1097,6 +1101,8 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_split_kernel(in
   int tm, tn;
   tile_coords(blockIdx.x, Mp / kTile, Np / kTile, tm, tn);
   const int m0 = tm * kTile, n0 = tn * kTile;
+
+  C += int64_t(blockIdx.y) * M * ldc;
 
   {
     unsigned *const least = reinterpret_cast<unsigned *>(lds);
@@ -1118,7 +1124,7 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_split_kernel(in
         const int ms = m0 + wm * kWaveRows + sub / (W / 2) * 64, ns = n0 + wn * kWaveRows + sub % (W / 2) * 64;
         if (ms >= M || ns >= N) continue;
         f32x4 acc[4][4];
-        direct_tile<kF32, 4>(M, N, K, A, lda, B, ldb, ms, ns, lane, 0, 1, acc);
+        direct_tile<kF32, 4>(M, N, K, A, lda, B, ldb, ms, ns, lane, int(blockIdx.y), slices, acc);
         store_tile<4>(M, N, C, ldc, ms, ns, lane, acc);
       }
       return;
@@ -1129,11 +1135,12 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_split_kernel(in
   const int rows_p = wave < 2 ? Mp : Np;
   const char *const from = wave < 2 ? X + int64_t(m0) * 32 : Y + int64_t(n0) * 32;
   const int part_stride = rows_p * 32;
-  const int stages = Kp / kSplitK;
+  const int first = slice_begin(Kp / kSplitK, blockIdx.y, slices);
+  const int stages = slice_begin(Kp / kSplitK, blockIdx.y + 1, slices) - first;
   const unsigned voff = unsigned(lane) * 16;
   auto dma = [&](int ks, int buf) {
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char *>(from) + int64_t(ks) * 3 * part_stride, 0, 2 * part_stride + kPartB, 0x00020000);
+        const_cast<char *>(from) + int64_t(first + ks) * 3 * part_stride, 0, 2 * part_stride + kPartB, 0x00020000);
     char *const l = lds + buf + (wave >> 1) * kSplitPanelB;
 #pragma unroll
     for (int i = 0; i < 3 * W; ++i) {
@@ -1224,6 +1231,58 @@ __global__ __launch_bounds__(256) void zero_matrix_kernel(float *__restrict__ C,
   C[(i / N) * ldc + i % N] = 0.0f;
 }
 
+// C = the sum of `slices` partial results [M][N] in their order, four values per thread. Bound by its launch
+// (64 x 64 of 16 slices) or its reads (1024 x 1024 of 4: 16 MiB).
+__global__ __launch_bounds__(256) void sum_slices_kernel(const float *__restrict__ part, int64_t n, int slices,
+                                                         int N, float *__restrict__ C, int ldc) {
+  const int64_t i = (int64_t(blockIdx.x) * 256 + threadIdx.x) * 4;
+  if (i >= n) return;
+  const float *p = part + i;
+  if (i + 4 <= n) {
+    f4u v = *reinterpret_cast<const f4u *>(p);
+#pragma unroll 4
+    for (int s = 1; s < slices; ++s) v += *reinterpret_cast<const f4u *>(p + int64_t(s) * n);
+    const int64_t r = i / N, c = i % N;
+    if (ldc == N || c + 4 <= N) {
+      *reinterpret_cast<f4u *>(C + r * ldc + c) = v;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) C[(i + e) / N * ldc + (i + e) % N] = v[e];
+    }
+  } else {
+    for (int e = 0; i + e < n; ++e) {
+      float v = p[e];
+      for (int s = 1; s < slices; ++s) v += p[int64_t(s) * n + e];
+      C[(i + e) / N * ldc + (i + e) % N] = v;
+    }
+  }
+}
+
+// Where the workgroups of a product write: C, or partial results in the stream's scratch behind `used`
+// bytes of operands. Without room for them in a captured stream's scratch, K stays whole.
+struct Target {
+  char *scratch;
+  float *out;
+  int ld, slices;
+
+  Target(cs_stream *stream, int64_t used, int M, int N, float *C, int ldc, int wanted) : slices(wanted) {
+    used = round_up(used, 256);
+    int64_t total = used;
+    if (slices > 1) total += int64_t(slices) * M * N * 4;
+    if (slices > 1 && !scratch_fits(stream, size_t(total))) slices = 1, total = used;
+    scratch = total ? static_cast<char *>(stream_scratch(stream, size_t(total))) : nullptr;
+    out = slices > 1 ? reinterpret_cast<float *>(scratch + used) : C;
+    ld = slices > 1 ? N : ldc;
+  }
+  void combine(cs_stream *stream, int M, int N, float *C, int ldc) const {
+    const int64_t n = int64_t(M) * N;
+    if (slices > 1)
+      hipLaunchKernelGGL(sum_slices_kernel, dim3(unsigned((n + 1023) / 1024)), dim3(256), 0, stream->stream, out, n,
+                         slices, N, C, ldc);
+    CS_HIP(hipGetLastError());
+  }
+};
+
 // The packed kernel's row offsets are 32 bits wide; K is held to that on every path.
 template <int KIND>
 void check_depth(int K) {
@@ -1235,7 +1294,7 @@ void check_depth(int K) {
 
 template <int KIND, int W, int kBufs>
 void run_lds(cs_stream *stream, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
-             int ldc) {
+             int ldc, int slices) {
   using P = Pipe<KIND>;
   constexpr int kTile = tile_edge(W);
   const int64_t Mp = round_up(M, kTile), Np = round_up(N, kTile), Kp = round_up(K, P::kK);
@@ -1243,8 +1302,8 @@ void run_lds(cs_stream *stream, int M, int N, int K, const float *A, int lda, co
   const int64_t xbytes = Mp * rowb, ybytes = Np * rowb;
   int64_t total = xbytes + ybytes + 4096;
   if (KIND == kFP8) total += (Mp + Np) * (Kp / 128) + 4096;
-  char *base = static_cast<char *>(stream_scratch(stream, static_cast<size_t>(total)));
-  char *x = base, *y = base + xbytes;
+  const Target to(stream, total, M, N, C, ldc, slices);
+  char *const base = to.scratch, *x = base, *y = base + xbytes;
   uint8_t *sx = nullptr, *sy = nullptr;
   hipStream_t s = stream->stream;
   if constexpr (KIND == kFP8) {
@@ -1275,22 +1334,26 @@ void run_lds(cs_stream *stream, int M, int N, int K, const float *A, int lda, co
     return true;
   }();
   (void)configured;
-  const unsigned grid = static_cast<unsigned>((Mp / kTile) * (Np / kTile));
-  hipLaunchKernelGGL((gemm_lds_kernel<KIND, W, kBufs>), dim3(grid), dim3(kThreads), lds_bytes(W, kBufs), s, M, N, int(Kp), int(Mp),
-                     int(Np), x, y, sx, sy, C, ldc);
-  CS_HIP(hipGetLastError());
+  const dim3 grid(static_cast<unsigned>((Mp / kTile) * (Np / kTile)), unsigned(to.slices));
+  hipLaunchKernelGGL((gemm_lds_kernel<KIND, W, kBufs>), grid, dim3(kThreads), lds_bytes(W, kBufs), s, M, N, int(Kp),
+                     int(Mp), int(Np), x, y, sx, sy, to.out, to.ld, to.slices);
+  to.combine(stream, M, N, C, ldc);
 }
 
-// FP32 from three BF16 parts. False when the operands are too tall for its 32-bit offsets.
+// FP32 from three BF16 parts. False when the operands are too tall for its 32-bit offsets or, in a
+// captured stream, too large for its scratch (three parts are 6 bytes of a value, the FP32 kernel's 4).
 template <int W>
 bool run_split(cs_stream *stream, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
-               int ldc) {
+               int ldc, int slices) {
   constexpr int kTile = tile_edge(W);
   const int64_t Mp = round_up(M, kTile), Np = round_up(N, kTile), Kp = round_up(K, kSplitK);
   if (std::max(Mp, Np) * 96 >= (int64_t(1) << 31)) return false;
   const int64_t xbytes = Mp * Kp * 6, ybytes = Np * Kp * 6, chunks = (Kp + 63) / 64;
   const int64_t ebytes = (Mp + Np) / 64 * chunks;
-  char *base = static_cast<char *>(stream_scratch(stream, static_cast<size_t>(xbytes + ybytes + ebytes + 4096)));
+  const int64_t total = xbytes + ybytes + ebytes + 4096;
+  if (!scratch_fits(stream, size_t(total))) return false;
+  const Target to(stream, total, M, N, C, ldc, slices);
+  char *const base = to.scratch;
   SplitArgs p;
   p.a = A, p.b = B, p.m = M, p.n = N, p.k = K, p.lda = lda, p.ldb = ldb, p.mp = int(Mp), p.np = int(Np), p.kp = int(Kp);
   p.x = base, p.y = base + xbytes;
@@ -1304,23 +1367,24 @@ bool run_split(cs_stream *stream, int M, int N, int K, const float *A, int lda, 
     return true;
   }();
   (void)configured;
-  hipLaunchKernelGGL(gemm_split_kernel<W>, dim3(unsigned((Mp / kTile) * (Np / kTile))), dim3(kThreads),
-                     split_lds_bytes(W),
-                     stream->stream, M, N, K, int(Kp), int(Mp), int(Np), p.x, p.y, p.ea, p.eb, A, lda, B, ldb, C, ldc);
-  CS_HIP(hipGetLastError());
+  const dim3 grid(unsigned((Mp / kTile) * (Np / kTile)), unsigned(to.slices));
+  hipLaunchKernelGGL(gemm_split_kernel<W>, grid, dim3(kThreads), split_lds_bytes(W), stream->stream, M, N, K, int(Kp),
+                     int(Mp), int(Np), p.x, p.y, p.ea, p.eb, A, lda, B, ldb, to.out, to.ld, to.slices);
+  to.combine(stream, M, N, C, ldc);
   return true;
 }
 
 template <int KIND, int T, int kWK>
 void run_direct(cs_stream *stream, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
-                int ldc) {
+                int ldc, int slices) {
   const int64_t rows = 16 * T * (kWK == 1 ? 4 : 1);  // of C per workgroup
   const int64_t tiles_m = (M + rows - 1) / rows, tiles_n = (N + 16 * T - 1) / (16 * T);
   const size_t lds = kWK == 1 ? 0 : size_t(kWK) * 256 * T * T * sizeof(float);
-  hipLaunchKernelGGL((gemm_direct_kernel<KIND, T, kWK>), dim3(unsigned(tiles_m * tiles_n)),
-                     dim3(kWK == 1 ? 256 : 64 * kWK), lds, stream->stream, M, N, K, A, lda, B, ldb, C, ldc,
-                     int(tiles_m));
-  CS_HIP(hipGetLastError());
+  const Target to(stream, 0, M, N, C, ldc, slices);
+  hipLaunchKernelGGL((gemm_direct_kernel<KIND, T, kWK>), dim3(unsigned(tiles_m * tiles_n), unsigned(to.slices)),
+                     dim3(kWK == 1 ? 256 : 64 * kWK), lds, stream->stream, M, N, K, A, lda, B, ldb, to.out, to.ld,
+                     int(tiles_m), to.slices);
+  to.combine(stream, M, N, C, ldc);
 }
 
 // The direct kernel's launch shape. Where the lines lie (FP32 calls, in us, "T.kWK"):
@@ -1366,6 +1430,10 @@ bool overlap(const float *a, int64_t rows_a, int64_t cols_a, int lda, const floa
 // LDS), 128 x 128 tiles (two stages, two workgroups on a CU) or 128 x 128 tiles with four stages, one
 // workgroup on a CU.
 enum Path { kDirect, kTiles256, kTiles128, kDeep128 };
+struct Plan {
+  Path path;
+  int slices;  // of K, each with workgroups of its own, added by a launch after them
+};
 
 // Each path's time is estimated from what it was measured to take (us): the direct kernel's from the
 // flops of its padded tiles at the rate of its tile size, with the CUs its last round leaves idle; the
@@ -1381,10 +1449,14 @@ enum Path { kDirect, kTiles256, kTiles128, kDeep128 };
 //           655 / 356 / 377 / 326
 //   FP8     512^3 6.5 / 10.2 / 9.8 / 20, 2048^3 259 / 28 / 24 / 46, 2500^3 522 / 40 / 46 / 61, 4096^3
 //           2024 / 99 / 110 / 95
-// With 128 tiles on 64 of the CUs (1024x1024x4096) a stage of two waits for the DMA of the next: BF16
+// Where a path starts too few workgroups for the CUs, K is cut into slices with workgroups of their own,
+// counted at 3 us of launches and 8 bytes of traffic per partial result, and taken where that gains 5%
+// (1 / chosen slices): FP32 64x64x4096 11.2 / 7.1 (16 of the direct kernel), 632x1305x3146 103 / 59 (128
+// tiles, 4), BF16 128x1024x4096 27 / 20 (8), 1024x1024x4096 40 / 29 (3), FP8 64x64x4096 16.2 / 6.8.
+// With 128 tiles on 64 of the CUs (1024x1024x4096, unsliced) a stage of two waits for the DMA of the next: BF16
 // 55 us, with four 40; FP8 38 / 29.
 template <int KIND>
-Path choose_path(double cus, double M, double N, double K, const DirectPlan &p) {
+Plan choose_path(double cus, double M, double N, double K, const DirectPlan &p) {
   struct Rates {
     double direct[3];   // TFLOP/s of T = 1, 2, 4
     double base;        // of a packed call, and what 256 x 256 tiles add
@@ -1404,22 +1476,34 @@ Path choose_path(double cus, double M, double N, double K, const DirectPlan &p) 
   const double e = 16.0 * p.t, blocks = p.wk == 1 ? std::ceil(std::ceil(M / e) / 4) * std::ceil(N / e) : tiles(e);
   const double packed = r.base + r.pack * (M + N) * K + 0.5e-6 * M * N;
   const double t256 = tiles(256), r128 = rounds(tiles(128)), pairs = std::floor(r128 / 2);
+  const double flops = 2e-6 * tiles(e) * e * e * K / r.direct[p.t / 2], out = (KIND == kF32 ? 0.5e-6 : 1.2e-6) * M * N;
+  auto direct = [&](double slices) { return 4 + flops * rounds(blocks * slices) * cus / (blocks * slices) + out; };
   const double time[] = {
-      4 + 2e-6 * tiles(e) * e * e * K / r.direct[p.t / 2] * rounds(blocks) * cus / blocks +
-          (KIND == kF32 ? 0.5e-6 : 1.2e-6) * M * N,
+      direct(1),
       packed + r.base_256 + K * rounds(t256) * (t256 <= 0.75 * cus ? r.t256_few : r.t256),
       packed + K * (pairs * r.t128_pair + (r128 - 2 * pairs) * r.t128),
       r128 == 1 ? packed + K * r.deep : 1e30,  // in several rounds nothing hides their ends
   };
-  return Path(std::min_element(time, time + 4) - time);
+  const int path = int(std::min_element(time, time + 4) - time);
+  Plan best = {Path(path), 1};
+  double least = time[path];
+  auto consider = [&](Path candidate, int slices, double t) {
+    t += 3 + 1.2e-6 * slices * M * N;
+    if (t < 0.95 * least) best = {candidate, slices}, least = t;
+  };
+  const double steps = K / (KIND == kF32 ? 16 : KIND == kFP8 ? 128 : 32);
+  for (int s = 2; s <= 16 && blocks * s <= cus && p.wk * s <= steps; s *= 2) consider(kDirect, s, direct(s));
+  for (int s = 2; s <= 8 && tiles(128) * s <= cus && 128 * s <= K; ++s)
+    consider(KIND == kF32 ? kTiles128 : kDeep128, s, packed + K / s * (KIND == kF32 ? r.t128 : r.deep));
+  return best;
 }
 
 template <int KIND, int W, int kBufs>
 void run_packed(cs_stream *stream, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
-                int ldc, bool over) {
+                int ldc, bool over, int slices) {
   if constexpr (KIND == kF32)
-    if (!over && run_split<W>(stream, M, N, K, A, lda, B, ldb, C, ldc)) return;
-  run_lds<KIND, W, kBufs>(stream, M, N, K, A, lda, B, ldb, C, ldc);
+    if (!over && run_split<W>(stream, M, N, K, A, lda, B, ldb, C, ldc, slices)) return;
+  run_lds<KIND, W, kBufs>(stream, M, N, K, A, lda, B, ldb, C, ldc, slices);
 }
 
 template <int KIND>
@@ -1429,24 +1513,25 @@ void run(cs_stream *stream, int M, int N, int K, const float *A, int lda, const 
   const DirectPlan p = plan_direct(KIND, cus, M, N, K);
   // A C that overlaps A or B is written only from copies of both.
   const bool over = overlap(A, M, K, lda, C, M, N, ldc) || overlap(B, K, N, ldb, C, M, N, ldc);
-  Path path = choose_path<KIND>(double(cus), M, N, K, p);
-  if (over && path == kDirect) path = kTiles128;
-  if (path == kTiles256) return run_packed<KIND, 4, 2>(stream, M, N, K, A, lda, B, ldb, C, ldc, over);
-  if (path == kTiles128) return run_packed<KIND, 2, 2>(stream, M, N, K, A, lda, B, ldb, C, ldc, over);
+  Plan plan = choose_path<KIND>(double(cus), M, N, K, p);
+  if (over && plan.path == kDirect) plan = {kTiles128, 1};
+  const int z = plan.slices;
+  if (plan.path == kTiles256) return run_packed<KIND, 4, 2>(stream, M, N, K, A, lda, B, ldb, C, ldc, over, z);
+  if (plan.path == kTiles128) return run_packed<KIND, 2, 2>(stream, M, N, K, A, lda, B, ldb, C, ldc, over, z);
   if constexpr (KIND != kF32)
-    if (path == kDeep128) return run_packed<KIND, 2, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc, over);
+    if (plan.path == kDeep128) return run_packed<KIND, 2, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc, over, z);
   switch (p.t * 100 + p.wk) {
-    case 101: return run_direct<KIND, 1, 1>(stream, M, N, K, A, lda, B, ldb, C, ldc);
-    case 104: return run_direct<KIND, 1, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc);
-    case 201: return run_direct<KIND, 2, 1>(stream, M, N, K, A, lda, B, ldb, C, ldc);
-    case 204: return run_direct<KIND, 2, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc);
+    case 101: return run_direct<KIND, 1, 1>(stream, M, N, K, A, lda, B, ldb, C, ldc, z);
+    case 104: return run_direct<KIND, 1, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc, z);
+    case 201: return run_direct<KIND, 2, 1>(stream, M, N, K, A, lda, B, ldb, C, ldc, z);
+    case 204: return run_direct<KIND, 2, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc, z);
   }
   if constexpr (KIND != kFP8) {
     switch (p.t * 100 + p.wk) {
-      case 116: return run_direct<KIND, 1, 16>(stream, M, N, K, A, lda, B, ldb, C, ldc);
-      case 208: return run_direct<KIND, 2, 8>(stream, M, N, K, A, lda, B, ldb, C, ldc);
-      case 401: return run_direct<KIND, 4, 1>(stream, M, N, K, A, lda, B, ldb, C, ldc);
-      case 404: return run_direct<KIND, 4, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc);
+      case 116: return run_direct<KIND, 1, 16>(stream, M, N, K, A, lda, B, ldb, C, ldc, z);
+      case 208: return run_direct<KIND, 2, 8>(stream, M, N, K, A, lda, B, ldb, C, ldc, z);
+      case 401: return run_direct<KIND, 4, 1>(stream, M, N, K, A, lda, B, ldb, C, ldc, z);
+      case 404: return run_direct<KIND, 4, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc, z);
     }
   }
   fail(CS_INVALID_OPERATION, "no direct GEMM kernel for this plan");

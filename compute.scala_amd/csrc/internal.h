@@ -201,6 +201,8 @@ namespace csmi {
 // synchronizes the stream, so the first call of a given size must not be under capture.
 // The buffer it replaces stays allocated until the stream is destroyed.
 void *stream_scratch(cs_stream *stream, size_t bytes);
+// Whether stream_scratch gives that much now: it is there already, or the stream is not capturing.
+bool scratch_fits(cs_stream *stream, size_t bytes);
 // FP64 block partials of a sum in the stream's scratch (n of them), and the fixed-order FP64
 // combine that turns n partials into *out (FP32, nullable) and *out64 (nullable).
 double *sum_partials(cs_stream *stream, size_t n);

@@ -264,12 +264,18 @@ std::vector<StreamEvent> record_on_all_streams(cs_device *device) {
   return evs;
 }
 
-void *stream_scratch(cs_stream *stream, size_t bytes) {
-  if (stream->scratch_bytes >= bytes) return stream->scratch;
+bool scratch_fits(cs_stream *stream, size_t bytes) {
+  if (stream->scratch_bytes >= bytes) return true;
   set_device(stream->device);
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   CS_HIP(hipStreamIsCapturing(stream->stream, &cap));
-  if (cap != hipStreamCaptureStatusNone)
+  return cap == hipStreamCaptureStatusNone;
+}
+
+void *stream_scratch(cs_stream *stream, size_t bytes) {
+  if (stream->scratch_bytes >= bytes) return stream->scratch;
+  set_device(stream->device);
+  if (!scratch_fits(stream, bytes))
     fail(CS_INVALID_OPERATION, "stream scratch must grow outside graph capture; run the call once first");
   CS_HIP(hipStreamSynchronize(stream->stream));
   // kept, not freed: graphs captured earlier on this stream may still address it

@@ -304,7 +304,17 @@ bool tiled_launch(const Dag &dag, const Options &o);
 // same (Emitter::ragged). In us against the widest dividing width, at about 4 million elements: view
 // chain with rows of 5 12.1 / 17.3, of 6 11.1 / 14.1, of 10 10.8 / 14.1, of 33 10.7 / 11.1, of 510
 // 9.0 / 9.8; a*b+c 10.6 / 12.3; 2049 x 2050 transpose plus matrix 13.8 / 18.9; their sums 11.9 / 17.5.
+// A join of several outputs gains nothing by it (below).
 constexpr int64_t kRaggedRow = 5;
+
+// The default vector width of a kernel with `outputs` joined outputs, where it divides the rows. A
+// thread's vector of V elements is V * outputs consecutive floats: up to four are one store, and a
+// wave's stores fill whole lines; longer runs leave each store instruction pieces of lines as far apart
+// as the runs are long. In us at V = 1 / 2 / 4, 4 million elements of a*c+b: 2 outputs 11.7 / 8.0 / 13.3,
+// 3 13.7 / 15.4 / 19.4, 4 12.6 / 18.0 / 25.0, 8 29.2 / 42.6 / 44.2, 12 50.9 / 61.5 / 61.9; from 14 on
+// level (71.7 / 70.7 / 71.5, 16 85.9 / 90.2 / 84.4). A 3 x 3 convolution of 800 x 48 x 48 to 6 filters
+// 16.4 / 20.8 / 30.6; 2048 x 2048 transposes joined 4 times 17.4 / 20.3 / 28.2.
+int joined_width(size_t outputs) { return outputs == 1 || outputs > 12 ? 4 : outputs == 2 ? 2 : 1; }
 
 Options resolve_options(const cs_fused_options *o, const Dag &dag) {
   Options r;
@@ -329,10 +339,10 @@ Options resolve_options(const cs_fused_options *o, const Dag &dag) {
   // A large body holds hundreds of values per element, so it defaults to 1 and 1 (the convolution
   // idiom: 9.3 us at V=1 against 25 us at V=2 and 50 us at V=4; two vectors per thread spill, 129 us).
   const bool large = dag.nodes.size() > kLargeBody;
-  if (r.V == 0 && !large && last >= kRaggedRow && last % 4 != 0) {
+  if (r.V == 0 && !large && dag.outputs.size() == 1 && last >= kRaggedRow && last % 4 != 0) {
     r.V = 4;  // the last vector of a row overlaps the one before (Emitter::ragged)
   } else {
-    if (r.V == 0) r.V = large ? 1 : 4;
+    if (r.V == 0) r.V = large ? 1 : joined_width(dag.outputs.size());
     if (r.V != 1 && r.V != 2 && r.V != 4 && r.V != 8) fail(CS_INVALID_VALUE, "vector_width must be 1, 2, 4 or 8");
     while (r.V > 1 && last % r.V != 0) r.V /= 2;
   }

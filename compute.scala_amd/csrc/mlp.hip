@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <utility>
 #include <vector>
 
 #include "internal.h"
@@ -115,205 +116,259 @@ __global__ __launch_bounds__(kB) void adam_kernel(float *__restrict__ p, const f
 // every layer, forward and back, with the activations and deltas in LDS, so that nothing but the
 // inputs, the parameters and the gradients' partial sums crosses memory. With the gradient, each
 // workgroup adds its samples' share of every parameter's gradient into its own row of `partial`,
-// and reduce_grads_kernel adds the rows. The forward sums run in the order of linear_fwd (bias
-// first, inputs in order), so activations are the same bits on either path. Bound by the latency of
-// the chain of layers in one workgroup (about 13 us for 23-64-64-64-1, of which the forward pass
-// takes 5): a gradient of 512 samples takes 19.7 us in two launches, against 820 us in twelve with
-// one thread per weight summing over all samples. Eight samples and 512 threads a workgroup: four
-// samples double the rows to add (25.5 us), 1024 threads change nothing.
+// and reduce_grads_kernel adds the rows.
+//
+// All three products run on the FP32 matrix instructions of K = 1, each a fused multiply-add per
+// element, so a sum keeps the order of its chain of them: the forward sums that of linear_fwd (bias
+// first, inputs in order), so activations are the same bits on either path. The 4x4x1 form, whose 16
+// blocks take one block's rows, multiplies four samples by 64 units, with the weights read from LDS
+// once for four samples and 16 inputs of the samples in one register; with a thread per sum each
+// multiply-add read its weight and its input, and LDS was the bound. The 16x16x1 form adds the outer
+// products of the weights' gradient, 16 inputs by 64 units. Bound by latency, that of the chain of layers
+// in one workgroup (18 cycles for each of a sum's terms), of the first loads and of fetching its
+// instructions, for which the loops are short (29 KiB unrolled 22.8 us, 10 KiB 17.5, at 512 samples of
+// 23-64-64-64-1; with a thread per sum 19.7). A gradient of 92 samples of 14-99-99-99-1 22.0 us (with a
+// thread per sum 37.7), of 512 of 32-128-128-128-1 38.8 (42.4); 512 samples of 23-64-64-64-1 took 820 us
+// in twelve launches with one thread per weight summing over all samples.
+// Eight samples and 512 threads a workgroup: four samples double the rows to add.
+// Evaluation of more than kManySamples takes four times as many, so that every wave has units of its own
+// (262144 samples of 23-64-64-64-1 191 us, with eight 406; at 4096 11.9 and 11.8, below eight are ahead).
 constexpr int kSamples = 8;  // per workgroup
+constexpr int kManySamples = 4096;
 constexpr int kNet = 512;      // threads of its kernel
+constexpr int kNetWaves = kNet / 64;
 constexpr int kMaxLayers = 15;
 
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef float f16 __attribute__((ext_vector_type(16)));
+
+// A layer: its widths, its parameters (W, then b) in the flat array and in LDS, and the LDS offsets of
+// its input and output activations.
+struct NetLayer {
+  int din, dout, params, lds, in, out, unused[2];
+};
 struct NetShape {
-  int layers;                      // L: widths[0] -> ... -> widths[L]
-  int widths[kMaxLayers + 1];
-  int w_off[kMaxLayers];           // of layer l + 1 in the flat parameters: W, then b
-  int act_off[kMaxLayers + 1];     // LDS offset of layer l's activations (0: the input)
-  int unit_off[kMaxLayers + 1];    // likewise of the activations by unit
-  int act_floats, unit_floats, delta_floats;  // LDS floats of both forms and of one delta buffer
-  int count;                       // parameters
-  int resident;                    // all parameters stay in LDS, else one layer's at a time
+  int layers;  // L
+  int count;   // parameters
+  int unit_floats, delta_floats, weight_floats;  // LDS floats of all activations, one delta buffer, parameters
+  int resident;  // all parameters stay in LDS, else one layer's at a time
+  NetLayer layer[kMaxLayers];
 };
 
-__host__ __device__ __forceinline__ int padded(int width) { return (width + 3) & ~3; }
+// In LDS widths are padded with zeros to a multiple of 16, the steps of sum_units. Rows of weights are an
+// odd number of 16-byte pieces: 64 consecutive floats of a row, and pieces of 16 rows, lie in different banks.
+__host__ __device__ __forceinline__ int padded(int width) { return (width + 15) & ~15; }
+__host__ __device__ __forceinline__ int pitch(int width) { return padded(width) + 4; }
 
-// Copies n floats of global memory to LDS, four 16-byte loads of a thread in flight (src at any
-// 4-byte boundary, dst at 16 bytes).
-__device__ __forceinline__ void copy_to_lds(float *dst, const float *__restrict__ src, int n) {
+// Copies the parameters of layers from .. to (any 4-byte boundary) to LDS, that of layer l to dst + its lds:
+// the bias first, then W. The waves take 1024 floats each in turn, through the layers.
+__device__ __forceinline__ void copy_to_lds(float *dst, const float *__restrict__ params, const NetShape &net,
+                                            int from, int to, int wave, int lane) {
   typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-  const f4u *s4 = reinterpret_cast<const f4u *>(src);
-  f4u *d4 = reinterpret_cast<f4u *>(dst);
-  const int nv = n / 4;
-  int i = threadIdx.x;
-  for (; i + 3 * kNet < nv; i += 4 * kNet) {
-    f4u v[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = s4[i + k * kNet];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) d4[i + k * kNet] = v[k];
-  }
-  for (; i < nv; i += kNet) d4[i] = s4[i];
-  for (int j = nv * 4 + threadIdx.x; j < n; j += kNet) dst[j] = src[j];
-}
-
-// LDS: activations by sample [layer][sample][padded width] and by unit [layer][unit, then a one for
-// the bias][sample], two delta buffers [sample][widest], parameters.
-template <bool kGrad>
-__global__ __launch_bounds__(kNet) void network_kernel(NetShape net, const float *__restrict__ params,
-                                                       const float *__restrict__ X, const float *__restrict__ target,
-                                                       int64_t n, float *__restrict__ y, float *__restrict__ partial,
-                                                       double *__restrict__ partial_loss) {
-  extern __shared__ __attribute__((aligned(16))) float lds[];
-  float *const acts = lds, *const by_unit = lds + net.act_floats;
-  float *const deltas = by_unit + net.unit_floats, *const weights = deltas + 2 * net.delta_floats;
-  const int t = threadIdx.x, L = net.layers;
-  const int last = net.widths[L];
-  if (net.resident) copy_to_lds(weights, params, net.count);
-  // Layer l's parameters in LDS, for every thread of the workgroup.
-  auto layer_weights = [&](int l) -> const float * {
-    const int from = net.w_off[l - 1];
-    if (net.resident) return weights + from;
-    __syncthreads();  // the previous layer's are no longer read
-    copy_to_lds(weights, params + from, (net.widths[l - 1] + 1) * net.widths[l]);
-    return weights;
-  };
-  double loss = 0.0;
-  bool first = true;
-  for (int64_t s0 = int64_t(blockIdx.x) * kSamples; s0 < n; s0 += int64_t(gridDim.x) * kSamples, first = false) {
-    const int live = n - s0 < kSamples ? static_cast<int>(n - s0) : kSamples;  // samples past n are zeros
-    const int din0 = net.widths[0], pad0 = padded(din0);
-    __syncthreads();  // the activations of the samples before are no longer read
-    if (kGrad && first)
-      for (int l = 0; l < L; ++l)  // the bias's input, after each layer's units
-        if (t < kSamples) by_unit[net.unit_off[l] + net.widths[l] * kSamples + t] = 1.0f;
-    for (int i = t; i < kSamples * pad0; i += kNet) {
-      const int s = i / pad0, c = i % pad0;
-      const float x = s < live && c < din0 ? X[(s0 + s) * din0 + c] : 0.0f;
-      acts[i] = x;
-      if (kGrad && c < din0) by_unit[c * kSamples + s] = x;
+  int mine = wave;  // chunks until this wave's next one
+#pragma unroll 1
+  for (int l = from; l <= to; ++l) {
+    const NetLayer y = net.layer[l - 1];
+    const int width = y.dout, n = y.din * width, chunks = (n + 1023) / 1024, row = pitch(width);
+    const float *const src = params + y.params;
+    float *const out = dst + y.lds;
+    const float inverse = 1.0f / float(width);
+    // (e + 0.5) / width is at least 0.5 / width from a whole number, and e < 2^16
+    auto at = [&](int e) {
+      const int r = int((float(e) + 0.5f) * inverse);
+      return e + (r + 1) * row - r * width;
+    };
+    if (mine == 0) {
+      for (int j = lane; j < width; j += 64) out[j] = src[n + j];
+      if (n < 4 && lane < n) out[at(lane)] = src[lane];
     }
-    for (int l = 1; l <= L; ++l) {
-      const int din = net.widths[l - 1], dout = net.widths[l], pin = padded(din), pout = padded(dout);
-      const float *const w = layer_weights(l), *const b = w + din * dout;
-      const float *const in = acts + net.act_off[l - 1];
-      float *const out = acts + net.act_off[l], *const out_unit = by_unit + net.unit_off[l];
-      __syncthreads();
-      for (int o = t; o < dout * kSamples; o += kNet) {
-        const int s = o / dout, j = o - s * dout;
-        const float *const x = in + s * pin, *wj = w + j;
-        float acc = b[j];
-        int i = 0;
-        for (; i + 16 <= din; i += 16, wj += 16 * dout) {
-          float4 xs[4];
-          float v[16];
+#pragma unroll 1
+    for (; n >= 4 && mine < chunks; mine += kNetWaves) {  // the last vector overlaps the one before
+      const int e0 = mine * 1024 + 4 * lane;
+      f4u v[4];
 #pragma unroll
-          for (int k = 0; k < 4; ++k) xs[k] = *reinterpret_cast<const float4 *>(x + i + 4 * k);
+      for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const f4u *>(src + min(e0 + 256 * k, n - 4));
 #pragma unroll
-          for (int k = 0; k < 16; ++k) v[k] = wj[k * dout];
-          __builtin_amdgcn_sched_barrier(0);  // all reads out before the first use
+      for (int k = 0; k < 4; ++k) {
+        const int e = min(e0 + 256 * k, n - 4);
 #pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            acc = fmaf(xs[k].x, v[4 * k], acc);
-            acc = fmaf(xs[k].y, v[4 * k + 1], acc);
-            acc = fmaf(xs[k].z, v[4 * k + 2], acc);
-            acc = fmaf(xs[k].w, v[4 * k + 3], acc);
-          }
-        }
-        for (; i < din; ++i, wj += dout) acc = fmaf(x[i], *wj, acc);
-        if (l < L) acc = fmaxf(acc, 0.0f);
-        out[s * pout + j] = acc;
-        if (kGrad) out_unit[j * kSamples + s] = acc;
+        for (int i = 0; i < 4; ++i) out[at(e + i)] = v[k][i];
       }
     }
-    __syncthreads();
-    const float *const pred = acts + net.act_off[L];
-    if constexpr (!kGrad) {
-      for (int i = t; i < live * last; i += kNet) y[s0 * last + i] = pred[(i / last) * padded(last) + i % last];
+    mine = (mine - chunks) & (kNetWaves - 1);
+  }
+}
+
+// acc[r] += x[k][r] w[k] for 16 units k in order: a holds unit k of sample r in lane 4 k + r.
+template <int... I>
+__device__ __forceinline__ void chain(float a, const float (&w)[16], f4 &acc, std::integer_sequence<int, I...>) {
+  ((acc = __builtin_amdgcn_mfma_f32_4x4x1f32(a, w[I], acc, 4, I, 0)), ...);
+}
+
+// acc[r] + sum_k x[k][r] v[k], k = 0 .. n - 1 in order, for four samples r and each lane's v: consecutive
+// values (kRow, 16-byte aligned) or values `stride` apart. x: the samples' values by unit, kS apart.
+// Both are zeros from n to the next multiple of 16.
+template <bool kRow, int kS>
+__device__ __forceinline__ f4 sum_units(const float *x, const float *v, int stride, int n, f4 acc) {
+  const int lane = threadIdx.x & 63;
+  const float *p = x + (lane >> 2) * kS + (lane & 3);
+#pragma unroll 1
+  for (int k0 = 0; k0 < n; k0 += 16) {
+    const float a = p[k0 * kS];
+    float w[16];
+    if constexpr (kRow) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const f4 q = reinterpret_cast<const f4 *>(v + k0)[k];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[4 * k + e] = q[e];
+      }
     } else {
-      // delta[s][j]: the loss's gradient by layer l's output before its ReLU
+#pragma unroll
+      for (int k = 0; k < 16; ++k) w[k] = v[k * stride];
+      v += 16 * stride;
+    }
+    chain(a, w, acc, std::make_integer_sequence<int, 16>());
+  }
+  return acc;
+}
+
+// LDS: activations [layer][unit][sample], two delta buffers [unit][sample], parameters by layer: the bias,
+// then W's rows.
+template <bool kGrad, int kS>
+__global__ __launch_bounds__(kNet) void network_kernel(NetShape net, const float *__restrict__ params,
+                                                       const float *__restrict__ X, const float *__restrict__ target,
+                                                       int64_t n, float *__restrict__ result,
+                                                       float *__restrict__ partial, double *__restrict__ partial_loss) {
+  static_assert(!kGrad || kS == 8, "the weights' gradient adds two registers of four samples");
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  float *const units = lds, *const deltas = units + net.unit_floats, *const weights = deltas + 2 * net.delta_floats;
+  const int t = threadIdx.x, L = net.layers;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
+  const int last = net.layer[L - 1].dout, din0 = net.layer[0].din;
+  // In sums over units a wave takes four samples and 64 units, then the next units that no wave has taken.
+  constexpr int kQuads = kS / 4, kStep = kNetWaves / kQuads * 64;
+  const int q = wave % kQuads * 4, first_unit = wave / kQuads * 64 + lane;
+  // Layer l's parameters in LDS, for every thread of the workgroup.
+  auto layer_weights = [&](int l, const NetLayer &layer) -> const float * {
+    if (net.resident) return weights + layer.lds;
+    __syncthreads();  // the previous layer's are no longer read
+    for (int i = t * 4; i < net.weight_floats; i += kNet * 4) *reinterpret_cast<f4 *>(weights + i) = f4{};
+    __syncthreads();
+    copy_to_lds(weights - layer.lds, params, net, l, l, wave, lane);
+    return weights;
+  };
+  for (int i = t * 4; i < net.unit_floats + 2 * net.delta_floats + net.weight_floats; i += kNet * 4)
+    *reinterpret_cast<f4 *>(lds + i) = f4{};
+  __syncthreads();
+  double loss = 0.0;
+  bool first = true;
+#pragma unroll 1
+  for (int64_t s0 = int64_t(blockIdx.x) * kS; s0 < n; s0 += int64_t(gridDim.x) * kS, first = false) {
+    const int live = n - s0 < kS ? static_cast<int>(n - s0) : kS;  // samples past n are zeros
+    const float wanted = kGrad && t < live ? target[s0 + t] : 0.0f;
+    if (!first) __syncthreads();  // the activations of the samples before are no longer read
+    for (int s = wave; s < kS; s += kNetWaves)
+      for (int c = lane; c < din0; c += 64) units[c * kS + s] = s < live ? X[(s0 + s) * din0 + c] : 0.0f;
+    if (first && net.resident) copy_to_lds(weights, params, net, 1, L, wave, lane);
+    NetLayer y = net.layer[0];
+#pragma unroll 1
+    for (int l = 1; l <= L; ++l) {
+      const NetLayer following = net.layer[l < L ? l : L - 1];  // read while this layer runs
+      const float *const w = layer_weights(l, y);
+      __syncthreads();
+#pragma unroll 1
+      for (int j = first_unit; j - lane < y.dout; j += kStep) {
+        const float *const wj = w + min(j, y.dout - 1);
+        const float b = wj[0];
+        f4 acc = sum_units<false, kS>(units + y.in + q, wj + pitch(y.dout), pitch(y.dout), y.din, f4{b, b, b, b});
+        if (l < L)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[e] = fmaxf(acc[e], 0.0f);
+        if (j < y.dout) *reinterpret_cast<f4 *>(units + y.out + j * kS + q) = acc;
+      }
+      y = following;
+    }
+    __syncthreads();
+    const float *const pred = units + y.out;
+    if constexpr (!kGrad) {
+      for (int s = wave; s < live; s += kNetWaves)
+        for (int c = lane; c < last; c += 64) result[(s0 + s) * last + c] = pred[c * kS + s];
+    } else {
+      // delta[j][s]: the loss's gradient by layer l's output before its ReLU
       float *cur = deltas, *next = deltas + net.delta_floats;
-      if (t < kSamples) {
-        const float d = t < live ? pred[t * padded(last)] - target[s0 + t] : 0.0f;
+      if (t < 16 * kS) {
+        const float d = t < live ? pred[t] - wanted : 0.0f;
         cur[t] = 2.0f * d / float(n);
         loss += double(d) * double(d);
       }
+#pragma unroll 1
       for (int l = L; l >= 1; --l) {
-        const int din = net.widths[l - 1], dout = net.widths[l], pin = padded(din);
-        const float *const in = acts + net.act_off[l - 1], *const in_unit = by_unit + net.unit_off[l - 1];
-        const float *const w = l > 1 ? layer_weights(l) : nullptr;
+        const NetLayer following = net.layer[l > 1 ? l - 2 : 0];
+        const int din = y.din, dout = y.dout;
+        const float *const in = units + y.in;
+        const float *const w = l > 1 ? layer_weights(l, y) : nullptr;
         __syncthreads();
-        // dW[i][j] = sum_s in[s][i] delta[s][j]; row din is the bias's, whose input is 1. A thread
-        // keeps a column j (several in turn where there are more than threads) and takes every
-        // `rows`-th row.
-        float *const row = partial + int64_t(blockIdx.x) * net.count + net.w_off[l - 1];
-        const int rows = dout < kNet ? kNet / dout : 1, side = dout < kNet ? dout : kNet;
-        const int i0 = t / side;
-        for (int j = t - i0 * side; j < dout && i0 < rows; j += side) {
-          float g[kSamples];
+        // dX[s][i] = sum_j delta[s][j] W[i][j], then the ReLU of layer l - 1: 64 inputs at a time
+        if (l > 1)
+#pragma unroll 1
+          for (int i = first_unit; i - lane < din; i += kStep) {
+            f4 acc = sum_units<true, kS>(cur + q, w + (min(i, din - 1) + 1) * pitch(dout), 1, dout, f4{});
+            const f4 x = *reinterpret_cast<const f4 *>(in + min(i, din - 1) * kS + q);
 #pragma unroll
-          for (int s = 0; s < kSamples; ++s) g[s] = cur[s * dout + j];
-          auto add = [&](int i, float acc) {
-            const float4 *const u = reinterpret_cast<const float4 *>(in_unit + i * kSamples);
+            for (int e = 0; e < 4; ++e) acc[e] = x[e] <= 0.0f || i >= din ? 0.0f : acc[e];
+            if (i < padded(din)) *reinterpret_cast<f4 *>(next + i * kS + q) = acc;
+          }
+        // dW[i][j] = sum_s in[s][i] delta[s][j]; row din is the bias's, whose input is 1. 16 inputs and 64
+        // units at a time, from the first wave without a sum above on. Inputs and units past the end have
+        // results of their own, which lie out of the buffer's range.
+        const __amdgpu_buffer_rsrc_t row = __builtin_amdgcn_make_buffer_rsrc(
+            partial + int64_t(blockIdx.x) * net.count + y.params, 0, (din + 1) * dout * 4, 0x00020000);
+        const int l16 = lane & 15, quad = lane >> 4, busy = l > 1 ? (din + 63) / 64 * kQuads : 0;
+#pragma unroll 1
+        for (int i0 = ((wave - busy) & (kNetWaves - 1)) * 16; i0 <= din; i0 += kNetWaves * 16) {
+          const int i = i0 + l16;
+          const float *const x = in + min(i, din - 1) * kS + quad;
+          const float a0 = i < din ? x[0] : 1.0f, a1 = i < din ? x[4] : 1.0f;
+#pragma unroll 1
+          for (int j0 = 0; j0 < dout; j0 += 64) {
+            const f4 *const d = reinterpret_cast<const f4 *>(cur + min(j0 + lane, dout - 1) * kS);
+            const f4 d0 = d[0], d1 = d[1];
+            int at[16];
 #pragma unroll
-            for (int s = 0; s < kSamples / 4; ++s) {
-              const float4 x = u[s];
-              acc = fmaf(x.x, g[4 * s], acc);
-              acc = fmaf(x.y, g[4 * s + 1], acc);
-              acc = fmaf(x.z, g[4 * s + 2], acc);
-              acc = fmaf(x.w, g[4 * s + 3], acc);
+            for (int e = 0; e < 16; ++e) {
+              const int j = j0 + e / 4 * 16 + l16;
+              at[e] = j < dout ? ((i0 + 4 * quad + e % 4) * dout + j) * 4 : 0x7ffffffc;
             }
-            return acc;
-          };
-          if (first) {
-#pragma unroll 4
-            for (int i = i0; i <= din; i += rows) row[i * dout + j] = add(i, 0.0f);
-          } else {
-            for (int i = i0; i <= din; i += rows) row[i * dout + j] = add(i, row[i * dout + j]);
+            f16 acc = {};
+            if (!first)
+#pragma unroll
+              for (int e = 0; e < 16; ++e)
+                acc[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(row, at[e], 0, 0));
+            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a0, d0[0], acc, 2, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a0, d0[1], acc, 2, 1, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a0, d0[2], acc, 2, 2, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a0, d0[3], acc, 2, 3, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a1, d1[0], acc, 2, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a1, d1[1], acc, 2, 1, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a1, d1[2], acc, 2, 2, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a1, d1[3], acc, 2, 3, 0);
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+              __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[e]), row, at[e], 0, 0);
           }
         }
-        if (l > 1) {
-          // dX[s][i] = sum_j delta[s][j] W[i][j], from a different j on for each i and round, so
-          // that the rows of W that a wave reads at once lie in different banks; then the ReLU of
-          // layer l - 1
-          const bool quads = dout % 4 == 0 && net.w_off[l - 1] % 4 == 0;
-          for (int o = t; o < kSamples * din; o += kNet) {
-            const int s = o / din, i = o - s * din;
-            const float *const wi = w + i * dout, *const gs = cur + s * dout;
-            float acc = 0.0f;
-            if (quads) {
-              const int nq = dout / 4;
-              int q = i % nq;
-#pragma unroll 4
-              for (int k = 0; k < nq; ++k) {
-                const float4 g = reinterpret_cast<const float4 *>(gs)[q], v = reinterpret_cast<const float4 *>(wi)[q];
-                acc = fmaf(g.x, v.x, acc);
-                acc = fmaf(g.y, v.y, acc);
-                acc = fmaf(g.z, v.z, acc);
-                acc = fmaf(g.w, v.w, acc);
-                q = q + 1 == nq ? 0 : q + 1;
-              }
-            } else {
-              int j = i % dout;
-#pragma unroll 8
-              for (int k = 0; k < dout; ++k) {
-                acc = fmaf(gs[j], wi[j], acc);
-                j = j + 1 == dout ? 0 : j + 1;
-              }
-            }
-            next[s * din + i] = in[s * pin + i] <= 0.0f ? 0.0f : acc;
-          }
-          float *const swap = cur;
-          cur = next;
-          next = swap;
-        }
+        float *const swap = cur;
+        cur = next;
+        next = swap;
+        y = following;
       }
     }
   }
   if constexpr (kGrad) {
-    // the samples' losses are in the first kSamples lanes of wave 0
+    // the samples' losses are in the first kS lanes of wave 0
 #pragma unroll
-    for (int off = kSamples / 2; off >= 1; off >>= 1) loss += __shfl_xor(loss, off, 64);
+    for (int off = kS / 2; off >= 1; off >>= 1) loss += __shfl_xor(loss, off, 64);
     if (t == 0) partial_loss[blockIdx.x] = loss;
   }
 }
@@ -405,60 +460,71 @@ void forward(cs_stream *stream, cs_mlp *net, const float *X, int64_t n) {
 }
 
 // The whole-network kernel's shape, and its LDS bytes: 0 when the network does not fit.
-size_t network_shape(const cs_mlp *net, bool grad, NetShape *shape) {
+size_t network_shape(const cs_mlp *net, bool grad, int samples, NetShape *shape) {
   const int L = static_cast<int>(net->widths.size()) - 1;
   if (L > kMaxLayers || net->count > (1 << 24)) return 0;
   shape->layers = L;
   shape->count = static_cast<int>(net->count);
-  int act = 0, unit = 0, widest = 1, layer = 0;
-  for (int l = 0; l <= L; ++l) {
-    const int w = net->widths[l];
-    shape->widths[l] = w;
-    shape->act_off[l] = act;
-    shape->unit_off[l] = unit;
-    act += kSamples * padded(w);
-    if (grad) unit += kSamples * padded(w + 1);
-    widest = std::max(widest, w);
-    if (l == 0) continue;
-    shape->w_off[l - 1] = static_cast<int>(net->w_off[l - 1]);
-    layer = std::max(layer, (net->widths[l - 1] + 1) * w);
+  int unit = samples * padded(net->widths[0]), from = 0, weights = 0, widest = net->widths[0], layer = 0;
+  for (int l = 1; l <= L; ++l) {
+    NetLayer &y = shape->layer[l - 1];
+    y.din = net->widths[l - 1], y.dout = net->widths[l];
+    y.params = static_cast<int>(net->w_off[l - 1]);
+    y.lds = weights;
+    y.in = from, y.out = from = unit;
+    unit += samples * padded(y.dout);
+    widest = std::max(widest, y.dout);
+    const int size = (padded(y.din) + 1) * pitch(y.dout);
+    if (size > (1 << 16)) return 0;
+    weights += size;
+    layer = std::max(layer, size);
   }
-  shape->act_floats = act;
   shape->unit_floats = unit;
-  shape->delta_floats = grad ? kSamples * padded(widest) : 0;
-  const size_t fixed = size_t(act + unit + 2 * shape->delta_floats) * 4, budget = net->device->props.sharedMemPerBlock;
-  shape->resident = fixed + size_t(net->count) * 4 <= budget;
-  const size_t bytes = fixed + size_t(shape->resident ? shape->count : layer) * 4;
+  shape->delta_floats = grad ? samples * padded(widest) : 0;
+  const size_t fixed = size_t(unit + 2 * shape->delta_floats) * 4, budget = net->device->props.sharedMemPerBlock;
+  shape->resident = fixed + size_t(weights) * 4 <= budget;
+  shape->weight_floats = shape->resident ? weights : layer;
+  const size_t bytes = fixed + size_t(shape->weight_floats) * 4;
   return bytes <= budget ? bytes : 0;
 }
 
-template <bool kGrad>
+// Workgroups for n samples: one each kS, up to `per_cu` on every CU (they take further samples in turn).
+// With the gradient one: each has a row of `partial` to write and to add.
+template <int kS>
+unsigned network_grid(cs_stream *stream, int64_t n, int64_t per_cu) {
+  return static_cast<unsigned>(
+      std::min<int64_t>((n + kS - 1) / kS, per_cu * stream->device->props.multiProcessorCount));
+}
+
+template <bool kGrad, int kS>
 void launch_network(cs_stream *stream, const NetShape &shape, size_t lds, unsigned grid, const cs_mlp *net,
                     const float *X, const float *target, int64_t n, float *y, float *partial, double *partial_loss) {
   static const bool configured = [] {
-    CS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&network_kernel<kGrad>),
+    CS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&network_kernel<kGrad, kS>),
                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10));
     return true;
   }();
   (void)configured;
-  hipLaunchKernelGGL(network_kernel<kGrad>, dim3(grid), dim3(kNet), lds, stream->stream, shape, net->params, X, target, n,
-                     y, partial, partial_loss);
+  hipLaunchKernelGGL((network_kernel<kGrad, kS>), dim3(grid), dim3(kNet), lds, stream->stream, shape, net->params, X,
+                     target, n, y, partial, partial_loss);
 }
 
-// Workgroups for n samples: one each kSamples, up to `per_cu` on every CU (they take further samples
-// in turn). With the gradient one: each has a row of `partial` to write and to add.
-unsigned network_grid(cs_stream *stream, int64_t n, int64_t per_cu) {
-  return static_cast<unsigned>(std::min<int64_t>((n + kSamples - 1) / kSamples,
-                                                 per_cu * stream->device->props.multiProcessorCount));
-}
+// Evaluation alone, of very many samples on a tiny network: the layer kernels, a thread per unit and
+// sample, are ahead (262144 samples, us, layers / whole: 8-16-1, 161 parameters, 33 / 61; 16-16-1, 289,
+// 42 / 62; 12-14-14-1, 407, 82 / 80; 16-24-1, 433, 65 / 69; 30-30-30-30-1, 2821, 373 / 129).
+bool prefer_layers(const NetShape &shape, int64_t n) { return n > 65536 && shape.count <= 400; }
 
-// Evaluation alone, of very many samples on a network too narrow to give every thread a unit: the
-// layer kernels, whose threads do not wait for one another, are ahead (262144 samples through
-// 8-16-1: 34 us against 45; through 23-64-64-64-1 they are behind, 872 against 650).
-bool prefer_layers(const NetShape &shape, int64_t n) {
-  int widest = 1;
-  for (int l = 1; l <= shape.layers; ++l) widest = std::max(widest, shape.widths[l]);
-  return n > 65536 && widest * kSamples < kNet;
+// Evaluation with kS samples per workgroup, where the network fits.
+template <int kS>
+bool evaluate(cs_stream *stream, cs_mlp *net, const float *X, int64_t n, float *y) {
+  NetShape shape;
+  const size_t lds = network_shape(net, false, kS, &shape);
+  if (!lds || prefer_layers(shape, n)) return false;
+  const int64_t per_cu = std::max<int64_t>(1, std::min<int64_t>(4, int64_t(160 << 10) / int64_t(lds)));
+  launch_network<false, kS>(stream, shape, lds, network_grid<kS>(stream, n, per_cu), net, X, nullptr, n, y, nullptr,
+                            nullptr);
+  CS_HIP(hipGetLastError());
+  return true;
 }
 
 }  // namespace
@@ -539,16 +605,11 @@ cs_status cs_mlp_forward(cs_stream *stream, cs_mlp *mlp, const float *X, int64_t
     if (!stream || !mlp || !X || !y) fail(CS_INVALID_VALUE, "null argument");
     if (n <= 0) fail(CS_INVALID_VALUE, "no samples");
     set_device(stream->device);
-    NetShape shape;
-    const size_t lds = network_shape(mlp, false, &shape);
     // y over X's memory: the layer kernels have read X before y is written
     const bool over = y < X + n * mlp->widths.front() && X < y + n * mlp->widths.back();
-    if (lds && !over && !prefer_layers(shape, n)) {
-      const int64_t per_cu = std::max<int64_t>(1, std::min<int64_t>(4, int64_t(160 << 10) / int64_t(lds)));
-      launch_network<false>(stream, shape, lds, network_grid(stream, n, per_cu), mlp, X, nullptr, n, y, nullptr, nullptr);
-      CS_HIP(hipGetLastError());
+    if (!over && ((n > kManySamples && evaluate<4 * kSamples>(stream, mlp, X, n, y)) ||
+                  evaluate<kSamples>(stream, mlp, X, n, y)))
       return;
-    }
     forward(stream, mlp, X, n);
     const int L = static_cast<int>(mlp->widths.size()) - 1;
     CS_HIP(hipMemcpyAsync(y, mlp->acts + act_offset(mlp, L, n), size_t(n) * mlp->widths[L] * 4,
@@ -565,13 +626,13 @@ cs_status cs_mlp_backward(cs_stream *stream, cs_mlp *mlp, const float *X, const 
     if (mlp->widths[L] != 1) fail(CS_INVALID_VALUE, "the loss needs a single output");
     set_device(stream->device);
     NetShape shape;
-    if (const size_t lds = network_shape(mlp, true, &shape)) {
-      const unsigned grid = network_grid(stream, n, 1);
+    if (const size_t lds = network_shape(mlp, true, kSamples, &shape)) {
+      const unsigned grid = network_grid<kSamples>(stream, n, 1);
       // partial losses (FP64), then one row of gradients per workgroup
       ensure(&mlp->deltas, &mlp->deltas_capacity, int64_t(grid) * (2 + mlp->count));
       double *partial_loss = reinterpret_cast<double *>(mlp->deltas);
       float *partial = mlp->deltas + 2 * grid;
-      launch_network<true>(stream, shape, lds, grid, mlp, X, target, n, nullptr, partial, partial_loss);
+      launch_network<true, kSamples>(stream, shape, lds, grid, mlp, X, target, n, nullptr, partial, partial_loss);
       hipLaunchKernelGGL(reduce_grads_kernel, dim3(blocks(kGradLanes * mlp->count) + 1), dim3(kB), 0, stream->stream, partial,
                          static_cast<int>(mlp->count), static_cast<int>(grid), partial_loss, n, grads, loss);
       CS_HIP(hipGetLastError());

@@ -1292,6 +1292,14 @@ void check_depth(int K) {
                            "value must stay below 8 MiB)");
 }
 
+// Scratch of the operands of run_lds.
+template <int KIND, int W>
+int64_t packed_bytes(int M, int N, int K) {
+  using P = Pipe<KIND>;
+  const int64_t rows = round_up(M, tile_edge(W)) + round_up(N, tile_edge(W)), Kp = round_up(K, P::kK);
+  return rows * Kp * P::kBytesPerK + 4096 + (KIND == kFP8 ? rows * (Kp / 128) + 4096 : 0);
+}
+
 template <int KIND, int W, int kBufs>
 void run_lds(cs_stream *stream, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
              int ldc, int slices) {
@@ -1300,9 +1308,7 @@ void run_lds(cs_stream *stream, int M, int N, int K, const float *A, int lda, co
   const int64_t Mp = round_up(M, kTile), Np = round_up(N, kTile), Kp = round_up(K, P::kK);
   const int64_t rowb = Kp * P::kBytesPerK;
   const int64_t xbytes = Mp * rowb, ybytes = Np * rowb;
-  int64_t total = xbytes + ybytes + 4096;
-  if (KIND == kFP8) total += (Mp + Np) * (Kp / 128) + 4096;
-  const Target to(stream, total, M, N, C, ldc, slices);
+  const Target to(stream, packed_bytes<KIND, W>(M, N, K), M, N, C, ldc, slices);
   char *const base = to.scratch, *x = base, *y = base + xbytes;
   uint8_t *sx = nullptr, *sy = nullptr;
   hipStream_t s = stream->stream;
@@ -1498,12 +1504,15 @@ Plan choose_path(double cus, double M, double N, double K, const DirectPlan &p) 
   return best;
 }
 
+// False where a captured stream's scratch has no room for the operands (but for a C that needs the copies).
 template <int KIND, int W, int kBufs>
-void run_packed(cs_stream *stream, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
+bool run_packed(cs_stream *stream, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
                 int ldc, bool over, int slices) {
   if constexpr (KIND == kF32)
-    if (!over && run_split<W>(stream, M, N, K, A, lda, B, ldb, C, ldc, slices)) return;
+    if (!over && run_split<W>(stream, M, N, K, A, lda, B, ldb, C, ldc, slices)) return true;
+  if (!over && !scratch_fits(stream, size_t(packed_bytes<KIND, W>(M, N, K)))) return false;
   run_lds<KIND, W, kBufs>(stream, M, N, K, A, lda, B, ldb, C, ldc, slices);
+  return true;
 }
 
 template <int KIND>
@@ -1515,11 +1524,20 @@ void run(cs_stream *stream, int M, int N, int K, const float *A, int lda, const 
   const bool over = overlap(A, M, K, lda, C, M, N, ldc) || overlap(B, K, N, ldb, C, M, N, ldc);
   Plan plan = choose_path<KIND>(double(cus), M, N, K, p);
   if (over && plan.path == kDirect) plan = {kTiles128, 1};
-  const int z = plan.slices;
-  if (plan.path == kTiles256) return run_packed<KIND, 4, 2>(stream, M, N, K, A, lda, B, ldb, C, ldc, over, z);
-  if (plan.path == kTiles128) return run_packed<KIND, 2, 2>(stream, M, N, K, A, lda, B, ldb, C, ldc, over, z);
-  if constexpr (KIND != kF32)
-    if (plan.path == kDeep128) return run_packed<KIND, 2, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc, over, z);
+  int z = plan.slices;
+  if (plan.path == kDirect) {
+    // a call sizes the scratch for calls of up to its size under capture, one that copies its operands too
+    const size_t bytes = size_t(packed_bytes<KIND, 2>(M, N, K));
+    if (scratch_fits(stream, bytes)) stream_scratch(stream, bytes);
+  } else {
+    bool done = false;
+    if (plan.path == kTiles256) done = run_packed<KIND, 4, 2>(stream, M, N, K, A, lda, B, ldb, C, ldc, over, z);
+    if (plan.path == kTiles128) done = run_packed<KIND, 2, 2>(stream, M, N, K, A, lda, B, ldb, C, ldc, over, z);
+    if constexpr (KIND != kF32)
+      if (plan.path == kDeep128) done = run_packed<KIND, 2, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc, over, z);
+    if (done) return;
+    z = 1;
+  }
   switch (p.t * 100 + p.wk) {
     case 101: return run_direct<KIND, 1, 1>(stream, M, N, K, A, lda, B, ldb, C, ldc, z);
     case 104: return run_direct<KIND, 1, 4>(stream, M, N, K, A, lda, B, ldb, C, ldc, z);

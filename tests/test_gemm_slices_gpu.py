@@ -77,3 +77,37 @@ def test_captured_without_scratch(gpu_tensors):
     capi.check(capi.lib.cs_stream_destroy(s))
     for h in (ba, bb, bc):
         h.release()
+
+
+@pytest.mark.parametrize("variant", sorted(VARIANTS))
+def test_captured_after_a_larger_call(gpu_tensors, variant):
+    """A stream's first call is large without operand copies; a smaller product is then captured whose plan
+    has them, and one whose result lies over an operand."""
+    T = gpu_tensors
+    s = ctypes.c_void_p()
+    capi.check(capi.lib.cs_stream_create(T.device, ctypes.byref(s)))
+    big, M, N, K = 1500, 1400, 1300, 60
+    a, b = inputs.uniform(M * K, 4087).reshape(M, K), inputs.uniform(K * N, 4088).reshape(K, N)
+    ba, bb, bc = upload(T, a), upload(T, b), alloc(T, big * big)
+    xa = upload(T, np.zeros(big * big, np.float32))
+    n = 96
+    sq = inputs.uniform(n * n, 4089).reshape(n, n)
+    bs = upload(T, sq)
+    capi.check(capi.lib.cs_stream_synchronize(T.stream))
+    capi.check(capi.lib.cs_gemm(s, VARIANTS[variant], big, 1, big, xa.ptr, big, xa.ptr, 1, bc.ptr, 1))
+    capi.check(capi.lib.cs_stream_synchronize(s))
+    g = ctypes.c_void_p()
+    capi.check(capi.lib.cs_graph_begin_capture(s))
+    capi.check(capi.lib.cs_gemm(s, VARIANTS[variant], M, N, K, ba.ptr, K, bb.ptr, N, bc.ptr, N))
+    capi.check(capi.lib.cs_gemm(s, VARIANTS[variant], n, n, n, bs.ptr, n, bb.ptr, n, bs.ptr, n))
+    capi.check(capi.lib.cs_graph_end_capture(s, ctypes.byref(g)))
+    capi.check(capi.lib.cs_graph_launch(s, g))
+    capi.check(capi.lib.cs_stream_synchronize(s))
+    c = download(T, bc, M * N).reshape(M, N)
+    assert fp64.gemm_normalized_error(c, a, b) <= BOUND[variant]
+    right = b.ravel()[:n * n].reshape(n, n).copy()
+    assert fp64.gemm_normalized_error(download(T, bs, n * n).reshape(n, n), sq, right) <= BOUND[variant]
+    capi.check(capi.lib.cs_graph_release(g))
+    capi.check(capi.lib.cs_stream_destroy(s))
+    for h in (ba, bb, bc, xa, bs):
+        h.release()

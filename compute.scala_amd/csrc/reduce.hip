@@ -234,20 +234,13 @@ __device__ __forceinline__ void add_vector(f4u v, Acc &a, float &m) {
 }
 
 // One row's share of a lane: vectors lane, lane + kStep, ... of p, four loads in flight. The
-// cols % 4 elements after the last whole vector are the end of one more vector that overlaps it,
-// so that they ride with the other loads. kShort: at most one vector per lane; what a launch of few
-// short rows waits for is mostly its own instructions, so it gets a kernel of few.
+// cols % 4 elements after the last whole vector ride with the other loads: in a wave or less as the end
+// of one more vector that overlaps it (120011 x 77 12.0 us, one by one 13.1), in a workgroup one by one,
+// which is shorter (3000 x 2500 8.9 us, as a vector 9.2). kShort: at most one vector per lane; what a
+// launch of few short rows waits for is mostly its own instructions, so it gets a kernel of few.
 template <int kStep, bool kShort, class Index>
 __device__ __forceinline__ void read_row(const float *__restrict__ p, Index cols, int lane, Acc &a, float &m) {
   const Index nv = cols / 4;
-  const int tail = static_cast<int>(cols % 4);
-  if (nv == 0) {
-    for (int j = lane; j < tail; j += kStep) {
-      a.add(p[j]);
-      m = nanmax(m, p[j]);
-    }
-    return;
-  }
   Index i = lane;
   if (!kShort) {
     const f4u *p4 = reinterpret_cast<const f4u *>(p);
@@ -260,23 +253,52 @@ __device__ __forceinline__ void read_row(const float *__restrict__ p, Index cols
     }
   }
   constexpr int kVecs = kShort ? 1 : 4;
-  const Index all = nv + (tail ? 1 : 0);
-  if (i >= all) return;
   f4u v[kVecs];
+  if constexpr (kStep > 64) {
+    float x;
+    const bool one = 4 * nv + lane < cols;
+    if (one) x = p[4 * nv + lane];
+    if (i < nv) {
 #pragma unroll
-  for (int k = 0; k < kVecs; ++k) {
-    const Index c = i + k * kStep;
-    if (c < all) v[k] = __builtin_nontemporal_load(reinterpret_cast<const f4u *>(p + (c < nv ? 4 * c : cols - 4)));
-  }
+      for (int k = 0; k < kVecs; ++k)
+        if (i + k * kStep < nv)
+          v[k] = __builtin_nontemporal_load(reinterpret_cast<const f4u *>(p + 4 * (i + k * kStep)));
 #pragma unroll
-  for (int k = 0; k < kVecs; ++k) {
-    const Index c = i + k * kStep;
-    if (c < all) {
-      const int again = c < nv ? 0 : 4 - tail;  // elements that the vector before has added
+      for (int k = 0; k < kVecs; ++k)
+        if (i + k * kStep < nv) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        a.add(e >= again ? v[k][e] : 0.0f);
-        m = nanmax(m, e >= again ? v[k][e] : __builtin_nanf(""));
+          for (int e = 0; e < 4; ++e) a.add(v[k][e]);
+          m = nanmax(m, nanmax(nanmax(v[k].x, v[k].y), nanmax(v[k].z, v[k].w)));
+        }
+    }
+    if (one) {
+      a.add(x);
+      m = nanmax(m, x);
+    }
+  } else {
+    const int tail = static_cast<int>(cols % 4);
+    if (nv == 0) {
+      for (int j = lane; j < tail; j += kStep) {
+        a.add(p[j]);
+        m = nanmax(m, p[j]);
+      }
+      return;
+    }
+    const Index all = nv + (tail ? 1 : 0);
+    if (i >= all) return;
+#pragma unroll
+    for (int k = 0; k < kVecs; ++k) {
+      const Index c = i + k * kStep;
+      if (c < all) v[k] = __builtin_nontemporal_load(reinterpret_cast<const f4u *>(p + (c < nv ? 4 * c : cols - 4)));
+    }
+#pragma unroll
+    for (int k = 0; k < kVecs; ++k) {
+      const Index c = i + k * kStep;
+      if (c < all) {
+        const int again = c < nv ? 0 : 4 - tail;  // elements that the vector before has added
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a.add(e >= again ? v[k][e] : 0.0f);
+        m = nanmax(m, nanmax(nanmax(v[k].x, v[k].y), nanmax(v[k].z, v[k].w)));  // twice changes no maximum
       }
     }
   }

@@ -999,7 +999,7 @@ constexpr unsigned kMinExponent = 24, kMinProduct = 254 - 110;
 struct SplitArgs {
   const float *a, *b;
   int m, n, k, lda, ldb, mp, np, kp;
-  char *x, *y;         // [kp / 16][3][mp or np][16] BF16
+  char *x, *y;         // [kp / 16][3][2][mp or np][8] BF16
   uint8_t *ea, *eb;    // least exponents: [mp / 64][chunks] and [np / 64][chunks], chunks of 64 K
   unsigned row_blocks;
 };
@@ -1028,7 +1028,7 @@ __device__ __forceinline__ unsigned split_store(const float (&v)[16], char *dst,
       r[2 * e + 1] -= __uint_as_float(h & 0xffff0000u);
     }
     *reinterpret_cast<i32x4 *>(dst + part * part_stride) = w[0];
-    *reinterpret_cast<i32x4 *>(dst + part * part_stride + 16) = w[1];
+    *reinterpret_cast<i32x4 *>(dst + part * part_stride + part_stride / 2) = w[1];
   }
   return least;
 }
@@ -1072,7 +1072,7 @@ __global__ __launch_bounds__(256) void split_operands_kernel(SplitArgs p) {
       }
     }
     const int64_t part_stride = int64_t(is_a ? p.mp : p.np) * 32;
-    char *dst = (is_a ? p.x : p.y) + int64_t(k / 16) * 3 * part_stride + int64_t(row) * 32;
+    char *dst = (is_a ? p.x : p.y) + int64_t(k / 16) * 3 * part_stride + int64_t(row) * 16;
     const unsigned e = split_store(v, dst, part_stride);
     if (e < 255) atomicMin(&least, e);
   }
@@ -1085,8 +1085,9 @@ __global__ __launch_bounds__(256) void split_operands_kernel(SplitArgs p) {
 // values: (W = 4) 96 MFMAs per wave, in six groups of 16 that use every accumulator once. Three stages
 // live in LDS: while stage s computes, the fragments of s + 1 replace those of s as their last group
 // has issued, and stage s + 2 streams into the buffer of s - 1 (six stages of W = 2 gain nothing:
-// 2048^3 101.9 us against 103.5). The operands are packed so that each part of a stage is contiguous:
-// DMA and fragment reads are linear in LDS, without bank conflicts.
+// 2048^3 101.9 us against 103.5). The operands are packed so that each half (eight K values) of each
+// part of a stage is contiguous: DMA and fragment reads are linear in LDS, without bank conflicts (with
+// whole rows of 16 K contiguous a read met two rows in a bank: 2048^3 103.6 us, 102.0 without).
 template <int W>
 __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_split_kernel(
     int M, int N, int K, int Kp, int Mp, int Np, const char *__restrict__ X, const char *__restrict__ Y,
@@ -1133,27 +1134,29 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_split_kernel(
 
   // Waves 0 and 1 stream A's panel, 2 and 3 B's: 3W chunks of 1 KiB each per stage.
   const int rows_p = wave < 2 ? Mp : Np;
-  const char *const from = wave < 2 ? X + int64_t(m0) * 32 : Y + int64_t(n0) * 32;
+  const char *const from = wave < 2 ? X + int64_t(m0) * 16 : Y + int64_t(n0) * 16;
   const int part_stride = rows_p * 32;
   const int first = slice_begin(Kp / kSplitK, blockIdx.y, slices);
   const int stages = slice_begin(Kp / kSplitK, blockIdx.y + 1, slices) - first;
   const unsigned voff = unsigned(lane) * 16;
   auto dma = [&](int ks, int buf) {
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char *>(from) + int64_t(first + ks) * 3 * part_stride, 0, 2 * part_stride + kPartB, 0x00020000);
+        const_cast<char *>(from) + int64_t(first + ks) * 3 * part_stride, 0,
+        5 * (part_stride / 2) + kPartB / 2, 0x00020000);
     char *const l = lds + buf + (wave >> 1) * kSplitPanelB;
 #pragma unroll
     for (int i = 0; i < 3 * W; ++i) {
       const int q = (wave & 1) * 3 * W + i;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)(l + q * 1024), 16, voff,
-                                               unsigned(q / (2 * W) * part_stride + q % (2 * W) * 1024), 0, 0);
+                                               unsigned(q / W * (part_stride / 2) + q % W * 1024), 0, 0);
     }
   };
-  const int arow = (wm * kWaveRows + l32) * 32 + half * 16, brow = kSplitPanelB + (wn * kWaveRows + l32) * 32 + half * 16;
+  const int arow = (wm * kWaveRows + l32) * 16 + half * (kPartB / 2);
+  const int brow = kSplitPanelB + (wn * kWaveRows + l32) * 16 + half * (kPartB / 2);
   auto frags = [&](bf16x8 (&f)[W], int buf, int row, int part) {
 #pragma unroll
     for (int i = 0; i < W; ++i)
-      f[i] = *reinterpret_cast<const bf16x8 *>(lds + buf + part * kPartB + row + i * 1024);
+      f[i] = *reinterpret_cast<const bf16x8 *>(lds + buf + part * kPartB + row + i * 512);
   };
 
   f32x16 acc[W][W];

@@ -37,7 +37,10 @@ sys.path.insert(0, ROOT)
 
 METRIC = "fused-expr HBM GB/s (% of 8 TB/s); GEMM TFLOP/s at err≤1e-5 vs FP64; vs plain"
 HBM_PEAK_GBS = 8000.0
-PEAK_TFLOPS = {"fp32": 157.3, "bf16": 2500.0, "bf16x3": 2500.0, "fp8": 5000.0}
+# Peak of the matrix instructions that each GEMM variant runs on at 4096^3, and its products of them: FP32
+# multiplies three BF16 parts of each operand, six products.
+PEAK_TFLOPS = {"fp32": 2500.0, "bf16": 2500.0, "bf16x3": 2500.0, "fp8": 5000.0}
+MFMA_PRODUCTS = {"fp32": 6, "bf16": 1, "bf16x3": 3, "fp8": 1}
 # Input/output sets the headline rotates through: 16 x 32 MiB = 512 MiB, twice the 256 MB
 # Infinity Cache, and within the GPU's TLB reach (past 16 sets the headline kernel, whose
 # permuted read touches every 2 MiB page of X from the first wave, slows by a fifth).
@@ -583,7 +586,7 @@ def bench_gemm(T, capi, variants, reps=10, streams=2):
         tflops = 2.0 * n ** 3 * reps / (ms * 1e-3) / 1e12
         out[name] = {"tflops": tflops, "ms": ms / reps, "normalized_error": errs["uniform"],
                      "normalized_error_row_scaled": errs["row_scaled"],
-                     "mfma_util": tflops * (3 if name == "bf16x3" else 1) / PEAK_TFLOPS[name]}
+                     "mfma_util": tflops * MFMA_PRODUCTS[name] / PEAK_TFLOPS[name]}
         if streams > 1:
             # independent calls (the same operands, an output per stream) spread over
             # `streams` streams, each with its own operand scratch: one call's operand packing

@@ -545,8 +545,8 @@ struct RowPlan {
 
 // Where the lines lie (whole calls with the total, in us: a workgroup per row against the rule):
 //   * up to 2048 columns a row is 8 vectors per lane of one wave, so a workgroup per row spends
-//     its time starting and combining: 120011 x 77 109.0 / 12.5, 524288 x 8 463 / 9.4,
-//     60000 x 128 57.8 / 9.4, 16384 x 1024 19.3 / 14.8, 16000 x 1025 21.6 / 15.7; equal at
+//     its time starting and combining: 120011 x 77 109.0 / 11.9, 524288 x 8 464 / 8.7,
+//     60000 x 128 57.8 / 8.9, 16384 x 1024 19.5 / 14.3, 16000 x 1025 21.6 / 15.7; equal at
 //     2047 columns (15.4 / 15.6); at 4096 the workgroup per row is ahead (43.3 / 45.8).
 //   * few rows (at most 8 per CU, all resident at once) of more than 256 columns keep a workgroup
 //     per row, since nothing else fills the chip: 2000 x 2000 7.5 / 7.2.

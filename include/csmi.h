@@ -411,7 +411,9 @@ cs_status cs_fill_normal(cs_stream *stream, float *out, int64_t n, uint32_t seed
  * The reference builds this from split/broadcast/join (README.md:301-362,
  * TensorsSpec.scala:468-528); every variant here accumulates in FP32. */
 typedef enum cs_gemm_variant {
-  CS_GEMM_FP32 = 0,     /* FP32 operands, FP32 products and sums (reference semantics) */
+  CS_GEMM_FP32 = 0,     /* FP32 operands, FP32 sums (reference semantics). Large products multiply three
+                           BF16 parts of each operand, exact together, but for the three smallest of
+                           the nine products of parts; operands out of their range FP32 itself */
   CS_GEMM_BF16 = 1,     /* operands rounded to BF16, BF16 MFMA, FP32 accumulate */
   CS_GEMM_BF16X3 = 2,   /* split-BF16x3: A=Ah+Al, B=Bh+Bl, AhBh + AhBl + AlBh, FP32 accumulate */
   CS_GEMM_FP8 = 3       /* FP8 e4m3 with one scale per 128-wide K block of each row of A

@@ -1485,7 +1485,11 @@ Plan choose_path(double cus, double M, double N, double K, const DirectPlan &p) 
   const double e = 16.0 * p.t, blocks = p.wk == 1 ? std::ceil(std::ceil(M / e) / 4) * std::ceil(N / e) : tiles(e);
   const double packed = r.base + r.pack * (M + N) * K + 0.5e-6 * M * N;
   const double t256 = tiles(256), r128 = rounds(tiles(128)), pairs = std::floor(r128 / 2);
-  const double flops = 2e-6 * tiles(e) * e * e * K / r.direct[p.t / 2], out = (KIND == kF32 ? 0.5e-6 : 1.2e-6) * M * N;
+  const double steps = std::ceil(K / (KIND == kF32 ? 16 : KIND == kFP8 ? 128 : 32));  // of the direct kernel
+  // where a workgroup has idle waves nothing hides the padding of FP8's K steps of 128 (1x100000x64: 44 us,
+  // packed 19; 3547x68x20, whose four waves have tiles, 5.9 / 8.3)
+  const double deep = KIND == kFP8 && p.wk == 1 && M <= 3 * e ? 128 * steps : K;
+  const double flops = 2e-6 * tiles(e) * e * e * deep / r.direct[p.t / 2], out = (KIND == kF32 ? 0.5e-6 : 1.2e-6) * M * N;
   auto direct = [&](double slices) { return 4 + flops * rounds(blocks * slices) * cus / (blocks * slices) + out; };
   const double time[] = {
       direct(1),
@@ -1500,7 +1504,6 @@ Plan choose_path(double cus, double M, double N, double K, const DirectPlan &p) 
     t += 3 + 1.2e-6 * slices * M * N;
     if (t < 0.95 * least) best = {candidate, slices}, least = t;
   };
-  const double steps = K / (KIND == kF32 ? 16 : KIND == kFP8 ? 128 : 32);
   for (int s = 2; s <= 16 && blocks * s <= cus && p.wk * s <= steps; s *= 2) consider(kDirect, s, direct(s));
   for (int s = 2; s <= 8 && tiles(128) * s <= cus && 128 * s <= K; ++s)
     consider(KIND == kF32 ? kTiles128 : kDeep128, s, packed + K / s * (KIND == kF32 ? r.t128 : r.deep));

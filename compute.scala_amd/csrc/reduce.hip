@@ -377,6 +377,7 @@ __global__ __launch_bounds__(kBlock) void reduce_short_rows_kernel(const float *
 // combine (5.9 TB/s), 20011 x 1003 19.0 us against 26.3 us with one column per thread and one
 // thread per column in the combine, 524288 x 8 9.9 us against 169 us (a wave with two active
 // lanes).
+template <bool kFew>
 __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(const float *__restrict__ in, int64_t rows,
                                                              int64_t cols, int across, int64_t rows_per_slice,
                                                              double *partial64, float *col_sum) {
@@ -430,10 +431,9 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(const float *__rest
     for (int k = 0; k < 4; ++k) part[(rl * across + cl) * 4 + k] = a[k].result64();
   }
   __syncthreads();
-  const int t = threadIdx.x;
-  if (t < across * 4) {
-    // thread t adds column t of the workgroup's columns; in an overlapping group the column sits
-    // nearer to the group's end
+  for (int t = threadIdx.x; t < across * 4; t += kBlock) {
+    // column t of the workgroup's columns; in an overlapping group the column sits nearer to the
+    // group's end
     const int64_t col = int64_t(blockIdx.x) * across * 4 + t;
     if (col < cols) {
       const int64_t group = col - t % 4;
@@ -443,6 +443,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(const float *__rest
       if (col_sum) col_sum[col] = float(s);
       else partial64[int64_t(blockIdx.y) * cols + col] = s;
     }
+    if (!kFew) break;  // at most 64 threads across
   }
 }
 
@@ -632,7 +633,8 @@ struct ColPlan {
 //   * at least eight rows per row lane (60000 x 128: 11.0; with 32 13.8).
 //   * up to 32 rows per row lane in one slice, which needs no combine (116 x 2588: 4.2 against
 //     6.8 with two launches); 128 leave one workgroup busy too long (1000 x 100: 13.3 against 6.7).
-//   * 64 threads across, for whole rows of 1 KiB per wave; up to 1024 rows fewer, down to 16, as
+//   * 64 threads across, for whole rows of 1 KiB per wave, more where there are fewer rows than row
+//     lanes (1 x 16000000: 27.3 against 72.8, 2 x 8000000 25.0 against 39.9); up to 1024 rows fewer, down to 16, as
 //     long as that brings workgroups (300 x 16384: 6.1 against 7.9; 116 x 2588: 4.2 against 6.4).
 //     Taller matrices lose by it (20011 x 1003: 22.8 against 19.0).
 constexpr int64_t kMinRowsPerLane = 8, kOneSliceRowsPerLane = 32, kNarrowRows = 1024;
@@ -642,6 +644,7 @@ ColPlan plan_cols(cs_stream *stream, int64_t rows, int64_t cols) {
   const int64_t cus = stream->device->props.multiProcessorCount;
   const int64_t quads = (cols + 3) / 4;
   int64_t most = 64;
+  while (most * 2 * std::max<int64_t>(rows, 1) <= kBlock) most *= 2;
   while (rows <= kNarrowRows && most > 16 && (quads + most - 1) / most < cus) most /= 2;
   p.groups = (quads + most - 1) / most;
   if (p.groups > 0x7fffffff) fail(CS_INVALID_VALUE, "too many columns");
@@ -768,11 +771,12 @@ cs_status cs_reduce_cols(cs_stream *stream, const float *in, int64_t rows, int64
     if (p.slices == 1) {
       // none needed, but a call sizes the scratch for smaller ones under capture
       if (scratch_fits(stream, 4096)) scratch_for(stream, 0);
-      hipLaunchKernelGGL(reduce_cols_kernel, grid, dim3(kBlock), 0, stream->stream, in, rows, cols, p.across,
-                         p.rows_per_slice, static_cast<double *>(nullptr), col_sum);
+      hipLaunchKernelGGL((p.across > 64 ? reduce_cols_kernel<true> : reduce_cols_kernel<false>), grid, dim3(kBlock), 0,
+                         stream->stream, in, rows, cols, p.across, p.rows_per_slice, static_cast<double *>(nullptr),
+                         col_sum);
     } else {
       ReduceScratch s = scratch_for(stream, static_cast<size_t>(p.slices * cols));
-      hipLaunchKernelGGL(reduce_cols_kernel, grid, dim3(kBlock), 0, stream->stream, in, rows, cols, p.across,
+      hipLaunchKernelGGL(reduce_cols_kernel<false>, grid, dim3(kBlock), 0, stream->stream, in, rows, cols, p.across,
                          p.rows_per_slice, s.partial64, static_cast<float *>(nullptr));
       const int64_t width = kBlock / p.finish_lanes;
       hipLaunchKernelGGL(finish_cols_kernel, dim3(static_cast<unsigned>((cols + width - 1) / width)), dim3(kBlock), 0,

@@ -233,6 +233,15 @@ __device__ __forceinline__ void add_vector(f4u v, Acc &a, float &m) {
   m = nanmax(m, nanmax(nanmax(v.x, v.y), nanmax(v.z, v.w)));
 }
 
+// Where the row kernels write, each nullable: a row's sum and maximum, the workgroups' partial sums, and
+// the total where there is one workgroup. One argument, since a small call takes as long as its launches.
+struct RowOutputs {
+  float *row_sum, *row_max;
+  double *partial64;
+  float *total;
+  double *total64;
+};
+
 // One row's share of a lane: vectors lane, lane + kStep, ... of p, four loads in flight. The
 // cols % 4 elements after the last whole vector ride with the other loads: in a wave or less as the end
 // of one more vector that overlaps it (120011 x 77 12.0 us, one by one 13.1), in a workgroup one by one,
@@ -308,18 +317,17 @@ __device__ __forceinline__ void read_row(const float *__restrict__ p, Index cols
 // partial of the row for the total.
 template <int kThreads, bool kShort>
 __global__ __launch_bounds__(kThreads) void reduce_rows_kernel(const float *__restrict__ in, int64_t cols,
-                                                               float *row_sum, float *row_max, double *partial64,
-                                                               float *total, double *total64) {
+                                                               RowOutputs out) {
   const int64_t row = blockIdx.x;
   Acc a;
   float m = __builtin_nanf("");
   read_row<kThreads, kShort>(in + row * cols, cols, threadIdx.x, a, m);
   block_reduce<kThreads / 64>(a, m);
   if (threadIdx.x == 0) {
-    if (row_sum) row_sum[row] = a.result();
-    if (row_max) row_max[row] = m;
-    if (partial64 && gridDim.x == 1) write_total(a.result64(), total, total64);
-    else if (partial64) partial64[row] = a.result64();
+    if (out.row_sum) out.row_sum[row] = a.result();
+    if (out.row_max) out.row_max[row] = m;
+    if (out.partial64 && gridDim.x == 1) write_total(a.result64(), out.total, out.total64);
+    else if (out.partial64) out.partial64[row] = a.result64();
   }
 }
 
@@ -330,9 +338,7 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_kernel(const float *__re
 // 109 us when every row had a workgroup; 16000 x 1025 15.7 us (4.2 TB/s) against 25.2.
 template <int kG, bool kShort>
 __global__ __launch_bounds__(kBlock) void reduce_short_rows_kernel(const float *__restrict__ in, int64_t rows,
-                                                                   int64_t cols, int tiles, float *row_sum,
-                                                                   float *row_max, double *partial64, float *total,
-                                                                   double *total64) {
+                                                                   int64_t cols, int tiles, RowOutputs out) {
   __shared__ double lw[kWaves];
   const int lane = threadIdx.x % kG, group = threadIdx.x / kG;
   double sum = 0.0;  // of this lane's rows
@@ -348,12 +354,12 @@ __global__ __launch_bounds__(kBlock) void reduce_short_rows_kernel(const float *
       m = nanmax(m, m2);
     }
     if (lane == 0 && row < rows) {
-      if (row_sum) row_sum[row] = a.result();
-      if (row_max) row_max[row] = m;
+      if (out.row_sum) out.row_sum[row] = a.result();
+      if (out.row_max) out.row_max[row] = m;
       sum += a.result64();
     }
   }
-  if (!partial64) return;
+  if (!out.partial64) return;
 #pragma unroll
   for (int off = 32; off >= kG; off >>= 1) sum += __shfl_xor(sum, off, 64);  // lane 0 of each row group holds a value
   if ((threadIdx.x & 63) == 0) lw[threadIdx.x >> 6] = sum;
@@ -362,8 +368,8 @@ __global__ __launch_bounds__(kBlock) void reduce_short_rows_kernel(const float *
     double s = lw[0];
 #pragma unroll
     for (int w = 1; w < kWaves; ++w) s += lw[w];
-    if (gridDim.x == 1) write_total(s, total, total64);
-    else partial64[blockIdx.x] = s;
+    if (gridDim.x == 1) write_total(s, out.total, out.total64);
+    else out.partial64[blockIdx.x] = s;
   }
 }
 
@@ -579,25 +585,24 @@ RowPlan plan_rows(cs_stream *stream, int64_t rows, int64_t cols) {
 
 template <int kG, bool kShort>
 void launch_short_rows(cs_stream *stream, const RowPlan &p, const float *in, int64_t rows, int64_t cols,
-                       float *row_sum, float *row_max, double *partial64, float *total, double *total64) {
+                       const RowOutputs &out) {
   hipLaunchKernelGGL((reduce_short_rows_kernel<kG, kShort>), dim3(static_cast<unsigned>(p.grid)), dim3(kBlock), 0,
-                     stream->stream, in, rows, cols, p.tiles, row_sum, row_max, partial64, total, total64);
+                     stream->stream, in, rows, cols, p.tiles, out);
 }
 
 template <int kThreads, bool kShort>
-void launch_long_rows(cs_stream *stream, const RowPlan &p, const float *in, int64_t cols, float *row_sum,
-                      float *row_max, double *partial64, float *total, double *total64) {
+void launch_long_rows(cs_stream *stream, const RowPlan &p, const float *in, int64_t cols,
+                      const RowOutputs &out) {
   hipLaunchKernelGGL((reduce_rows_kernel<kThreads, kShort>), dim3(static_cast<unsigned>(p.grid)), dim3(kThreads), 0,
-                     stream->stream, in, cols, row_sum, row_max, partial64, total, total64);
+                     stream->stream, in, cols, out);
 }
 
 // The row pass of a plan and, when partial64 is not null, the combine of its plan.grid partials (one
 // workgroup writes the total itself).
-void launch_rows(cs_stream *stream, const RowPlan &p, const float *in, int64_t rows, int64_t cols, float *row_sum,
-                 float *row_max, double *partial64, float *total, double *total64) {
+void launch_rows(cs_stream *stream, const RowPlan &p, const float *in, int64_t rows, int64_t cols,
+                 const RowOutputs &out) {
 #define CSMI_ROWS(kG) \
-  (cols <= 4 * kG ? launch_short_rows<kG, true> : launch_short_rows<kG, false>)(stream, p, in, rows, cols, row_sum, \
-                                                                             row_max, partial64, total, total64)
+  (cols <= 4 * kG ? launch_short_rows<kG, true> : launch_short_rows<kG, false>)(stream, p, in, rows, cols, out)
   switch (p.lanes) {
     case 2: CSMI_ROWS(2); break;
     case 4: CSMI_ROWS(4); break;
@@ -608,11 +613,10 @@ void launch_rows(cs_stream *stream, const RowPlan &p, const float *in, int64_t r
     default:
       (p.wide                ? launch_long_rows<1024, false>
        : cols <= 4 * kBlock  ? launch_long_rows<kBlock, true>
-                             : launch_long_rows<kBlock, false>)(stream, p, in, cols, row_sum, row_max, partial64,
-                                                                total, total64);
+                             : launch_long_rows<kBlock, false>)(stream, p, in, cols, out);
   }
 #undef CSMI_ROWS
-  if (partial64 && p.grid > 1) launch_finish_sum(stream, partial64, p.grid, total, total64);
+  if (out.partial64 && p.grid > 1) launch_finish_sum(stream, out.partial64, p.grid, out.total, out.total64);
 }
 }  // namespace
 
@@ -727,7 +731,7 @@ cs_status cs_reduce_rows(cs_stream *stream, const float *in, int64_t rows, int64
     }
     const RowPlan plan = plan_rows(stream, rows, cols);
     ReduceScratch s = scratch_for(stream, want_total ? static_cast<size_t>(plan.grid) : 0);
-    launch_rows(stream, plan, in, rows, cols, row_sum, row_max, want_total ? s.partial64 : nullptr, total, total64);
+    launch_rows(stream, plan, in, rows, cols, {row_sum, row_max, want_total ? s.partial64 : nullptr, total, total64});
     CS_HIP(hipGetLastError());
   });
 }
@@ -754,7 +758,7 @@ cs_status cs_reduce_rows_noalloc(cs_stream *stream, const float *in, int64_t row
     }
     // every partial the combine reads is written by this call's row kernel first
     double *partial64 = want_total ? noalloc_scratch(stream->device) : nullptr;
-    launch_rows(stream, plan_rows(stream, rows, cols), in, rows, cols, row_sum, row_max, partial64, total, total64);
+    launch_rows(stream, plan_rows(stream, rows, cols), in, rows, cols, {row_sum, row_max, partial64, total, total64});
     CS_HIP(hipGetLastError());
   });
 }

@@ -1337,12 +1337,9 @@ void run_lds(cs_stream *stream, int M, int N, int K, const float *A, int lda, co
     const int64_t blocks = int64_t(pa.row_blocks) + int64_t(pa.cols_gx) * col_tiles_k;
     hipLaunchKernelGGL(pack_operands_kernel<KIND>, dim3(unsigned(blocks)), dim3(256), 0, s, pa);
   }
-  static const bool configured = [] {
-    CS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_lds_kernel<KIND, W, kBufs>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes(W, kBufs))));
-    return true;
-  }();
-  (void)configured;
+  static std::atomic<uint64_t> allowed{0};
+  allow_lds(allowed, stream->device->ordinal, reinterpret_cast<const void *>(&gemm_lds_kernel<KIND, W, kBufs>),
+            lds_bytes(W, kBufs));
   const dim3 grid(static_cast<unsigned>((Mp / kTile) * (Np / kTile)), unsigned(to.slices));
   hipLaunchKernelGGL((gemm_lds_kernel<KIND, W, kBufs>), grid, dim3(kThreads), lds_bytes(W, kBufs), s, M, N, int(Kp),
                      int(Mp), int(Np), x, y, sx, sy, to.out, to.ld, to.slices);
@@ -1370,12 +1367,9 @@ bool run_split(cs_stream *stream, int M, int N, int K, const float *A, int lda, 
   p.row_blocks = unsigned(Mp / 64 * chunks);
   const int64_t blocks = int64_t(p.row_blocks) + Np / 64 * chunks;
   hipLaunchKernelGGL(split_operands_kernel, dim3(unsigned(blocks)), dim3(256), 0, stream->stream, p);
-  static const bool configured = [] {
-    CS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_split_kernel<W>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(split_lds_bytes(W))));
-    return true;
-  }();
-  (void)configured;
+  static std::atomic<uint64_t> allowed{0};
+  allow_lds(allowed, stream->device->ordinal, reinterpret_cast<const void *>(&gemm_split_kernel<W>),
+            split_lds_bytes(W));
   const dim3 grid(unsigned((Mp / kTile) * (Np / kTile)), unsigned(to.slices));
   hipLaunchKernelGGL(gemm_split_kernel<W>, grid, dim3(kThreads), split_lds_bytes(W), stream->stream, M, N, K, int(Kp),
                      int(Mp), int(Np), p.x, p.y, p.ea, p.eb, A, lda, B, ldb, to.out, to.ld, to.slices);
@@ -1489,7 +1483,8 @@ Plan choose_path(double cus, double M, double N, double K, const DirectPlan &p) 
   // where a workgroup has idle waves nothing hides the padding of FP8's K steps of 128 (1x100000x64: 44 us,
   // packed 19; 3547x68x20, whose four waves have tiles, 5.9 / 8.3)
   const double deep = KIND == kFP8 && p.wk == 1 && M <= 3 * e ? 128 * steps : K;
-  const double flops = 2e-6 * tiles(e) * e * e * deep / r.direct[p.t / 2], out = (KIND == kF32 ? 0.5e-6 : 1.2e-6) * M * N;
+  const double flops = 2e-6 * tiles(e) * e * e * deep / r.direct[p.t / 2];
+  const double out = (KIND == kF32 ? 0.5e-6 : 1.2e-6) * M * N;
   auto direct = [&](double slices) { return 4 + flops * rounds(blocks * slices) * cus / (blocks * slices) + out; };
   const double time[] = {
       direct(1),

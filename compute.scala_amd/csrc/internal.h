@@ -197,6 +197,14 @@ struct cs_graph {
 };
 
 namespace csmi {
+// Lets `kernel` take `bytes` of dynamic LDS on device `ordinal`, the current one; `done` holds the devices
+// where it has been called.
+inline void allow_lds(std::atomic<uint64_t> &done, int ordinal, const void *kernel, size_t bytes) {
+  const uint64_t bit = uint64_t(1) << (ordinal & 63);
+  if (done.load(std::memory_order_relaxed) & bit) return;
+  CS_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)));
+  done.fetch_or(bit, std::memory_order_relaxed);
+}
 // Stream-owned scratch of at least `bytes`, zero-filled when (re)allocated. Growing it
 // synchronizes the stream, so the first call of a given size must not be under capture.
 // The buffer it replaces stays allocated until the stream is destroyed.

@@ -499,12 +499,8 @@ unsigned network_grid(cs_stream *stream, int64_t n, int64_t per_cu) {
 template <bool kGrad, int kS>
 void launch_network(cs_stream *stream, const NetShape &shape, size_t lds, unsigned grid, const cs_mlp *net,
                     const float *X, const float *target, int64_t n, float *y, float *partial, double *partial_loss) {
-  static const bool configured = [] {
-    CS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&network_kernel<kGrad, kS>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10));
-    return true;
-  }();
-  (void)configured;
+  static std::atomic<uint64_t> allowed{0};
+  allow_lds(allowed, stream->device->ordinal, reinterpret_cast<const void *>(&network_kernel<kGrad, kS>), 160 << 10);
   hipLaunchKernelGGL((network_kernel<kGrad, kS>), dim3(grid), dim3(kNet), lds, stream->stream, shape, net->params, X,
                      target, n, y, partial, partial_loss);
 }
@@ -633,7 +629,8 @@ cs_status cs_mlp_backward(cs_stream *stream, cs_mlp *mlp, const float *X, const 
       double *partial_loss = reinterpret_cast<double *>(mlp->deltas);
       float *partial = mlp->deltas + 2 * grid;
       launch_network<true, kSamples>(stream, shape, lds, grid, mlp, X, target, n, nullptr, partial, partial_loss);
-      hipLaunchKernelGGL(reduce_grads_kernel, dim3(blocks(kGradLanes * mlp->count) + 1), dim3(kB), 0, stream->stream, partial,
+      hipLaunchKernelGGL(reduce_grads_kernel, dim3(blocks(kGradLanes * mlp->count) + 1), dim3(kB), 0, stream->stream,
+                         partial,
                          static_cast<int>(mlp->count), static_cast<int>(grid), partial_loss, n, grads, loss);
       CS_HIP(hipGetLastError());
       return;

@@ -66,8 +66,7 @@ struct Slab {
   size_t in_use = 0;
 };
 
-// An event recorded on a stream (nullptr: the null stream) when a block was released; without an
-// event, the block is free once all work queued on the stream by then is done.
+// An event recorded on a stream (nullptr: the null stream) when a block was released.
 struct StreamEvent {
   hipStream_t stream;
   hipEvent_t event;
@@ -215,8 +214,8 @@ bool scratch_fits(cs_stream *stream, size_t bytes);
 // combine that turns n partials into *out (FP32, nullable) and *out64 (nullable).
 double *sum_partials(cs_stream *stream, size_t n);
 void launch_finish_sum(cs_stream *stream, const double *partials, int64_t n, float *out, double *out64);
-// Events recorded now on every live stream of the device (for stream-ordered frees).
-std::vector<StreamEvent> record_on_all_streams(cs_device *device);
+// Events recorded now on every live stream of the device that has work queued (for stream-ordered frees).
+std::vector<StreamEvent> record_on_busy_streams(cs_device *device);
 // Makes `device` current on the calling thread.
 void set_device(cs_device *device);
 // hiprtc build of `source` for the device's arch; throws Error with the log on failure.

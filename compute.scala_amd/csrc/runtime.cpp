@@ -96,17 +96,7 @@ void Arena::drain_pending(bool wait) {
     PendingFree &p = pending_.front();
     bool done = true;
     for (const StreamEvent &se : p.events) {
-      if (!se.event) {
-        // ordered on se.stream, without an event: complete once that stream is (it waited for
-        // itself before a capture began)
-        if (!wait) {
-          done = false;
-          break;
-        }
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        CS_HIP(hipStreamIsCapturing(se.stream, &cap));
-        if (cap == hipStreamCaptureStatusNone) CS_HIP(hipStreamSynchronize(se.stream));
-      } else if (wait) {
+      if (wait) {
         CS_HIP(hipEventSynchronize(se.event));
       } else if (hipEventQuery(se.event) != hipSuccess) {
         (void)hipGetLastError();
@@ -115,8 +105,7 @@ void Arena::drain_pending(bool wait) {
       }
     }
     if (!done) return;
-    for (const StreamEvent &se : p.events)
-      if (se.event) (void)hipEventDestroy(se.event);
+    for (const StreamEvent &se : p.events) (void)hipEventDestroy(se.event);
     give_back(p.block);
     pending_.pop_front();
   }
@@ -129,8 +118,7 @@ void Arena::hand_back_ordered(hipStream_t stream) {
   // the blocks it takes (its own events need no wait: its work is ordered).
   while (!pending_.empty()) {
     PendingFree &p = pending_.front();
-    for (const StreamEvent &se : p.events)
-      if (se.event) retired_.push_back(se);  // without one: this stream's own work, or work it waited for when created
+    for (const StreamEvent &se : p.events) retired_.push_back(se);
     give_back(p.block);
     pending_.pop_front();
   }
@@ -229,13 +217,18 @@ void Arena::trim() {
   }
 }
 
-std::vector<StreamEvent> record_on_all_streams(cs_device *device) {
+std::vector<StreamEvent> record_on_busy_streams(cs_device *device) {
   std::vector<StreamEvent> evs;
   auto record = [&](hipStream_t s) {
+    // Nothing to wait for on an idle stream (the null stream is idle when the blocking streams are, too):
+    // creating, recording and destroying the events of two idle streams took 14 of the 17 us of an
+    // allocation and its release.
+    if (hipStreamQuery(s) == hipSuccess) return;
+    (void)hipGetLastError();
     hipEvent_t ev;
     CS_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    CS_HIP(hipEventRecord(ev, s));
     evs.push_back(StreamEvent{s, ev});
+    CS_HIP(hipEventRecord(ev, s));
   };
   // A stream that is capturing a graph is skipped: an event recorded there would become a
   // node of the graph, and capture starts on an idle stream (cs_graph_begin_capture waits
@@ -250,15 +243,6 @@ std::vector<StreamEvent> record_on_all_streams(cs_device *device) {
   }
   // The null stream covers raw launches made outside library streams; it is left alone
   // while a capture is open.
-  // With one library stream and an idle null stream the block is ordered on that stream alone, and
-  // no event is needed: later work on it comes after, a stream created later first waits for it
-  // (cs_stream_create), and an allocation that waits on the host waits for the stream. Recording two
-  // events and destroying them again took 14 of the 17 us of an allocation and its release.
-  if (!capturing && live.size() == 1 && hipStreamQuery(nullptr) == hipSuccess) {
-    evs.push_back(StreamEvent{live.front(), nullptr});
-    return evs;
-  }
-  (void)hipGetLastError();  // of a null stream that is not ready
   if (!capturing) record(nullptr);
   for (hipStream_t s : live) record(s);
   return evs;
@@ -613,21 +597,6 @@ cs_status cs_stream_create(cs_device *device, cs_stream **stream) {
     s->device = device;
     s->stream = hs;
     std::lock_guard<std::recursive_mutex> l(device->mu);
-    if (device->streams.size() == 1) {
-      // Blocks released while there was one stream carry no event: what the new stream is handed may
-      // still be in use by work on the first, so it begins after that work.
-      hipStream_t first = (*device->streams.begin())->stream;
-      hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-      CS_HIP(hipStreamIsCapturing(first, &cap));
-      if (cap == hipStreamCaptureStatusNone) {
-        hipEvent_t ev = nullptr;
-        CS_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-        hipError_t r = hipEventRecord(ev, first);
-        if (r == hipSuccess) r = hipStreamWaitEvent(hs, ev, 0);
-        (void)hipEventDestroy(ev);
-        CS_HIP(r);
-      }
-    }
     device->streams.insert(s.get());
     *stream = s.release();
   });
@@ -815,7 +784,7 @@ cs_status cs_buffer_release(cs_buffer *buffer) {
       cs_device *d = buffer->device;
       set_device(d);
       std::lock_guard<std::recursive_mutex> l(d->mu);
-      d->arena->release(buffer->block, record_on_all_streams(d));
+      d->arena->release(buffer->block, record_on_busy_streams(d));
       delete buffer;
     }
   });
@@ -1121,7 +1090,9 @@ cs_status cs_graph_begin_capture(cs_stream *stream) {
     set_device(stream->device);
     // Capture starts on an idle stream, so buffers released during the capture are not in
     // use by work queued on it before (their release events skip capturing streams). The lock
-    // keeps releases from coming between the wait and the capture.
+    // keeps releases from coming between the wait and the capture; the first wait is without it, so
+    // that other threads are not held up by this stream's work.
+    CS_HIP(hipStreamSynchronize(stream->stream));
     std::lock_guard<std::recursive_mutex> l(stream->device->mu);
     CS_HIP(hipStreamSynchronize(stream->stream));
     CS_HIP(hipStreamBeginCapture(stream->stream, hipStreamCaptureModeThreadLocal));

@@ -1362,6 +1362,10 @@ struct cs_fused {
   int max_block = 1024;      // the kernel's launch bound
   Dag dag;                   // kept for batches, which re-emit the body
   Options opts;
+  // The same expression at a width that divides its rows, once a launch has needed it (LaunchKernel).
+  // Not in the cache: it lives, its code loaded, as long as the kernel that stands for it.
+  std::atomic<cs_fused *> dividing{nullptr};
+  ~cs_fused() { delete dividing.load(); }
 };
 
 struct cs_batch {
@@ -1486,9 +1490,8 @@ static void one_block_sum(const Dag &dag, Options *o) {
   if (dag.nodes.size() <= kLargeBody && per_thread <= 4) o->U = static_cast<int>(std::max<int64_t>(per_thread, 1));
 }
 
-// Compiles the kernel of `dag` under `o` into the device's cache (or takes the one another thread
-// has put there meanwhile); the caller gets a reference.
-static cs_fused *build_fused(cs_device *device, Dag dag, const Options &o, const std::string &key) {
+// Compiles the kernel of `dag` under `o`.
+static std::unique_ptr<cs_fused> build_fused(cs_device *device, Dag dag, const Options &o, const std::string &key) {
   int64_t vectors = 0;
   const std::string name = kernel_name(key, o);
   std::string src = Emitter(dag, o).generate(&vectors, name);
@@ -1514,54 +1517,32 @@ static cs_fused *build_fused(cs_device *device, Dag dag, const Options &o, const
   f->grid = static_cast<uint32_t>((vectors + per_block - 1) / per_block);
   f->dag = std::move(dag);
   f->opts = o;
-  std::lock_guard<std::recursive_mutex> l(device->mu);
-  auto it = device->fused_cache.find(key);
-  if (it != device->fused_cache.end()) {  // another thread won the race
-    it->second->refs++;
-    return it->second;
-  }
-  f->refs = 2;  // one for the cache, one for the caller
-  device->fused_cache.emplace(key, f.get());
-  return f.release();
+  return f;
 }
 
 // The kernel that a launch of `fused` into `out` runs: `fused` itself, or, where its rows are ragged
-// and the output lies over a leaf, the same expression at a width that divides the rows (compiled on
-// the first such launch, which may be under capture). Holds a reference while it lives.
+// and the output lies over a leaf, the same expression at a width that divides the rows, compiled on
+// the first such launch (which may be under capture) and owned by `fused`.
 class LaunchKernel {
  public:
   LaunchKernel(cs_fused *fused, const void *const *leaves, const void *out) : f_(fused) {
-    if (!ragged_rows(fused->dag, fused->opts) || !over_leaf(fused, leaves, out)) {
-      f_->refs++;
-      return;
-    }
+    if (!ragged_rows(fused->dag, fused->opts) || !over_leaf(fused, leaves, out)) return;
+    if ((f_ = fused->dividing.load())) return;
     Options o = fused->opts;
     const int64_t last = fused->dag.out_shape.back();
     while (o.V > 1 && last % o.V != 0) o.V /= 2;
-    const std::string key = canonical_key(fused->dag, o);
-    cs_device *device = fused->device;
-    {
-      std::lock_guard<std::recursive_mutex> l(device->mu);
-      auto it = device->fused_cache.find(key);
-      if (it != device->fused_cache.end()) {
-        f_ = it->second;
-        f_->refs++;
-        return;
-      }
-    }
+    std::unique_ptr<cs_fused> built;
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     CS_HIP(hipThreadExchangeStreamCaptureMode(&mode));
     try {
-      f_ = build_fused(device, fused->dag, o, key);
+      built = build_fused(fused->device, fused->dag, o, canonical_key(fused->dag, o));
     } catch (...) {
       (void)hipThreadExchangeStreamCaptureMode(&mode);
       throw;
     }
     CS_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+    if (fused->dividing.compare_exchange_strong(f_, built.get())) f_ = built.release();  // else another thread's
   }
-  ~LaunchKernel() { (void)cs_fused_release(f_); }
-  LaunchKernel(const LaunchKernel &) = delete;
-  LaunchKernel &operator=(const LaunchKernel &) = delete;
   cs_fused *operator->() const { return f_; }
 
  private:
@@ -1601,7 +1582,17 @@ static cs_status compile_fused(cs_device *device, const cs_node *nodes, int nnod
         return;
       }
     }
-    *fused = build_fused(device, std::move(dag), o, key);
+    std::unique_ptr<cs_fused> f = build_fused(device, std::move(dag), o, key);
+    std::lock_guard<std::recursive_mutex> l(device->mu);
+    auto it = device->fused_cache.find(key);
+    if (it != device->fused_cache.end()) {  // another thread won the race
+      it->second->refs++;
+      *fused = it->second;
+      return;
+    }
+    f->refs = 2;  // one for the cache, one for the caller
+    device->fused_cache.emplace(key, f.get());
+    *fused = f.release();
   });
 }
 

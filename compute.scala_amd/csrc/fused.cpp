@@ -748,12 +748,16 @@ class Emitter {
   // 48.1 / 47.7. Longer or odd runs leave each instruction every other piece of a line, which written
   // through becomes partial-line writes: those stay plain or plainly non-temporal, as do the bodies
   // of a batch, whose kernel ends once.
+  // A store of more than two registers reads them up to two wait states after it has issued. The compiler
+  // keeps later writes of them that far behind its own stores, but does not look into the assembly, so
+  // the wait is written there.
   std::string store(const std::string &addr, const std::string &val, const std::string &type, int run) {
     const bool whole = (run == 4 && type != "float") || (run == 1 && type == "float");
     if (whole && (o_.nt || gq_.empty())) {
-      const std::string op = type != "float" ? "global_store_dwordx4" : "global_store_dword";
-      return "asm volatile(\"" + op + " %0, %1, off sc1" + (o_.nt ? " nt" : "") + "\" :: \"v\"((" + gq_ + type +
-             "*)(" + addr + ")), \"v\"(" + val + ") : \"memory\");";
+      const bool wide = type != "float";
+      return std::string("asm volatile(\"") + (wide ? "global_store_dwordx4" : "global_store_dword") + " %0, %1, off sc1" +
+             (o_.nt ? " nt" : "") + (wide ? "\\n\\ts_nop 1" : "") + "\" :: \"v\"((" + gq_ + type + "*)(" + addr +
+             ")), \"v\"(" + val + ") : \"memory\");";
     }
     if (o_.nt) return "__builtin_nontemporal_store(" + val + ", (" + gq_ + type + "*)(" + addr + "));";
     return "*(" + gq_ + type + "*)(" + addr + ") = " + val + ";";

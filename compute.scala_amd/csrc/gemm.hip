@@ -984,35 +984,45 @@ __global__ __launch_bounds__(kWK == 1 ? 256 : 64 * kWK) void gemm_direct_kernel(
 // meet in one rounding instead of two: relative to |C|, U(-1,1), K = 16 3.2e-8 / 7.4e-8, 256
 // 2.3e-7 / 2.9e-7, 1024 4.8e-7 / 5.7e-7, 4096 1.0e-6 / 1.1e-6.
 // The split is exact, and the products' sums are FP32's, only in a range: not for infinities and
-// NaN, values that round to an infinite BF16, parts below BF16's normal range and products near
-// FP32's. The pre-pass keeps the least exponent of each of its pieces of A and B (0 for values out of
-// range), and a tile of C whose rows or columns leave the range is computed from A and B on the FP32
-// matrix cores (direct_tile).
+// NaN, values that round to an infinite BF16, parts below BF16's normal range, products near FP32's
+// least and sums near its greatest (h may be above x, and hh overflow where ab does not). The pre-pass
+// keeps the least and the greatest exponent of each of its pieces of A and B (0 as the least for values
+// out of range), and a tile of C whose rows or columns leave the range is computed from A and B on the
+// FP32 matrix cores (direct_tile).
 constexpr int kSplitK = 16;  // K values of a stage
 // One part of an operand's stage (W = 4: 8 KiB); h, m and l of both operands are a stage (48 KiB), and
 // three stages are in LDS (144 KiB).
 constexpr int part_bytes(int W) { return tile_edge(W) * kSplitK * 2; }
 constexpr size_t split_lds_bytes(int W) { return size_t(18) * part_bytes(W); }
-// Least exponents (biased) of the operands, and of a product of both, that stay on the BF16 path.
-constexpr unsigned kMinExponent = 24, kMinProduct = 254 - 110;
+// Exponents (biased) of the operands, and of a product of both, that stay on the BF16 path: 2^21 products
+// at most (check_depth) of less than 2^(76 + 2) stay far below an overflow.
+constexpr unsigned kMinExponent = 24, kMinProduct = 254 - 110, kMaxProduct = 254 + 76;
+// The exponents of a piece of an operand: 255 less the least (0 for zeros alone, 255 where a value is out
+// of range), and the greatest. Those of several pieces together are the maxima.
+typedef uint16_t Exponents __attribute__((ext_vector_type(2)));
 
 struct SplitArgs {
   const float *a, *b;
   int m, n, k, lda, ldb, mp, np, kp;
   char *x, *y;         // [kp / 16][3][2][mp or np][8] BF16
-  uint8_t *ea, *eb;    // least exponents: [mp / 64][chunks] and [np / 64][chunks], chunks of 64 K
+  Exponents *ea, *eb;  // [mp / 64][chunks] and [np / 64][chunks], chunks of 64 K
   unsigned row_blocks;
 };
 
-// Splits 16 consecutive K values of one row of an operand, stores them and returns their least
-// exponent: 255 for zeros, 0 for a value out of range.
-__device__ __forceinline__ unsigned split_store(const float (&v)[16], char *dst, int64_t part_stride) {
-  unsigned least = 255;
+__device__ __forceinline__ bool in_split_range(Exponents a, Exponents b) {
+  return 255u - a[0] >= kMinExponent && 255u - b[0] >= kMinExponent && 510u - a[0] - b[0] >= kMinProduct &&
+         unsigned(a[1]) + b[1] <= kMaxProduct;
+}
+
+// Splits 16 consecutive K values of one row of an operand, stores them and returns their exponents.
+__device__ __forceinline__ Exponents split_store(const float (&v)[16], char *dst, int64_t part_stride) {
+  unsigned least = 255, greatest = 0;
 #pragma unroll
   for (int e = 0; e < 16; ++e) {
     const uint32_t bits = __float_as_uint(v[e]) & 0x7fffffffu;
     const unsigned x = bits >= 0x7f7f8000u ? 0u : bits == 0 ? 255u : bits >> 23;
     least = min(least, x);
+    greatest = max(greatest, bits);
   }
   float r[16];
 #pragma unroll
@@ -1030,17 +1040,16 @@ __device__ __forceinline__ unsigned split_store(const float (&v)[16], char *dst,
     *reinterpret_cast<i32x4 *>(dst + part * part_stride) = w[0];
     *reinterpret_cast<i32x4 *>(dst + part * part_stride + part_stride / 2) = w[1];
   }
-  return least;
+  return Exponents{uint16_t(255 - least), uint16_t(greatest >> 23)};
 }
 
 // Workgroups [0, row_blocks) split 64 rows x 64 K of A (a thread per 16 K of a row), the others 64
 // columns x 64 K of B (a thread per 16 K of a column: each load of a wave is 256 contiguous bytes).
 // Rows, columns and K values past the source are zeros.
 __global__ __launch_bounds__(256) void split_operands_kernel(SplitArgs p) {
-  __shared__ unsigned least;
+  __shared__ Exponents waves[4];
   const int t = threadIdx.x;
-  if (t == 0) least = 255;
-  __syncthreads();
+  Exponents exponents = {0, 0};
   const unsigned chunks = unsigned(p.kp + 63) / 64;
   const bool is_a = blockIdx.x < p.row_blocks;
   const unsigned block = is_a ? blockIdx.x : blockIdx.x - p.row_blocks;
@@ -1073,12 +1082,17 @@ __global__ __launch_bounds__(256) void split_operands_kernel(SplitArgs p) {
     }
     const int64_t part_stride = int64_t(is_a ? p.mp : p.np) * 32;
     char *dst = (is_a ? p.x : p.y) + int64_t(k / 16) * 3 * part_stride + int64_t(row) * 16;
-    const unsigned e = split_store(v, dst, part_stride);
-    if (e < 255) atomicMin(&least, e);
+    exponents = split_store(v, dst, part_stride);
   }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1)
+    exponents = __builtin_elementwise_max(
+        exponents, __builtin_bit_cast(Exponents, __shfl_xor(__builtin_bit_cast(int, exponents), off, 64)));
+  if (t % 64 == 0) waves[t / 64] = exponents;
   __syncthreads();
   if (t == 0)
-    (is_a ? p.ea : p.eb)[int64_t(strip) * chunks + chunk] = static_cast<uint8_t>(least);
+    (is_a ? p.ea : p.eb)[int64_t(strip) * chunks + chunk] = __builtin_elementwise_max(
+        __builtin_elementwise_max(waves[0], waves[1]), __builtin_elementwise_max(waves[2], waves[3]));
 }
 
 // 4 waves in 2x2 per output tile, W x W MFMA tiles each, as in gemm_lds_kernel. A stage is 16 K
@@ -1091,7 +1105,7 @@ __global__ __launch_bounds__(256) void split_operands_kernel(SplitArgs p) {
 template <int W>
 __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_split_kernel(
     int M, int N, int K, int Kp, int Mp, int Np, const char *__restrict__ X, const char *__restrict__ Y,
-    const uint8_t *__restrict__ ea, const uint8_t *__restrict__ eb, const float *__restrict__ A, int lda,
+    const Exponents *__restrict__ ea, const Exponents *__restrict__ eb, const float *__restrict__ A, int lda,
     const float *__restrict__ B, int ldb, float *__restrict__ C, int ldc, int slices) {
   constexpr int kTile = tile_edge(W), kWaveRows = 32 * W, kPartB = part_bytes(W), kSplitPanelB = 3 * kPartB,
                 kSplitStageB = 2 * kSplitPanelB;
@@ -1106,21 +1120,23 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_split_kernel(
   C += int64_t(blockIdx.y) * M * ldc;
 
   {
-    unsigned *const least = reinterpret_cast<unsigned *>(lds);
-    if (threadIdx.x < 2) least[threadIdx.x] = 255;
-    __syncthreads();
+    Exponents *const waves = reinterpret_cast<Exponents *>(lds);  // [operand][wave]
     const int pieces = (Kp + 63) / 64 * W;  // of the tile's rows, and of its columns
-    unsigned la = 255, lb = 255;
+    Exponents a = {0, 0}, b = {0, 0};
     for (int i = threadIdx.x; i < pieces; i += kThreads) {
-      la = min(la, unsigned(ea[int64_t(tm) * pieces + i]));
-      lb = min(lb, unsigned(eb[int64_t(tn) * pieces + i]));
+      a = __builtin_elementwise_max(a, ea[int64_t(tm) * pieces + i]);
+      b = __builtin_elementwise_max(b, eb[int64_t(tn) * pieces + i]);
     }
-    atomicMin(&least[0], la);
-    atomicMin(&least[1], lb);
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+      a = __builtin_elementwise_max(a, __builtin_bit_cast(Exponents, __shfl_xor(__builtin_bit_cast(int, a), off, 64)));
+      b = __builtin_elementwise_max(b, __builtin_bit_cast(Exponents, __shfl_xor(__builtin_bit_cast(int, b), off, 64)));
+    }
+    if (lane == 0) waves[wave] = a, waves[4 + wave] = b;
     __syncthreads();
-    la = least[0], lb = least[1];
+    for (int w = 0; w < 4; ++w) a = __builtin_elementwise_max(a, waves[w]), b = __builtin_elementwise_max(b, waves[4 + w]);
     __syncthreads();  // before the stages overwrite them
-    if (la < kMinExponent || lb < kMinExponent || la + lb < kMinProduct) {
+    if (!in_split_range(a, b)) {
       for (int sub = 0; sub < W * W / 4; ++sub) {
         const int ms = m0 + wm * kWaveRows + sub / (W / 2) * 64, ns = n0 + wn * kWaveRows + sub % (W / 2) * 64;
         if (ms >= M || ns >= N) continue;
@@ -1355,7 +1371,7 @@ bool run_split(cs_stream *stream, int M, int N, int K, const float *A, int lda, 
   const int64_t Mp = round_up(M, kTile), Np = round_up(N, kTile), Kp = round_up(K, kSplitK);
   if (std::max(Mp, Np) * 96 >= (int64_t(1) << 31)) return false;
   const int64_t xbytes = Mp * Kp * 6, ybytes = Np * Kp * 6, chunks = (Kp + 63) / 64;
-  const int64_t ebytes = (Mp + Np) / 64 * chunks;
+  const int64_t ebytes = (Mp + Np) / 64 * chunks * int64_t(sizeof(Exponents));
   const int64_t total = xbytes + ybytes + ebytes + 4096;
   if (!scratch_fits(stream, size_t(total))) return false;
   const Target to(stream, total, M, N, C, ldc, slices);
@@ -1363,7 +1379,7 @@ bool run_split(cs_stream *stream, int M, int N, int K, const float *A, int lda, 
   SplitArgs p;
   p.a = A, p.b = B, p.m = M, p.n = N, p.k = K, p.lda = lda, p.ldb = ldb, p.mp = int(Mp), p.np = int(Np), p.kp = int(Kp);
   p.x = base, p.y = base + xbytes;
-  p.ea = reinterpret_cast<uint8_t *>(base + xbytes + ybytes), p.eb = p.ea + Mp / 64 * chunks;
+  p.ea = reinterpret_cast<Exponents *>(base + xbytes + ybytes), p.eb = p.ea + Mp / 64 * chunks;
   p.row_blocks = unsigned(Mp / 64 * chunks);
   const int64_t blocks = int64_t(p.row_blocks) + Np / 64 * chunks;
   hipLaunchKernelGGL(split_operands_kernel, dim3(unsigned(blocks)), dim3(256), 0, stream->stream, p);

@@ -987,13 +987,18 @@ __global__ __launch_bounds__(kWK == 1 ? 256 : 64 * kWK) void gemm_direct_kernel(
 // NaN, values that round to an infinite BF16, parts below BF16's normal range, products near FP32's
 // least and sums near its greatest (h may be above x, and hh overflow where ab does not). The pre-pass
 // keeps the least and the greatest exponent of each of its pieces of A and B (0 as the least for values
-// out of range), and a tile of C whose rows or columns leave the range is computed from A and B on the
-// FP32 matrix cores (direct_tile).
+// out of range), and a tile of C adds the chunks of 64 K where its rows or columns leave the range from A
+// and B on the FP32 matrix cores, whose accumulators lie as the BF16 ones' do.
+// A chunk costs about 2.7 times its split form there: 2048^3 with one value out of range 97 us against 95,
+// with one in every chunk 166 (180 both when such tiles left the split whole); 4096^3 611 (1345) and
+// 1059 (1258; 983 to 1020 in a kernel of FP32 MFMAs alone).
 constexpr int kSplitK = 16;  // K values of a stage
 // One part of an operand's stage (W = 4: 8 KiB); h, m and l of both operands are a stage (48 KiB), and
 // three stages are in LDS (144 KiB).
 constexpr int part_bytes(int W) { return tile_edge(W) * kSplitK * 2; }
-constexpr size_t split_lds_bytes(int W) { return size_t(18) * part_bytes(W); }
+// The chunks of K whose values are out of range follow, a bit each (check_depth bounds K).
+constexpr int kMaxChunks = 1 << 15;
+constexpr size_t split_lds_bytes(int W) { return size_t(18) * part_bytes(W) + kMaxChunks / 8; }
 // Exponents (biased) of the operands, and of a product of both, that stay on the BF16 path: 2^21 products
 // at most (check_depth) of less than 2^(76 + 2) stay far below an overflow.
 constexpr unsigned kMinExponent = 24, kMinProduct = 254 - 110, kMaxProduct = 254 + 76;
@@ -1119,45 +1124,40 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_split_kernel(
 
   C += int64_t(blockIdx.y) * M * ldc;
 
-  {
-    Exponents *const waves = reinterpret_cast<Exponents *>(lds);  // [operand][wave]
-    const int pieces = (Kp + 63) / 64 * W;  // of the tile's rows, and of its columns
+  const int chunks = (Kp + 63) / 64;
+  uint64_t *const out_of_range = reinterpret_cast<uint64_t *>(lds + 3 * kSplitStageB);
+  for (int c = threadIdx.x; c - lane < chunks; c += kThreads) {
     Exponents a = {0, 0}, b = {0, 0};
-    for (int i = threadIdx.x; i < pieces; i += kThreads) {
-      a = __builtin_elementwise_max(a, ea[int64_t(tm) * pieces + i]);
-      b = __builtin_elementwise_max(b, eb[int64_t(tn) * pieces + i]);
-    }
+    if (c < chunks) {
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-      a = __builtin_elementwise_max(a, __builtin_bit_cast(Exponents, __shfl_xor(__builtin_bit_cast(int, a), off, 64)));
-      b = __builtin_elementwise_max(b, __builtin_bit_cast(Exponents, __shfl_xor(__builtin_bit_cast(int, b), off, 64)));
-    }
-    if (lane == 0) waves[wave] = a, waves[4 + wave] = b;
-    __syncthreads();
-    for (int w = 0; w < 4; ++w) a = __builtin_elementwise_max(a, waves[w]), b = __builtin_elementwise_max(b, waves[4 + w]);
-    __syncthreads();  // before the stages overwrite them
-    if (!in_split_range(a, b)) {
-      for (int sub = 0; sub < W * W / 4; ++sub) {
-        const int ms = m0 + wm * kWaveRows + sub / (W / 2) * 64, ns = n0 + wn * kWaveRows + sub % (W / 2) * 64;
-        if (ms >= M || ns >= N) continue;
-        f32x4 acc[4][4];
-        direct_tile<kF32, 4>(M, N, K, A, lda, B, ldb, ms, ns, lane, int(blockIdx.y), slices, acc);
-        store_tile<4>(M, N, C, ldc, ms, ns, lane, acc);
+      for (int i = 0; i < W; ++i) {  // strips of 64 rows, and of 64 columns
+        a = __builtin_elementwise_max(a, ea[int64_t(tm * W + i) * chunks + c]);
+        b = __builtin_elementwise_max(b, eb[int64_t(tn * W + i) * chunks + c]);
       }
-      return;
     }
+    const uint64_t bits = __ballot(!in_split_range(a, b));
+    if (lane == 0) out_of_range[c / 64] = bits;
   }
+  __syncthreads();
+  // The first chunk from c on that is out of range (out) or in it, at most `chunks`.
+  auto next_chunk = [&](int c, bool out) {
+    while (c < chunks) {
+      const uint64_t bits = out_of_range[c / 64] ^ (out ? 0 : ~uint64_t(0));
+      const int at = __ffsll(static_cast<unsigned long long>(bits >> (c % 64)));
+      if (at) return __builtin_amdgcn_readfirstlane(min(c + at - 1, chunks));
+      c = c / 64 * 64 + 64;
+    }
+    return chunks;
+  };
 
   // Waves 0 and 1 stream A's panel, 2 and 3 B's: 3W chunks of 1 KiB each per stage.
   const int rows_p = wave < 2 ? Mp : Np;
   const char *const from = wave < 2 ? X + int64_t(m0) * 16 : Y + int64_t(n0) * 16;
   const int part_stride = rows_p * 32;
-  const int first = slice_begin(Kp / kSplitK, blockIdx.y, slices);
-  const int stages = slice_begin(Kp / kSplitK, blockIdx.y + 1, slices) - first;
   const unsigned voff = unsigned(lane) * 16;
   auto dma = [&](int ks, int buf) {
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char *>(from) + int64_t(first + ks) * 3 * part_stride, 0,
+        const_cast<char *>(from) + int64_t(ks) * 3 * part_stride, 0,
         5 * (part_stride / 2) + kPartB / 2, 0x00020000);
     char *const l = lds + buf + (wave >> 1) * kSplitPanelB;
 #pragma unroll
@@ -1192,42 +1192,130 @@ __global__ __launch_bounds__(kThreads, W == 4 ? 1 : 2) void gemm_split_kernel(
   };
 
   int cur = 0, nxt = kSplitStageB, nn = 2 * kSplitStageB;  // buffers of stages s, s + 1, s + 2
-  dma(0, cur);
-  if (stages > 1) dma(1, nxt);
-  publish_stage<0>();
   bf16x8 ah[W], am[W], al[W], bm[W], bl[W], bh[2][W];
-  frags(al, cur, arow, 2);
-  frags(bh[0], cur, brow, 0);
-  frags(bl, cur, brow, 2);
-  frags(am, cur, arow, 1);
-  frags(bm, cur, brow, 1);
-  auto stage = [&](int ks, auto parity) {
-    constexpr int P = decltype(parity)::value;
-    frags(ah, cur, arow, 0);
-    if (ks + 2 < stages) dma(ks + 2, nn);
-    // past the last stage the reads below fetch what no MFMA uses
-    group(al, bh[P]);
-    frags(al, nxt, arow, 2);
-    group(ah, bl);
-    frags(bl, nxt, brow, 2);
-    group(am, bm);
-    frags(bh[P ^ 1], nxt, brow, 0);
-    group(am, bh[P]);
-    frags(am, nxt, arow, 1);
-    group(ah, bm);
-    frags(bm, nxt, brow, 1);
-    group(ah, bh[P]);
-    // stage s + 2 has landed (own DMAs, then everybody's), and nobody reads stage s any more
+  // Stages [begin, end).
+  auto split_stages = [&](int begin, int end) {
+    dma(begin, cur);
+    if (begin + 1 < end) dma(begin + 1, nxt);
     publish_stage<0>();
-    const int free = cur;
-    cur = nxt, nxt = nn, nn = free;
+    frags(al, cur, arow, 2);
+    frags(bh[0], cur, brow, 0);
+    frags(bl, cur, brow, 2);
+    frags(am, cur, arow, 1);
+    frags(bm, cur, brow, 1);
+    auto stage = [&](int ks, auto parity) {
+      constexpr int P = decltype(parity)::value;
+      frags(ah, cur, arow, 0);
+      if (ks + 2 < end) dma(ks + 2, nn);
+      // past the last stage the reads below fetch what no MFMA uses
+      group(al, bh[P]);
+      frags(al, nxt, arow, 2);
+      group(ah, bl);
+      frags(bl, nxt, brow, 2);
+      group(am, bm);
+      frags(bh[P ^ 1], nxt, brow, 0);
+      group(am, bh[P]);
+      frags(am, nxt, arow, 1);
+      group(ah, bm);
+      frags(bm, nxt, brow, 1);
+      group(ah, bh[P]);
+      // stage s + 2 has landed (own DMAs, then everybody's), and nobody reads stage s any more
+      publish_stage<0>();
+      const int free = cur;
+      cur = nxt, nxt = nn, nn = free;
+    };
+    int ks = begin;
+    for (; ks + 1 < end; ks += 2) {
+      stage(ks, std::integral_constant<int, 0>());
+      stage(ks + 1, std::integral_constant<int, 1>());
+    }
+    if (ks < end) stage(ks, std::integral_constant<int, 0>());
   };
-  int ks = 0;
-  for (; ks + 1 < stages; ks += 2) {
-    stage(ks, std::integral_constant<int, 0>());
-    stage(ks + 1, std::integral_constant<int, 1>());
+  // K values [begin, end), from a multiple of 16 on, on the FP32 matrix cores: per step of 8 a lane holds four
+  // consecutive K values of one row and of one column of each MFMA tile, straight from A and B, and MFMA t
+  // takes value t of both halves. Rows and columns past the end repeat the
+  // last one (their results are not stored); K values past the end are zeros.
+  auto fp32_values = [&](int begin, int end) {
+    const float *ap[W], *bp[W];
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      ap[i] = A + int64_t(min(m0 + wm * kWaveRows + 32 * i + l32, M - 1)) * lda + 4 * half;
+      bp[i] = B + int64_t(4 * half) * ldb + min(n0 + wn * kWaveRows + 32 * i + l32, N - 1);
+    }
+    struct Step {
+      f4u a[W], b[W];
+    };
+    // The loads that go out behind the MFMAs of tile row i and value t: all in the first quarter of a step of
+    // W = 4, whose one wave per SIMD has nothing else to cover them (4096^3, all out of range, 1080 us, spread
+    // over the step 1121), and spread over one of W = 2, where two waves would wait for the same burst
+    // (5000^3 2590 us, in the first quarter 4290).
+    auto load = [&](int k, int t, int i, Step &f) {
+      if (t == 0) f.a[i] = *reinterpret_cast<const f4u *>(ap[i] + k);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (W == 4 ? t == 0 : t == u) f.b[i][u] = bp[i][int64_t(k + u) * ldb];
+      CSMI_SCHED_FENCE();
+    };
+    // Multiplies f and loads `next` from k on.
+    auto step = [&](const Step &f, int k, Step &next) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < W; ++i) {
+#pragma unroll
+          for (int j = 0; j < W; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(f.a[i][t], f.b[j][t], acc[i][j], 0, 0, 0);
+          load(k, t, i, next);
+        }
+    };
+    const int stop = min(end, K), full = begin + (stop - begin) / 16 * 16;
+    if (begin < full) {
+      Step f[2];
+#pragma unroll
+      for (int t = 0; t < 4; ++t)  // in the loop's order, whose waits would be for the last of them otherwise
+#pragma unroll
+        for (int i = 0; i < W; ++i) load(begin, t, i, f[0]);
+#pragma unroll 1
+      for (int k = begin; k < full; k += 16) {
+        step(f[0], k + 8, f[1]);
+        step(f[1], min(k + 16, full - 8), f[0]);  // the last values are not used
+      }
+    }
+#pragma unroll 1
+    for (int k = full; k < stop; k += 8) {
+      Step f;
+#pragma unroll
+      for (int i = 0; i < W; ++i)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const int at = min(k + t, K - 1 - 4 * half);  // negative in the upper half where K < 5: in bounds all the same
+          const bool inside = k + t + 4 * half < K;
+          const float x = ap[i][at], y = bp[i][int64_t(at) * ldb];
+          f.a[i][t] = inside ? x : 0.0f;
+          f.b[i][t] = inside ? y : 0.0f;
+        }
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < W; ++i)
+#pragma unroll
+          for (int j = 0; j < W; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(f.a[i][t], f.b[j][t], acc[i][j], 0, 0, 0);
+    }
+  };
+  constexpr int kPerChunk = 64 / kSplitK;  // stages
+  const int last = slice_begin(Kp / kSplitK, blockIdx.y + 1, slices);
+#pragma unroll 1
+  for (int s = slice_begin(Kp / kSplitK, blockIdx.y, slices); s < last;) {
+    const int out = min(next_chunk(s / kPerChunk, true) * kPerChunk, last);
+    if (s < out) split_stages(s, out);
+    s = max(s, out);
+    const int in = min(next_chunk(s / kPerChunk, false) * kPerChunk, last);
+    if (s < in) {
+      fp32_values(s * kSplitK, in * kSplitK);
+      s = in;
+    }
   }
-  if (ks < stages) stage(ks, std::integral_constant<int, 0>());
 
   // acc[i][j][e]: row = 8*(e/4) + 4*half + e%4, col = l32 of the 32x32 tile (i, j)
 #pragma unroll

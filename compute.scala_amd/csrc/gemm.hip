@@ -1620,13 +1620,24 @@ bool run_packed(cs_stream *stream, int M, int N, int K, const float *A, int lda,
   return true;
 }
 
+// Rows and columns of C computed together.
+constexpr int64_t kMaxEdge = int64_t(1) << 26;
+
 template <int KIND>
 void run(cs_stream *stream, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C, int ldc) {
   check_depth<KIND>(K);
   const int64_t cus = stream->device->props.multiProcessorCount;
-  const DirectPlan p = plan_direct(KIND, cus, M, N, K);
   // A C that overlaps A or B is written only from copies of both.
   const bool over = overlap(A, M, K, lda, C, M, N, ldc) || overlap(B, K, N, ldb, C, M, N, ldc);
+  // A launch holds fewer than 2^32 threads, of which a narrow product takes one per value.
+  if (!over && std::max(M, N) > kMaxEdge) {
+    for (int64_t m = 0; m < M; m += kMaxEdge)
+      for (int64_t n = 0; n < N; n += kMaxEdge)
+        run<KIND>(stream, int(std::min<int64_t>(M - m, kMaxEdge)), int(std::min<int64_t>(N - n, kMaxEdge)), K,
+                  A + m * lda, lda, B + n, ldb, C + m * ldc + n, ldc);
+    return;
+  }
+  const DirectPlan p = plan_direct(KIND, cus, M, N, K);
   Plan plan = choose_path<KIND>(double(cus), M, N, K, p);
   if (over && plan.path == kDirect) plan = {kTiles128, 1};
   int z = plan.slices;

@@ -1643,8 +1643,7 @@ void run(cs_stream *stream, int M, int N, int K, const float *A, int lda, const 
   int z = plan.slices;
   if (plan.path == kDirect) {
     // a call sizes the scratch for calls of up to its size under capture, one that copies its operands too
-    const size_t bytes = size_t(packed_bytes<KIND, 2>(M, N, K));
-    if (scratch_fits(stream, bytes)) stream_scratch(stream, bytes);
+    reserve_scratch(stream, size_t(packed_bytes<KIND, 2>(M, N, K)));
   } else {
     bool done = false;
     if (plan.path == kTiles256) done = run_packed<KIND, 4, 2>(stream, M, N, K, A, lda, B, ldb, C, ldc, over, z);

@@ -206,10 +206,13 @@ inline void allow_lds(std::atomic<uint64_t> &done, int ordinal, const void *kern
 }
 // Stream-owned scratch of at least `bytes`, zero-filled when (re)allocated. Growing it
 // synchronizes the stream, so the first call of a given size must not be under capture.
-// The buffer it replaces stays allocated until the stream is destroyed.
+// The buffer it replaces stays allocated until the stream is destroyed, and in use if the growth fails.
 void *stream_scratch(cs_stream *stream, size_t bytes);
 // Whether stream_scratch gives that much now: it is there already, or the stream is not capturing.
 bool scratch_fits(cs_stream *stream, size_t bytes);
+// For calls that need no scratch themselves but size it for others under capture: grows it to `bytes`
+// where that can be done.
+void reserve_scratch(cs_stream *stream, size_t bytes);
 // FP64 block partials of a sum in the stream's scratch (n of them), and the fixed-order FP64
 // combine that turns n partials into *out (FP32, nullable) and *out64 (nullable).
 double *sum_partials(cs_stream *stream, size_t n);

@@ -774,7 +774,7 @@ cs_status cs_reduce_cols(cs_stream *stream, const float *in, int64_t rows, int64
     const dim3 grid(static_cast<unsigned>(p.groups), static_cast<unsigned>(p.slices));
     if (p.slices == 1) {
       // none needed, but a call sizes the scratch for smaller ones under capture
-      if (scratch_fits(stream, 4096)) scratch_for(stream, 0);
+      reserve_scratch(stream, 4096);
       hipLaunchKernelGGL((p.across > 64 ? reduce_cols_kernel<true> : reduce_cols_kernel<false>), grid, dim3(kBlock), 0,
                          stream->stream, in, rows, cols, p.across, p.rows_per_slice, static_cast<double *>(nullptr),
                          col_sum);

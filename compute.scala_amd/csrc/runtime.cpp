@@ -262,16 +262,25 @@ void *stream_scratch(cs_stream *stream, size_t bytes) {
   if (!scratch_fits(stream, bytes))
     fail(CS_INVALID_OPERATION, "stream scratch must grow outside graph capture; run the call once first");
   CS_HIP(hipStreamSynchronize(stream->stream));
+  size_t n = round_up(bytes, 1u << 20);
+  void *grown = nullptr;
+  CS_HIP(hipMalloc(&grown, n));
   // kept, not freed: graphs captured earlier on this stream may still address it
   if (stream->scratch) stream->retired_scratch.push_back(stream->scratch);
-  stream->scratch = nullptr;
+  stream->scratch = grown;
   stream->scratch_bytes = 0;
-  size_t n = round_up(bytes, 1u << 20);
-  CS_HIP(hipMalloc(&stream->scratch, n));
-  CS_HIP(hipMemsetAsync(stream->scratch, 0, n, stream->stream));
+  CS_HIP(hipMemsetAsync(grown, 0, n, stream->stream));
   CS_HIP(hipStreamSynchronize(stream->stream));
   stream->scratch_bytes = n;
-  return stream->scratch;
+  return grown;
+}
+
+void reserve_scratch(cs_stream *stream, size_t bytes) {
+  if (!scratch_fits(stream, bytes)) return;
+  try {
+    stream_scratch(stream, bytes);
+  } catch (const Error &) {
+  }
 }
 
 // ------------------------------------------------------------------------ hiprtc

@@ -1372,11 +1372,15 @@ struct Target {
   float *out;
   int ld, slices;
 
-  Target(cs_stream *stream, int64_t used, int M, int N, float *C, int ldc, int wanted) : slices(wanted) {
+  // `reserve`: what the scratch is sized to besides, where it can be: for calls of up to this size under
+  // capture, whatever their path.
+  Target(cs_stream *stream, int64_t used, int64_t reserve, int M, int N, float *C, int ldc, int wanted)
+      : slices(wanted) {
     used = round_up(used, 256);
     int64_t total = used;
     if (slices > 1) total += int64_t(slices) * M * N * 4;
     if (slices > 1 && !scratch_fits(stream, size_t(total))) slices = 1, total = used;
+    reserve_scratch(stream, size_t(std::max(total, reserve)));
     scratch = total ? static_cast<char *>(stream_scratch(stream, size_t(total))) : nullptr;
     out = slices > 1 ? reinterpret_cast<float *>(scratch + used) : C;
     ld = slices > 1 ? N : ldc;
@@ -1415,7 +1419,7 @@ void run_lds(cs_stream *stream, int M, int N, int K, const float *A, int lda, co
   const int64_t Mp = round_up(M, kTile), Np = round_up(N, kTile), Kp = round_up(K, P::kK);
   const int64_t rowb = Kp * P::kBytesPerK;
   const int64_t xbytes = Mp * rowb, ybytes = Np * rowb;
-  const Target to(stream, packed_bytes<KIND, W>(M, N, K), M, N, C, ldc, slices);
+  const Target to(stream, packed_bytes<KIND, W>(M, N, K), packed_bytes<KIND, 4>(M, N, K), M, N, C, ldc, slices);
   char *const base = to.scratch, *x = base, *y = base + xbytes;
   uint8_t *sx = nullptr, *sy = nullptr;
   hipStream_t s = stream->stream;
@@ -1462,7 +1466,7 @@ bool run_split(cs_stream *stream, int M, int N, int K, const float *A, int lda, 
   const int64_t ebytes = (Mp + Np) / 64 * chunks * int64_t(sizeof(Exponents));
   const int64_t total = xbytes + ybytes + ebytes + 4096;
   if (!scratch_fits(stream, size_t(total))) return false;
-  const Target to(stream, total, M, N, C, ldc, slices);
+  const Target to(stream, total, packed_bytes<kF32, 4>(M, N, K), M, N, C, ldc, slices);
   char *const base = to.scratch;
   SplitArgs p;
   p.a = A, p.b = B, p.m = M, p.n = N, p.k = K, p.lda = lda, p.ldb = ldb, p.mp = int(Mp), p.np = int(Np), p.kp = int(Kp);
@@ -1487,7 +1491,7 @@ void run_direct(cs_stream *stream, int M, int N, int K, const float *A, int lda,
   const int64_t rows = 16 * T * (kWK == 1 ? 4 : 1);  // of C per workgroup
   const int64_t tiles_m = (M + rows - 1) / rows, tiles_n = (N + 16 * T - 1) / (16 * T);
   const size_t lds = kWK == 1 ? 0 : size_t(kWK) * 256 * T * T * sizeof(float);
-  const Target to(stream, 0, M, N, C, ldc, slices);
+  const Target to(stream, 0, packed_bytes<KIND, 4>(M, N, K), M, N, C, ldc, slices);
   hipLaunchKernelGGL((gemm_direct_kernel<KIND, T, kWK>), dim3(unsigned(tiles_m * tiles_n), unsigned(to.slices)),
                      dim3(kWK == 1 ? 256 : 64 * kWK), lds, stream->stream, M, N, K, A, lda, B, ldb, to.out, to.ld,
                      int(tiles_m), to.slices);
@@ -1641,10 +1645,7 @@ void run(cs_stream *stream, int M, int N, int K, const float *A, int lda, const 
   Plan plan = choose_path<KIND>(double(cus), M, N, K, p);
   if (over && plan.path == kDirect) plan = {kTiles128, 1};
   int z = plan.slices;
-  if (plan.path == kDirect) {
-    // a call sizes the scratch for calls of up to its size under capture, one that copies its operands too
-    reserve_scratch(stream, size_t(packed_bytes<KIND, 2>(M, N, K)));
-  } else {
+  if (plan.path != kDirect) {
     bool done = false;
     if (plan.path == kTiles256) done = run_packed<KIND, 4, 2>(stream, M, N, K, A, lda, B, ldb, C, ldc, over, z);
     if (plan.path == kTiles128) done = run_packed<KIND, 2, 2>(stream, M, N, K, A, lda, B, ldb, C, ldc, over, z);

@@ -730,6 +730,8 @@ cs_status cs_reduce_rows(cs_stream *stream, const float *in, int64_t rows, int64
       return;
     }
     const RowPlan plan = plan_rows(stream, rows, cols);
+    // sized for calls of up to as many rows under capture, which may have a partial per row
+    if (want_total) reserve_scratch(stream, static_cast<size_t>(rows) * 8 + 4096);
     ReduceScratch s = scratch_for(stream, want_total ? static_cast<size_t>(plan.grid) : 0);
     launch_rows(stream, plan, in, rows, cols, {row_sum, row_max, want_total ? s.partial64 : nullptr, total, total64});
     CS_HIP(hipGetLastError());

@@ -295,6 +295,10 @@ __global__ __launch_bounds__(kNet) void network_kernel(NetShape net, const float
       for (int s = wave; s < live; s += kNetWaves)
         for (int c = lane; c < last; c += 64) result[(s0 + s) * last + c] = pred[c * kS + s];
     } else {
+      // samples past n add nothing, whatever infinite parameters have made of their zeros
+      if (live < kS)
+        for (int i = t; i < net.unit_floats; i += kNet)
+          if (i % kS >= live) units[i] = 0.0f;
       // delta[j][s]: the loss's gradient by layer l's output before its ReLU
       float *cur = deltas, *next = deltas + net.delta_floats;
       if (t < 16 * kS) {

@@ -25,6 +25,7 @@ struct cs_mlp {
   int64_t acts_capacity = 0;
   float *deltas = nullptr;  // two ping-pong gradient buffers of n x max width
   int64_t deltas_capacity = 0;
+  std::vector<float *> retired;  // workspaces outgrown under capture
 };
 
 namespace csmi {
@@ -433,11 +434,22 @@ uint32_t hash32(uint32_t v) {
   return v;
 }
 
-void ensure(float **buf, int64_t *cap, int64_t need) {
+// A workspace of `need` floats. Under capture one that grows is kept as well, since the calls captured
+// before use it; allocating there needs the relaxed capture mode.
+void ensure(cs_stream *stream, cs_mlp *net, float **buf, int64_t *cap, int64_t need) {
   if (*cap >= need) return;
-  if (*buf) CS_HIP(hipFree(*buf));
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  CS_HIP(hipStreamIsCapturing(stream->stream, &status));
+  const bool capturing = status != hipStreamCaptureStatusNone;
+  if (*buf && capturing) net->retired.push_back(*buf);
+  if (*buf && !capturing) CS_HIP(hipFree(*buf));
   *buf = nullptr;
-  CS_HIP(hipMalloc(reinterpret_cast<void **>(buf), static_cast<size_t>(need) * 4));
+  *cap = 0;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  if (capturing) CS_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  const hipError_t r = hipMalloc(reinterpret_cast<void **>(buf), static_cast<size_t>(need) * 4);
+  if (capturing) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  CS_HIP(r);
   *cap = need;
 }
 
@@ -451,7 +463,7 @@ void forward(cs_stream *stream, cs_mlp *net, const float *X, int64_t n) {
   const int L = static_cast<int>(net->widths.size()) - 1;
   int64_t total = 0;
   for (int l = 1; l <= L; ++l) total += n * net->widths[l];
-  ensure(&net->acts, &net->acts_capacity, total);
+  ensure(stream, net, &net->acts, &net->acts_capacity, total);
   const float *in = X;
   for (int l = 1; l <= L; ++l) {
     float *out = net->acts + act_offset(net, l, n);
@@ -629,7 +641,7 @@ cs_status cs_mlp_backward(cs_stream *stream, cs_mlp *mlp, const float *X, const 
     if (const size_t lds = network_shape(mlp, true, kSamples, &shape)) {
       const unsigned grid = network_grid<kSamples>(stream, n, 1);
       // partial losses (FP64), then one row of gradients per workgroup
-      ensure(&mlp->deltas, &mlp->deltas_capacity, int64_t(grid) * (2 + mlp->count));
+      ensure(stream, mlp, &mlp->deltas, &mlp->deltas_capacity, int64_t(grid) * (2 + mlp->count));
       double *partial_loss = reinterpret_cast<double *>(mlp->deltas);
       float *partial = mlp->deltas + 2 * grid;
       launch_network<true, kSamples>(stream, shape, lds, grid, mlp, X, target, n, nullptr, partial, partial_loss);
@@ -642,7 +654,7 @@ cs_status cs_mlp_backward(cs_stream *stream, cs_mlp *mlp, const float *X, const 
     forward(stream, mlp, X, n);
     int wmax = 1;
     for (int w : mlp->widths) wmax = std::max(wmax, w);
-    ensure(&mlp->deltas, &mlp->deltas_capacity, 2 * n * wmax);
+    ensure(stream, mlp, &mlp->deltas, &mlp->deltas_capacity, 2 * n * wmax);
     float *d_cur = mlp->deltas, *d_next = mlp->deltas + n * wmax;
     const float *pred = mlp->acts + act_offset(mlp, L, n);
     hipLaunchKernelGGL(mse_grad, dim3(1), dim3(1024), 0, stream->stream, pred, target, n, d_cur, loss);
@@ -682,6 +694,7 @@ cs_status cs_mlp_release(cs_mlp *mlp) {
     set_device(mlp->device);
     for (float *p : {mlp->params, mlp->m, mlp->v, mlp->acts, mlp->deltas})
       if (p) (void)hipFree(p);
+    for (float *p : mlp->retired) (void)hipFree(p);
     delete mlp;
   });
 }

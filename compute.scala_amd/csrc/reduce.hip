@@ -641,7 +641,13 @@ struct ColPlan {
 //     lanes (1 x 16000000: 27.3 against 72.8, 2 x 8000000 25.0 against 39.9); up to 1024 rows fewer, down to 16, as
 //     long as that brings workgroups (300 x 16384: 6.1 against 7.9; 116 x 2588: 4.2 against 6.4).
 //     Taller matrices lose by it (20011 x 1003: 22.8 against 19.0).
+//   * from half as many groups as CUs on, one slice leaves CUs idle, or a few with two workgroups: up to
+//     eight slices there, as the estimate has it, by which 0.8 of the CUs fill the memory and a slice costs
+//     3% (4000 x 33000, 129 groups: 1 slice 122.8, 2 110.6, 3 89.2, 4 106.6; 4000 x 44000, 172 groups: 125.6,
+//     112.3, 127.7, 108.5; 2000 x 70000, 274 groups: 107.1, 105.8, 98.4, 95.5; 4000 x 60000, 235 groups: 137.1,
+//     141.0, 145.0, 146.2).
 constexpr int64_t kMinRowsPerLane = 8, kOneSliceRowsPerLane = 32, kNarrowRows = 1024;
+constexpr int kMaxWideSlices = 8;
 
 ColPlan plan_cols(cs_stream *stream, int64_t rows, int64_t cols) {
   ColPlan p;
@@ -655,7 +661,17 @@ ColPlan plan_cols(cs_stream *stream, int64_t rows, int64_t cols) {
   p.across = static_cast<int>((quads + p.groups - 1) / p.groups);
   const int64_t lanes = kBlock / p.across;
   if (rows > lanes * kOneSliceRowsPerLane) {
-    int64_t slices = std::min(cus / p.groups, rows / (lanes * kMinRowsPerLane));
+    int64_t slices = cus / p.groups;
+    if (slices <= 1 && rows > kNarrowRows) {
+      // the time of s slices in rounds over all rows: what memory delivers, or the CU with most workgroups
+      const double full = double(p.groups) / (0.8 * double(cus));
+      double least = 1e30;
+      for (int s = 1; s <= kMaxWideSlices; ++s) {
+        const double t = std::max(full, double((p.groups * s + cus - 1) / cus) / s) + 0.03 * s;
+        if (t < 0.95 * least) least = t, slices = s;
+      }
+    }
+    slices = std::min(slices, rows / (lanes * kMinRowsPerLane));
     slices = std::max<int64_t>(1, std::min<int64_t>(slices, 65535));
     p.rows_per_slice = (rows + slices - 1) / slices;
     p.slices = (rows + p.rows_per_slice - 1) / p.rows_per_slice;
@@ -774,9 +790,11 @@ cs_status cs_reduce_cols(cs_stream *stream, const float *in, int64_t rows, int64
     set_device(stream->device);
     const ColPlan p = plan_cols(stream, rows, cols);
     const dim3 grid(static_cast<unsigned>(p.groups), static_cast<unsigned>(p.slices));
+    // sized for smaller calls under capture as well: only matrices of up to two groups per CU are cut into
+    // slices that take more than the least scratch
+    const int64_t widest = rows > kNarrowRows ? std::min<int64_t>(cols, 512 * stream->device->props.multiProcessorCount) : 0;
+    reserve_scratch(stream, static_cast<size_t>(widest * kMaxWideSlices * 8 + 4096));
     if (p.slices == 1) {
-      // none needed, but a call sizes the scratch for smaller ones under capture
-      reserve_scratch(stream, 4096);
       hipLaunchKernelGGL((p.across > 64 ? reduce_cols_kernel<true> : reduce_cols_kernel<false>), grid, dim3(kBlock), 0,
                          stream->stream, in, rows, cols, p.across, p.rows_per_slice, static_cast<double *>(nullptr),
                          col_sum);

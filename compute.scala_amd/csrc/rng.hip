@@ -123,10 +123,11 @@ __device__ __forceinline__ void sincos_turn(float theta, const NormalTables &tab
 // arithmetic, a third of it FP64: 16777259 values (67 MB) take 27.7 us, against 59 us with the
 // device library's log, cos and sin, which serve the whole range of their arguments. (One copy of the
 // tables per LDS lane, against bank conflicts, took 32.5 us: filling them costs more than it saves.)
-__global__ __launch_bounds__(kBlock) void random_normal_kernel(float *out, int64_t pairs, uint32_t seed) {
+__global__ __launch_bounds__(kBlock) void random_normal_kernel(float *out, int64_t pairs, uint32_t seed,
+                                                                int64_t stride) {
   __shared__ NormalTables tables;
   fill_tables(tables);
-  for (int64_t i = (int64_t(blockIdx.x) * kBlock + threadIdx.x) * 2; i < pairs; i += int64_t(gridDim.x) * kBlock * 2) {
+  for (int64_t i = (int64_t(blockIdx.x) * kBlock + threadIdx.x) * 2; i < pairs; i += stride) {
     f4u v;
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
@@ -207,7 +208,7 @@ cs_status cs_random_normal(cs_stream *stream, float *out, int64_t n, uint32_t se
     // workgroups to fill every CU, each with pairs enough to pay for its table
     const unsigned grid = std::min<unsigned>(blocks_for((pairs + 1) / 2), 8 * stream->device->props.multiProcessorCount);
     hipLaunchKernelGGL(random_normal_kernel, dim3(grid), dim3(kBlock), 0, stream->stream, out,
-                       pairs, seed);
+                       pairs, seed, int64_t(grid) * kBlock * 2);
     CS_HIP(hipGetLastError());
   });
 }

@@ -521,17 +521,37 @@ void launch_network(cs_stream *stream, const NetShape &shape, size_t lds, unsign
                      target, n, y, partial, partial_loss);
 }
 
-// Evaluation alone, of very many samples on a tiny network: the layer kernels, a thread per unit and
-// sample, are ahead (262144 samples, us, layers / whole: 8-16-1, 161 parameters, 33 / 61; 16-16-1, 289,
-// 42 / 62; 12-14-14-1, 407, 82 / 80; 16-24-1, 433, 65 / 69; 30-30-30-30-1, 2821, 373 / 129).
-bool prefer_layers(const NetShape &shape, int64_t n) { return n > 65536 && shape.count <= 400; }
+// Whether the layer kernels, a thread per unit and sample, are ahead of the whole-network kernel in evaluating
+// many samples on a network of few units: by estimates in us, of which the layers' is 2.2 for a launch and, for
+// each input of a unit, the latency of one step of its loop or the rate of all CUs (1.7 times slower where rows
+// of inputs straddle lines), or what L2 delivers where the rows that the waves of a CU read together outgrow
+// its L1. The whole network's is per sample and 4 us. Measured (layers / whole; samples): 64-8-1 17.8 / 25.2
+// (65536), 71 / 108 (300000); 1000-1 199 / 595, 2934 / 3042; 512-8 109 / 160, 585 / 889; 32-16-1 18.1 / 19.7,
+// 62 / 84; 16-8-8-1 13.5 / 22.7 (65536); 256-4-1 52 / 71, 353 / 329; 200-8-1 59 / 55, 280 / 248; 64-16-1
+// 27 / 25, 111 / 108; 12-14-14-1 26 / 23; 30-30-1 37 / 21. Above 65536 samples networks of up to 400
+// parameters stay with the layers.
+bool prefer_layers(const cs_mlp *net, const NetShape &shape, size_t lds, int samples, int64_t n) {
+  const double cus = net->device->props.multiProcessorCount;
+  double layers = 0.0;
+  for (int l = 0; l < shape.layers; ++l) {
+    const int din = shape.layer[l].din, dout = shape.layer[l].dout;
+    const double threads = double(n) * dout, waves = std::min(32.0, threads / 64 / cus);
+    double step = std::max(0.17, (din % 16 && dout <= 16 ? 1.7e-4 : 1e-4) * threads / cus);
+    if (waves * std::max(1, 64 / dout) * std::min(128, 4 * din) > 36000)
+      step = std::max(step, 4.9e-6 * double(n) * std::min(1.0, din / 32.0));
+    layers += 2.2 + step * din;
+  }
+  const double crowded = samples < 4 * kSamples && n > kManySamples ? 2.4 : size_t(160 << 10) / lds < 2 ? 1.35 : 1.0;
+  const double whole = 4 + double(n) * (1e-4 + 3.6e-6 * shape.layer[0].din + 6e-5 * (shape.layers - 1)) * crowded;
+  return layers < 0.95 * whole || (n > 65536 && shape.count <= 400);
+}
 
 // Evaluation with kS samples per workgroup, where the network fits.
 template <int kS>
 bool evaluate(cs_stream *stream, cs_mlp *net, const float *X, int64_t n, float *y) {
   NetShape shape;
   const size_t lds = network_shape(net, false, kS, &shape);
-  if (!lds || prefer_layers(shape, n)) return false;
+  if (!lds || prefer_layers(net, shape, lds, kS, n)) return false;
   const int64_t per_cu = std::max<int64_t>(1, std::min<int64_t>(4, int64_t(160 << 10) / int64_t(lds)));
   launch_network<false, kS>(stream, shape, lds, network_grid<kS>(stream, n, per_cu), net, X, nullptr, n, y, nullptr,
                             nullptr);

@@ -427,11 +427,22 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(const float *__rest
           a[3].add(v[k].w);
         }
     } else {
-      for (int64_t r = r0 + rl; r < r1; r += lanes) {
-        a[0].add(in[r * cols]);
-        if (cols > 1) a[1].add(in[r * cols + 1]);
-        if (cols > 2) a[2].add(in[r * cols + 2]);
+      // the slice is one run of values: a thread takes every 256th (255th of three columns), all of one column
+      // (5054 x 2 one row at a time 9.2 us)
+      const int span = cols == 3 ? 255 : 256, mine = cols == 1 ? 0 : cols == 2 ? rl & 1 : rl % 3;
+      const int64_t n = rl < span ? (r1 - r0) * cols : 0;
+      const float *p = in + r0 * cols;
+      Acc b;
+      for (int64_t i = rl; i < n; i += 8 * span) {
+        float v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = i + k * span < n ? p[i + k * span] : 0.0f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) b.add(v[k]);
       }
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        if (mine == k) a[k] = b;
     }
   }
   if (rl < lanes) {
@@ -645,7 +656,8 @@ struct ColPlan {
 //   * 64 threads across, for whole rows of 1 KiB per wave, more where there are fewer rows than row
 //     lanes (1 x 16000000: 27.3 against 72.8, 2 x 8000000 25.0 against 39.9); up to 1024 rows fewer, down to 16, as
 //     long as that brings workgroups (300 x 16384: 6.1 against 7.9; 116 x 2588: 4.2 against 6.4).
-//     Taller matrices lose by it (20011 x 1003: 22.8 against 19.0).
+//     Taller matrices lose by it (20011 x 1003: 22.8 against 19.0). Where that would leave a few CUs with two
+//     workgroups, as many as the CUs' number needs (1022 x 19058: 19 across 17.8, 16 across 22.2).
 //   * from half as many groups as CUs on, one slice leaves CUs idle, or a few with two workgroups: up to
 //     eight slices there, as the estimate has it, by which 0.8 of the CUs fill the memory and a slice costs
 //     3% (4000 x 33000, 129 groups: 1 slice 122.8, 2 110.6, 3 89.2, 4 106.6; 4000 x 44000, 172 groups: 125.6,
@@ -660,12 +672,16 @@ ColPlan plan_cols(cs_stream *stream, int64_t rows, int64_t cols) {
   const int64_t quads = (cols + 3) / 4;
   int64_t most = 64;
   while (most * 2 * std::max<int64_t>(rows, 1) <= kBlock) most *= 2;
-  while (rows <= kNarrowRows && most > 16 && (quads + most - 1) / most < cus) most /= 2;
+  if (rows <= kNarrowRows) {
+    while (most > 16 && (quads + most - 1) / most < cus) most /= 2;
+    if (most < 64 && quads > most * cus && quads * 5 < most * cus * 6) most = (quads + cus - 1) / cus;
+  }
   p.groups = (quads + most - 1) / most;
   if (p.groups > 0x7fffffff) fail(CS_INVALID_VALUE, "too many columns");
   p.across = static_cast<int>((quads + p.groups - 1) / p.groups);
   const int64_t lanes = kBlock / p.across;
-  if (rows > lanes * kOneSliceRowsPerLane) {
+  // of fewer than four columns a thread has values, not rows: 64 each in one slice (8191 x 3 9.7 us cut, 11.0 whole)
+  if (cols < 4 ? rows * cols > 2 * lanes * kOneSliceRowsPerLane : rows > lanes * kOneSliceRowsPerLane) {
     int64_t slices = cus / p.groups;
     if (slices <= 1 && rows > kNarrowRows) {
       // the time of s slices in rounds over all rows: what memory delivers, or the CU with most workgroups

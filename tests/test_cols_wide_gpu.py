@@ -1,4 +1,5 @@
-"""Column sums of matrices with about as many groups of columns as CUs, cut into a few slices of rows."""
+"""Column sums of matrices with about as many groups of columns as CUs, cut into a few slices of rows or a
+number of columns to a workgroup that no power of two gives, and of fewer than four columns."""
 import ctypes
 
 import numpy as np
@@ -17,7 +18,10 @@ def column_sums(T, x, rows, cols, out):
     capi.check(lib.cs_reduce_cols(T.stream, x.ptr, rows, cols, out.ptr))
 
 
-@pytest.mark.parametrize("shape", [(1025, 32768), (1025, 32769), (1030, 33001), (1100, 44003), (1027, 66000), (1026, 102401)])
+@pytest.mark.parametrize("shape", [(1025, 32768), (1025, 32769), (1030, 33001), (1100, 44003), (1027, 66000), (1026, 102401),
+                                   (1022, 19058), (515, 19661), (1024, 9601),
+                                   (1, 3), (84, 3), (85, 3), (86, 3), (5462, 3), (5461, 3), (8192, 2), (8193, 2),
+                                   (255, 1), (257, 1), (16384, 1), (16385, 1), (300007, 3)])
 def test_slices(gpu_tensors, shape):
     T, (rows, cols) = gpu_tensors, shape
     a = inputs.uniform(rows * cols, 31).reshape(shape)

@@ -19,3 +19,14 @@ def test_wide_stores_wait(width, items, nontemporal):
     stores = re.findall(r'"global_store_dwordx4 ([^"]*)"', src)
     assert stores and all(s.endswith("\\n\\ts_nop 1") for s in stores)
     compiles(src)
+
+
+@pytest.mark.parametrize("items", [1, 2, 3])
+def test_values_come_before_the_stores(items):
+    """With several vectors per thread no value is left to be computed behind the first store."""
+    T = Tensors(offline=True, items_per_thread=items)
+    a, b = (T.Tensor.fill(0.0, (64, 256)).nonInline for _ in range(2))
+    src = T.kernel_source((a * b + a).closure, (64, 256))
+    first_store = src.index('asm volatile("global_store_dwordx4')
+    assert ('asm volatile("" :: "v"(' in src[:first_store]) == (items > 1)
+    compiles(src)

@@ -1494,14 +1494,17 @@ BatchPlan plan_batch(const std::vector<BatchExpr> &members, int block, int math_
 
 }  // namespace
 
-// Up to four vectors per thread, where that makes one workgroup of a sum: it writes the result
-// itself and the call is one launch (2048 elements of an 18-node expression: 3.9 us against 6.4 in
-// two). From eight on the one workgroup takes longer than the second launch.
-static void one_block_sum(const Dag &dag, Options *o) {
+// The vectors per thread of a sum. Up to four where that makes one workgroup: it writes the result itself and
+// the call is one launch (2048 elements of an 18-node expression: 3.9 us against 6.4 in two). From eight on the
+// one workgroup takes longer than the second launch. Otherwise two from 2^22 elements, with a transcendental
+// function too: a sum has no stores to cover, and one vector leaves twice the partials (the sum of exp of 4
+// million elements 6.9 us, with one vector 7.6; of 8 million 9.2 and 11.4).
+static void choose_sum_items(const Dag &dag, Options *o) {
+  if (dag.nodes.size() > kLargeBody) return;
   int64_t total = 1;
   for (auto d : dag.out_shape) total *= d;
   const int64_t per_thread = (total + int64_t(o->V) * o->block - 1) / (int64_t(o->V) * o->block);
-  if (dag.nodes.size() <= kLargeBody && per_thread <= 4) o->U = static_cast<int>(std::max<int64_t>(per_thread, 1));
+  o->U = per_thread <= 4 ? static_cast<int>(std::max<int64_t>(per_thread, 1)) : total >= (int64_t(1) << 22) ? 2 : 1;
 }
 
 // Compiles the kernel of `dag` under `o`.
@@ -1584,7 +1587,7 @@ static cs_status compile_fused(cs_device *device, const cs_node *nodes, int nnod
     Dag dag = canonicalize(nodes, nnodes, outputs, noutputs, out_rank, out_shape);
     o = resolve_options(options, dag);
     o.sum = sum;
-    if (sum && (!options || options->items_per_thread == 0)) one_block_sum(dag, &o);
+    if (sum && (!options || options->items_per_thread == 0)) choose_sum_items(dag, &o);
     if (sum && dag.outputs.size() != 1) fail(CS_INVALID_VALUE, "a fused sum takes one output");
     key = canonical_key(dag, o);
     {

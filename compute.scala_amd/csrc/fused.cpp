@@ -307,6 +307,23 @@ bool tiled_launch(const Dag &dag, const Options &o);
 // A join of several outputs gains nothing by it (below).
 constexpr int64_t kRaggedRow = 5;
 
+// Whether every leaf is read at the place that is computed (no view but the identity), and the leaves and the
+// output outgrow the caches: such a kernel takes what memory delivers to whole lines, which the vectors of a
+// ragged row straddle. In us ragged / at the dividing width: a*b+c of 4096 x 2050 (134 MB) 20.5 / 19.5, of
+// 16384 x 2050 100.4 / 93.0, a*b 74.8 / 70.2; at a width of one, of 8192 x 4099 101.7 / 88.0 and 75.6 / 68.0, but
+// of 4096 x 4097 38.5 / 39.7 and, with one leaf, 2a+1 of 8192 x 4099 40.3 / 43.5. In the caches a*b of 2048 x
+// 2050 5.8 / 8.4, 2a+1 of 4096 x 2050 8.5 / 10.9. With views ragged vectors stay ahead (view chain of
+// [512,128,510] 49.7 / 57.0).
+bool streams(const Dag &dag, int64_t total) {
+  for (const cs_node &n : dag.nodes) {
+    if (n.op != CS_OP_EXTRACT) continue;
+    const cs_node &leaf = dag.nodes[static_cast<size_t>(n.a)];
+    if (leaf.op != CS_OP_PARAMETER || dag.leaf_shape[static_cast<size_t>(leaf.param)] != dag.out_shape) return false;
+  }
+  const bool odd = dag.out_shape.back() % 2 != 0;
+  return dag.nleaves > (odd ? 1 : 0) && 4 * total * (dag.nleaves + 1) >= (int64_t(odd ? 256 : 120) << 20);
+}
+
 // The default vector width of a kernel with `outputs` joined outputs, where it divides the rows. A
 // thread's vector of V elements is V * outputs consecutive floats: up to four are one store, and a
 // wave's stores fill whole lines; longer runs leave each store instruction pieces of lines as far apart
@@ -316,7 +333,7 @@ constexpr int64_t kRaggedRow = 5;
 // 16.4 / 20.8 / 30.6; 2048 x 2048 transposes joined 4 times 17.4 / 20.3 / 28.2.
 int joined_width(size_t outputs) { return outputs == 1 || outputs > 12 ? 4 : outputs == 2 ? 2 : 1; }
 
-Options resolve_options(const cs_fused_options *o, const Dag &dag) {
+Options resolve_options(const cs_fused_options *o, const Dag &dag, bool sum = false) {
   Options r;
   if (o) {
     r.math_mode = o->math_mode;
@@ -339,7 +356,8 @@ Options resolve_options(const cs_fused_options *o, const Dag &dag) {
   // A large body holds hundreds of values per element, so it defaults to 1 and 1 (the convolution
   // idiom: 9.3 us at V=1 against 25 us at V=2 and 50 us at V=4; two vectors per thread spill, 129 us).
   const bool large = dag.nodes.size() > kLargeBody;
-  if (r.V == 0 && !large && dag.outputs.size() == 1 && last >= kRaggedRow && last % 4 != 0) {
+  if (r.V == 0 && !large && dag.outputs.size() == 1 && last >= kRaggedRow && last % 4 != 0 &&
+      (sum || !streams(dag, total))) {
     r.V = 4;  // the last vector of a row overlaps the one before (Emitter::ragged)
   } else {
     if (r.V == 0) r.V = large ? 1 : joined_width(dag.outputs.size());
@@ -1585,7 +1603,7 @@ static cs_status compile_fused(cs_device *device, const cs_node *nodes, int nnod
     Options o;
     std::string key;
     Dag dag = canonicalize(nodes, nnodes, outputs, noutputs, out_rank, out_shape);
-    o = resolve_options(options, dag);
+    o = resolve_options(options, dag, sum);
     o.sum = sum;
     if (sum && (!options || options->items_per_thread == 0)) choose_sum_items(dag, &o);
     if (sum && dag.outputs.size() != 1) fail(CS_INVALID_VALUE, "a fused sum takes one output");

@@ -778,8 +778,15 @@ class Emitter {
   // A store of more than two registers reads them up to two wait states after it has issued. The compiler
   // keeps later writes of them that far behind its own stores, but does not look into the assembly, so
   // the wait is written there.
-  bool written_through(int run) const { return (run == 1 || run == 4) && (o_.nt || gq_.empty()); }
-
+  // Single floats (rows of one to three elements) only where leaves and output outgrow the L2s' 32 MiB: in us
+  // plain / written through, a*b+c of 1.5 million 3.6 / 3.8, a*b of 2.5 million 4.5 / 5.1, 2a+1 of 4 million 6.1 /
+  // 7.0, but a*b+c of 2.5 million 7.0 / 5.3 and a*b of 4 million 9.5 / 7.7.
+  bool written_through(int run) const {
+    if (o_.nt) return run == 1 || run == 4;
+    int64_t total = 1;
+    for (auto d : dag_.out_shape) total *= d;
+    return gq_.empty() && (run == 4 || (run == 1 && 4 * total * (dag_.nleaves + 1) >= (int64_t(32) << 20)));
+  }
   std::string store(const std::string &addr, const std::string &val, const std::string &type, int run) {
     if (written_through(run) && (run == 1 || type != "float")) {
       const bool wide = type != "float";

@@ -30,3 +30,10 @@ def test_values_come_before_the_stores(items):
     first_store = src.index('asm volatile("global_store_dwordx4')
     assert ('asm volatile("" :: "v"(' in src[:first_store]) == (items > 1)
     compiles(src)
+
+
+@pytest.mark.parametrize("rows,through", [((1 << 22) - 1, False), (1 << 22, True)])
+def test_single_floats_write_through_past_the_caches(rows, through):
+    T = Tensors(offline=True)
+    a = T.Tensor.fill(0.0, (rows, 1)).nonInline
+    assert ("global_store_dword %0" in T.kernel_source((a * a).closure, (rows, 1))) == through

@@ -979,10 +979,12 @@ __global__ __launch_bounds__(kWK == 1 ? 256 : 64 * kWK) void gemm_direct_kernel(
 // Large FP32 products on the BF16 matrix cores, which do 16 times the FP32 ones' work per cycle. A
 // 24-bit significand is exactly three 8-bit ones, x = h + m + l (each the BF16 nearest to what is
 // left; Henry, Tang & Heinecke 2019), and of the nine products the six of hh, hm, mh, mm, hl and lh
-// are summed in FP32: what the others would add is below 2^-25 of |a||b|, half an FP32 rounding of
-// one product. The error against FP64 is that of the FP32 matrix cores or less, since 16 products
-// meet in one rounding instead of two: relative to |C|, U(-1,1), K = 16 3.2e-8 / 7.4e-8, 256
-// 2.3e-7 / 2.9e-7, 1024 4.8e-7 / 5.7e-7, 4096 1.0e-6 / 1.1e-6.
+// are summed in FP32: what the others would add is below 2^-24 of |a||b|, one unit roundoff, and all but
+// that for a = b = 1 + 2^-8 - 2^-17, say. Products that FP32 holds exactly lose nothing. The error against
+// FP64 of arbitrary values is that of the FP32 matrix cores or less, since 16 products meet in one rounding
+// instead of two: relative to |C|, U(-1,1), K = 16 3.2e-8 / 7.4e-8, 256 2.3e-7 / 2.9e-7, 1024 4.8e-7 /
+// 5.7e-7, 4096 1.0e-6 / 1.1e-6. Where all values are that one, FP32 sums round alike (5.9e-8 at K = 4096), and
+// the parts' sums do not (3.8e-6).
 // The split is exact, and the products' sums are FP32's, only in a range: not for infinities and
 // NaN, values that round to an infinite BF16, parts below BF16's normal range, products near FP32's
 // least and sums near its greatest (h may be above x, and hh overflow where ab does not). The pre-pass

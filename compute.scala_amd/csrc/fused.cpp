@@ -298,8 +298,6 @@ struct Options {
 // size (launch_bound) and launched by default at one element per vector and per thread.
 constexpr size_t kLargeBody = 256;
 
-bool tiled_launch(const Dag &dag, const Options &o);
-
 // Rows longer than a vector of four that four does not divide are cut into vectors of four all the
 // same (Emitter::ragged). In us against the widest dividing width, at about 4 million elements: view
 // chain with rows of 5 12.1 / 17.3, of 6 11.1 / 14.1, of 10 10.8 / 14.1, of 33 10.7 / 11.1, of 510
@@ -307,21 +305,26 @@ bool tiled_launch(const Dag &dag, const Options &o);
 // A join of several outputs gains nothing by it (below).
 constexpr int64_t kRaggedRow = 5;
 
-// Whether every leaf is read at the place that is computed (no view but the identity), and the leaves and the
-// output outgrow the caches: such a kernel takes what memory delivers to whole lines, which the vectors of a
-// ragged row straddle. In us ragged / at the dividing width: a*b+c of 4096 x 2050 (134 MB) 20.5 / 19.5, of
-// 16384 x 2050 100.4 / 93.0, a*b 74.8 / 70.2; at a width of one, of 8192 x 4099 101.7 / 88.0 and 75.6 / 68.0, but
-// of 4096 x 4097 38.5 / 39.7 and, with one leaf, 2a+1 of 8192 x 4099 40.3 / 43.5. In the caches a*b of 2048 x
-// 2050 5.8 / 8.4, 2a+1 of 4096 x 2050 8.5 / 10.9. With views ragged vectors stay ahead (view chain of
-// [512,128,510] 49.7 / 57.0).
-bool streams(const Dag &dag, int64_t total) {
+// Whether every leaf is read at the place that is computed: no view but the identity.
+bool reads_in_place(const Dag &dag) {
   for (const cs_node &n : dag.nodes) {
     if (n.op != CS_OP_EXTRACT) continue;
     const cs_node &leaf = dag.nodes[static_cast<size_t>(n.a)];
     if (leaf.op != CS_OP_PARAMETER || dag.leaf_shape[static_cast<size_t>(leaf.param)] != dag.out_shape) return false;
   }
+  return true;
+}
+
+// Whether a kernel only streams leaves and an output that outgrow the caches: it takes what memory delivers to
+// whole lines, which the vectors of a ragged row straddle. In us ragged / at the dividing width: a*b+c of 4096 x
+// 2050 (134 MB) 20.5 / 19.5, of 16384 x 2050 100.4 / 93.0, a*b 74.8 / 70.2; at a width of one, of 8192 x 4099
+// 101.7 / 88.0 and 75.6 / 68.0, but of 4096 x 4097 38.5 / 39.7 and, with one leaf, 2a+1 of 8192 x 4099 40.3 / 43.5.
+// In the caches a*b of 2048 x 2050 5.8 / 8.4, 2a+1 of 4096 x 2050 8.5 / 10.9. With views ragged vectors stay ahead
+// (view chain of [512,128,510] 49.7 / 57.0).
+bool streams(const Dag &dag, int64_t total) {
   const bool odd = dag.out_shape.back() % 2 != 0;
-  return dag.nleaves > (odd ? 1 : 0) && 4 * total * (dag.nleaves + 1) >= (int64_t(odd ? 256 : 120) << 20);
+  return dag.nleaves > (odd ? 1 : 0) && 4 * total * (dag.nleaves + 1) >= (int64_t(odd ? 256 : 120) << 20) &&
+         reads_in_place(dag);
 }
 
 // The default vector width of a kernel with `outputs` joined outputs, where it divides the rows. A
@@ -349,10 +352,11 @@ Options resolve_options(const cs_fused_options *o, const Dag &dag, bool sum = fa
   int64_t last = dag.out_shape.empty() ? 1 : dag.out_shape.back();
   int64_t total = 1;
   for (auto s : dag.out_shape) total *= s;
-  // Defaults: 4 elements per vector, 2 vectors per thread from 2^22 elements; from 2^23 with a
-  // transcendental function outside 2-D tiles, where the arithmetic of one vector covers the loads of
-  // another wave's (us, 1 / 2 vectors: view chain of 4 million elements 7.1 / 7.6, of 32 million
-  // 57.8 / 53.5; a*b+c of 4 million 10.7 / 10.6; 2048 x 2048 transpose plus matrix 12.6 / 10.9).
+  // Defaults: 4 elements per vector, 2 vectors per thread from 2^22 elements; from 2^23 with a transcendental
+  // function of leaves read in place, where the arithmetic of one vector covers the loads of another wave's,
+  // while views leave each vector several loads to wait for (us, 1 / 2 vectors: exp(a)*tanh(b) of 4 million
+  // elements 8.5 / 8.8, of 8 million 15.5 / 16.1; view chain of 4 million 7.0 / 6.5, of 4.7 million ragged 8.1 /
+  // 7.6, of 17 million 29.1 / 27.0; 2048 x 2048 transpose plus matrix 12.4 / 10.1).
   // A large body holds hundreds of values per element, so it defaults to 1 and 1 (the convolution
   // idiom: 9.3 us at V=1 against 25 us at V=2 and 50 us at V=4; two vectors per thread spill, 129 us).
   const bool large = dag.nodes.size() > kLargeBody;
@@ -367,7 +371,7 @@ Options resolve_options(const cs_fused_options *o, const Dag &dag, bool sum = fa
   if (r.U == 0) {
     bool heavy = false;
     for (const cs_node &n : dag.nodes) heavy = heavy || n.op == CS_OP_TANH || n.op == CS_OP_EXP || n.op == CS_OP_LOG;
-    const int from = heavy && !tiled_launch(dag, r) ? 23 : 22;
+    const int from = heavy && reads_in_place(dag) ? 23 : 22;
     r.U = !large && total >= (int64_t(1) << from) ? 2 : 1;
   }
   if (r.U < 1 || r.U > 8) fail(CS_INVALID_VALUE, "items_per_thread must be 1..8");
@@ -510,13 +514,6 @@ class Emitter {
   }
 
   int nleaves() const { return dag_.nleaves; }
-
-  // Whether the automatic launch order takes 2-D tiles for this expression.
-  bool tiled() const {
-    int64_t rows = 1;
-    for (size_t i = 0; i + 1 < dag_.out_shape.size(); ++i) rows *= dag_.out_shape[i];
-    return choose_order(rows * row_vectors()).tiled;
-  }
 
  private:
   void header(std::ostringstream &s, bool with_prelude) {
@@ -1357,8 +1354,6 @@ class Emitter {
   std::map<std::string, RowGroup> row_groups_;          // rows read together, by leaf and leading indices
   std::map<int, std::string> in_group_;                 // gather node -> its row group
 };
-
-bool tiled_launch(const Dag &dag, const Options &o) { return Emitter(dag, o).tiled(); }
 
 // FAST mirrors -cl-unsafe-math-optimizations (OpenCL.scala:1131-1135): reassociation,
 // reciprocals, no signed zeros and contraction, but not finite-math-only, so infinities and

@@ -233,7 +233,7 @@ typedef struct cs_fused_options {
  * multiple of 4, the last vector of a row overlaps the one before, unless the expression only
  * streams operands that outgrow the caches; then, and where a vector_width is given, it is halved
  * until it divides the extent), items_per_thread 2 from 2^22 output positions (2^23 with
- * exp, tanh or log, unless the launch order takes tiles) and 1 below, 256 threads. An expression of
+ * exp, tanh or log of leaves that are read without a view) and 1 below, 256 threads. An expression of
  * more than 256 canonical nodes (such as the convolution idiom) holds hundreds of values per
  * element: it gets vector_width 1 and items_per_thread 1, and is compiled for its own
  * workgroup size (a larger launch of it is CS_INVALID_WORK_GROUP_SIZE). */

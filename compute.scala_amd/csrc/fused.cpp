@@ -606,7 +606,7 @@ class Emitter {
   // Rows that the vector width does not divide: a row has one vector more than fit, and the last one
   // starts early, so that it ends with the row. Its first again[u] elements repeat the ones before
   // with the same values (a sum leaves them out), so loads and stores stay 16 bytes wide, at any
-  // 4-byte boundary. The view chain of [251,37,509] takes 8.4 us this way, against 9.2 us one element
+  // 4-byte boundary. The view chain of [251,37,509] takes 7.75 us this way, against 10.5 us one element
   // at a time; without the repeated stores each row would end in a narrower one, and the partly
   // written lines cost more than the rest together (12.1 us, with rows of 33 31 us against 11).
   // A kernel whose output lies over one of its leaves must not repeat elements, as the repetition may
@@ -766,8 +766,8 @@ class Emitter {
   // per vector) it writes through at device scope (`sc1`, a vector store): no dirty line is left in
   // L2 for the release at the end of the kernel, which otherwise writes it back between this launch
   // and the next. The lines stay in L2 for a kernel that reads them, unless the caller asks for
-  // non-temporal stores (`sc1 nt`). In us, plain / written through / and non-temporal: view chain of
-  // [256,64,256] 8.9 / 7.6 / 7.5, of [251,37,509] 9.6 / 8.3 / 10.2, of [300,100,33] 6.3 / 4.0 / 4.3;
+  // non-temporal stores (`sc1 nt`). In us, plain / written through / and non-temporal, at one vector
+  // per thread: view chain of [256,64,256] 7.6 / 7.1 / 7.1, of [251,37,509] 8.8 / 7.9 / 8.6, of [300,100,33] 6.3 / 4.0 / 4.3;
   // a 2048 x 2048 producer followed by its consumer 21.9 / 20.7 / 23.0; a*b+c of 16 million 47.9 /
   // 48.1 / 47.7. Longer or odd runs leave each instruction every other piece of a line, which written
   // through becomes partial-line writes: those stay plain or plainly non-temporal, as do the bodies

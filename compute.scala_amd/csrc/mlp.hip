@@ -3,8 +3,8 @@
 //
 // The reference has no counterpart (it has no tuning). Layout: parameters are one flat
 // FP32 array [W1 (d0 x d1), b1 (d1), W2 (d1 x d2), b2, ...]; W is row-major [in][out]; ReLU
-// follows every layer but the last. Every reduction runs in a fixed order (one thread per
-// output sum), so results are deterministic.
+// follows every layer but the last. Every sum has a fixed order, so results are
+// deterministic.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

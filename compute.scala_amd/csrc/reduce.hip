@@ -336,7 +336,7 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_kernel(const float *__re
 // Short rows: kG lanes per row, kBlock / kG consecutive rows per workgroup at a time, so that a
 // wave reads whole rows one after another; `tiles` such groups of rows per workgroup. The FP64
 // values of its rows are added in a fixed order into one partial per workgroup. Bound by HBM once
-// the grid fills the chip: 120011 x 77 (37 MB) takes 12.5 us with its combine, 3.0 TB/s, against
+// the grid fills the chip: 120011 x 77 (37 MB) takes 12.0 us with its combine, 3.1 TB/s, against
 // 109 us when every row had a workgroup; 16000 x 1025 15.7 us (4.2 TB/s) against 25.2.
 template <int kG, bool kShort>
 __global__ __launch_bounds__(kBlock) void reduce_short_rows_kernel(const float *__restrict__ in, int64_t rows,
@@ -565,7 +565,7 @@ struct RowPlan {
 
 // Where the lines lie (whole calls with the total, in us: a workgroup per row against the rule):
 //   * up to 2048 columns a row is 8 vectors per lane of one wave, so a workgroup per row spends
-//     its time starting and combining: 120011 x 77 109.0 / 11.9, 524288 x 8 464 / 8.7,
+//     its time starting and combining: 120011 x 77 109.0 / 12.0, 524288 x 8 464 / 8.7,
 //     60000 x 128 57.8 / 8.9, 16384 x 1024 19.5 / 14.3, 16000 x 1025 21.6 / 15.7; equal at
 //     2047 columns (15.4 / 15.6); at 4096 the workgroup per row is ahead (43.3 / 45.8).
 //   * few rows (at most 8 per CU, all resident at once) of more than 256 columns keep a workgroup

@@ -120,7 +120,7 @@ __device__ __forceinline__ void sincos_turn(float theta, const NormalTables &tab
 // Pair i writes buffer[2i], buffer[2i+1] (Tensors.scala:409-425). Every FP32 operation is
 // correctly rounded: log, cos and sin are evaluated in FP64 and rounded once, as a correctly
 // rounded libm does on the host. Two pairs per thread and step, one 16-byte store. Bound by
-// arithmetic, a third of it FP64: 16777259 values (67 MB) take 27.7 us, against 59 us with the
+// arithmetic, a third of it FP64: 16777259 values (67 MB) take 25.0 us, against 58.4 us with the
 // device library's log, cos and sin, which serve the whole range of their arguments. (One copy of the
 // tables per LDS lane, against bank conflicts, took 32.5 us: filling them costs more than it saves.)
 __global__ __launch_bounds__(kBlock) void random_normal_kernel(float *out, int64_t pairs, uint32_t seed,
